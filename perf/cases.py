@@ -249,3 +249,69 @@ def tolerance(case):
     """About four times what the present code is off from the same sums in 64 bits (fp16 inputs, weights and outputs,
     32-bit sums); blocks pass fp16 intermediates on, one after the other."""
     return {"rel": {"layer": 2e-3, "train_layer": 1.5e-3, "train_block": 4.5e-3, "decode": 1e-2}[case["kind"]]}
+
+
+# ---------------------------------------------------------------------------------------------------- in 64 bits
+def _dense64(layer):
+    """The layer's weights, scale * (code - zero - 1), in 64 bits."""
+    shifts = 4 * torch.arange(8, device="cuda", dtype=torch.int32)
+    codes = ((layer.qweight.unsqueeze(1) >> shifts.view(1, 8, 1)) & 15).reshape(-1, layer.qweight.shape[1])
+    zeros = ((layer.qzeros.unsqueeze(2) >> shifts) & 15).reshape(layer.qzeros.shape[0], -1) + 1
+    g = layer.g_idx.long()
+    return layer.scales.double()[g] * (codes - zeros[g]).double()
+
+
+def _keep64(rows, cols, seed, p):
+    """The adapter's dropout factors: 0 where the 15-bit draw of (seed, row, column) lies below p, else 1 / (1 - p)."""
+    m32 = 0xFFFFFFFF
+
+    def mul(a, b):                                           # 32-bit product without leaving 64-bit integers
+        return ((a & 0xFFFF) * b + ((((a >> 16) * b) & 0xFFFF) << 16)) & m32
+    row = (mul(torch.arange(rows, device="cuda"), 0x9E3779B1) + (seed & m32)) & m32
+    pair = (mul(torch.arange(cols // 2, device="cuda"), 0x85EBCA6B) + ((seed >> 32) & m32)) & m32
+    h = row.view(-1, 1) ^ pair
+    h = mul(h ^ (h >> 16), 0x7FEB352D)
+    h = mul(h ^ (h >> 15), 0x846CA68B)
+    h = h ^ (h >> 16)
+    draws = torch.stack([h & 0x7FFF, (h >> 16) & 0x7FFF], dim=-1).view(rows, cols)
+    threshold = round(p * 32768)
+    return (draws >= threshold).double() / (1.0 - threshold / 32768.0)
+
+
+def exact(case, seed):
+    """What `run` returns, from the same inputs with every weight, product and sum in 64 bits."""
+    state = prepare({**case, "graph": False}, seed)
+    training = case["kind"].startswith("train")
+    x = state["x"].detach().double().requires_grad_(training)
+    params = [p.detach().double().requires_grad_(True) for p in state.get("params", [])]
+    left = list(params)
+    p = case.get("dropout", 0.0)
+    torch.default_generator.manual_seed(seed)
+
+    def linear(layer, t):
+        y = t @ _dense64(layer)
+        if hasattr(layer, "lora_A"):
+            a, b = (left.pop(0), left.pop(0)) if training else (m["default"].weight.detach().double() for m in (layer.lora_A, layer.lora_B))
+            if training and p > 0.0:
+                t = t * _keep64(t.shape[0], t.shape[1], int(torch.randint(0, 2 ** 62, (1,)).item()), p)
+            y = y + layer.scaling["default"] * ((t @ a.t()) @ b.t())
+        return y
+
+    def block(m, t):
+        n, attn, mlp = F.rms_norm(t, t.shape[-1:], eps=torch.finfo(torch.float32).eps), m.self_attn, m.mlp
+        q, k, v = linear(attn.q_proj, n), linear(attn.k_proj, n), linear(attn.v_proj, n)
+        t = t + linear(attn.o_proj, v * torch.sigmoid(q + k))
+        n = F.rms_norm(t, t.shape[-1:], eps=torch.finfo(torch.float32).eps)
+        return t + linear(mlp.down_proj, F.silu(linear(mlp.gate_proj, n)) * linear(mlp.up_proj, n))
+
+    with torch.set_grad_enabled(training):
+        y = x
+        if "layer" in case["kind"]:
+            y = linear(state["model"], y)
+        else:
+            for m in state["model"]:
+                y = block(m, y)
+    if not training:
+        return y
+    y.backward(state["dy"].double())
+    return [y.detach(), x.grad] + [t.grad for t in params]
