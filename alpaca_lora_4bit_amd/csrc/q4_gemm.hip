@@ -73,15 +73,14 @@ struct GemmArgs {
 //    a single L2 channel; workgroups marching through the reduction in lockstep then queue on that one
 //    channel.  Row tile r therefore starts its (cyclic) reduction loop phase_step * r steps later.
 struct TileMap {
-    int tile_c, tile_r, phase;
+    int tile_c, tile_r;
 };
-__device__ __forceinline__ TileMap map_tile(int phase_step, int nsteps, int col_tile0) {   // nsteps: steps of THIS workgroup
+__device__ __forceinline__ TileMap map_tile(int phase_step, int col_tile0) {
     const int nc = gridDim.x, nr = gridDim.y, total = nc * nr;
     int id = blockIdx.y * nc + blockIdx.x;
     if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
     TileMap m;
     const int rg = phase_step >> 8;                   // row tiles per group (0: column-major over all row tiles)
-    phase_step &= 0xff;
     const int grouped = rg > 0 ? (nr / rg) * rg * nc : 0;
     if (id < grouped) {
         // groups of rg row tiles: all column tiles of a group, then the next group
@@ -94,7 +93,6 @@ __device__ __forceinline__ TileMap map_tile(int phase_step, int nsteps, int col_
         m.tile_r = base + (rem - m.tile_c * left);
     }
     m.tile_c += col_tile0;
-    m.phase = (m.tile_r * phase_step) % nsteps;
     return m;
 }
 // Split-K: gridDim.z workgroups share an output tile; workgroup z owns `cnt` consecutive steps from `begin`.
@@ -359,11 +357,13 @@ struct BwdSlab {
 //   2  backward: from an LDS table of the tile's group, filled once (needs the 128 output rows of a tile in one
 //      group and room for 4 bytes per column n in dynamic LDS)
 // WGN: wavefronts along N (2 or 4), each 64 columns wide: the tile is BM x 64*WGN.
-// The body of the kernels below.  `tm`: the output tile; `sr`: this workgroup's share of the reduction; `zsplit` of
-// `nsplit`: which share that is (share 0 carries bias and adapter term); `zpart`: index of its fp32 partial tile.
-template <int BM, int WGM, bool FWD, bool GIDX, int SZ, int WGN>
-__device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, const StepRange sr, const int zsplit,
-                                          const int nsplit, const int zpart) {
+// The body of the kernels below.  `tm`: the output tile; `share`: this workgroup's steps of the reduction; `zsplit` of
+// `nsplit`: which share that is (share 0 carries the bias) and the index of its fp32 partial tile.
+// With MULTI the reduction is that of `nlay` layers one after the other (grad-input: dx = sum_i dy_i @ W_i^T), `share`
+// counts their concatenated steps, and the share that holds a layer's first step carries its adapter term.
+template <int BM, int WGM, bool FWD, bool GIDX, int SZ, int WGN, bool MULTI = false>
+__device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay, const TileMap tm, const StepRange share,
+                                          const int zsplit, const int nsplit) {
     constexpr int BNT = 64 * WGN;                     // columns of the tile
     static_assert(SZ == 0 || (!GIDX && ((FWD && SZ == 1) || (!FWD && SZ == 2))), "unsupported scale/zero mode");
     extern __shared__ __attribute__((aligned(16))) unsigned char sz_tab[];
@@ -383,12 +383,37 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
     const int wm = wave / WGN, wn = wave % WGN;
-    const int NOUT = FWD ? a.N : a.K;
-    const int RED = FWD ? a.K : a.N;
+    const GemmArgs& a0 = layers[0];          // what all layers share: M, the output, the partial tiles
+    const int NOUT = FWD ? a0.N : a0.K;
     const int m0 = tm.tile_r * BM;
     const int c0 = tm.tile_c * BNT;          // first output column of the tile
-    const int rows_valid = min(BM, a.M - m0);
+    const int rows_valid = min(BM, a0.M - m0);
 
+    // bias of this lane's two output columns, requested before everything else: its latency hides under the
+    // prologue instead of sitting in the epilogue
+    float bias_v[2] = {0.f, 0.f};
+    if (FWD && a0.bias) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bias_v[j] = (float)a0.bias[c0 + wn * 64 + 32 * j + (lane & 31)];
+    }
+
+    float16_t acc[TM][2];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    // the steps `sr` of one layer's reduction onto the accumulators
+    auto run_layer = [&](const GemmArgs& a, const StepRange sr, const bool lora_here) {
+    // MULTI: opaque per layer, or everything derived from it is kept in registers over the loop (and spills)
+    int t = threadIdx.x;
+    if constexpr (MULTI) asm volatile("" : "+v"(t));
+    const int lane = t & 63, wave = t >> 6;
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int RED = FWD ? a.K : a.N;
+    const int phase = (tm.tile_r * (a.phase_step & 0xff)) % sr.cnt;
     // buffer descriptors: activations of this workgroup's rows (rows beyond M read as zero), weights
     const rsrc_t rs_a = make_rsrc(a.a + (size_t)m0 * RED, (unsigned)rows_valid * (unsigned)RED * 2u);
     SlabRsrc rs;
@@ -419,22 +444,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
     slab[0].init(t, a, c0);
     slab[1].init(t, a, c0);
     typename Slab::Prep prep;
-
-    // bias of this lane's two output columns, requested before everything else: its latency hides under the
-    // prologue instead of sitting in the epilogue
-    float bias_v[2] = {0.f, 0.f};
-    if (FWD && a.bias) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) bias_v[j] = (float)a.bias[c0 + wn * 64 + 32 * j + (lane & 31)];
-    }
-
-    float16_t acc[TM][2];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
     const int lr = lane & 31, lk = (lane >> 5) * 8;
     const int a_off = (wm * WROWS + lr) * LDS_STRIDE + lk;
@@ -470,8 +479,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
         // fragment set 0 is reloaded right after the barrier: every MFMA of sub-step KS-2 (its last
         // user in this step) must have been issued by then
         static_assert(BAR >= (KS - 1) * TM * 2 - 1, "barrier placed before the last use of fragment set 0");
-        const int red_next2 = red_of(s + 2, sr, tm.phase);
-        const int red_next1 = red_of(s + 1, sr, tm.phase);
+        const int red_next2 = red_of(s + 2, sr, phase);
+        const int red_next1 = red_of(s + 1, sr, phase);
         const half_t* const a_cur = CUR ? sA1 : sA0;
         const half_t* const b_cur = CUR ? sB1 : sB0;
         half_t* const a_nxt = CUR ? sA0 : sA1;
@@ -517,7 +526,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
 
     // rank-R adapter step: activations [M, R] (columns beyond R are zero) and the adapter matrix go through the LDS
     // buffers pa / pb like one more reduction step
-    auto lora_step = [&](half_t* pa, half_t* pb) {
+    auto stage_lora = [&](half_t* pa, half_t* pb) {
         __syncthreads();
         const rsrc_t rs_l = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
 #pragma unroll
@@ -528,19 +537,37 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
         }
         slab[0].store_lora(a, c0, pb, t);
         __syncthreads();
-        for (int ks = 0; ks < (a.R + 15) / 16; ++ks) {
-            read_frags(af[0], bf[0], pa, pb, ks);
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0][i], bf[0][j], acc[i][j], 0, 0, 0);
-        }
     };
-    const bool lora_here = a.R > 0 && zsplit == 0;
     const bool lora_masked = lora_here && a.drop.thr15 != 0;              // uniform
 
-    const int red0 = red_of(0, sr, tm.phase), red1 = red_of(1, sr, tm.phase);
+    if (lora_masked) {
+        // Dropout on the adapter input: the adapter's share of out[m, c] exists only where the mask keeps (m, c).
+        // It is summed by itself, one 32 x 32 tile at a time, masked, and added to the accumulators (before
+        // anything of the main loop is live: with its loads in flight the registers would not do); the main loop adds
+        // the unmasked product on top.  The kept values carry 1/(1-p) through lb_scale.
+        stage_lora(sA1, sB1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                float16_t term;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) term[r] = 0.f;
+                for (int ks = 0; ks < (a.R + 15) / 16; ++ks)
+                    term = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8_t*>(sA1 + a_off + 32 * i * LDS_STRIDE + 16 * ks),
+                                                                  *reinterpret_cast<const half8_t*>(sB1 + b_off + 32 * j * LDS_STRIDE + 16 * ks),
+                                                                  term, 0, 0, 0);
+                const int col = c0 + wn * 64 + 32 * j + (lane & 31);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + (lane >> 5) * 4 + (r & 3);
+                    const uint32_t w = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)col >> 1);
+                    acc[i][j][r] += ((w >> (16 * (col & 1))) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[r];
+                }
+                __builtin_amdgcn_sched_barrier(0);                // one tile's masks and term at a time
+            }
+    }
+    const int red0 = red_of(0, sr, phase), red1 = red_of(1, sr, phase);
     // Same order as inside a step (weights, scale, zero, then the activations): the compiler's wait counts at the
     // head of the main loop are the merge of this path and the loop's own, and with the activations of stage 1
     // requested BEFORE its weights that merge makes every even step wait for ALL loads of the step before it.
@@ -569,26 +596,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
         slab[0].fetch_tab(sz_tab, red0);
         slab[1].fetch_tab(sz_tab, red1);
     }
-    if (lora_masked) {
-        // Dropout on the adapter input: the adapter's share of out[m, c] exists only where the mask keeps (m, c).
-        // So the adapter step runs FIRST, into the zeroed accumulators (through the second pair of LDS buffers,
-        // while the loads of the first two stages are in flight), the accumulators are masked, and the main
-        // loop adds the unmasked product on top.  The kept values carry 1/(1-p) through lb_scale.
-        lora_step(sA1, sB1);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + (lane >> 5) * 4 + (r & 3);
-                const uint32_t key = drop_row_key(a.drop, (uint32_t)m);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int col = c0 + wn * 64 + 32 * j + (lane & 31);
-                    const uint32_t w = drop_word(a.drop, key, (uint32_t)col >> 1);
-                    if (((w >> (16 * (col & 1))) & 0x7FFFu) < a.drop.thr15) acc[i][j][r] = 0.f;
-                }
-            }
-    }
     store_a(areg[0], sA0);
     prep = slab[0].make_prep(c0);
     static_for<0, NSL>([&](auto jc) { slab[0].template store_slice<decltype(jc)::value>(a, c0, red0, sB0, prep); });
@@ -599,7 +606,35 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
         step(s + 1, std::integral_constant<int, 1>{});
     }
     if (sr.cnt & 1) step(sr.cnt - 1, std::integral_constant<int, 0>{});   // an even number of steps precedes it: LDS[0]
-    if (lora_here && !lora_masked) lora_step(sA0, sB0);
+    if (lora_here && !lora_masked) {
+        stage_lora(sA0, sB0);
+        for (int ks = 0; ks < (a.R + 15) / 16; ++ks) {
+            read_frags(af[0], bf[0], sA0, sB0, ks);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0][i], bf[0][j], acc[i][j], 0, 0, 0);
+        }
+    }
+    };  // run_layer
+
+    if constexpr (MULTI) {
+        bool first = true;
+        int base = 0;                                             // concatenated step at which the layer begins
+#pragma unroll 1
+        for (int li = 0; li < nlay; ++li) {
+            const int steps = (FWD ? layers[li].K : layers[li].N) / BK;
+            const int lo = max(share.begin, base) - base, hi = min(share.begin + share.cnt, base + steps) - base;
+            base += steps;
+            if (lo >= hi) continue;                               // uniform
+            if (!first) __syncthreads();                          // every wavefront has read the last layer's tiles
+            first = false;
+            run_layer(layers[li], StepRange{lo, hi - lo}, layers[li].R > 0 && lo == 0);
+        }
+    } else {
+        run_layer(a0, share, a0.R > 0 && zsplit == 0);
+    }
 
     // epilogue: acc[i][j][r] is row 8*(r/4) + 4*(lane/32) + r%4, column lane%32 of its 32x32 tile.
     // Each wavefront transposes one 32 x 64 block at a time through its own 4.5 KB of LDS
@@ -608,7 +643,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
     if (nsplit > 1) {
         // split-K: fp32 partial sums straight from the accumulators (32 lanes cover one 128-byte row segment);
         // the bias rides with split 0, the reduction kernel adds the splits in order and rounds once
-        float* const pz = a.part + (size_t)zpart * a.M * a.part_cols - (size_t)a.col_tile0 * BNT;
+        float* const pz = a0.part + (size_t)zsplit * a0.M * a0.part_cols - (size_t)a0.col_tile0 * BNT;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -618,7 +653,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + lrow + (r & 3);
-                    if (m < a.M) pz[(size_t)m * a.part_cols + col] = acc[i][j][r] + bv;
+                    if (m < a0.M) pz[(size_t)m * a0.part_cols + col] = acc[i][j][r] + bv;
                 }
             }
         return;
@@ -645,7 +680,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
             const int rr = orow + 8 * p;
             const int m = m0 + wm * WROWS + 32 * i + rr;
             const uint4_t v = *reinterpret_cast<const uint4_t*>(stage + rr * LDS_STRIDE + ocol);
-            if (m < a.M) *reinterpret_cast<uint4_t*>(a.out + (size_t)m * NOUT + c0 + wn * 64 + ocol) = v;
+            if (m < a0.M) *reinterpret_cast<uint4_t*>(a0.out + (size_t)m * NOUT + c0 + wn * 64 + ocol) = v;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -657,40 +692,36 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a, const TileMap tm, c
 template <int BM, int WGM, bool FWD, bool GIDX, int SZ = 0, int WGN = 2>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs a) {
     const StepRange sr = split_steps((FWD ? a.K : a.N) / BK, blockIdx.z, gridDim.z);
-    gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(a, map_tile(a.phase_step, sr.cnt, a.col_tile0), sr, blockIdx.z, gridDim.z,
-                                           blockIdx.z);
+    gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(&a, 1, map_tile(a.phase_step, a.col_tile0), sr, blockIdx.z, gridDim.z);
 }
 
 // Up to kGemmGroup layers that share M, K, the group size and (forward) the activations -- q|k|v, gate|up -- in ONE
 // grid, each on its own tensors.
 //   forward:    blockIdx.x walks the column tiles of layer 0, then of layer 1, ...; every workgroup computes one tile of
 //               one layer's own output, over the whole reduction (no split).
-//   grad-input: dx = sum_i dy_i @ W_i^T.  The layers are the "splits" of one launch: blockIdx.z = layer * zs + share,
-//               every workgroup leaves an fp32 partial tile (adapter term and dropout mask of ITS layer included) and
-//               the ordered reduction adds them all into dx: one launch and one reduction instead of one of each per
-//               layer plus the additions of the per-layer results.
+//   grad-input: dx = sum_i dy_i @ W_i^T is ONE reduction over the layers' columns one after the other: a workgroup
+//               walks the layers (all of them, or its share of the concatenated steps where the tiles are few) with
+//               the sum in its accumulators, adapter term and dropout mask of each layer included.
 constexpr int kGemmGroup = 4;
 struct GemmGroupArgs {
     GemmArgs layer[kGemmGroup];
     int tile_end[kGemmGroup];          // forward: running total of column tiles (tile width of the launch)
-    int zs;                            // grad-input: reduction shares per layer
+    int n;
 };
 
 template <int BM, int WGM, bool FWD, bool GIDX, int SZ = 0, int WGN = 2>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_group_kernel(GemmGroupArgs g) {
+    TileMap tm = map_tile(g.layer[0].phase_step, g.layer[0].col_tile0);
     if constexpr (FWD) {
-        const GemmArgs& a0 = g.layer[0];
-        const StepRange sr = split_steps(a0.K / BK, 0, 1);
-        TileMap tm = map_tile(a0.phase_step, sr.cnt, 0);
         const int li = (tm.tile_c >= g.tile_end[0]) + (tm.tile_c >= g.tile_end[1]) + (tm.tile_c >= g.tile_end[2]);   // uniform
         tm.tile_c -= li == 0 ? 0 : g.tile_end[li - 1];
         const GemmArgs a = g.layer[li];
-        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(a, tm, sr, 0, 1, 0);
+        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(&a, 1, tm, split_steps(a.K / BK, 0, 1), 0, 1);
     } else {
-        const int li = blockIdx.z / g.zs, zz = blockIdx.z - li * g.zs;
-        const GemmArgs a = g.layer[li];
-        const StepRange sr = split_steps(a.N / BK, zz, g.zs);
-        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(a, map_tile(a.phase_step, sr.cnt, 0), sr, zz, gridDim.z, blockIdx.z);
+        int nsteps = 0;
+        for (int i = 0; i < g.n; ++i) nsteps += g.layer[i].N / BK;
+        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN, true>(g.layer, g.n, tm, split_steps(nsteps, blockIdx.z, gridDim.z),
+                                                     blockIdx.z, gridDim.z);
     }
 }
 
@@ -751,21 +782,40 @@ static void launch_tiles(const GemmArgs& a, dim3 grid, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_kernel<BM, WGM, FWD, GIDX, 0>), grid, block, 0, stream, a);
 }
 
+// fp32 partial tiles of the columns [col0, col0 + part_cols) of out, added in order
+static void launch_reduce_cols(const GemmArgs& a, int part_cols, int out_cols, int col0, int splits, hipStream_t stream) {
+    const long total = (long)a.M * part_cols;
+    hipLaunchKernelGGL(gemm_splitk_reduce_cols_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream,
+                       a.part, a.out, a.M, part_cols, out_cols, col0, splits);
+}
+
+// The last tail_cols column tiles of 128 as a launch of 256 x 128 tiles whose reduction is split tail_splits ways.
+template <bool FWD, bool GIDX>
+static void launch_tail(GemmArgs a, int nout, int tail_cols, int tail_splits, hipStream_t stream) {
+    a.col_tile0 = nout / BN - tail_cols;
+    a.part_cols = tail_cols * BN;
+    launch_tiles<256, 4, FWD, GIDX>(a, dim3(tail_cols, (a.M + 255) / 256, tail_splits), stream);
+    if (tail_splits > 1) launch_reduce_cols(a, a.part_cols, nout, a.col_tile0 * BN, tail_splits, stream);
+}
+
 // 256 x 256 tiles (8 wavefronts of 128 x 64): half the activation traffic and 30 % less LDS traffic per MFMA than the
 // 256 x 128 tile; for outputs with enough such tiles to fill the CUs.  No split, no second launch; the tile buffers
 // take 144 KB of LDS, so the grad-input kernel keeps its per-step scale / zero loads.
+// tail_cols > 0: the last tail_cols tiles of 128 columns are left to a second launch of 256 x 128 tiles, with the
+// reduction split tail_splits ways (see wide_tail).
 template <bool FWD, bool GIDX>
-static hipError_t launch_gemm_wide(GemmArgs a, int nout, hipStream_t stream) {
-    const dim3 grid(nout / 256, (a.M + 255) / 256, 1), block(512);
+static hipError_t launch_gemm_wide(GemmArgs a, int nout, int tail_cols, int tail_splits, hipStream_t stream) {
+    const int nr = (a.M + 255) / 256;
+    const dim3 grid((nout - tail_cols * BN) / 256, nr, 1), block(512);
     a.col_tile0 = 0;
     a.part_cols = nout;
+    bool sz1 = false;
     if constexpr (FWD && !GIDX) {
-        if (a.groupsize % 128 == 0 && (a.K / BK) % 2 == 0 && ((a.phase_step & 0xff) % 2) == 0) {
-            hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 1, 4>), grid, block, 0, stream, a);
-            return hipGetLastError();
-        }
+        sz1 = a.groupsize % 128 == 0 && (a.K / BK) % 2 == 0 && ((a.phase_step & 0xff) % 2) == 0;
+        if (sz1) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 1, 4>), grid, block, 0, stream, a);
     }
-    hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 0, 4>), grid, block, 0, stream, a);
+    if (!sz1) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 0, 4>), grid, block, 0, stream, a);
+    if (tail_cols > 0) launch_tail<FWD, GIDX>(a, nout, tail_cols, tail_splits, stream);
     return hipGetLastError();
 }
 
@@ -782,20 +832,13 @@ static hipError_t launch_gemm(GemmArgs a, int nout, int splits, int tail_cols, i
         hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream,
                            a.part, a.out, total, splits);
     }
-    if (tail_cols > 0) {
-        a.col_tile0 = nc - tail_cols;
-        a.part_cols = tail_cols * BN;
-        launch_tiles<BM, WGM, FWD, GIDX>(a, dim3(tail_cols, nr, tail_splits), stream);
-        const long total = (long)a.M * a.part_cols;
-        hipLaunchKernelGGL(gemm_splitk_reduce_cols_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream,
-                           a.part, a.out, a.M, a.part_cols, nout, a.col_tile0 * BN, tail_splits);
-    }
+    if (tail_cols > 0) launch_tail<FWD, GIDX>(a, nout, tail_cols, tail_splits, stream);
     return hipGetLastError();
 }
 
 struct GemmPlan {
     int cfg, splits;
-    int tail_cols, tail_splits;      // cfg 2 only: column tiles of the split second launch (0: none)
+    int tail_cols, tail_splits;      // cfg 2, 3: 128-column tiles of the second launch (0: none), its reduction split
 };
 
 template <bool FWD, bool GIDX>
@@ -803,7 +846,7 @@ static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout
     switch (p.cfg) {
         case 0: return launch_gemm<128, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 128 x 128, 4 wavefronts of 64 x 64
         case 1: return launch_gemm<256, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 256 x 128, 4 wavefronts of 128 x 64
-        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, stream);                        // 256 x 256, 8 wavefronts of 128 x 64
+        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, p.tail_cols, p.tail_splits, stream);                        // 256 x 256, 8 wavefronts of 128 x 64
         default: return launch_gemm<256, 4, FWD, GIDX>(a, nout, p.splits, p.tail_cols, p.tail_splits, stream);   // 256 x 128, 8 wavefronts of 64 x 64
     }
 }
@@ -811,6 +854,31 @@ static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout
 // What TileMap is told: row tile r starts its reduction loop kPhaseStep * r steps later; tiles are ordered in groups
 // of kRowTilesPerGroup row tiles (measured optimum over the benchmark shapes).
 constexpr int kPhaseStep = 2, kRowTilesPerGroup = 2;
+
+// More 256 x 256 tiles than whole rounds of the CUs: the wide tiles of the whole rounds run as they are, and the columns
+// left over go to a second launch of 256 x 128 tiles that is one round at most, its reduction split when even that
+// leaves CUs idle.  A full round of wide tiles takes 1.75-1.85 us per reduction step, one of narrow tiles 0.9-1.05, so the
+// remainder costs at most 0.6 of the round of wide tiles, or half of the two narrow ones, that it would cost otherwise:
+// 2048 x (4096 -> 11008), 344 tiles: three rounds of narrow tiles 186 us, 118 + 57 us; grad-input of 4096 x
+// (5120 -> 13824), 864 tiles: four rounds of wide tiles 561 us, 447 + 79 us.
+// Taken for remainders of 1/8 to 1/2 of a round: below that the narrow tiles with their own remainder launch lose
+// little, above it the remainder does not fit a round of narrow tiles.
+struct WideTail { int tail_cols, tail_splits; };     // 128-column tiles; 0: does not apply
+static WideTail wide_tail(int M, int nsteps, int nout, bool may_split, size_t workspace_bytes) {
+    WideTail w{0, 1};
+    const int nr = (M + 255) / 256, nc = nout / 256;
+    const long t = (long)nc * nr;
+    if (nout % 256 != 0 || t <= 256) return w;
+    const int main_cols = (int)((t / 256) * 256 / nr);
+    const long left = (long)(nc - main_cols) * nr;
+    if (main_cols < 1 || left < 32 || left > 128) return w;
+    int s = (int)(256 / (2 * left));
+    while (s > 1 && (!may_split || nsteps < 8 * s ||
+                     (size_t)s * (size_t)M * (size_t)(nc - main_cols) * 256 * sizeof(float) > workspace_bytes)) --s;
+    w.tail_cols = 2 * (nc - main_cols);
+    w.tail_splits = s;
+    return w;
+}
 
 // Launch plan shared by q4_launch_gemm and q4_gemm_plan_workspace.  Few output tiles (small M) leave most CUs
 // idle while each tile walks the whole reduction: the reduction is then split over gridDim.z workgroups that
@@ -831,6 +899,13 @@ static GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes) {
     // fill theirs better: 3072 x (4096 -> 11008) has 516 wide tiles = 3 rounds for 2.02 rounds of work and stays
     // with the narrow ones (270 against 294 us), 4096 rows have 688 (313 against 356 us).
     const long twide = (nout % 256 == 0) ? (long)(nout / 256) * ((M + 255) / 256) : 0;
+    const WideTail wt = wide_tail(M, nsteps, nout, true, workspace_bytes);
+    if (wt.tail_cols > 0) {
+        p.cfg = 3; p.splits = 1;
+        p.tail_cols = wt.tail_cols;
+        p.tail_splits = wt.tail_splits;
+        return p;
+    }
     if (twide >= 144 &&
         (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) {
         p.cfg = 3; p.splits = 1;
@@ -946,12 +1021,17 @@ extern "C" int q4_launch_gemm(int fwd, const void* act, const int32_t* qweight, 
 
 // ---- several layers in one launch (sequential groups only) ---------------------------------------------------------
 namespace q4 {
-struct GroupPlan { int cfg; int zs; };      // cfg as in launch_gemm_cfg (0: 128 x 128, 2: 256 x 128, 3: 256 x 256); -1: not applicable
+// cfg as in launch_gemm_cfg (2: 256 x 128 tiles, 3: 256 x 256 tiles; -1: not applicable), the split of the reduction,
+// and for cfg 3 the second launch (see wide_tail).
+struct GroupPlan { int cfg, splits, tail_cols, tail_splits; };
 
 // Forward: one tile of one layer per workgroup, no split, so the launch needs enough tiles by itself.
-// Grad-input: every layer is a share of the reduction (times zs shares per layer when the tiles are few).
+// Grad-input: one reduction over all layers' columns; of the tilings and splits the one with the shortest estimate
+// (us: rounds of the CUs x steps x time per step, prologue and epilogue of a workgroup, and the traffic of the partial
+// sums where the reduction is split).  Against one partial tile per layer and their sum: 4096 rows, two layers 5120 ->
+// 13824: 1151 us + 46 us for the sums became 752 + 233 + 8 us; three layers 5120 -> 5120: 694 + 34 became 504 + 140 + 8 us.
 static GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
-    GroupPlan p{-1, 1};
+    GroupPlan p{-1, 1, 0, 1};
     if (n < 2 || n > kGemmGroup || M <= 128) return p;
     const int nr = (M + 255) / 256;
     if (fwd) {
@@ -959,19 +1039,39 @@ static GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
         bool all256 = true;
         for (int i = 0; i < n; ++i) { tot += N[i]; all256 = all256 && N[i] % 256 == 0; }
         const long twide = all256 ? (tot / 256) * nr : 0, t256 = (tot / BN) * nr;
-        if (twide >= 144 && (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) p.cfg = 3;
+        const WideTail wt = all256 && tot < (1l << 30) ? wide_tail(M, K / BK, (int)tot, false, 0) : WideTail{0, 1};
+        if (wt.tail_cols > 0) { p.cfg = 3; p.tail_cols = wt.tail_cols; }
+        else if (twide >= 144 && (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) p.cfg = 3;
         else if (t256 >= 192) p.cfg = 2;
         return p;
     }
-    const long twide = K % 256 == 0 ? (long)(K / 256) * nr * n : 0, t256 = (long)(K / BN) * nr * n;
-    if (twide >= 144 && twide <= 256) { p.cfg = 3; return p; }
-    p.cfg = 2;
-    if (t256 < 192) {
-        int mn = N[0];
-        for (int i = 1; i < n; ++i) mn = N[i] < mn ? N[i] : mn;
-        if (mn / BK >= 16) p.zs = 2;                     // at least eight steps per workgroup
+    constexpr double kWide = 1.7, kNarrow = 1.0, kEnds = 4.0, kReduce = 4.0, kBytesPerUs = 4.5e6;
+    long nsteps = 0;
+    for (int i = 0; i < n; ++i) nsteps += N[i] / BK;
+    double best = 0.0;
+    auto offer = [&](double us, GroupPlan q) { if (p.cfg < 0 || us < best) { best = us; p = q; } };
+    for (int cfg = 3; cfg >= 2; --cfg) {
+        const int tw = cfg == 3 ? 256 : BN;
+        if (K % tw != 0) continue;
+        const long t = (long)(K / tw) * nr;
+        for (int s = 1; s <= 8 && (s == 1 || (t * s <= 256 && nsteps >= 8 * s)); ++s)
+            offer((double)((t * s + 255) / 256) * ((nsteps + s - 1) / s * (cfg == 3 ? kWide : kNarrow) + kEnds) +
+                  (s > 1 ? kReduce + 8.0 * s * M * K / kBytesPerUs : 0.0), GroupPlan{cfg, s, 0, 1});
+    }
+    const WideTail wt = wide_tail(M, nsteps < 1 << 24 ? (int)nsteps : 1 << 24, K, true, ~(size_t)0);
+    if (wt.tail_cols > 0) {
+        const int ts = wt.tail_splits;
+        const long t = (long)(K / 256 - wt.tail_cols / 2) * nr;
+        offer((double)((t + 255) / 256) * (nsteps * kWide + kEnds) + (nsteps + ts - 1) / ts * kNarrow + kEnds + kReduce +
+              (ts > 1 ? kReduce + 8.0 * ts * M * wt.tail_cols * BN / kBytesPerUs : 0.0), GroupPlan{3, 1, wt.tail_cols, ts});
     }
     return p;
+}
+static size_t group_workspace(const GroupPlan& p, int M, int K) {
+    const size_t main = p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)K * sizeof(float) : 0;
+    const size_t tail = p.tail_cols > 0 && p.tail_splits > 1
+        ? (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float) : 0;
+    return main > tail ? main : tail;
 }
 
 template <int BM, int WGM, bool FWD, int WGN>
@@ -1007,7 +1107,7 @@ extern "C" int q4_gemm_group_applicable(int fwd, int n, int M, int K, const int*
 extern "C" size_t q4_gemm_group_plan_workspace(int fwd, int n, int M, int K, const int* N) {
     const q4::GroupPlan p = q4::plan_gemm_group(fwd, n, M, K, N);
     if (fwd || p.cfg < 0) return 0;
-    return (size_t)n * p.zs * (size_t)M * (size_t)K * sizeof(float);
+    return q4::group_workspace(p, M, K);
 }
 
 // act: forward the shared x (act[i] may all be the same pointer), grad-input dy_i.  out: forward y_i, grad-input out[0] = dx.
@@ -1020,11 +1120,10 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
     using namespace q4;
     const GroupPlan p = plan_gemm_group(fwd, n, M, K, N);
     if (p.cfg < 0) return -2;
-    const size_t need = fwd ? 0 : (size_t)n * p.zs * (size_t)M * (size_t)K * sizeof(float);
+    const size_t need = fwd ? 0 : group_workspace(p, M, K);
     if (need > 0 && (!workspace || workspace_bytes < need)) return -3;
     GemmGroupArgs g;
-    const int tile_w = p.cfg == 3 ? 256 : BN;
-    int tiles = 0;
+    int tiles[2] = {0, 0}, ends[2][kGemmGroup];         // running totals of column tiles, 256 and 128 columns wide
     for (int i = 0; i < kGemmGroup; ++i) {
         const int j = i < n ? i : n - 1;                // unused slots repeat the last layer (never selected)
         GemmArgs& a = g.layer[i];
@@ -1048,23 +1147,32 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
         a.part = reinterpret_cast<float*>(workspace);
         a.col_tile0 = 0;
         a.part_cols = fwd ? N[j] : K;
-        if (i < n) tiles += N[i] / tile_w;
-        g.tile_end[i] = i < n ? tiles : 0x7fffffff;
+        for (int w = 0; w < 2; ++w) {
+            if (i < n) tiles[w] += N[i] / (w == 0 ? 256 : BN);
+            ends[w][i] = i < n ? tiles[w] : 0x7fffffff;
+        }
     }
-    g.zs = p.zs;
-    const int bm = p.cfg == 0 ? 128 : 256;
-    const int nr = (M + bm - 1) / bm;
-    const dim3 grid(fwd ? tiles : K / tile_w, nr, fwd ? 1 : n * p.zs);
-    if (fwd) {
-        if (p.cfg == 3) launch_group_tiles<256, 2, true, 4>(g, n, grid, stream);
-        else launch_group_tiles<256, 4, true, 2>(g, n, grid, stream);
-    } else {
-        if (p.cfg == 3) launch_group_tiles<256, 2, false, 4>(g, n, grid, stream);
+    g.n = n;
+    const int nr = (M + 255) / 256;
+    // `count` column tiles from `first` on, in tiles of 256 x 256 (wide) or 256 x 128
+    auto launch = [&](bool wide, int first, int count, int splits, int part_cols) {
+        for (int i = 0; i < kGemmGroup; ++i) {
+            g.layer[i].col_tile0 = first;
+            if (!fwd) g.layer[i].part_cols = part_cols;
+            g.tile_end[i] = ends[wide ? 0 : 1][i];
+        }
+        const dim3 grid(count, nr, splits);
+        if (fwd && wide) launch_group_tiles<256, 2, true, 4>(g, n, grid, stream);
+        else if (fwd) launch_group_tiles<256, 4, true, 2>(g, n, grid, stream);
+        else if (wide) launch_group_tiles<256, 2, false, 4>(g, n, grid, stream);
         else launch_group_tiles<256, 4, false, 2>(g, n, grid, stream);
-        const long total = (long)M * K;
-        hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream,
-                           g.layer[0].part, g.layer[0].out, total, n * p.zs);
-    }
+        if (splits > 1) launch_reduce_cols(g.layer[0], part_cols, K, first * (wide ? 256 : BN), splits, stream);
+    };
+    const bool wide = p.cfg == 3;
+    const int narrow_total = fwd ? tiles[1] : K / BN;
+    const int main_tiles = wide ? (narrow_total - p.tail_cols) / 2 : narrow_total;
+    launch(wide, 0, main_tiles, p.splits, K);
+    if (p.tail_cols > 0) launch(false, narrow_total - p.tail_cols, p.tail_cols, p.tail_splits, p.tail_cols * BN);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -1074,7 +1182,7 @@ extern "C" size_t q4_gemm_plan_workspace(int fwd, int M, int K, int N) {
     const int nout = fwd ? N : K;
     const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, ~(size_t)0);
     size_t need = p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)nout * sizeof(float) : 0;
-    if (p.tail_cols > 0) need = (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float);
+    if (p.tail_cols > 0 && p.tail_splits > 1) need = (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float);
     if (fwd && M > 16 && M <= 64) {               // the skinny kernel's partial rows (it may or may not apply)
         const size_t sk = q4_skinny_workspace(M, K, N);
         if (sk > need) need = sk;

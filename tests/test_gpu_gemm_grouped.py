@@ -176,3 +176,91 @@ def test_grouped_block_matches_the_ungrouped_block_forward_and_gradients(oracle,
                 assert float((a.float() - b.float()).abs().max() / b.float().abs().max()) <= 2e-3
     assert calls["fwd"] == 2
     assert ungroup(grouped) == 1 and "_q4_group" not in grouped.k_proj.__dict__
+
+
+def _dense(quant_hip, t, gs):
+    return quant_hip.dequant(t["qweight"], t["qzeros"], t["scales"], t["g_idx"], gs).float()
+
+
+@pytest.mark.parametrize("M,K,Ns,gs,r,p", [
+    (200, 4096, (256, 384), 128, 8, 0.05),          # one row tile: shares that begin and end inside a layer, 10 steps in all
+    (1000, 4096, (1024, 640, 512), 64, 16, 0.05),   # ragged rows, shares across three layers, no scale / zero table
+    (4500, 4096, (512, 256), 128, 8, 0.1),          # 288 wide tiles: whole rounds and a remainder launch
+    (300, 384, (1024, 1024), 128, 0, 0.0),          # K not a multiple of 256: narrow tiles only
+])
+def test_grouped_grad_input_is_one_reduction_over_the_layers(oracle, M, K, Ns, gs, r, p):
+    """dx over the concatenated reduction (adapter terms and their dropout masks included) against fp32 products with
+    the bit-exact dense weights.  Bound: inputs and weights are the same fp16 values on both sides, so what differs is the
+    fp16 rounding of the result (2^-11), of the scaled adapter matrix (2^-11 of the smaller adapter term) and the order
+    of the 32-bit sums: 2e-3 of the largest value."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    ts = [to_cuda_layer(oracle.make_layer(K, N, gs, seed=K + N + i)) for i, N in enumerate(Ns)]
+    g = torch.Generator(device="cuda").manual_seed(M)
+    dys, layers, ref = [], [], 0.0
+    for i, (t, N) in enumerate(zip(ts, Ns)):
+        dy = torch.randn((M, N), device="cuda", generator=g).half()
+        dyb = A = drop = None
+        ref = ref + dy.float() @ _dense(quant_hip, t, gs).t()
+        if r and i != 1:
+            A = torch.randn((r, K), device="cuda", generator=g) * 0.05
+            dyb = torch.randn((M, r), device="cuda", generator=g).half()
+            drop = (77 + i, p)
+            keep = quant_hip.dropout_keep_mask(M, K, 77 + i, p, dy.device).float()
+            ref = ref + keep * quant_hip.dropout_scale(p) * 2.0 * (dyb.float() @ A)
+        dys.append(dy)
+        layers.append((t["qweight"], t["qzeros"], t["scales"], dyb, A, 2.0 if A is not None else 1.0, drop))
+    dx = quant_hip.gemm_grouped_bwd_dx(dys, layers, gs)
+    assert float((dx.float() - ref).abs().max() / ref.abs().max()) <= 2e-3
+    assert torch.equal(dx, quant_hip.gemm_grouped_bwd_dx(dys, layers, gs))
+
+
+def test_grouped_forward_remainder_launch(oracle):
+    """344 wide tiles: 256 of them as they are, the columns left over (inside the second layer) as 256 x 128 tiles."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    M, K, Ns = 1000, 512, (11008, 11008)
+    ts = [to_cuda_layer(oracle.make_layer(K, N, 128, seed=N + i)) for i, N in enumerate(Ns)]
+    x = torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).half()
+    bias = [None, torch.randn(Ns[1], device="cuda").half()]
+    ys = quant_hip.gemm_grouped_fwd(x, [(t["qweight"], t["qzeros"], t["scales"], b, None, None, 1.0) for t, b in zip(ts, bias)], 128)
+    for t, b, y in zip(ts, bias, ys):
+        ref = x.float() @ _dense(quant_hip, t, 128) + (0.0 if b is None else b.float())
+        assert float((y.float() - ref).abs().max() / ref.abs().max()) <= 2e-3
+
+
+@pytest.mark.parametrize("M,red,nout,gs,act,tail_cols,splits", [
+    (2000, 512, 11008, 128, False, 22, 1),      # 8 x 43 wide tiles: 11 columns left, one round of narrow tiles
+    (2000, 512, 11008, 64, False, 22, 1),
+    (4500, 1536, 4096, 128, True, 4, 3),        # 18 x 16: 2 columns left (36 tiles), reduction split
+    (4096, 2048, 5120, 256, False, 8, 2),       # 16 x 20: 4 columns left (64 tiles)
+])
+def test_wide_tiles_with_a_remainder_launch(oracle, M, red, nout, gs, act, tail_cols, splits):
+    """Forward (bias, adapter) and grad-input (adapter with dropout) where the last columns are a launch of narrow tiles."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    r = 8
+    for fwd in (True, False):
+        K, N = (red, nout) if fwd else (nout, red)
+        want = splits * M * tail_cols * 128 * 4 if splits > 1 else 0
+        assert _lib.lib().q4_gemm_workspace_bytes(int(fwd), M, K, N) == want
+        t = to_cuda_layer(oracle.make_layer(K, N, gs, act_order=act, seed=M))
+        W = _dense(quant_hip, t, gs)
+        g = torch.Generator(device="cuda").manual_seed(M)
+        A, B = (torch.randn(s, device="cuda", generator=g) * 0.05 for s in ((r, K), (N, r)))
+        a = torch.randn((M, red), device="cuda", generator=g).half()
+        small = torch.randn((M, r), device="cuda", generator=g).half()
+        if fwd:
+            bias = torch.randn(N, device="cuda", generator=g).half()
+            got = quant_hip.gemm_fwd(a, t["qweight"], t["qzeros"], t["scales"], t["g_idx"] if act else None, gs, bias=bias,
+                                     xa=small, lora_bt=B.t(), lora_scale=2.0)
+            ref = a.float() @ W + bias.float() + 2.0 * (small.float() @ B.t())
+        else:
+            drop = None if act else (5, 0.1)
+            got = quant_hip.gemm_bwd_dx(a, t["qweight"], t["qzeros"], t["scales"], t["g_idx"] if act else None, gs, dyb=small,
+                                        lora_a=A, lora_scale=2.0, dropout=drop)
+            term = 2.0 * (small.float() @ A)
+            if drop:
+                term = term * quant_hip.dropout_keep_mask(M, K, 5, 0.1, a.device).float() * quant_hip.dropout_scale(0.1)
+            ref = a.float() @ W.t() + term
+        assert float((got.float() - ref).abs().max() / ref.abs().max()) <= 2e-3
