@@ -1025,7 +1025,8 @@ namespace q4 {
 // and for cfg 3 the second launch (see wide_tail).
 struct GroupPlan { int cfg, splits, tail_cols, tail_splits; };
 
-// Forward: one tile of one layer per workgroup, no split, so the launch needs enough tiles by itself.
+// Forward: one tile of one layer per workgroup, no split, so the launch needs enough tiles by itself: from 96 tiles of
+// 256 x 128 on (q|k|v of 4096 features at 129..256 rows), below which the split launches per layer are shorter.
 // Grad-input: one reduction over all layers' columns; of the tilings and splits the one with the shortest estimate
 // (us: rounds of the CUs x steps x time per step, prologue and epilogue of a workgroup, and the traffic of the partial
 // sums where the reduction is split).  Against one partial tile per layer and their sum: 4096 rows, two layers 5120 ->
@@ -1042,7 +1043,7 @@ static GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
         const WideTail wt = all256 && tot < (1l << 30) ? wide_tail(M, K / BK, (int)tot, false, 0) : WideTail{0, 1};
         if (wt.tail_cols > 0) { p.cfg = 3; p.tail_cols = wt.tail_cols; }
         else if (twide >= 144 && (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) p.cfg = 3;
-        else if (t256 >= 192) p.cfg = 2;
+        else if (t256 >= 96) p.cfg = 2;
         return p;
     }
     constexpr double kWide = 1.7, kNarrow = 1.0, kEnds = 4.0, kReduce = 4.0, kBytesPerUs = 4.5e6;

@@ -164,6 +164,8 @@ class _MemberGroup:
         if not quant_hip.gemm_grouped_applicable(True, rows, member.in_features, Ns) or \
                 (grad and not quant_hip.gemm_grouped_applicable(False, rows, member.in_features, Ns)):
             return None
+        if not grad and sum(Ns) // 128 * ((rows + 255) // 256) < 192:
+            return None                                      # forward alone: the streaming kernels per layer (200 rows, q|k|v: 51 us)
         if self._gemm_ok is None:
             self._gemm_ok = all(quant_hip._group_layer_ok(l, self.groupsize) for l in layers)
         if not self._gemm_ok:
