@@ -490,6 +490,22 @@ at::Tensor lora_down(const at::Tensor& inp, const at::Tensor& w, const c10::opti
     return o;
 }
 
+// y += alpha * (x @ a^T) @ b^T in place (x @ a^T in fp16), two launches
+void lora_update(const at::Tensor& x, const at::Tensor& a, const at::Tensor& b, const at::Tensor& y, double alpha) {
+    TORCH_CHECK_VALUE(y.is_cuda() && y.scalar_type() == at::kHalf && y.dim() == 2 && y.is_contiguous() && y.device() == x.device() &&
+                      x.dim() == 2 && y.size(0) == x.size(0), "y must be a contiguous float16 [M, N] tensor beside x [M, K]");
+    TORCH_CHECK_VALUE(b.dim() == 2 && b.size(0) == y.size(1) && b.size(1) == a.size(0) && b.device() == y.device(),
+                      "b must be an [N, R] view on the same device");
+    TORCH_CHECK_VALUE(b.scalar_type() == at::kHalf || b.scalar_type() == at::kFloat, "b must be float16 or float32");
+    TORCH_CHECK_VALUE(b.stride(0) >= 1 && b.stride(1) >= 1, "b must have positive strides");
+    const at::Tensor xa = lora_down(x, a, c10::nullopt);
+    if (y.size(0) == 0) return;
+    Launch L(y.device());
+    const int rc = q4_lora_up_f16(xa.data_ptr(), b.data_ptr(), (int)b.stride(0), (int)b.stride(1), b.scalar_type() == at::kFloat,
+                                  y.data_ptr(), (float)alpha, (int)y.size(0), (int)y.size(1), (int)a.size(0), L.stream);
+    if (rc != Q4_OK) raise_q4(rc, "q4_lora_up_f16");
+}
+
 std::pair<at::Tensor, at::Tensor> lora_grad_pair(const at::Tensor& p1, const at::Tensor& in1, const at::Tensor& p2,
                                                  const at::Tensor& in2, double alpha,
                                                  const c10::optional<std::pair<int64_t, double>>& dropout) {
@@ -571,6 +587,7 @@ PYBIND11_MODULE(_q4_host, m) {
     m.def("gemm_grouped_bwd_dx", &gemm_grouped_bwd_dx, py::arg("dys"), py::arg("layers"), py::arg("groupsize"),
           py::arg("out_shape") = py::none());
     m.def("lora_down", &lora_down, py::arg("inp"), py::arg("w"), py::arg("dropout") = py::none());
+    m.def("lora_update", &lora_update, py::arg("x"), py::arg("a"), py::arg("b"), py::arg("y"), py::arg("alpha"));
     m.def("lora_grad_pair", &lora_grad_pair, py::arg("p1"), py::arg("inp1"), py::arg("p2"), py::arg("inp2"), py::arg("alpha"),
           py::arg("dropout") = py::none());
     m.def("mlp_decode", &mlp_decode, py::arg("x"), py::arg("gate"), py::arg("up"), py::arg("down"), py::arg("groupsize"),

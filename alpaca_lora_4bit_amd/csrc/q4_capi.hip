@@ -24,6 +24,7 @@ int q4_launch_lora_grad(const void*, const void*, float*, int, int, float, int, 
                         hipStream_t);
 int q4_launch_lora_grad_pair(const void*, const void*, float*, int, int, int, const void*, const void*, float*, int, int, int,
                              float, int, int, const q4_drop_args*, void*, hipStream_t);
+int q4_launch_lora_up(const void*, const void*, int, int, int, void*, float, int, int, int, hipStream_t);
 size_t q4_lora_grad_workspace(int, int, int);
 int q4_launch_gemv_group(int, const void* const*, const int32_t* const*, const int32_t* const*, const void* const*,
                          void* const*, const int*, int, int, int, int, int, void*, hipStream_t);
@@ -77,7 +78,7 @@ int check_layer(const void* qweight, const void* qzeros, const void* scales, con
 }
 }  // namespace
 
-extern "C" int q4_abi_version(void) { return 14; }
+extern "C" int q4_abi_version(void) { return 15; }
 
 extern "C" const char* q4_error_string(int code) {
     switch (code) {
@@ -426,6 +427,15 @@ extern "C" int q4_lora_down_f16(const void* in, const void* w, int w_sr, int w_s
     if (misaligned(in) || (reinterpret_cast<uintptr_t>(out) & 1u) || (reinterpret_cast<uintptr_t>(w) & (w_is_f32 ? 3u : 1u)))
         return Q4_ERR_MISALIGNED;
     return q4_launch_lora_down(in, w, w_sr, w_sc, w_is_f32, out, M, C, R, dp, (hipStream_t)stream);
+}
+
+extern "C" int q4_lora_up_f16(const void* xa, const void* w, int w_sn, int w_sr, int w_is_f32, void* y, float alpha,
+                              int M, int N, int R, void* stream) {
+    if (!xa || !w || !y) return Q4_ERR_NULL_POINTER;
+    if (M < 1 || M > 262140 || N < 1 || R < 1 || R > 64 || w_sn < 1 || w_sr < 1) return Q4_ERR_BAD_SHAPE;
+    if (((reinterpret_cast<uintptr_t>(xa) | reinterpret_cast<uintptr_t>(y)) & 1u) ||
+        (reinterpret_cast<uintptr_t>(w) & (w_is_f32 ? 3u : 1u))) return Q4_ERR_MISALIGNED;
+    return q4_launch_lora_up(xa, w, w_sn, w_sr, w_is_f32, y, alpha, M, N, R, (hipStream_t)stream);
 }
 
 extern "C" size_t q4_lora_grad_workspace_bytes(int M, int C, int R) {

@@ -227,6 +227,58 @@ __global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(const half_t
     }
 }
 
+// ---- rank-R update of a few rows -----------------------------------------------------------
+// y[m, n] += alpha * sum_r xa[m, r] * B[n, r] in place, one rounding: the second half of the adapter at decode sizes.
+// Launch-bound (a few hundred KB at most): one thread per column, kUpRows rows per workgroup, B read in place with its
+// strides and in its own type, xa from LDS.  At 4 x 4096, R = 8 it stands for a library product of 6.9 us (whose 256-row
+// tile is mostly padding) and for the fp16 copy of B that it needed: 8 blocks of the 7B step at 4 rows with adapters on q
+// and v, called one by one, 1289 -> 937 us.
+constexpr int kUpRows = 4, kUpCols = 64;
+
+template <bool F32, bool VEC>           // VEC: B rows contiguous, R % 4 == 0, 16 (fp32) / 8 (fp16) byte aligned
+__global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restrict__ xa, const void* __restrict__ w, int w_sn, int w_sr,
+                                                          half_t* __restrict__ y, float alpha, int M, int N, int R) {
+    __shared__ float sx[kUpRows][64];
+    const int m0 = blockIdx.y * kUpRows, rows = min(kUpRows, M - m0);
+    for (int i = threadIdx.x; i < kUpRows * R; i += kUpCols) {
+        const int m = i / R, r = i - m * R;
+        sx[m][r] = m < rows ? (float)xa[(size_t)(m0 + m) * R + r] : 0.f;
+    }
+    __syncthreads();
+    const int n = blockIdx.x * kUpCols + threadIdx.x;
+    if (n >= N) return;
+    float old[kUpRows];
+#pragma unroll
+    for (int m = 0; m < kUpRows; ++m) old[m] = m < rows ? (float)y[(size_t)(m0 + m) * N + n] : 0.f;
+    float acc[kUpRows] = {0.f, 0.f, 0.f, 0.f};
+    const size_t base = (size_t)n * w_sn;
+    auto add = [&](float b, int r) {
+#pragma unroll
+        for (int m = 0; m < kUpRows; ++m) acc[m] = fmaf(sx[m][r], b, acc[m]);
+    };
+    if constexpr (VEC) {
+        for (int r = 0; r < R; r += 4) {
+            if constexpr (F32) {
+                const float4_t b = *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(w) + base + r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) add(b[e], r + e);
+            } else {
+                const half4_t b = *reinterpret_cast<const half4_t*>(reinterpret_cast<const half_t*>(w) + base + r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) add((float)b[e], r + e);
+            }
+        }
+    } else {
+        for (int r = 0; r < R; ++r) {
+            const size_t i = base + (size_t)r * w_sr;
+            add(F32 ? reinterpret_cast<const float*>(w)[i] : (float)reinterpret_cast<const half_t*>(w)[i], r);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < kUpRows; ++m)
+        if (m < rows) y[(size_t)(m0 + m) * N + n] = (half_t)fmaf(alpha, acc[m], old[m]);
+}
+
 // ---- gradient of an adapter matrix --------------------------------------------------------
 // out[j, c] = alpha * sum_m P[m, j] * in[m, c] as v_mfma_f32_16x16x32_f16 products whose reduction index is the ROW m:
 //   A operand  P^T: lane (j = l % 16, kk = l / 16) holds P[mb + 8*kk .. + 7][j]   (rows j >= R are zero)
@@ -501,6 +553,20 @@ extern "C" int q4_launch_lora_down(const void* in, const void* w, int w_sr, int 
         if (w_is_f32) launch_down_rb<kAny, true>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
         else launch_down_rb<kAny, false>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
     }
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+extern "C" int q4_launch_lora_up(const void* xa, const void* w, int w_sn, int w_sr, int w_is_f32, void* y, float alpha,
+                                 int M, int N, int R, hipStream_t stream) {
+    using namespace q4;
+    const half_t* xp = reinterpret_cast<const half_t*>(xa);
+    half_t* yp = reinterpret_cast<half_t*>(y);
+    const dim3 grid((N + kUpCols - 1) / kUpCols, (M + kUpRows - 1) / kUpRows), block(kUpCols);
+    const bool vec = w_sr == 1 && R % 4 == 0 && w_sn % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & (w_is_f32 ? 15u : 7u)) == 0;
+    if (w_is_f32 && vec) hipLaunchKernelGGL((lora_up_kernel<true, true>), grid, block, 0, stream, xp, w, w_sn, w_sr, yp, alpha, M, N, R);
+    else if (w_is_f32) hipLaunchKernelGGL((lora_up_kernel<true, false>), grid, block, 0, stream, xp, w, w_sn, w_sr, yp, alpha, M, N, R);
+    else if (vec) hipLaunchKernelGGL((lora_up_kernel<false, true>), grid, block, 0, stream, xp, w, w_sn, w_sr, yp, alpha, M, N, R);
+    else hipLaunchKernelGGL((lora_up_kernel<false, false>), grid, block, 0, stream, xp, w, w_sn, w_sr, yp, alpha, M, N, R);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

@@ -845,6 +845,27 @@ def lora_down(inp, w, dropout=None):
     return out
 
 
+def lora_update(x, a, b, y, alpha):
+    """y fp16 [M, N] += alpha * (x @ a^T) @ b^T in place, for x fp16 [M, K], a = lora_A.weight [R, K] and
+    b = lora_B.weight [N, R] (fp16/fp32, any positive strides): the adapter of a few rows in two launches (models.py:66).
+    x @ a^T is rounded to fp16, the update once, onto y."""
+    if _host is not None:
+        return _host.lora_update(x, a, b, y, alpha)
+    _require(y.is_cuda and y.dtype == torch.float16 and y.dim() == 2 and y.is_contiguous() and y.device == x.device
+             and x.dim() == 2 and y.shape[0] == x.shape[0], "y must be a contiguous float16 [M, N] tensor beside x [M, K]")
+    _require(b.dim() == 2 and b.shape == (y.shape[1], a.shape[0]) and b.device == y.device, "b must be an [N, R] view on the same device")
+    f32 = _adapter_dtype_flag(b, "b")
+    sn, sr = b.stride()
+    _require(sn >= 1 and sr >= 1, "b must have positive strides")
+    xa = lora_down(x, a)
+    if y.shape[0] == 0:
+        return
+    with _device_ctx(y.device):
+        rc = _lib.lib().q4_lora_up_f16(xa.data_ptr(), b.data_ptr(), int(sn), int(sr), f32, y.data_ptr(), float(alpha),
+                                       y.shape[0], y.shape[1], a.shape[0], _stream(y.device))
+    _lib.check(rc, "q4_lora_up_f16")
+
+
 def lora_grad(p, inp, alpha, transposed=False, dropout=None):
     """alpha * p^T @ inp in fp32 for p fp16 [M, R], inp fp16 [M, C], R in LORA_GRAD_RANKS.  Returns [R, C], or
     with transposed=True the same values stored as a contiguous [C, R] tensor (lora_B.weight's layout).

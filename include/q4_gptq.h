@@ -301,6 +301,11 @@ Q4_API int q4_gemm_grouped_bwd_dx_f16(const q4_gemm_layer_t *layers, int n_layer
 Q4_API int q4_lora_down_f16(const void *in, const void *w, int w_sr, int w_sc, int w_is_f32, void *out,
                      int M, int C, int R, const q4_dropout_t *drop, void *stream);
 
+/* y fp16 [M, N] += alpha * xa fp16 [M, R] @ B^T in place, one rounding; B (element (n, r) at w[n*w_sn + r*w_sr], fp16 or
+ * fp32) is lora_B.weight: the second half of the adapter at decode sizes (models.py:66).  R <= 64; sums in fp32. */
+Q4_API int q4_lora_up_f16(const void *xa, const void *w, int w_sn, int w_sr, int w_is_f32, void *y, float alpha,
+                   int M, int N, int R, void *stream);
+
 /* Gradient of an adapter matrix:  out fp32 [j*o_sr + c*o_sc] = alpha * sum_m p[m, j] * in[m, c]
  * with p fp16 [M, R] and in fp16 [M, C]:  dA = scaling * dyb^T @ x (out = [R, K], o_sr = K, o_sc = 1) and
  * dB = scaling * dy^T @ xa (out = lora_B.weight.grad [N, R], o_sr = 1, o_sc = R) -- what torch autograd

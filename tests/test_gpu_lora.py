@@ -130,3 +130,27 @@ def test_lora_grad_pair_equals_the_two_single_launches(M, C1, C2, R):
     assert torch.equal(got1, want1) and torch.equal(got2, want2)
     ref1 = 2.0 * p1.float().t() @ in1.float()
     assert float((got1 - ref1).abs().max() / ref1.abs().max()) <= 1e-3
+
+
+@pytest.mark.parametrize("M,K,N,r,dtype,strided", [(1, 4096, 4096, 8, "float32", False), (4, 256, 4096, 8, "float16", False),
+                                                   (16, 5120, 13824, 64, "float32", False), (5, 128, 200, 3, "float32", False),
+                                                   (7, 96, 65, 16, "float16", True), (3, 128, 384, 12, "float32", True)])
+def test_rank_r_update_of_a_few_rows(M, K, N, r, dtype, strided):
+    """y += alpha * (x @ A^T) @ B^T in place: edges of the 4-row and 64-column blocks, every layout of B.  The same fp16
+    values enter the reference, so the bound is the one rounding of y (2^-11) plus what 32-bit sums of r terms lose."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    g = torch.Generator(device="cuda").manual_seed(M * N + r)
+    dt = getattr(torch, dtype)
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    A = (torch.randn((r, K), device="cuda", generator=g) * 0.1).to(dt)
+    B = (torch.randn((r, N) if strided else (N, r), device="cuda", generator=g) * 0.1).to(dt)
+    B = B.t() if strided else B
+    y0 = torch.randn((M, N), device="cuda", generator=g).half()
+    guard = torch.zeros((M + 1, N), device="cuda", dtype=torch.float16)
+    y = guard[:M]
+    y.copy_(y0)
+    quant_hip.lora_update(x, A, B, y, 2.0)
+    ref = y0.double() + 2.0 * (quant_hip.lora_down(x, A).double() @ B.double().t())
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 1e-5).all())
+    assert not bool(guard[M].any())
