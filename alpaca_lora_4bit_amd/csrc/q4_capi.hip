@@ -438,8 +438,11 @@ extern "C" int q4_lora_up_f16(const void* xa, const void* w, int w_sn, int w_sr,
     return q4_launch_lora_up(xa, w, w_sn, w_sr, w_is_f32, y, alpha, M, N, R, (hipStream_t)stream);
 }
 
+static bool lora_grad_rank(int R) { return R >= 2 && R <= 32 && (R & 1) == 0; }
+static bool lora_grad_pair_rank(int R) { return lora_grad_rank(R) || (R > 32 && R <= 64 && R % 8 == 0); }
+
 extern "C" size_t q4_lora_grad_workspace_bytes(int M, int C, int R) {
-    if (M < 1 || C < 8 || R < 2 || R > 32 || (R & 1)) return 0;
+    if (M < 1 || C < 8 || !(lora_grad_rank(R) || lora_grad_pair_rank(R))) return 0;
     return q4_lora_grad_workspace(M, C, R);
 }
 
@@ -469,7 +472,8 @@ extern "C" int q4_lora_grad_pair_f32(const void* p1, const void* in1, float* out
     q4_drop_args da;
     const q4_drop_args* dp;
     if (!make_drop(drop1, &da, &dp)) return Q4_ERR_BAD_SHAPE;
-    if (M < 1 || R < 2 || R > 32 || (R & 1)) return Q4_ERR_BAD_SHAPE;
+    if (M < 1 || !lora_grad_pair_rank(R)) return Q4_ERR_BAD_SHAPE;
+    if (R > 32 && (long long)M * R * 2 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;          /* 32-bit buffer offsets of p */
     const int Cs[2] = {C1, C2};
     const int strides[4] = {o1_sr, o1_sc, o2_sr, o2_sc};
     for (int i = 0; i < 2; ++i) {

@@ -293,10 +293,14 @@ __global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restri
 // fp32 partial tiles [split][strip][R][128] that lora_grad_reduce_kernel adds in a fixed order (bit-reproducible).
 constexpr int kG2Waves = 4, kG2Cols = 128, kG2PadRows = 40;
 
-// One or two gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
-// independent, so they go out side by side.  Workgroups beyond a problem's own grid leave at once.
+// Up to four gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
+// independent, so they go out side by side; above 32 adapter rows (the accumulators of one wavefront) each is two problems
+// on the first 32 and the remaining columns of P, which reads `in` twice: 2 x 16 MB at 2048 x 4096, where the library
+// products this replaces also needed the dropout mask and the masked input in memory.  Workgroups beyond a problem's own
+// grid leave at once.
 struct GradProb {
-    const half_t* P;          // [M, R]
+    const half_t* P;          // [M, R] of a row pitch of p_ld
+    int R, p_ld;              // both even
     const half_t* in;         // [M, C]
     float* out;               // through o_sr, o_sc
     float* part;              // partial tiles [splits][col_blocks][R][128]
@@ -304,7 +308,7 @@ struct GradProb {
     DropArgs drop;            // dropout mask applied to `in` (thr15 == 0: none); the result carries drop.scale
 };
 struct GradArgs {
-    GradProb p[2];
+    GradProb p[4];
     float alpha;
     int M;
 };
@@ -314,8 +318,9 @@ template <int NPL>
 struct G2Regs { uint4_t d[8]; uint32_t p[NPL]; };
 
 template <bool DROP, int RB>    // RB = ceil(R / 16) A operands (1 or 2); R is even
-__global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga, int R) {
+__global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
     const GradProb& q = ga.p[blockIdx.z];
+    const int R = q.R;
     if ((int)blockIdx.x >= q.col_blocks || (int)blockIdx.y >= q.splits) return;       // uniform over the workgroup
     constexpr int NPL = 4 * RB;                                                       // 4-byte loads of P per lane and block
     __shared__ float red[kG2Waves][16][kG2Cols];                                      // 32 KB
@@ -329,7 +334,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga, i
     const int m_wg = blockIdx.y * q.rows_per_wg;
     const int m_end = min(m_wg + q.rows_per_wg, M);
     const rsrc_t rs_in = make_rsrc(q.in, (unsigned)m_end * (unsigned)row_bytes);       // rows past m_end read as zero
-    const rsrc_t rs_p = make_rsrc(q.P, (unsigned)m_end * (unsigned)(R * 2));
+    const rsrc_t rs_p = make_rsrc(q.P, ((unsigned)(m_end - 1) * (unsigned)q.p_ld + (unsigned)R) * 2u);
     int voff[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) voff[e] = c0 < C ? (8 * kk + e) * row_bytes + c0 * 2 : kFarOffset;
@@ -340,7 +345,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga, i
 #pragma unroll
     for (int t = 0; t < NPL; ++t) {
         const int i = lane + 64 * t, m = i / hr, j = 2 * (i - m * hr);
-        pvoff[t] = i < 32 * hr ? i * 4 : kFarOffset;
+        pvoff[t] = i < 32 * hr ? (m * q.p_ld + j) * 2 : kFarOffset;
         pdst[t] = i < 32 * hr ? j * kG2PadRows + m : -1;
     }
     half_t* const ptw = &pt[wave][0][0];
@@ -357,7 +362,7 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga, i
     auto load_block = [&](G2Regs<NPL>& x, int mb) {
         const bool live = mb < m_end;
         const int soff = live ? mb * row_bytes : kFarOffset;
-        const int soff_p = live ? mb * R * 2 : kFarOffset;
+        const int soff_p = live ? mb * q.p_ld * 2 : kFarOffset;
 #pragma unroll
         for (int t = 0; t < NPL; ++t) x.p[t] = buf_load32(rs_p, pvoff[t], soff_p);
 #pragma unroll
@@ -449,8 +454,9 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga, i
 }
 
 // Adds the `splits` partial tiles of every strip in order and writes the scaled result through the caller's strides.
-__global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga, int R) {
+__global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga) {
     const GradProb& q = ga.p[blockIdx.y];
+    const int R = q.R;
     const int total = q.col_blocks * R * kG2Cols;              // one split's tiles: [strip][j][column]
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (q.splits <= 1 || t >= total) return;                   // a single split was written directly
@@ -575,11 +581,12 @@ extern "C" size_t q4_lora_grad_workspace(int M, int C, int R) {
     return g.splits == 1 ? 0 : (size_t)g.splits * g.col_blocks * R * q4::kG2Cols * sizeof(float);
 }
 
-static q4::GradProb make_grad_prob(const void* P, const void* in, float* out, int o_sr, int o_sc, int M, int C, int R,
+static q4::GradProb make_grad_prob(const void* P, int p_ld, const void* in, float* out, int o_sr, int o_sc, int M, int C, int R,
                                    float* part, const q4::DropArgs* drop = nullptr) {
     const q4::GradPlan g = q4::plan_grad(M, C);
     q4::GradProb q;
     q.P = reinterpret_cast<const q4::half_t*>(P);
+    q.R = R; q.p_ld = p_ld;
     q.in = reinterpret_cast<const q4::half_t*>(in);
     q.out = out;
     q.part = part;
@@ -589,38 +596,38 @@ static q4::GradProb make_grad_prob(const void* P, const void* in, float* out, in
     return q;
 }
 
-static int launch_grad(const q4::GradArgs& ga, int nprob, int R, hipStream_t stream) {
+static int launch_grad(const q4::GradArgs& ga, int nprob, hipStream_t stream) {
     using namespace q4;
-    int gx = 0, gy = 0, rx = 0;
+    int gx = 0, gy = 0, rx = 0, R = 0;
     bool any_split = false, any_drop = false;
     for (int i = 0; i < nprob; ++i) {
+        R = ga.p[i].R > R ? ga.p[i].R : R;
         gx = ga.p[i].col_blocks > gx ? ga.p[i].col_blocks : gx;
         gy = ga.p[i].splits > gy ? ga.p[i].splits : gy;
-        const int rb = (ga.p[i].col_blocks * R * kG2Cols + 255) / 256;
+        const int rb = (ga.p[i].col_blocks * ga.p[i].R * kG2Cols + 255) / 256;
         rx = rb > rx ? rb : rx;
         any_split = any_split || ga.p[i].splits > 1;
         any_drop = any_drop || ga.p[i].drop.thr15 != 0;
     }
     const dim3 grid(gx, gy, nprob), block(64 * kG2Waves);
     if (R <= 16) {
-        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 1>), grid, block, 0, stream, ga, R);
-        else hipLaunchKernelGGL((lora_grad_kernel<false, 1>), grid, block, 0, stream, ga, R);
+        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 1>), grid, block, 0, stream, ga);
+        else hipLaunchKernelGGL((lora_grad_kernel<false, 1>), grid, block, 0, stream, ga);
     } else {
-        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 2>), grid, block, 0, stream, ga, R);
-        else hipLaunchKernelGGL((lora_grad_kernel<false, 2>), grid, block, 0, stream, ga, R);
+        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 2>), grid, block, 0, stream, ga);
+        else hipLaunchKernelGGL((lora_grad_kernel<false, 2>), grid, block, 0, stream, ga);
     }
-    if (any_split) hipLaunchKernelGGL(lora_grad_reduce_kernel, dim3(rx, nprob), dim3(256), 0, stream, ga, R);
+    if (any_split) hipLaunchKernelGGL(lora_grad_reduce_kernel, dim3(rx, nprob), dim3(256), 0, stream, ga);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 extern "C" int q4_launch_lora_grad(const void* P, const void* in, float* out, int o_sr, int o_sc, float alpha,
                                    int M, int C, int R, const q4::DropArgs* drop, void* workspace, hipStream_t stream) {
     q4::GradArgs ga;
-    ga.p[0] = make_grad_prob(P, in, out, o_sr, o_sc, M, C, R, reinterpret_cast<float*>(workspace), drop);
-    ga.p[1] = ga.p[0];
+    ga.p[0] = make_grad_prob(P, R, in, out, o_sr, o_sc, M, C, R, reinterpret_cast<float*>(workspace), drop);
     ga.alpha = alpha;
     ga.M = M;
-    return launch_grad(ga, 1, R, stream);
+    return launch_grad(ga, 1, stream);
 }
 
 extern "C" int q4_launch_dropout_keep(uint8_t* keep, int M, int C, const q4::DropArgs* drop, hipStream_t stream) {
@@ -637,10 +644,18 @@ extern "C" int q4_launch_lora_grad_pair(const void* P1, const void* in1, float* 
                                         hipStream_t stream) {
     q4::GradArgs ga;
     float* ws = reinterpret_cast<float*>(workspace);
-    ga.p[0] = make_grad_prob(P1, in1, out1, o1_sr, o1_sc, M, C1, R, ws, drop1);      // the mask applies to in1 only
-    ga.p[1] = make_grad_prob(P2, in2, out2, o2_sr, o2_sc, M, C2, R,
-                             ws ? ws + q4_lora_grad_workspace(M, C1, R) / sizeof(float) : nullptr);
+    int n = 0;
+    auto add = [&](const void* P, const void* in, float* out, int o_sr, int o_sc, int C, const q4::DropArgs* drop) {
+        for (int r0 = 0; r0 < R; r0 += 32) {
+            const int rq = R - r0 < 32 ? R - r0 : 32;
+            ga.p[n++] = make_grad_prob(reinterpret_cast<const q4::half_t*>(P) + r0, R, in, out + (size_t)r0 * o_sr, o_sr, o_sc,
+                                       M, C, rq, ws, drop);
+            if (ws) ws += q4_lora_grad_workspace(M, C, rq) / sizeof(float);
+        }
+    };
+    add(P1, in1, out1, o1_sr, o1_sc, C1, drop1);                                     // the mask applies to in1 only
+    add(P2, in2, out2, o2_sr, o2_sc, C2, nullptr);
     ga.alpha = alpha;
     ga.M = M;
-    return launch_grad(ga, 2, R, stream);
+    return launch_grad(ga, n, stream);
 }

@@ -817,6 +817,7 @@ def gemm_bwd_dx(dy, qweight, qzeros, scales, g_idx=None, groupsize=None, dyb=Non
 
 
 LORA_GRAD_RANKS = tuple(range(2, 33, 2))
+LORA_GRAD_PAIR_RANKS = LORA_GRAD_RANKS + (40, 48, 56, 64)
 
 
 def lora_down(inp, w, dropout=None):
@@ -900,7 +901,7 @@ def lora_grad(p, inp, alpha, transposed=False, dropout=None):
 def lora_grad_pair(p1, inp1, p2, inp2, alpha, dropout=None, outs=None):
     """Both adapter gradients of a layer in one launch: returns (alpha * p1^T @ inp1 as [R, C1],
     alpha * p2^T @ inp2 stored as a contiguous [C2, R] tensor) -- dA from (dyb, x) and dB in lora_B.weight's
-    layout from (xa, dy).  Same requirements as lora_grad; p1 and p2 share their shape.
+    layout from (xa, dy).  Same requirements as lora_grad, R also 40, 48, 56 and 64; p1 and p2 share their shape.
     dropout=(seed, p): inp1 is replaced by dropout(inp1) (inp2 is left as it is)."""
     if _host is not None and outs is None:
         return _host.lora_grad_pair(p1, inp1, p2, inp2, float(alpha),
@@ -913,7 +914,8 @@ def lora_grad_pair(p1, inp1, p2, inp2, alpha, dropout=None, outs=None):
     _require(p1.shape == p2.shape and p1.device == p2.device, "the two rank-R operands must share shape and device")
     M, R = p1.shape
     C1, C2 = inp1.shape[1], inp2.shape[1]
-    _require(R in LORA_GRAD_RANKS and C1 % 8 == 0 and C2 % 8 == 0, "lora_grad needs an even R in 2..32 and C % 8 == 0")
+    _require(R in LORA_GRAD_PAIR_RANKS and C1 % 8 == 0 and C2 % 8 == 0,
+             "lora_grad_pair needs an even R in 2..32 or a multiple of 8 up to 64, and C % 8 == 0")
     dev = p1.device
     if M == 0:
         return (torch.zeros((R, C1), dtype=torch.float32, device=dev), torch.zeros((C2, R), dtype=torch.float32, device=dev))

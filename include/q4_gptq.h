@@ -309,7 +309,7 @@ Q4_API int q4_lora_up_f16(const void *xa, const void *w, int w_sn, int w_sr, int
 /* Gradient of an adapter matrix:  out fp32 [j*o_sr + c*o_sc] = alpha * sum_m p[m, j] * in[m, c]
  * with p fp16 [M, R] and in fp16 [M, C]:  dA = scaling * dyb^T @ x (out = [R, K], o_sr = K, o_sc = 1) and
  * dB = scaling * dy^T @ xa (out = lora_B.weight.grad [N, R], o_sr = 1, o_sc = R) -- what torch autograd
- * computes for the two adapter Linears of models.py:66.  R even, 2 <= R <= 32; C % 8 == 0.
+ * computes for the two adapter Linears of models.py:66.  R even, 2 <= R <= 32 (the pair also 40, 48, 56, 64); C % 8 == 0.
  * `workspace`: q4_lora_grad_workspace_bytes(M, C, R) bytes (0 for small M: then it may be NULL), 256-byte
  * aligned, contents irrelevant before and after the call: it carries fp32 partial sums of row blocks,
  * which a second kernel adds in a fixed order (bit-reproducible).  With `drop`, `in` is replaced by dropout(in)

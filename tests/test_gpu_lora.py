@@ -154,3 +154,19 @@ def test_rank_r_update_of_a_few_rows(M, K, N, r, dtype, strided):
     ref = y0.double() + 2.0 * (quant_hip.lora_down(x, A).double() @ B.double().t())
     assert bool(((y.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + 1e-5).all())
     assert not bool(guard[M].any())
+
+
+@pytest.mark.parametrize("M,C1,C2,R,p", [(2048, 4096, 4096, 64, 0.05), (300, 1408, 512, 40, 0.0), (70, 136, 5120, 56, 0.1), (1000, 512, 4096, 48, 0.0)])
+def test_lora_grad_pair_above_32_rows(M, C1, C2, R, p):
+    """Ranks that are two problems per gradient: every row of both against fp32 products (bound as for the smaller ranks)."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    g = torch.Generator().manual_seed(M + C1 + R)
+    p1, p2 = (torch.randn(M, R, generator=g).half().cuda() for _ in range(2))
+    in1, in2 = torch.randn(M, C1, generator=g).half().cuda(), torch.randn(M, C2, generator=g).half().cuda()
+    got1, got2 = quant_hip.lora_grad_pair(p1, in1, p2, in2, 2.0, dropout=(9, p) if p else None)
+    x1 = in1.float()
+    if p:
+        x1 = x1 * quant_hip.dropout_keep_mask(M, C1, 9, p, in1.device).float() * quant_hip.dropout_scale(p)
+    for got, ref in ((got1, 2.0 * p1.float().t() @ x1), (got2, 2.0 * in2.float().t() @ p2.float())):
+        assert got.shape == ref.shape and float((got - ref).abs().max() / ref.abs().max()) <= 1e-3
