@@ -334,7 +334,7 @@ class AutogradMatmul4bitLora(torch.autograd.Function):
         """(dA, dB) = scaling * (dyb^T @ dropout(x), dy^T @ xa) in the parameters' dtypes (None where not needed)."""
         da = db = None
         r = dyb.shape[1]
-        if need_a and need_b and r in quant_hip.LORA_GRAD_PAIR_RANKS:
+        if need_a and need_b and quant_hip.lora_grad_pair_takes(x2.shape[0], x2.shape[1], dy.shape[1], r):
             da, db = quant_hip.lora_grad_pair(dyb, x2, xa, dy, scaling, dropout=dropout)   # one launch for both gradients
         else:
             if need_a:

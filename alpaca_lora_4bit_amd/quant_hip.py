@@ -820,6 +820,12 @@ LORA_GRAD_RANKS = tuple(range(2, 33, 2))
 LORA_GRAD_PAIR_RANKS = LORA_GRAD_RANKS + (40, 48, 56, 64)
 
 
+def lora_grad_pair_takes(rows, c1, c2, r):
+    """Whether both adapter gradients of a layer go to lora_grad_pair.  The kernel addresses its operands with 32-bit
+    byte offsets (q4_lora_grad_pair_f32 refuses more); ranks above 32 have library products to fall back on there."""
+    return r in LORA_GRAD_PAIR_RANKS and (r <= 32 or (max(c1, c2) <= 1 << 20 and 2 * rows * max(c1, c2, r) < 0x70000000))
+
+
 def lora_down(inp, w, dropout=None):
     """out fp16 [M, R] = inp fp16 [M, C] @ w^T for an adapter matrix view w [R, C] (fp16/fp32, any positive
     strides): xa = x @ A^T with w = lora_A.weight, dyb = dy @ B with w = lora_B.weight.t()  (models.py:66).

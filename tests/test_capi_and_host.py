@@ -164,6 +164,30 @@ def test_streaming_kernel_selection_rules_need_no_gpu():
     assert not fwd(128, 131072, 4096, 128, 0) and not dx(128, 4096, 131072, 128, 0)   # beyond the 32-bit offsets
 
 
+def test_gradients_of_ranks_above_32_beyond_the_kernels_offsets_use_library_products(monkeypatch):
+    """67964 rows of 13824 features are the first that q4_lora_grad_pair_f32 refuses (32-bit byte offsets); the backward
+    of such a call takes the products it took before the kernel knew these ranks.  Meta tensors: shapes only."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    from alpaca_lora_4bit_amd.autograd_4bit import AutogradMatmul4bitLora
+    L, p, odd = _lib.lib(), 0x100000, 0x100001           # the misaligned operand ends every accepted call before a launch
+    C = 13824
+    pair = []
+    monkeypatch.setattr(quant_hip, "lora_grad_pair", lambda dyb, x, xa, dy, scaling, dropout=None: pair.append(1) or (
+        torch.empty((dyb.shape[1], x.shape[1]), device="meta"), torch.empty((dy.shape[1], dyb.shape[1]), device="meta")))
+    for r in (40, 64):
+        for rows, taken in ((67963, True), (67964, False)):
+            for c1, c2 in ((C, 4096), (4096, C)):
+                rc = L.q4_lora_grad_pair_f32(odd, p, p, c1, 1, c1, p, p, p, 1, r, c2, 1.0, rows, r, None, None, 0, None)
+                assert rc == (-5 if taken else -2) == (-5 if quant_hip.lora_grad_pair_takes(rows, c1, c2, r) else -2)
+                x, dy = (torch.empty((rows, c), dtype=torch.float16, device="meta") for c in (c1, c2))
+                small = torch.empty((rows, r), dtype=torch.float16, device="meta")
+                del pair[:]
+                da, db = AutogradMatmul4bitLora._adapter_grads(small, x, small, dy, 2.0, None, True, True, (torch.float32, torch.float16))
+                assert (da.shape, db.shape) == ((r, c1), (c2, r)) and (da.dtype, db.dtype) == (torch.float32, torch.float16)
+                assert bool(pair) == taken
+
+
 def test_compiled_host_binding_is_built_and_matches_the_library():
     """The pybind11 host module (csrc/host/q4_host.cpp) sits next to the library, was built against the same ABI
     version, and quant_hip routes its operators through it.  Its argument checks run without a GPU."""
