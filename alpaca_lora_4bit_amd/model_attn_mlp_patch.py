@@ -160,19 +160,27 @@ class _MemberGroup:
         if matmul_utils_4bit.use_dense_route(rows) or member.in_features % 128 or any(m.out_features % 128 for m in self.members):
             return None
         Ns = [m.out_features for m in self.members]
-        grad = torch.is_grad_enabled()
-        if not quant_hip.gemm_grouped_applicable(True, rows, member.in_features, Ns) or \
-                (grad and not quant_hip.gemm_grouped_applicable(False, rows, member.in_features, Ns)):
+        if not quant_hip.gemm_grouped_applicable(True, rows, member.in_features, Ns):
             return None
-        if not grad and sum(Ns) // 128 * ((rows + 255) // 256) < 192:
-            return None                                      # forward alone: the streaming kernels per layer (200 rows, q|k|v: 51 us)
+        parts = [self._gemm_spec(m, x) for m in self.members]
+        train = torch.is_grad_enabled() and (x.requires_grad or any(
+            t is not None and t.requires_grad for _, la, lb, _, _ in parts for t in (la, lb)))
+        if train:
+            if not quant_hip.gemm_grouped_applicable(False, rows, member.in_features, Ns):
+                return None
+        elif all(la is None for _, la, _, _, _ in parts) and quant_hip.streams_forward(rows, member.in_features, Ns, self.groupsize):
+            # nothing to differentiate and no adapter in the launch: layers that all have a whole-reduction streaming
+            # kernel run by themselves.  us apart against grouped: q|k|v of 4096 features at 136 / 200 / 256 rows 41.6 / 49.7 /
+            # 52.6 against 48.6 / 49.5 / 50.0, of 5120 at 136 rows 52.2 against 59.6.  Where one of them has none, the
+            # group wins (5120, 200 rows: 78.8 against 61.0; gate|up of 4096 -> 11008, 200 rows: 71.8 against 53.2), and with
+            # adapters always (q|k|v of 4096, 200 rows: 67.9 against 54.9).
+            return None
         if self._gemm_ok is None:
             self._gemm_ok = all(quant_hip._group_layer_ok(l, self.groupsize) for l in layers)
         if not self._gemm_ok:
             return None
         specs, tensors = [], []
-        for m, (qweight, qzeros, scales) in zip(self.members, layers):
-            bias, la, lb, scaling, drop_p = self._gemm_spec(m, x)
+        for (qweight, qzeros, scales), (bias, la, lb, scaling, drop_p) in zip(layers, parts):
             seed = int(torch.randint(0, 2 ** 62, (1,)).item()) if drop_p > 0.0 else 0
             specs.append((scaling, drop_p, seed))
             tensors += [qweight, scales, qzeros, bias, la, lb]

@@ -689,14 +689,23 @@ def gemm_fwd(x, qweight, qzeros, scales, g_idx=None, groupsize=None, bias=None, 
     return out
 
 
+ROUTE_STREAM = 2              # Q4_ROUTE_STREAM
+
+
 def gemm_grouped_applicable(fwd, M, K, Ns):
-    """True when gemm_grouped_fwd / gemm_grouped_bwd_dx take this shape (2..4 layers, more than 128 rows, enough tiles
-    for one launch); the layers must also have sequential groups and scales below 64 (checked by those calls)."""
+    """True when gemm_grouped_fwd / gemm_grouped_bwd_dx take this shape (2..4 layers, more than 128 rows, forward: enough
+    tiles for one launch), not that they are the faster choice; the layers must also have sequential groups and scales below 64 (checked by those calls)."""
     n = len(Ns)
     if not 2 <= n <= 4:
         return False
     arr = (ctypes.c_int * n)(*[int(v) for v in Ns])
     return bool(_lib.lib().q4_gemm_grouped_applicable(int(bool(fwd)), n, int(M), int(K), arr))
+
+
+def streams_forward(M, K, Ns, groupsize):
+    """True when every one of the sequential-group layers K -> N has a whole-reduction streaming kernel for M rows."""
+    L = _lib.lib()
+    return all(L.q4_gemm_route(1, int(M), int(K), int(N), int(groupsize), 0) == ROUTE_STREAM for N in Ns)
 
 
 def _group_layer_ok(lay, groupsize):

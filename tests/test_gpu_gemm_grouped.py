@@ -178,6 +178,57 @@ def test_grouped_block_matches_the_ungrouped_block_forward_and_gradients(oracle,
     assert ungroup(grouped) == 1 and "_q4_group" not in grouped.k_proj.__dict__
 
 
+@pytest.mark.parametrize("K,N,M,streams", [(4096, 4096, 200, True),        # 96 tiles, one row tile, all three layers stream
+                                           (1024, 5120, 200, False)])      # 120 tiles, too many strips to stream at this many rows
+def test_one_row_tile_is_grouped_by_what_there_is_to_train(oracle, K, N, M, streams, monkeypatch):
+    """129..256 rows of q|k|v: one grouped launch when something needs a gradient, when an adapter rides along or when the
+    layers have no streaming kernel of their own; a forward alone of layers that stream stays with them, whether or not
+    gradients are switched on.  Values and gradients against the block without grouping in every case."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_quant_attn
+    grouped, plain = _Block(oracle, K, N, 128, 0.0, 60), _Block(oracle, K, N, 128, 0.0, 60)
+    assert make_quant_attn(grouped) == 1
+    assert quant_hip.streams_forward(M, K, (N, N, N), 128) == streams
+    count = {"fwd": 0, "bwd": 0}
+    for name, key in (("gemm_grouped_fwd", "fwd"), ("gemm_grouped_bwd_dx", "bwd")):
+        real = getattr(quant_hip, name)
+        monkeypatch.setattr(quant_hip, name, (lambda real, key: lambda *a, **k: (count.__setitem__(key, count[key] + 1), real(*a, **k))[1])(real, key))
+    xh, gys = oracle.make_activations(M, K, seed=5), [_t(oracle.make_activations(M, N, seed=6 + i)) for i in range(3)]
+
+    def compare(grad_mode, x_needs_grad, want_fwd, want_bwd):
+        count.update(fwd=0, bwd=0)
+        results = []
+        for block in (grouped, plain):
+            block.zero_grad()
+            x = _t(xh).requires_grad_(x_needs_grad)
+            with torch.set_grad_enabled(grad_mode):
+                ys = block(x)
+            if any(y.requires_grad for y in ys):
+                torch.autograd.backward([y for y in ys if y.requires_grad], [g for y, g in zip(ys, gys) if y.requires_grad])
+            results.append([y.detach() for y in ys] + [g for g in [x.grad] + [p.grad for p in block.parameters() if p.requires_grad] if g is not None])
+        assert count == {"fwd": want_fwd, "bwd": want_bwd}
+        assert len(results[0]) == len(results[1])
+        for a, b in zip(*results):
+            assert float((a.float() - b.float()).abs().max() / b.float().abs().max()) <= 3e-3
+
+    compare(True, True, 1, 1)                          # training: grad_input and the adapters
+    compare(True, False, 1, 0)                         # the first block: adapters only
+    compare(False, False, 1, 0)                        # inference with the adapters
+    for block in (grouped, plain):
+        for m in (block.q_proj, block.v_proj):
+            for p in list(m.lora_A.parameters()) + list(m.lora_B.parameters()):
+                p.requires_grad_(False)
+    compare(True, False, 1, 0)                         # frozen adapters still ride in the launch
+    for block in (grouped, plain):
+        for m in (block.q_proj, block.v_proj):
+            m.enable_adapters(False)
+    alone = 0 if streams else 1
+    compare(True, True, 1, 1)
+    compare(True, False, alone, 0)                     # an evaluation that left gradients on
+    compare(False, False, alone, 0)
+
+
 def _dense(quant_hip, t, gs):
     return quant_hip.dequant(t["qweight"], t["qzeros"], t["scales"], t["g_idx"], gs).float()
 
