@@ -31,12 +31,12 @@
 // activation and whose B operand is the fp16 adapter matrix: no second pass over the output.
 // The epilogue transposes the accumulators through LDS so that y is written in 16-byte pieces.
 #include "q4_common.hpp"
+#include "q4_gemm_plan.hpp"
 #include <stdlib.h>
 #include <type_traits>
 
 namespace q4 {
 
-constexpr int BN = 128, BK = 64;
 constexpr int LDS_STRIDE = BK + 8;   // halves
 
 struct GemmArgs {
@@ -702,7 +702,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs a) {
 //   grad-input: dx = sum_i dy_i @ W_i^T is ONE reduction over the layers' columns one after the other: a workgroup
 //               walks the layers (all of them, or its share of the concatenated steps where the tiles are few) with
 //               the sum in its accumulators, adapter term and dropout mask of each layer included.
-constexpr int kGemmGroup = 4;
 struct GemmGroupArgs {
     GemmArgs layer[kGemmGroup];
     int tile_end[kGemmGroup];          // forward: running total of column tiles (tile width of the launch)
@@ -836,11 +835,6 @@ static hipError_t launch_gemm(GemmArgs a, int nout, int splits, int tail_cols, i
     return hipGetLastError();
 }
 
-struct GemmPlan {
-    int cfg, splits;
-    int tail_cols, tail_splits;      // cfg 2, 3: 128-column tiles of the second launch (0: none), its reduction split
-};
-
 template <bool FWD, bool GIDX>
 static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout, hipStream_t stream) {
     switch (p.cfg) {
@@ -854,98 +848,6 @@ static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout
 // What TileMap is told: row tile r starts its reduction loop kPhaseStep * r steps later; tiles are ordered in groups
 // of kRowTilesPerGroup row tiles (measured optimum over the benchmark shapes).
 constexpr int kPhaseStep = 2, kRowTilesPerGroup = 2;
-
-// More 256 x 256 tiles than whole rounds of the CUs: the wide tiles of the whole rounds run as they are, and the columns
-// left over go to a second launch of 256 x 128 tiles that is one round at most, its reduction split when even that
-// leaves CUs idle.  A full round of wide tiles takes 1.75-1.85 us per reduction step, one of narrow tiles 0.9-1.05, so the
-// remainder costs at most 0.6 of the round of wide tiles, or half of the two narrow ones, that it would cost otherwise:
-// 2048 x (4096 -> 11008), 344 tiles: three rounds of narrow tiles 186 us, 118 + 57 us; grad-input of 4096 x
-// (5120 -> 13824), 864 tiles: four rounds of wide tiles 561 us, 447 + 79 us.
-// Taken for remainders of 1/8 to 1/2 of a round: below that the narrow tiles with their own remainder launch lose
-// little, above it the remainder does not fit a round of narrow tiles.
-struct WideTail { int tail_cols, tail_splits; };     // 128-column tiles; 0: does not apply
-static WideTail wide_tail(int M, int nsteps, int nout, bool may_split, size_t workspace_bytes) {
-    WideTail w{0, 1};
-    const int nr = (M + 255) / 256, nc = nout / 256;
-    const long t = (long)nc * nr;
-    if (nout % 256 != 0 || t <= 256) return w;
-    const int main_cols = (int)((t / 256) * 256 / nr);
-    const long left = (long)(nc - main_cols) * nr;
-    if (main_cols < 1 || left < 32 || left > 128) return w;
-    int s = (int)(256 / (2 * left));
-    while (s > 1 && (!may_split || nsteps < 8 * s ||
-                     (size_t)s * (size_t)M * (size_t)(nc - main_cols) * 256 * sizeof(float) > workspace_bytes)) --s;
-    w.tail_cols = 2 * (nc - main_cols);
-    w.tail_splits = s;
-    return w;
-}
-
-// Launch plan shared by q4_launch_gemm and q4_gemm_plan_workspace.  Few output tiles (small M) leave most CUs
-// idle while each tile walks the whole reduction: the reduction is then split over gridDim.z workgroups that
-// write fp32 partial tiles, about 1.5 workgroups per CU in total.
-static GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes) {
-    GemmPlan p;
-    p.tail_cols = 0; p.tail_splits = 1;
-    const int nsteps = red / BK;
-    // Tiles of 256 rows (8 wavefronts, one dequantized slab of W for 256 activation rows) do about twice the work per
-    // CU and unit of time that 128-row tiles do, so they are used from 129 rows on: as they are when there are more
-    // than 128 of them (even 130 of them on 256 CUs beat 260 tiles of 128 rows), otherwise with the reduction split
-    // floor(256 / tiles) ways so that every CU gets one workgroup (never more than 256 workgroups: a second, nearly
-    // empty round costs more than the split gains).
-    const long t256 = (long)(nout / BN) * ((M + 255) / 256);
-    int splits = 1;
-    // 256 x 256 tiles from 144 of them on (a workgroup does the work of two 256 x 128 ones in about 1.7 times their
-    // time), unless their last round would leave more than a fifth of the CUs' slots empty where the narrower tiles
-    // fill theirs better: 3072 x (4096 -> 11008) has 516 wide tiles = 3 rounds for 2.02 rounds of work and stays
-    // with the narrow ones (270 against 294 us), 4096 rows have 688 (313 against 356 us).
-    const long twide = (nout % 256 == 0) ? (long)(nout / 256) * ((M + 255) / 256) : 0;
-    const WideTail wt = wide_tail(M, nsteps, nout, true, workspace_bytes);
-    if (wt.tail_cols > 0) {
-        p.cfg = 3; p.splits = 1;
-        p.tail_cols = wt.tail_cols;
-        p.tail_splits = wt.tail_splits;
-        return p;
-    }
-    if (twide >= 144 &&
-        (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) {
-        p.cfg = 3; p.splits = 1;
-        return p;
-    }
-    if (t256 > 128 && M > 128) {
-        p.cfg = 2;
-        // More tiles than CUs and a last round that fills at most half of them: the column tiles of that
-        // remainder run as a second launch with the reduction split so that it takes a fraction of a round.
-        const int nr = (M + 255) / 256;
-        const long rem = t256 % 256;
-        if (t256 > 256 && rem > 0) {
-            const int tcols = (int)((rem + nr - 1) / nr);
-            const long tt = (long)tcols * nr;
-            int ts = tt <= 128 ? (int)(256 / tt) : 1;
-            if (ts > 8) ts = 8;
-            while (ts > 1 && nsteps < 8 * ts) --ts;
-            if (ts > 1 && (size_t)ts * (size_t)M * (size_t)tcols * BN * sizeof(float) <= workspace_bytes) {
-                p.tail_cols = tcols;
-                p.tail_splits = ts;
-            }
-        }
-    } else if (t256 <= 128 && M > 128 && nsteps >= 8 * (int)(256 / t256) &&
-               (size_t)(256 / t256 > 8 ? 8 : 256 / t256) * (size_t)M * (size_t)nout * sizeof(float) <= workspace_bytes) {
-        p.cfg = 2;                                             // only with room for all its partial tiles
-        splits = (int)(256 / t256);
-        if (splits > 8) splits = 8;
-    } else {
-        p.cfg = 0;
-        const long tiles = (long)(nout / BN) * ((M + 127) / 128);
-        if (tiles < 192) {
-            splits = (int)((384 + tiles - 1) / tiles);
-            if (splits > 8) splits = 8;                        // measured: more splits only add prologues and partial tiles
-            if (splits > nsteps / 4) splits = nsteps / 4;      // at least four steps per workgroup
-        }
-    }
-    while (splits > 1 && (size_t)splits * (size_t)M * (size_t)nout * sizeof(float) > workspace_bytes) --splits;
-    p.splits = splits < 1 ? 1 : splits;
-    return p;
-}
 
 }  // namespace q4
 
@@ -1021,60 +923,6 @@ extern "C" int q4_launch_gemm(int fwd, const void* act, const int32_t* qweight, 
 
 // ---- several layers in one launch (sequential groups only) ---------------------------------------------------------
 namespace q4 {
-// cfg as in launch_gemm_cfg (2: 256 x 128 tiles, 3: 256 x 256 tiles; -1: not applicable), the split of the reduction,
-// and for cfg 3 the second launch (see wide_tail).
-struct GroupPlan { int cfg, splits, tail_cols, tail_splits; };
-
-// Forward: one tile of one layer per workgroup, no split, so the launch needs enough tiles by itself: from 96 tiles of
-// 256 x 128 on (q|k|v of 4096 features at 129..256 rows), below which the split launches per layer are shorter.
-// Grad-input: one reduction over all layers' columns; of the tilings and splits the one with the shortest estimate
-// (us: rounds of the CUs x steps x time per step, prologue and epilogue of a workgroup, and the traffic of the partial
-// sums where the reduction is split).  Against one partial tile per layer and their sum: 4096 rows, two layers 5120 ->
-// 13824: 1151 us + 46 us for the sums became 752 + 233 + 8 us; three layers 5120 -> 5120: 694 + 34 became 504 + 140 + 8 us.
-static GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
-    GroupPlan p{-1, 1, 0, 1};
-    if (n < 2 || n > kGemmGroup || M <= 128) return p;
-    const int nr = (M + 255) / 256;
-    if (fwd) {
-        long tot = 0;
-        bool all256 = true;
-        for (int i = 0; i < n; ++i) { tot += N[i]; all256 = all256 && N[i] % 256 == 0; }
-        const long twide = all256 ? (tot / 256) * nr : 0, t256 = (tot / BN) * nr;
-        const WideTail wt = all256 && tot < (1l << 30) ? wide_tail(M, K / BK, (int)tot, false, 0) : WideTail{0, 1};
-        if (wt.tail_cols > 0) { p.cfg = 3; p.tail_cols = wt.tail_cols; }
-        else if (twide >= 144 && (twide <= 256 || 5 * twide >= 4 * 256 * ((twide + 255) / 256))) p.cfg = 3;
-        else if (t256 >= 96) p.cfg = 2;
-        return p;
-    }
-    constexpr double kWide = 1.7, kNarrow = 1.0, kEnds = 4.0, kReduce = 4.0, kBytesPerUs = 4.5e6;
-    long nsteps = 0;
-    for (int i = 0; i < n; ++i) nsteps += N[i] / BK;
-    double best = 0.0;
-    auto offer = [&](double us, GroupPlan q) { if (p.cfg < 0 || us < best) { best = us; p = q; } };
-    for (int cfg = 3; cfg >= 2; --cfg) {
-        const int tw = cfg == 3 ? 256 : BN;
-        if (K % tw != 0) continue;
-        const long t = (long)(K / tw) * nr;
-        for (int s = 1; s <= 8 && (s == 1 || (t * s <= 256 && nsteps >= 8 * s)); ++s)
-            offer((double)((t * s + 255) / 256) * ((nsteps + s - 1) / s * (cfg == 3 ? kWide : kNarrow) + kEnds) +
-                  (s > 1 ? kReduce + 8.0 * s * M * K / kBytesPerUs : 0.0), GroupPlan{cfg, s, 0, 1});
-    }
-    const WideTail wt = wide_tail(M, nsteps < 1 << 24 ? (int)nsteps : 1 << 24, K, true, ~(size_t)0);
-    if (wt.tail_cols > 0) {
-        const int ts = wt.tail_splits;
-        const long t = (long)(K / 256 - wt.tail_cols / 2) * nr;
-        offer((double)((t + 255) / 256) * (nsteps * kWide + kEnds) + (nsteps + ts - 1) / ts * kNarrow + kEnds + kReduce +
-              (ts > 1 ? kReduce + 8.0 * ts * M * wt.tail_cols * BN / kBytesPerUs : 0.0), GroupPlan{3, 1, wt.tail_cols, ts});
-    }
-    return p;
-}
-static size_t group_workspace(const GroupPlan& p, int M, int K) {
-    const size_t main = p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)K * sizeof(float) : 0;
-    const size_t tail = p.tail_cols > 0 && p.tail_splits > 1
-        ? (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float) : 0;
-    return main > tail ? main : tail;
-}
-
 template <int BM, int WGM, bool FWD, int WGN>
 static void launch_group_tiles(const GemmGroupArgs& g, int n, dim3 grid, hipStream_t stream) {
     const GemmArgs& a = g.layer[0];
