@@ -32,6 +32,7 @@
 // The epilogue transposes the accumulators through LDS so that y is written in 16-byte pieces.
 #include "q4_common.hpp"
 #include "q4_gemm_plan.hpp"
+#include <initializer_list>
 #include <stdlib.h>
 #include <type_traits>
 
@@ -913,7 +914,7 @@ extern "C" int q4_launch_gemm(int fwd, const void* act, const int32_t* qweight, 
         workspace_bytes >= q4_skinny_dx_workspace(M, K, N))
         return q4_launch_skinny_dx(act, qweight, qzeros, scales, groupsize, out, M, K, N, G, workspace, stream);
     // tile configuration: 256-row tiles once they still give every CU a workgroup; split-K for few tiles
-    const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, workspace ? workspace_bytes : 0);
+    const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, workspace ? workspace_bytes : 0, gidx);
     a.part = reinterpret_cast<float*>(workspace);
     hipError_t e;
     if (fwd) e = gidx ? launch_gemm_cfg<true, true>(p, a, nout, stream) : launch_gemm_cfg<true, false>(p, a, nout, stream);
@@ -1029,9 +1030,11 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
 extern "C" size_t q4_gemm_plan_workspace(int fwd, int M, int K, int N) {
     using namespace q4;
     const int nout = fwd ? N : K;
-    const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, ~(size_t)0);
-    size_t need = p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)nout * sizeof(float) : 0;
-    if (p.tail_cols > 0 && p.tail_splits > 1) need = (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float);
+    size_t need = 0;                              // the query does not know the group order: room for either
+    for (const bool indexed : {false, true}) {
+        const size_t part = plan_workspace(plan_gemm(M, fwd ? K : N, nout, ~(size_t)0, indexed), M, nout);
+        need = part > need ? part : need;
+    }
     if (fwd && M > 16 && M <= 64) {               // the skinny kernel's partial rows (it may or may not apply)
         const size_t sk = q4_skinny_workspace(M, K, N);
         if (sk > need) need = sk;

@@ -42,7 +42,11 @@ inline WideTail wide_tail(int M, int nsteps, int nout, bool may_split, size_t wo
 // Launch plan shared by q4_launch_gemm and q4_gemm_plan_workspace.  Few output tiles (small M) leave most CUs
 // idle while each tile walks the whole reduction: the reduction is then split over gridDim.z workgroups that
 // write fp32 partial tiles, about 1.5 workgroups per CU in total.
-inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes) {
+// `indexed`: the kernels that look every row's group up (groups of 32, g_idx).  On them wide tiles of whole rounds with a
+// remainder launch are slower than the narrow tiles on every shape measured (30 shapes of groups of 32): forward by 37..53 %
+// (1969 x (4352 -> 9472): 420 against 290 us), grad-input by 11..16 % (2605 x (8704 -> 4352): 318 against 279 us, where the
+// wide kernel also spills 80 bytes a lane).
+inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes, bool indexed) {
     GemmPlan p;
     p.tail_cols = 0; p.tail_splits = 1;
     const int nsteps = red / BK;
@@ -58,7 +62,7 @@ inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes) {
     // fill theirs better: 3072 x (4096 -> 11008) has 516 wide tiles = 3 rounds for 2.02 rounds of work and stays
     // with the narrow ones (270 against 294 us), 4096 rows have 688 (313 against 356 us).
     const long twide = (nout % 256 == 0) ? (long)(nout / 256) * ((M + 255) / 256) : 0;
-    const WideTail wt = wide_tail(M, nsteps, nout, true, workspace_bytes);
+    const WideTail wt = indexed ? WideTail{0, 1} : wide_tail(M, nsteps, nout, true, workspace_bytes);
     if (wt.tail_cols > 0) {
         p.cfg = 3; p.splits = 1;
         p.tail_cols = wt.tail_cols;
@@ -104,6 +108,13 @@ inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes) {
     while (splits > 1 && (size_t)splits * (size_t)M * (size_t)nout * sizeof(float) > workspace_bytes) --splits;
     p.splits = splits < 1 ? 1 : splits;
     return p;
+}
+
+// fp32 partial sums of a plan
+inline size_t plan_workspace(const GemmPlan& p, int M, int nout) {
+    if (p.tail_cols > 0)
+        return p.tail_splits > 1 ? (size_t)p.tail_splits * (size_t)M * (size_t)p.tail_cols * BN * sizeof(float) : 0;
+    return p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)nout * sizeof(float) : 0;
 }
 
 // cfg as in launch_gemm_cfg (2: 256 x 128 tiles, 3: 256 x 256 tiles; -1: not applicable), the split of the reduction,

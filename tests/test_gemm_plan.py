@@ -9,8 +9,8 @@ from conftest import ROOT
 
 WRAPPER = r"""
 #include "q4_gemm_plan.hpp"
-extern "C" void plan(int M, int red, int nout, size_t workspace, int* out) {
-    const q4::GemmPlan p = q4::plan_gemm(M, red, nout, workspace);
+extern "C" void plan(int M, int red, int nout, size_t workspace, int indexed, int* out) {
+    const q4::GemmPlan p = q4::plan_gemm(M, red, nout, workspace, indexed != 0);
     out[0] = p.cfg; out[1] = p.splits; out[2] = p.tail_cols; out[3] = p.tail_splits;
 }
 """
@@ -25,14 +25,14 @@ def plans(tmp_path_factory):
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I" + os.path.join(ROOT, "alpaca_lora_4bit_amd", "csrc"),
                            str(tmp / "plan.cpp"), "-o", str(tmp / "plan.so")])
     lib = ctypes.CDLL(str(tmp / "plan.so"))
-    lib.plan.argtypes = [ctypes.c_int] * 3 + [ctypes.c_size_t, ctypes.POINTER(ctypes.c_int)]
+    lib.plan.argtypes = [ctypes.c_int] * 3 + [ctypes.c_size_t, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     lib.plan.restype = None
     return lib
 
 
-def _plan(lib, M, red, nout, workspace=ANY):
+def _plan(lib, M, red, nout, workspace=ANY, indexed=False):
     out = (ctypes.c_int * 4)()
-    lib.plan(M, red, nout, workspace, out)
+    lib.plan(M, red, nout, workspace, int(indexed), out)
     return tuple(out)
 
 
@@ -42,3 +42,39 @@ def test_up_to_128_rows_keep_the_128_row_tiles(plans, M, nout):
     """More wide tiles than CUs with a remainder, but half of every 256-row tile would be padding."""
     assert _plan(plans, M, 2048, nout)[0] == NARROW128
     assert _plan(plans, 129, 2048, nout)[0] == WIDE and _plan(plans, 129, 2048, nout)[2] > 0
+
+
+def _partials(plan, M, nout):
+    cfg, splits, tail_cols, tail_splits = plan
+    if tail_cols:
+        return 4 * tail_splits * M * tail_cols * 128 if tail_splits > 1 else 0
+    return 4 * splits * M * nout if splits > 1 else 0
+
+
+@pytest.mark.parametrize("M,red,nout", [(1969, 4352, 9472), (1576, 9600, 12800), (2605, 4352, 8704), (3950, 6784, 12800), (2048, 4096, 11008)])
+def test_indexed_groups_have_no_wide_remainder_route(plans, M, red, nout):
+    assert _plan(plans, M, red, nout)[0] == WIDE and _plan(plans, M, red, nout)[2] > 0
+    assert _plan(plans, M, red, nout, indexed=True)[0] == NARROW
+
+
+def test_a_plan_stays_inside_its_output_and_its_workspace(plans):
+    """Every plan over rows, features and scratch sizes: the second launch's columns lie inside the output, no share is
+    without a step, the partial sums fit the scratch given, and the query's size holds the plan of either group order."""
+    import random
+    from alpaca_lora_4bit_amd import _lib
+    rng = random.Random(3)
+    L = _lib.lib()
+    for _ in range(4000):
+        M = int(2 ** rng.uniform(0, 14))
+        red, nout = 128 * int(2 ** rng.uniform(0, 7.5)), 128 * int(2 ** rng.uniform(0, 10))
+        for indexed in (False, True):
+            whole = _plan(plans, M, red, nout, indexed=indexed)
+            assert _partials(whole, M, nout) <= L.q4_gemm_workspace_bytes(1, M, red, nout)
+            scratch = rng.choice([0, 1 << 20, _partials(whole, M, nout), max(_partials(whole, M, nout) - 1, 0)])
+            for p, room in ((whole, ANY), (_plan(plans, M, red, nout, scratch, indexed), scratch)):
+                cfg, splits, tail_cols, tail_splits = p
+                width = 256 if cfg == WIDE else 128
+                assert nout % width == 0 and 0 <= tail_cols * 128 < nout and (nout - tail_cols * 128) % width == 0
+                assert 1 <= splits <= max(red // 64, 1) and 1 <= tail_splits <= red // 64
+                assert splits == 1 or tail_cols == 0
+                assert _partials(p, M, nout) <= room
