@@ -1020,7 +1020,7 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
     };
     const bool wide = p.cfg == 3;
     const int narrow_total = fwd ? tiles[1] : K / BN;
-    const int main_tiles = wide ? (narrow_total - p.tail_cols) / 2 : narrow_total;
+    const int main_tiles = (narrow_total - p.tail_cols) / (wide ? 2 : 1);
     launch(wide, 0, main_tiles, p.splits, K);
     if (p.tail_cols > 0) launch(false, narrow_total - p.tail_cols, p.tail_cols, p.tail_splits, p.tail_cols * BN);
     return hipGetLastError() == hipSuccess ? 0 : -4;

@@ -117,16 +117,20 @@ inline size_t plan_workspace(const GemmPlan& p, int M, int nout) {
     return p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)nout * sizeof(float) : 0;
 }
 
-// cfg as in launch_gemm_cfg (2: 256 x 128 tiles, 3: 256 x 256 tiles; -1: not applicable), the split of the reduction,
-// and for cfg 3 the second launch (see wide_tail).
+// cfg as in launch_gemm_cfg (2: 256 x 128 tiles, 3: 256 x 256 tiles; -1: not applicable), the split of the reduction, and
+// the 128-column tiles of the second launch (0: none) with the split of its reduction.
 struct GroupPlan { int cfg, splits, tail_cols, tail_splits; };
 
 // Forward: one tile of one layer per workgroup, no split, so the launch needs enough tiles by itself: from 96 tiles of
-// 256 x 128 on (q|k|v of 4096 features at 129..256 rows), below which the split launches per layer are shorter.
-// Grad-input: one reduction over all layers' columns; of the tilings and splits the one with the shortest estimate
-// (us: rounds of the CUs x steps x time per step, prologue and epilogue of a workgroup, and the traffic of the partial
-// sums where the reduction is split).  Against one partial tile per layer and their sum: 4096 rows, two layers 5120 ->
-// 13824: 1151 us + 46 us for the sums became 752 + 233 + 8 us; three layers 5120 -> 5120: 694 + 34 became 504 + 140 + 8 us.
+// 256 x 128 on (q|k|v of 4096 features at 129..256 rows).  Forward + grad-input of 200 rows apart / grouped, us: 96 tiles
+// 110 / 92 (with adapters on q and v 143 / 101), 120 tiles of 5120 features 165 / 115.  Below the line, 90 tiles of 3840
+// features 124 / 88 and 48 of 2048 63 / 57: the line could lie lower for training.
+// Grad-input: one reduction over all layers' columns.  Of the tilings, splits and remainder launches the one with the
+// shortest estimate in us: the rounds of the CUs, each as long as a workgroup's steps (a round that leaves CUs idle runs up
+// to a fifth faster) plus its prologue and epilogue, a second launch, and the sum of the partial tiles where a reduction is
+// split.  Against every plan measured on 130 shapes (2..4 layers, 129..4096 rows, 2048..13824 features) the choice is
+// 0.2 % slower than the best on average and 3 % at most; splits of one round alone and remainders of wide tiles alone were
+// 4.9 % and up to 44 % slower (1006 rows, three layers 8832 -> 9600, 276 narrow tiles: 736 -> 553 us).
 inline GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
     GroupPlan p{-1, 1, 0, 1};
     if (n < 2 || n > kGemmGroup || M <= 128) return p;
@@ -142,25 +146,28 @@ inline GroupPlan plan_gemm_group(int fwd, int n, int M, int K, const int* N) {
         else if (t256 >= 96) p.cfg = 2;
         return p;
     }
-    constexpr double kWide = 1.7, kNarrow = 1.0, kEnds = 4.0, kReduce = 4.0, kBytesPerUs = 4.5e6;
+    constexpr double kWide = 1.6, kNarrow = 1.0, kEnds = 5.0, kIdle = 0.8, kLaunch = 3.0, kBytesPerUs = 4.5e6;
     long nsteps = 0;
     for (int i = 0; i < n; ++i) nsteps += N[i] / BK;
+    auto tiles_us = [&](int cfg, long tiles, int s) {
+        const double steps = (double)((nsteps + s - 1) / s) * (cfg == 3 ? kWide : kNarrow);
+        const long last = tiles * s % 256;
+        return (double)(tiles * s / 256) * (steps + kEnds) + (last ? steps * (kIdle + (1.0 - kIdle) * last / 256.0) + kEnds : 0.0);
+    };
+    auto sum_us = [&](int s, long cols) { return s > 1 ? kLaunch + 8.0 * s * M * cols / kBytesPerUs : 0.0; };
+    auto worth = [&](long tiles, int s) { return s == 1 || (tiles * s <= 512 && nsteps >= 8 * s); };
     double best = 0.0;
     auto offer = [&](double us, GroupPlan q) { if (p.cfg < 0 || us < best) { best = us; p = q; } };
     for (int cfg = 3; cfg >= 2; --cfg) {
         const int tw = cfg == 3 ? 256 : BN;
         if (K % tw != 0) continue;
         const long t = (long)(K / tw) * nr;
-        for (int s = 1; s <= 8 && (s == 1 || (t * s <= 256 && nsteps >= 8 * s)); ++s)
-            offer((double)((t * s + 255) / 256) * ((nsteps + s - 1) / s * (cfg == 3 ? kWide : kNarrow) + kEnds) +
-                  (s > 1 ? kReduce + 8.0 * s * M * K / kBytesPerUs : 0.0), GroupPlan{cfg, s, 0, 1});
-    }
-    const WideTail wt = wide_tail(M, nsteps < 1 << 24 ? (int)nsteps : 1 << 24, K, true, ~(size_t)0);
-    if (wt.tail_cols > 0) {
-        const int ts = wt.tail_splits;
-        const long t = (long)(K / 256 - wt.tail_cols / 2) * nr;
-        offer((double)((t + 255) / 256) * (nsteps * kWide + kEnds) + (nsteps + ts - 1) / ts * kNarrow + kEnds + kReduce +
-              (ts > 1 ? kReduce + 8.0 * ts * M * wt.tail_cols * BN / kBytesPerUs : 0.0), GroupPlan{3, 1, wt.tail_cols, ts});
+        for (int s = 1; s <= 8 && worth(t, s); ++s) offer(tiles_us(cfg, t, s) + sum_us(s, K), GroupPlan{cfg, s, 0, 1});
+        const int main_cols = (int)(t / 256 * 256 / nr), tail = (K / tw - main_cols) * (tw / BN);
+        if (main_cols < 1 || tail < 1) continue;
+        for (int s = 1; s <= 8 && worth((long)tail * nr, s); ++s)
+            offer(tiles_us(cfg, (long)main_cols * nr, 1) + kLaunch + tiles_us(2, (long)tail * nr, s) + sum_us(s, (long)tail * BN),
+                  GroupPlan{cfg, 1, tail, s});
     }
     return p;
 }

@@ -13,6 +13,10 @@ extern "C" void plan(int M, int red, int nout, size_t workspace, int indexed, in
     const q4::GemmPlan p = q4::plan_gemm(M, red, nout, workspace, indexed != 0);
     out[0] = p.cfg; out[1] = p.splits; out[2] = p.tail_cols; out[3] = p.tail_splits;
 }
+extern "C" void group_plan(int fwd, int n, int M, int K, const int* N, int* out) {
+    const q4::GroupPlan p = q4::plan_gemm_group(fwd, n, M, K, N);
+    out[0] = p.cfg; out[1] = p.splits; out[2] = p.tail_cols; out[3] = p.tail_splits;
+}
 """
 NARROW128, NARROW, WIDE = 0, 2, 3            # 128 x 128, 256 x 128 and 256 x 256 tiles
 ANY = 2 ** 62
@@ -26,13 +30,20 @@ def plans(tmp_path_factory):
                            str(tmp / "plan.cpp"), "-o", str(tmp / "plan.so")])
     lib = ctypes.CDLL(str(tmp / "plan.so"))
     lib.plan.argtypes = [ctypes.c_int] * 3 + [ctypes.c_size_t, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
-    lib.plan.restype = None
+    lib.group_plan.argtypes = [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int)] * 2
+    lib.plan.restype = lib.group_plan.restype = None
     return lib
 
 
 def _plan(lib, M, red, nout, workspace=ANY, indexed=False):
     out = (ctypes.c_int * 4)()
     lib.plan(M, red, nout, workspace, int(indexed), out)
+    return tuple(out)
+
+
+def _group_plan(lib, fwd, M, K, Ns):
+    out = (ctypes.c_int * 4)()
+    lib.group_plan(fwd, len(Ns), M, K, (ctypes.c_int * len(Ns))(*Ns), out)
     return tuple(out)
 
 
@@ -78,3 +89,47 @@ def test_a_plan_stays_inside_its_output_and_its_workspace(plans):
                 assert 1 <= splits <= max(red // 64, 1) and 1 <= tail_splits <= red // 64
                 assert splits == 1 or tail_cols == 0
                 assert _partials(p, M, nout) <= room
+
+
+@pytest.mark.parametrize("M,K,Ns,was", [
+    (1006, 8832, (9600, 9600, 9600), (NARROW, 1, 0, 1)),             # 276 narrow tiles: 1.08 rounds
+    (846, 10368, (11392, 11392, 11392), (NARROW, 1, 0, 1)),          # 324
+    (1086, 8064, (3712, 3712, 3712, 3712), (NARROW, 1, 0, 1)),       # 315
+])
+def test_grouped_grad_input_does_not_leave_a_second_round_nearly_empty(plans, M, K, Ns, was):
+    """Widths without wide tiles just beyond one round of narrow ones: a remainder launch (1.23..1.28 times faster)."""
+    cfg, splits, tail_cols, tail_splits = _group_plan(plans, 0, M, K, Ns)
+    row_tiles = (M + 255) // 256
+    assert (cfg, splits, tail_cols, tail_splits) != was
+    assert tail_cols > 0 and tail_splits > 1 and (K // 128 - tail_cols) * row_tiles <= 256
+
+
+def test_a_grouped_plan_stays_inside_its_output_and_its_workspace(plans):
+    import random
+    from alpaca_lora_4bit_amd import _lib
+    rng = random.Random(4)
+    L = _lib.lib()
+    seen = set()
+    for _ in range(6000):
+        n = rng.choice([2, 3, 4])
+        M, K = int(2 ** rng.uniform(7, 15)), 128 * int(2 ** rng.uniform(0, 8))
+        Ns = [128 * int(2 ** rng.uniform(0, 8)) for _ in range(n)]
+        arr = (ctypes.c_int * n)(*Ns)
+        for fwd in (0, 1):
+            cfg, splits, tail_cols, tail_splits = p = _group_plan(plans, fwd, M, K, Ns)
+            assert bool(L.q4_gemm_grouped_applicable(fwd, n, M, K, arr)) == (cfg >= 0)
+            if cfg < 0:
+                assert M <= 128 or fwd
+                continue
+            seen.add((fwd, cfg, splits > 1, tail_cols > 0, tail_splits > 1))
+            columns, steps = (sum(Ns), K // 64) if fwd else (K, sum(Ns) // 64)
+            width = 256 if cfg == WIDE else 128
+            assert all(c % width == 0 for c in (Ns if fwd else [K]))
+            assert 0 <= tail_cols * 128 < columns and (columns - tail_cols * 128) % width == 0
+            assert 1 <= splits <= 8 and 1 <= tail_splits <= 8 and max(splits, tail_splits) <= steps
+            assert (splits == 1 or tail_cols == 0) and (tail_splits == 1 or tail_cols > 0)
+            want = _partials(p, M, columns)
+            assert L.q4_gemm_grouped_workspace_bytes(fwd, n, M, K, arr) == want and (want == 0 or not fwd)
+    # what the estimate can choose came up: both widths, whole and split, and a remainder launch, split or not
+    whole, split, rest, rest_split = (False, False, False), (True, False, False), (False, True, False), (False, True, True)
+    assert {(0, NARROW, *k) for k in (whole, split, rest_split)} | {(0, WIDE, *k) for k in (whole, split, rest, rest_split)} <= seen
