@@ -17,7 +17,7 @@ def _t(a):
 @pytest.mark.parametrize("M,K,Ns,gs,lora", [
     (1024, 4096, (4096, 4096, 4096), 128, (8, 0, 8)),          # q|k|v of config 4: 192 wide tiles, adapters on q and v
     (1024, 4096, (11008, 11008), 128, (0, 0)),                 # gate|up of config 4
-    (600, 1024, (4096, 2048, 1024, 2048), 256, (16, 8, 0, 0)),  # four layers, ragged rows, narrow tiles, two shares per layer
+    (600, 1024, (4096, 2048, 1024, 2048), 256, (16, 8, 0, 0)),  # four layers, ragged rows, one row tile's worth of narrow tiles in eight shares
     (2048, 512, (4096, 4096), 64, (0, 8)),                     # groups of 64 rows
 ])
 def test_grouped_forward_and_grad_input(oracle, M, K, Ns, gs, lora):
@@ -233,19 +233,29 @@ def _dense(quant_hip, t, gs):
     return quant_hip.dequant(t["qweight"], t["qzeros"], t["scales"], t["g_idx"], gs).float()
 
 
-@pytest.mark.parametrize("M,K,Ns,gs,r,p", [
-    (200, 4096, (256, 384), 128, 8, 0.05),          # one row tile: shares that begin and end inside a layer, 10 steps in all
-    (1000, 4096, (1024, 640, 512), 64, 16, 0.05),   # ragged rows, shares across three layers, no scale / zero table
-    (4500, 4096, (512, 256), 128, 8, 0.1),          # 288 wide tiles: whole rounds and a remainder launch
-    (300, 384, (1024, 1024), 128, 0, 0.0),          # K not a multiple of 256: narrow tiles only
+@pytest.mark.parametrize("M,K,Ns,gs,r,p,bare,splits,tail_cols", [
+    (200, 4096, (256, 384), 128, 8, 0.05, 1, 1, 0),                    # 10 steps in all, walked whole
+    (1000, 4096, (1024, 640, 512), 64, 16, 0.05, 1, 1, 0),             # ragged rows, walked whole, no scale / zero table
+    (200, 4096, (2048, 1152, 1024), 128, 8, 0.05, 1, 6, 0),            # layers begin at steps 32 and 50, shares at multiples of 11
+    (200, 4096, (2048, 1152, 1024), 64, 16, 0.0, None, 6, 0),          # the same without the table, every layer with an adapter
+    (1000, 4096, (2048, 1152, 640), 64, 16, 0.05, 0, 2, 0),            # the second share begins in layer 0 and holds 1 and 2 whole
+    (4500, 4096, (512, 256), 128, 8, 0.1, 1, 1, 4),                    # 288 wide tiles: whole rounds and a remainder launch
+    (4500, 4096, (2048, 640), 128, 8, 0.1, None, 3, 4),                # its reduction in three shares, the last across both layers
+    (4500, 4096, (1152, 640), 128, 8, 0.0, None, 2, 4),                # unmasked adapters on the wide layer walk and on two shares
+    (300, 384, (1024, 1024), 128, 0, 0.0, None, 4, 0),                 # K not a multiple of 256: narrow tiles only
 ])
-def test_grouped_grad_input_is_one_reduction_over_the_layers(oracle, M, K, Ns, gs, r, p):
+def test_grouped_grad_input_is_one_reduction_over_the_layers(oracle, M, K, Ns, gs, r, p, bare, splits, tail_cols):
     """dx over the concatenated reduction (adapter terms and their dropout masks included) against fp32 products with
     the bit-exact dense weights.  Bound: inputs and weights are the same fp16 values on both sides, so what differs is the
     fp16 rounding of the result (2^-11), of the scaled adapter matrix (2^-11 of the smaller adapter term) and the order
-    of the 32-bit sums: 2e-3 of the largest value."""
+    of the 32-bit sums: 2e-3 of the largest value (an adapter term left out or counted twice is 10 to 40 times that).
+    The scratch query shows that the plan is the one the case stands for: `splits` shares of the whole output, or of the
+    last `tail_cols` column tiles.  `bare`: the layer without an adapter."""
+    import ctypes
     import torch
-    from alpaca_lora_4bit_amd import quant_hip
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    scratch = splits * M * (tail_cols * 128 or K) * 4 if splits > 1 else 0
+    assert _lib.lib().q4_gemm_grouped_workspace_bytes(0, len(Ns), M, K, (ctypes.c_int * len(Ns))(*Ns)) == scratch
     ts = [to_cuda_layer(oracle.make_layer(K, N, gs, seed=K + N + i)) for i, N in enumerate(Ns)]
     g = torch.Generator(device="cuda").manual_seed(M)
     dys, layers, ref = [], [], 0.0
@@ -253,12 +263,14 @@ def test_grouped_grad_input_is_one_reduction_over_the_layers(oracle, M, K, Ns, g
         dy = torch.randn((M, N), device="cuda", generator=g).half()
         dyb = A = drop = None
         ref = ref + dy.float() @ _dense(quant_hip, t, gs).t()
-        if r and i != 1:
+        if r and i != bare:
             A = torch.randn((r, K), device="cuda", generator=g) * 0.05
             dyb = torch.randn((M, r), device="cuda", generator=g).half()
-            drop = (77 + i, p)
-            keep = quant_hip.dropout_keep_mask(M, K, 77 + i, p, dy.device).float()
-            ref = ref + keep * quant_hip.dropout_scale(p) * 2.0 * (dyb.float() @ A)
+            term = 2.0 * (dyb.float() @ A)
+            if p:
+                drop = (77 + i, p)
+                term = term * quant_hip.dropout_keep_mask(M, K, 77 + i, p, dy.device).float() * quant_hip.dropout_scale(p)
+            ref = ref + term
         dys.append(dy)
         layers.append((t["qweight"], t["qzeros"], t["scales"], dyb, A, 2.0 if A is not None else 1.0, drop))
     dx = quant_hip.gemm_grouped_bwd_dx(dys, layers, gs)
