@@ -287,21 +287,22 @@ __global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restri
 // per 16 lanes and row), and turns the 8 x 8 block around in registers with 32 byte permutes; MFMA i of the eight
 // then multiplies column c0 + 8*cg + i.  A wavefront so consumes a block of 32 rows x 128 columns (8 KB) with 8
 // loads, 32 permutes and 8 MFMAs per 16 adapter rows; the kernel is bound by its loads.  P for the block (32 x R
-// values, R even and at most 32) is fetched with 4-byte loads and transposed through a wavefront-private LDS tile.
+// values) is fetched with 4-byte loads (R even, at most 32) or 16-byte ones (40, 48, 56, 64) and transposed through a
+// wavefront-private LDS tile.
 // Workgroup = 4 wavefronts on one 128-column strip and `rows_per_wg` rows (wavefront w takes the 32-row blocks
 // w, w + 4, ...); the sum over wavefronts goes through LDS, the sum over the gridDim.y workgroups of a strip through
 // fp32 partial tiles [split][strip][R][128] that lora_grad_reduce_kernel adds in a fixed order (bit-reproducible).
+// Above 32 adapter rows `in` is still read once, at the price of one workgroup per CU for ranks 56 and 64 (32 accumulator
+// tiles a wavefront).  As two problems of half the rank, each reading `in` and leaving partial tiles, both gradients of
+// 2048 rows of 13824 and 13824 features took 72 us at rank 64 (77.5 with dropout) where library products take 44; now 31
+// with dropout; 4096 x 4096 features 33.8 -> 20.5, 512 rows of 5120 and 13824 39 -> 17.  One block of 64 rows alone
+// takes longer (7.7 -> 10 us).
 constexpr int kG2Waves = 4, kG2Cols = 128, kG2PadRows = 40;
 
-// Up to four gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
-// independent, so they go out side by side; above 32 adapter rows (the accumulators of one wavefront) each is two problems
-// on the first 32 and the remaining columns of P, which reads `in` twice: 2 x 16 MB at 2048 x 4096, where the library
-// products this replaces also needed the dropout mask and the masked input in memory (2048 x 4096 x 4096, rank 64, dropout
-// 0.05, forward + backward: 296 -> 262 us).  Workgroups beyond a problem's own
-// grid leave at once.
+// One or two gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
+// independent, so they go out side by side.  Workgroups beyond a problem's own grid leave at once.
 struct GradProb {
-    const half_t* P;          // [M, R] of a row pitch of p_ld
-    int R, p_ld;              // both even
+    const half_t* P;          // [M, R]
     const half_t* in;         // [M, C]
     float* out;               // through o_sr, o_sc
     float* part;              // partial tiles [splits][col_blocks][R][128]
@@ -309,22 +310,25 @@ struct GradProb {
     DropArgs drop;            // dropout mask applied to `in` (thr15 == 0: none); the result carries drop.scale
 };
 struct GradArgs {
-    GradProb p[4];
+    GradProb p[2];
     float alpha;
     int M;
 };
 
+// Above 32 adapter rows a result whose adapter rows lie side by side (lora_B.weight's layout) goes out along them, partial
+// tiles included: 64-byte pieces instead of single words (64 rows of 4096 features at rank 64: 11.3 -> 10.6 us).
+__device__ __forceinline__ bool grad_jfast(const GradProb& q) { return q.o_sr < q.o_sc; }
 
-template <int NPL>
-struct G2Regs { uint4_t d[8]; uint32_t p[NPL]; };
+template <int RB>
+struct G2Regs { uint4_t d[8]; uint32_t p[4 * RB]; };
 
-template <bool DROP, int RB>    // RB = ceil(R / 16) A operands (1 or 2); R is even
-__global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
+template <bool DROP, int RB>    // RB = ceil(R / 16) A operands; R is even, above 32 a multiple of 8
+__global__ __launch_bounds__(64 * kG2Waves, RB == 3 ? 2 : 1) void lora_grad_kernel(GradArgs ga, int R) {
     const GradProb& q = ga.p[blockIdx.z];
-    const int R = q.R;
     if ((int)blockIdx.x >= q.col_blocks || (int)blockIdx.y >= q.splits) return;       // uniform over the workgroup
-    constexpr int NPL = 4 * RB;                                                       // 4-byte loads of P per lane and block
-    __shared__ float red[kG2Waves][16][kG2Cols];                                      // 32 KB
+    constexpr bool PV = RB > 2;                                                       // P in 16-byte pieces
+    constexpr int NPL = PV ? RB : 4 * RB;                                             // loads of P per lane and block
+    __shared__ __attribute__((aligned(16))) float red[kG2Waves][16][kG2Cols + (PV ? 4 : 0)];   // 32 KB; + 4: grad_jfast's reads
     __shared__ __attribute__((aligned(16))) half_t pt[kG2Waves][16 * RB][kG2PadRows]; // P^T of the current block
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -335,22 +339,26 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
     const int m_wg = blockIdx.y * q.rows_per_wg;
     const int m_end = min(m_wg + q.rows_per_wg, M);
     const rsrc_t rs_in = make_rsrc(q.in, (unsigned)m_end * (unsigned)row_bytes);       // rows past m_end read as zero
-    const rsrc_t rs_p = make_rsrc(q.P, ((unsigned)(m_end - 1) * (unsigned)q.p_ld + (unsigned)R) * 2u);
+    const rsrc_t rs_p = make_rsrc(q.P, (unsigned)m_end * (unsigned)(R * 2));
     int voff[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) voff[e] = c0 < C ? (8 * kk + e) * row_bytes + c0 * 2 : kFarOffset;
     // this lane's share of a block of P: the pairs i = lane, lane + 64, ... of the 32 x R block
-    // (row i / (R/2), columns 2 * (i % (R/2)) and the next)
+    // (row i / (R/2), columns 2 * (i % (R/2)) and the next); PV: row lane % 32, columns 16 * t + 8 * (lane / 32) and the
+    // seven next (32 lanes then write 64 contiguous bytes of P^T)
     const int hr = R >> 1;
     int pvoff[NPL], pdst[NPL];
 #pragma unroll
     for (int t = 0; t < NPL; ++t) {
-        const int i = lane + 64 * t, m = i / hr, j = 2 * (i - m * hr);
-        pvoff[t] = i < 32 * hr ? (m * q.p_ld + j) * 2 : kFarOffset;
-        pdst[t] = i < 32 * hr ? j * kG2PadRows + m : -1;
+        const int i = lane + 64 * t;
+        const int m = PV ? lane & 31 : i / hr, j = PV ? 16 * t + 8 * (lane >> 5) : 2 * (i - m * hr);
+        const bool mine = PV ? j < R : i < 32 * hr;
+        pvoff[t] = mine ? (m * R + j) * 2 : kFarOffset;
+        pdst[t] = mine || PV ? j * kG2PadRows + m : -1;             // PV: columns beyond R read as zero and fill their rows
     }
     half_t* const ptw = &pt[wave][0][0];
-    for (int i = lane; i < 16 * RB * kG2PadRows; i += 64) ptw[i] = (half_t)0.f;   // rows j >= R stay zero
+    if constexpr (!PV)
+        for (int i = lane; i < 16 * RB * kG2PadRows; i += 64) ptw[i] = (half_t)0.f;   // rows j >= R stay zero
     const DropArgs drop = q.drop;
     const uint32_t thr_pair = drop.thr15 | (drop.thr15 << 16);
 
@@ -360,16 +368,19 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[b][i] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    auto load_block = [&](G2Regs<NPL>& x, int mb) {
+    auto load_block = [&](G2Regs<RB>& x, int mb) {
         const bool live = mb < m_end;
         const int soff = live ? mb * row_bytes : kFarOffset;
-        const int soff_p = live ? mb * q.p_ld * 2 : kFarOffset;
+        const int soff_p = live ? mb * R * 2 : kFarOffset;
 #pragma unroll
-        for (int t = 0; t < NPL; ++t) x.p[t] = buf_load32(rs_p, pvoff[t], soff_p);
+        for (int t = 0; t < NPL; ++t) {
+            if constexpr (PV) *reinterpret_cast<uint4_t*>(&x.p[4 * t]) = buf_load128(rs_p, pvoff[t], soff_p);
+            else x.p[t] = buf_load32(rs_p, pvoff[t], soff_p);
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) x.d[e] = buf_load128(rs_in, voff[e], soff);
     };
-    auto consume = [&](G2Regs<NPL>& x, int mb) {
+    auto consume = [&](G2Regs<RB>& x, int mb) {
         if (DROP && drop.thr15) {                 // uniform: the mask belongs to one problem of a pair
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -383,9 +394,14 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
         }
 #pragma unroll
         for (int t = 0; t < NPL; ++t)
-            if (pdst[t] >= 0) {
-                ptw[pdst[t]] = __builtin_bit_cast(half_t, (uint16_t)(x.p[t] & 0xFFFFu));
-                ptw[pdst[t] + kG2PadRows] = __builtin_bit_cast(half_t, (uint16_t)(x.p[t] >> 16));
+            if (PV || pdst[t] >= 0) {
+                constexpr int W = PV ? 4 : 1;                                         // words of a load
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const uint32_t v = x.p[W * t + w];
+                    ptw[pdst[t] + 2 * w * kG2PadRows] = __builtin_bit_cast(half_t, (uint16_t)(v & 0xFFFFu));
+                    ptw[pdst[t] + (2 * w + 1) * kG2PadRows] = __builtin_bit_cast(half_t, (uint16_t)(v >> 16));
+                }
             }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -417,16 +433,26 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
 
     // blocks w, w + 4, ... of the workgroup's rows; the next block's loads are in flight while one is consumed
     const int step = 32 * kG2Waves;
-    G2Regs<NPL> xa, xb;
+    G2Regs<RB> xa, xb;
     int mb = m_wg + 32 * wave;
     load_block(xa, mb);
-    for (; mb < m_end; mb += 2 * step) {
-        load_block(xb, mb + step);
-        consume(xa, mb);
-        load_block(xa, mb + 2 * step);
-        if (mb + step < m_end) consume(xb, mb + step);
+    if constexpr (RB == 4) {                  // one copy of the products: with two the accumulators are copied between register
+                                              // files on the way (2048 rows, 4096 features: 22.1 against 20.5 us)
+        for (; mb < m_end; mb += step) {
+            load_block(xb, mb + step);
+            consume(xa, mb);
+            xa = xb;
+        }
+    } else {
+        for (; mb < m_end; mb += 2 * step) {
+            load_block(xb, mb + step);
+            consume(xa, mb);
+            load_block(xa, mb + 2 * step);
+            if (mb + step < m_end) consume(xb, mb + step);
+        }
     }
     const bool direct = q.splits == 1;
+    const bool jfast = PV && grad_jfast(q);
     const float alpha = ga.alpha * drop.scale;
     float* tile = q.part + ((size_t)blockIdx.y * q.col_blocks + blockIdx.x) * (size_t)(R * kG2Cols);
 #pragma unroll
@@ -442,23 +468,28 @@ __global__ __launch_bounds__(64 * kG2Waves) void lora_grad_kernel(GradArgs ga) {
         __syncthreads();
         const int nj = min(16, R - 16 * b);
         for (int o = threadIdx.x; o < nj * kG2Cols; o += 64 * kG2Waves) {
-            const int jl = o >> 7, cl = o & (kG2Cols - 1), j = 16 * b + jl;
+            int jl = o >> 7, cl = o & (kG2Cols - 1);
+            if (jfast) {                                                              // nj is 8 or 16
+                jl = o & (nj - 1);
+                cl = nj == 16 ? o >> 4 : o >> 3;
+            }
+            const int j = 16 * b + jl;
             const float v = (red[0][jl][cl] + red[1][jl][cl]) + (red[2][jl][cl] + red[3][jl][cl]);
             if (direct) {
                 const int cc = blockIdx.x * kG2Cols + cl;
                 if (cc < C) q.out[(size_t)j * q.o_sr + (size_t)cc * q.o_sc] = alpha * v;
             } else {
-                tile[j * kG2Cols + cl] = v;
+                tile[jfast ? cl * R + j : j * kG2Cols + cl] = v;
             }
         }
     }
 }
 
 // Adds the `splits` partial tiles of every strip in order and writes the scaled result through the caller's strides.
-__global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga) {
+template <bool WIDE>            // R > 32
+__global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga, int R) {
     const GradProb& q = ga.p[blockIdx.y];
-    const int R = q.R;
-    const int total = q.col_blocks * R * kG2Cols;              // one split's tiles: [strip][j][column]
+    const int total = q.col_blocks * R * kG2Cols;              // one split's tiles: [strip][j][column] or [strip][column][j]
     const int t = blockIdx.x * 256 + threadIdx.x;
     if (q.splits <= 1 || t >= total) return;                   // a single split was written directly
     const float* __restrict__ part = q.part;
@@ -473,7 +504,12 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga) {
     }
     for (; s < q.splits; ++s) v += part[(size_t)s * total + t];
     const int bx = t / (R * kG2Cols), o = t - bx * (R * kG2Cols);
-    const int j = o >> 7, cc = bx * kG2Cols + (o & (kG2Cols - 1));
+    int j = o >> 7, cl = o & (kG2Cols - 1);
+    if (WIDE && grad_jfast(q)) {
+        cl = o / R;
+        j = o - cl * R;
+    }
+    const int cc = bx * kG2Cols + cl;
     if (cc < q.C) q.out[(size_t)j * q.o_sr + (size_t)cc * q.o_sc] = ga.alpha * q.drop.scale * v;
 }
 
@@ -491,11 +527,14 @@ __global__ __launch_bounds__(256) void dropout_keep_kernel(uint8_t* __restrict__
 
 // 128-column strips; enough row splits for about two workgroups per CU over both problems of a pair (their partial
 // tiles cost 2 * splits * R * C * 4 bytes of traffic); rows per workgroup a multiple of 128 (4 wavefronts x 32 rows).
+// Above 32 adapter rows at most one workgroup per CU over two problems of this size: a second round costs more than the
+// parallel rows give (512 rows, two gradients of 5120 features at rank 64: 320 workgroups 27 us, 160 of them 16), and wide
+// strips then need no partial tiles at all (13824 features, 2048 rows: 45 -> 35 us).
 struct GradPlan { int col_blocks, splits, rows_per_wg; };
-inline GradPlan plan_grad(int M, int C) {
+inline GradPlan plan_grad(int M, int C, int R) {
     GradPlan g;
     g.col_blocks = (C + kG2Cols - 1) / kG2Cols;
-    int splits = (384 + g.col_blocks - 1) / g.col_blocks;
+    int splits = R > 32 ? 128 / g.col_blocks : (384 + g.col_blocks - 1) / g.col_blocks;
     if (splits > 64) splits = 64;
     if (splits < 1) splits = 1;
     const int unit = 32 * kG2Waves;
@@ -578,16 +617,15 @@ extern "C" int q4_launch_lora_up(const void* xa, const void* w, int w_sn, int w_
 }
 
 extern "C" size_t q4_lora_grad_workspace(int M, int C, int R) {
-    const q4::GradPlan g = q4::plan_grad(M, C);
+    const q4::GradPlan g = q4::plan_grad(M, C, R);
     return g.splits == 1 ? 0 : (size_t)g.splits * g.col_blocks * R * q4::kG2Cols * sizeof(float);
 }
 
-static q4::GradProb make_grad_prob(const void* P, int p_ld, const void* in, float* out, int o_sr, int o_sc, int M, int C, int R,
+static q4::GradProb make_grad_prob(const void* P, const void* in, float* out, int o_sr, int o_sc, int M, int C, int R,
                                    float* part, const q4::DropArgs* drop = nullptr) {
-    const q4::GradPlan g = q4::plan_grad(M, C);
+    const q4::GradPlan g = q4::plan_grad(M, C, R);
     q4::GradProb q;
     q.P = reinterpret_cast<const q4::half_t*>(P);
-    q.R = R; q.p_ld = p_ld;
     q.in = reinterpret_cast<const q4::half_t*>(in);
     q.out = out;
     q.part = part;
@@ -597,38 +635,45 @@ static q4::GradProb make_grad_prob(const void* P, int p_ld, const void* in, floa
     return q;
 }
 
-static int launch_grad(const q4::GradArgs& ga, int nprob, hipStream_t stream) {
+template <int RB>
+static void launch_grad_rb(const q4::GradArgs& ga, bool any_drop, dim3 grid, int R, hipStream_t stream) {
+    const dim3 block(64 * q4::kG2Waves);
+    if (any_drop) hipLaunchKernelGGL((q4::lora_grad_kernel<true, RB>), grid, block, 0, stream, ga, R);
+    else hipLaunchKernelGGL((q4::lora_grad_kernel<false, RB>), grid, block, 0, stream, ga, R);
+}
+
+static int launch_grad(const q4::GradArgs& ga, int nprob, int R, hipStream_t stream) {
     using namespace q4;
-    int gx = 0, gy = 0, rx = 0, R = 0;
+    int gx = 0, gy = 0, rx = 0;
     bool any_split = false, any_drop = false;
     for (int i = 0; i < nprob; ++i) {
-        R = ga.p[i].R > R ? ga.p[i].R : R;
         gx = ga.p[i].col_blocks > gx ? ga.p[i].col_blocks : gx;
         gy = ga.p[i].splits > gy ? ga.p[i].splits : gy;
-        const int rb = (ga.p[i].col_blocks * ga.p[i].R * kG2Cols + 255) / 256;
+        const int rb = (ga.p[i].col_blocks * R * kG2Cols + 255) / 256;
         rx = rb > rx ? rb : rx;
         any_split = any_split || ga.p[i].splits > 1;
         any_drop = any_drop || ga.p[i].drop.thr15 != 0;
     }
-    const dim3 grid(gx, gy, nprob), block(64 * kG2Waves);
-    if (R <= 16) {
-        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 1>), grid, block, 0, stream, ga);
-        else hipLaunchKernelGGL((lora_grad_kernel<false, 1>), grid, block, 0, stream, ga);
-    } else {
-        if (any_drop) hipLaunchKernelGGL((lora_grad_kernel<true, 2>), grid, block, 0, stream, ga);
-        else hipLaunchKernelGGL((lora_grad_kernel<false, 2>), grid, block, 0, stream, ga);
+    const dim3 grid(gx, gy, nprob);
+    switch ((R + 15) / 16) {
+        case 1: launch_grad_rb<1>(ga, any_drop, grid, R, stream); break;
+        case 2: launch_grad_rb<2>(ga, any_drop, grid, R, stream); break;
+        case 3: launch_grad_rb<3>(ga, any_drop, grid, R, stream); break;
+        default: launch_grad_rb<4>(ga, any_drop, grid, R, stream); break;
     }
-    if (any_split) hipLaunchKernelGGL(lora_grad_reduce_kernel, dim3(rx, nprob), dim3(256), 0, stream, ga);
+    if (any_split && R > 32) hipLaunchKernelGGL(lora_grad_reduce_kernel<true>, dim3(rx, nprob), dim3(256), 0, stream, ga, R);
+    else if (any_split) hipLaunchKernelGGL(lora_grad_reduce_kernel<false>, dim3(rx, nprob), dim3(256), 0, stream, ga, R);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 extern "C" int q4_launch_lora_grad(const void* P, const void* in, float* out, int o_sr, int o_sc, float alpha,
                                    int M, int C, int R, const q4::DropArgs* drop, void* workspace, hipStream_t stream) {
     q4::GradArgs ga;
-    ga.p[0] = make_grad_prob(P, R, in, out, o_sr, o_sc, M, C, R, reinterpret_cast<float*>(workspace), drop);
+    ga.p[0] = make_grad_prob(P, in, out, o_sr, o_sc, M, C, R, reinterpret_cast<float*>(workspace), drop);
+    ga.p[1] = ga.p[0];
     ga.alpha = alpha;
     ga.M = M;
-    return launch_grad(ga, 1, stream);
+    return launch_grad(ga, 1, R, stream);
 }
 
 extern "C" int q4_launch_dropout_keep(uint8_t* keep, int M, int C, const q4::DropArgs* drop, hipStream_t stream) {
@@ -645,18 +690,10 @@ extern "C" int q4_launch_lora_grad_pair(const void* P1, const void* in1, float* 
                                         hipStream_t stream) {
     q4::GradArgs ga;
     float* ws = reinterpret_cast<float*>(workspace);
-    int n = 0;
-    auto add = [&](const void* P, const void* in, float* out, int o_sr, int o_sc, int C, const q4::DropArgs* drop) {
-        for (int r0 = 0; r0 < R; r0 += 32) {
-            const int rq = R - r0 < 32 ? R - r0 : 32;
-            ga.p[n++] = make_grad_prob(reinterpret_cast<const q4::half_t*>(P) + r0, R, in, out + (size_t)r0 * o_sr, o_sr, o_sc,
-                                       M, C, rq, ws, drop);
-            if (ws) ws += q4_lora_grad_workspace(M, C, rq) / sizeof(float);
-        }
-    };
-    add(P1, in1, out1, o1_sr, o1_sc, C1, drop1);                                     // the mask applies to in1 only
-    add(P2, in2, out2, o2_sr, o2_sc, C2, nullptr);
+    ga.p[0] = make_grad_prob(P1, in1, out1, o1_sr, o1_sc, M, C1, R, ws, drop1);      // the mask applies to in1 only
+    ga.p[1] = make_grad_prob(P2, in2, out2, o2_sr, o2_sc, M, C2, R,
+                             ws ? ws + q4_lora_grad_workspace(M, C1, R) / sizeof(float) : nullptr);
     ga.alpha = alpha;
     ga.M = M;
-    return launch_grad(ga, n, stream);
+    return launch_grad(ga, 2, R, stream);
 }

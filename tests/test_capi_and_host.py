@@ -93,6 +93,8 @@ def test_error_codes_and_validation_need_no_gpu():
     assert L.q4_lora_grad_workspace_bytes(64, 4096, 8) == 0            # one row block: no partial sums
     assert L.q4_lora_grad_workspace_bytes(2048, 4096, 8) == 8 * 32 * 8 * 128 * 4      # 8 row blocks x 32 strips of [R, 128] fp32
     assert L.q4_lora_grad_workspace_bytes(2048, 4096, 12) == 8 * 32 * 12 * 128 * 4
+    assert L.q4_lora_grad_workspace_bytes(2048, 4096, 64) == 4 * 32 * 64 * 128 * 4     # above rank 32: a workgroup per CU over two such gradients
+    assert L.q4_lora_grad_workspace_bytes(2048, 13824, 64) == 0            # of wide ones, whole strips
     assert L.q4_lora_grad_workspace_bytes(2048, 4096, 7) == 0 and L.q4_lora_grad_workspace_bytes(2048, 4096, 34) == 0
     assert L.q4_lora_grad_f32(fake, fake, fake, 4096, 1, 1.0, 64, 4096, 7, None, fake, 1 << 20, None) == -2    # odd R
     assert L.q4_lora_grad_f32(fake, fake, fake, 4096, 1, 1.0, 64, 4096, 34, None, fake, 1 << 20, None) == -2   # R > 32

@@ -156,9 +156,11 @@ def test_rank_r_update_of_a_few_rows(M, K, N, r, dtype, strided):
     assert not bool(guard[M].any())
 
 
-@pytest.mark.parametrize("M,C1,C2,R,p", [(2048, 4096, 4096, 64, 0.05), (300, 1408, 512, 40, 0.0), (70, 136, 5120, 56, 0.1), (1000, 512, 4096, 48, 0.0)])
+@pytest.mark.parametrize("M,C1,C2,R,p", [(2048, 4096, 4096, 64, 0.05), (300, 1408, 512, 40, 0.0), (70, 136, 5120, 56, 0.1), (1000, 512, 4096, 48, 0.0),
+                                         (1, 8, 128, 64, 0.0), (161, 16640, 13824, 64, 0.05), (4200, 1024, 264, 40, 0.05)])
 def test_lora_grad_pair_above_32_rows(M, C1, C2, R, p):
-    """Ranks that are two problems per gradient: every row of both against fp32 products (bound as for the smaller ranks)."""
+    """Three and four operands of 16 adapter rows, with and without partial sums: every row of both gradients against fp32
+    products (bound as for the smaller ranks)."""
     import torch
     from alpaca_lora_4bit_amd import quant_hip
     g = torch.Generator().manual_seed(M + C1 + R)
