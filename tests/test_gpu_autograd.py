@@ -197,6 +197,29 @@ def test_lora_layer_decode_path_matches_the_composition(oracle, rows, wdtype):
         assert not torch.equal(y2, y)
 
 
+@pytest.mark.parametrize("kind", ["transposed", "expanded", "bfloat16"])
+def test_decode_with_a_lora_b_of_another_layout_or_type(oracle, kind):
+    """lora_B views with any positive strides are read in place; expanded ones (a stride of 0) and types the kernels do not
+    read go through an fp16 copy.  All give result + lora_B(lora_A(x)) * scaling."""
+    import torch
+    from alpaca_lora_4bit_amd import models
+    K, N, r, rows = 256, 384, 8, 3
+    layer = oracle.make_layer(K, N, 128, seed=37)
+    A, B = oracle.make_lora(K, N, r, seed=37)
+    m = models.Linear4bitLt("default", K, N, 128, False, r=r, lora_alpha=16).cuda().eval()
+    _fill(m, layer)
+    m.lora_A["default"].weight.data = torch.from_numpy(A).cuda()
+    b = torch.from_numpy(B).cuda()
+    b = {"transposed": b.t().contiguous().t(), "expanded": b[:, :1].expand(N, r), "bfloat16": b.bfloat16()}[kind]
+    m.lora_B["default"].weight.data = b
+    x = torch.from_numpy(oracle.make_activations(rows, K, seed=rows)).cuda()
+    W = oracle.dequant_v2(layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"]).astype(np.float64)
+    xd = x.double().cpu().numpy()
+    with torch.no_grad():
+        y = m(x)
+    assert rel_err(y.cpu().numpy(), xd @ W + 2.0 * (xd @ A.astype(np.float64).T) @ b.double().cpu().numpy().T) <= TOL
+
+
 def test_fuse_quant_linears_matches_separate_layers(oracle):
     """gate/up (or q/k/v) concatenated along N: one launch, same numbers."""
     import torch
