@@ -63,16 +63,12 @@ struct GemmArgs {
     DropArgs drop;            // thr15 != 0: the adapter term of out[m, c] is kept only where dropout keeps (m, c)
 };
 
-// Which output tile a workgroup computes, and where in the reduction it starts.
-//  * Workgroups are handed to the 8 XCDs round-robin in dispatch order.  The ids are permuted so that one
-//    XCD owns a contiguous range of tiles, ordered in groups of `rg` row tiles: all column tiles of a group,
-//    then the next group.  The 32 workgroups an XCD runs at a time then share 2 slabs of activations and 16
-//    column tiles of W (about 4 MB each at K = 4096, what its L2 holds) instead of every row tile of a few
-//    columns: with many row tiles the activations would otherwise stream from HBM once per column tile
-//    (8192 x 4096 x 4096: 306 -> 260 us; no shape slower).
-//  * Activation rows of a power-of-two pitch (K = 4096: 8 KB) put one reduction slab of ALL rows into
-//    a single L2 channel; workgroups marching through the reduction in lockstep then queue on that one
-//    channel.  Row tile r therefore starts its (cyclic) reduction loop phase_step * r steps later.
+// Which output tile a workgroup computes.  Workgroups are handed to the 8 XCDs round-robin in dispatch order.  The ids are
+// permuted so that one XCD owns a contiguous range of tiles, ordered in groups of `rg` row tiles: all column tiles of a
+// group, then the next group.  The 32 workgroups an XCD runs at a time then share 2 slabs of activations and 16 column
+// tiles of W (about 4 MB each at K = 4096, what its L2 holds) instead of every row tile of a few columns: with many row
+// tiles the activations would otherwise stream from HBM once per column tile (8192 x 4096 x 4096: 306 -> 260 us; no shape
+// slower).
 struct TileMap {
     int tile_c, tile_r;
 };
@@ -381,9 +377,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
     constexpr int APASS = NT / 8;                     // activation rows covered by one pass of the workgroup
     constexpr int KS = BK / 16;                       // MFMA reduction sub-steps per step
 
-    const int t = threadIdx.x;
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
+    // of the first and the last part; run_layer has its own
+    const int lane0 = threadIdx.x & 63, wave0 = threadIdx.x >> 6;
+    const int wm0 = wave0 / WGN, wn0 = wave0 % WGN;
     const GemmArgs& a0 = layers[0];          // what all layers share: M, the output, the partial tiles
     const int NOUT = FWD ? a0.N : a0.K;
     const int m0 = tm.tile_r * BM;
@@ -395,7 +391,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
     float bias_v[2] = {0.f, 0.f};
     if (FWD && a0.bias) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) bias_v[j] = (float)a0.bias[c0 + wn * 64 + 32 * j + (lane & 31)];
+        for (int j = 0; j < 2; ++j) bias_v[j] = (float)a0.bias[c0 + wn0 * 64 + 32 * j + (lane0 & 31)];
     }
 
     float16_t acc[TM][2];
@@ -408,216 +404,219 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
 
     // the steps `sr` of one layer's reduction onto the accumulators
     auto run_layer = [&](const GemmArgs& a, const StepRange sr, const bool lora_here) {
-    // MULTI: opaque per layer, or everything derived from it is kept in registers over the loop (and spills)
-    int t = threadIdx.x;
-    if constexpr (MULTI) asm volatile("" : "+v"(t));
-    const int lane = t & 63, wave = t >> 6;
-    const int wm = wave / WGN, wn = wave % WGN;
-    const int RED = FWD ? a.K : a.N;
-    const int phase = (tm.tile_r * (a.phase_step & 0xff)) % sr.cnt;
-    // buffer descriptors: activations of this workgroup's rows (rows beyond M read as zero), weights
-    const rsrc_t rs_a = make_rsrc(a.a + (size_t)m0 * RED, (unsigned)rows_valid * (unsigned)RED * 2u);
-    SlabRsrc rs;
-    rs.w = make_rsrc(a.qweight, (unsigned)(a.K >> 3) * (unsigned)a.N * 4u);
-    rs.s = make_rsrc(a.scales, (unsigned)a.G * (unsigned)a.N * 2u);
-    rs.z = make_rsrc(a.qzeros, (unsigned)a.G * (unsigned)(a.N >> 3) * 4u);
+        // MULTI: opaque per layer, or everything derived from it is kept in registers over the loop (and spills)
+        int t = threadIdx.x;
+        if constexpr (MULTI) asm volatile("" : "+v"(t));
+        const int lane = t & 63, wave = t >> 6;
+        const int wm = wave / WGN, wn = wave % WGN;
+        const int RED = FWD ? a.K : a.N;
+        // Activation rows of a power-of-two pitch (K = 4096: 8 KB) put one reduction slab of ALL rows into a single L2
+        // channel; workgroups marching through the reduction in lockstep then queue on that one channel.  Row tile r
+        // therefore starts its (cyclic) reduction loop phase_step * r steps later.
+        const int phase = (tm.tile_r * (a.phase_step & 0xff)) % sr.cnt;
+        // buffer descriptors: activations of this workgroup's rows (rows beyond M read as zero), weights
+        const rsrc_t rs_a = make_rsrc(a.a + (size_t)m0 * RED, (unsigned)rows_valid * (unsigned)RED * 2u);
+        SlabRsrc rs;
+        rs.w = make_rsrc(a.qweight, (unsigned)(a.K >> 3) * (unsigned)a.N * 4u);
+        rs.s = make_rsrc(a.scales, (unsigned)a.G * (unsigned)a.N * 2u);
+        rs.z = make_rsrc(a.qzeros, (unsigned)a.G * (unsigned)(a.N >> 3) * 4u);
 
-    // activation tile: BM rows x 64 reduction entries, 16 B per thread per pass.
-    // Two register sets (areg / slab): while stage s is multiplied out of LDS, stage s+1 sits in
-    // registers waiting to be dequantized into the other LDS buffer and stage s+2 is in flight.
-    const int arow = t >> 3, acol = (t & 7) * 8;
-    const int voff_a = (arow * RED + acol) * 2;
-    const int astride = APASS * RED * 2;
-    uint4_t areg[2][NA];
-    auto load_a = [&](uint4_t* dst, int red0) {
+        // activation tile: BM rows x 64 reduction entries, 16 B per thread per pass.
+        // Two register sets (areg / slab): while stage s is multiplied out of LDS, stage s+1 sits in
+        // registers waiting to be dequantized into the other LDS buffer and stage s+2 is in flight.
+        const int arow = t >> 3, acol = (t & 7) * 8;
+        const int voff_a = (arow * RED + acol) * 2;
+        const int astride = APASS * RED * 2;
+        uint4_t areg[2][NA];
+        auto load_a = [&](uint4_t* dst, int red0) {
 #pragma unroll
-        for (int i = 0; i < NA; ++i) dst[i] = buf_load128(rs_a, voff_a + i * astride, red0 * 2);
-    };
-    auto store_a = [&](const uint4_t* src, half_t* dst) {
+            for (int i = 0; i < NA; ++i) dst[i] = buf_load128(rs_a, voff_a + i * astride, red0 * 2);
+        };
+        auto store_a = [&](const uint4_t* src, half_t* dst) {
 #pragma unroll
-        for (int i = 0; i < NA; ++i)
-            *reinterpret_cast<uint4_t*>(dst + (arow + APASS * i) * LDS_STRIDE + acol) = src[i];
-    };
+            for (int i = 0; i < NA; ++i)
+                *reinterpret_cast<uint4_t*>(dst + (arow + APASS * i) * LDS_STRIDE + acol) = src[i];
+        };
 
-    using Slab = typename std::conditional<FWD, FwdSlab<GIDX, NT, BNT>, BwdSlab<GIDX, NT, SZ == 2, BNT>>::type;
-    constexpr int NSL = Slab::kSlices;
-    Slab slab[2];
-    slab[0].init(t, a, c0);
-    slab[1].init(t, a, c0);
-    typename Slab::Prep prep;
+        using Slab = typename std::conditional<FWD, FwdSlab<GIDX, NT, BNT>, BwdSlab<GIDX, NT, SZ == 2, BNT>>::type;
+        constexpr int NSL = Slab::kSlices;
+        Slab slab[2];
+        slab[0].init(t, a, c0);
+        slab[1].init(t, a, c0);
+        typename Slab::Prep prep;
 
-    const int lr = lane & 31, lk = (lane >> 5) * 8;
-    const int a_off = (wm * WROWS + lr) * LDS_STRIDE + lk;
-    const int b_off = (wn * 64 + lr) * LDS_STRIDE + lk;
-    auto read_frags = [&](half8_t* af, half8_t* bf, const half_t* pa, const half_t* pb, int ks) {
+        const int lr = lane & 31, lk = (lane >> 5) * 8;
+        const int a_off = (wm * WROWS + lr) * LDS_STRIDE + lk;
+        const int b_off = (wn * 64 + lr) * LDS_STRIDE + lk;
+        auto read_frags = [&](half8_t* af, half8_t* bf, const half_t* pa, const half_t* pb, int ks) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-            af[i] = *reinterpret_cast<const half8_t*>(pa + a_off + 32 * i * LDS_STRIDE + 16 * ks);
+            for (int i = 0; i < TM; ++i)
+                af[i] = *reinterpret_cast<const half8_t*>(pa + a_off + 32 * i * LDS_STRIDE + 16 * ks);
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-            bf[j] = *reinterpret_cast<const half8_t*>(pb + b_off + 32 * j * LDS_STRIDE + 16 * ks);
-    };
+            for (int j = 0; j < 2; ++j)
+                bf[j] = *reinterpret_cast<const half8_t*>(pb + b_off + 32 * j * LDS_STRIDE + 16 * ks);
+        };
 
-    half8_t af[2][TM], bf[2][2];              // operand fragments, double buffered over the sub-steps
+        half8_t af[2][TM], bf[2][2];              // operand fragments, double buffered over the sub-steps
 
-    // One pipeline step, branch-free.  CUR = LDS buffer / register set of the stage being multiplied:
-    //   registers[CUR]   <- global loads of stage s+2 (clamped to the last stage: a harmless reload)
-    //   LDS[CUR^1]       <- dequantized stage s+1 from registers[CUR^1]
-    //   acc              += LDS[CUR] (stage s); on entry af[0]/bf[0] already hold sub-step 0
-    auto step = [&](int s, auto cur_tag) {
-        constexpr int CUR = decltype(cur_tag)::value;
-        constexpr int NM = TM * 2 * KS;                        // MFMAs per step
-        constexpr int BAR = NM - 3;                   // MFMA index after which the barrier sits (NM-2 .. NM-5 measured: within 3 %)
-        // Side work of a step: NL global loads (stage s+2 -> register set CUR) and NC consumer items
-        // (stage s+1: register set CUR^1 -> LDS[CUR^1]; NSL dequantization slices with the NA activation
-        // stores spread evenly among them).  One load per MFMA slot from slot 0 on (never a burst: eight
-        // wavefronts issuing ten loads each at once stall on the address unit), the consumers spread over
-        // slots 0..BAR-2 so that the last LDS stores have two MFMAs to drain before the barrier.
-        constexpr int NLS = (SZ == 1 && CUR == 1) ? Slab::kLoads - 2 : Slab::kLoads;   // SZ 1: odd steps load no scale / zero
-        constexpr int NL = NLS + NA, NC = NSL + NA;
-        constexpr int SLOTS = BAR - 1;
-        static_assert(SLOTS >= 1, "too few MFMAs per step");
-        // fragment set 0 is reloaded right after the barrier: every MFMA of sub-step KS-2 (its last
-        // user in this step) must have been issued by then
-        static_assert(BAR >= (KS - 1) * TM * 2 - 1, "barrier placed before the last use of fragment set 0");
-        const int red_next2 = red_of(s + 2, sr, phase);
-        const int red_next1 = red_of(s + 1, sr, phase);
-        const half_t* const a_cur = CUR ? sA1 : sA0;
-        const half_t* const b_cur = CUR ? sB1 : sB0;
-        half_t* const a_nxt = CUR ? sA0 : sA1;
-        half_t* const b_nxt = CUR ? sB0 : sB1;
-        static_for<0, NM>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            constexpr int ks = i / (TM * 2), r = i % (TM * 2), ti = r / 2, tj = r % 2;
-            if constexpr (r == 0 && ks + 1 < KS)
-                read_frags(af[(ks + 1) & 1], bf[(ks + 1) & 1], a_cur, b_cur, ks + 1);
-            acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks & 1][ti], bf[ks & 1][tj], acc[ti][tj], 0, 0, 0);
-            // (scale, zero) terms of the stage dequantized in this step, in the shadow of the step's first MFMA;
-            // SZ 1: the odd stage (CUR == 0) shares the group of the even stage before it
-            if constexpr (i == 0 && (SZ != 1 || CUR == 1)) prep = slab[CUR ^ 1].make_prep(c0);
-            // load l goes out in slot l*SLOTS/NL (rounded down), consumer q in slot q*SLOTS/NC (rounded up)
-            static_for<0, NL>([&](auto lc) {
-                constexpr int l = decltype(lc)::value;
-                if constexpr (l * SLOTS / NL == i) {
-                    if constexpr (l < NLS) slab[CUR].template load_part<l>(a, rs, red_next2);
-                    else areg[CUR][l - NLS] = buf_load128(rs_a, voff_a + (l - NLS) * astride, red_next2 * 2);
+        // One pipeline step, branch-free.  CUR = LDS buffer / register set of the stage being multiplied:
+        //   registers[CUR]   <- global loads of stage s+2 (clamped to the last stage: a harmless reload)
+        //   LDS[CUR^1]       <- dequantized stage s+1 from registers[CUR^1]
+        //   acc              += LDS[CUR] (stage s); on entry af[0]/bf[0] already hold sub-step 0
+        auto step = [&](int s, auto cur_tag) {
+            constexpr int CUR = decltype(cur_tag)::value;
+            constexpr int NM = TM * 2 * KS;                        // MFMAs per step
+            constexpr int BAR = NM - 3;                   // MFMA index after which the barrier sits (NM-2 .. NM-5 measured: within 3 %)
+            // Side work of a step: NL global loads (stage s+2 -> register set CUR) and NC consumer items
+            // (stage s+1: register set CUR^1 -> LDS[CUR^1]; NSL dequantization slices with the NA activation
+            // stores spread evenly among them).  One load per MFMA slot from slot 0 on (never a burst: eight
+            // wavefronts issuing ten loads each at once stall on the address unit), the consumers spread over
+            // slots 0..BAR-2 so that the last LDS stores have two MFMAs to drain before the barrier.
+            constexpr int NLS = (SZ == 1 && CUR == 1) ? Slab::kLoads - 2 : Slab::kLoads;   // SZ 1: odd steps load no scale / zero
+            constexpr int NL = NLS + NA, NC = NSL + NA;
+            constexpr int SLOTS = BAR - 1;
+            static_assert(SLOTS >= 1, "too few MFMAs per step");
+            // fragment set 0 is reloaded right after the barrier: every MFMA of sub-step KS-2 (its last
+            // user in this step) must have been issued by then
+            static_assert(BAR >= (KS - 1) * TM * 2 - 1, "barrier placed before the last use of fragment set 0");
+            const int red_next2 = red_of(s + 2, sr, phase);
+            const int red_next1 = red_of(s + 1, sr, phase);
+            const half_t* const a_cur = CUR ? sA1 : sA0;
+            const half_t* const b_cur = CUR ? sB1 : sB0;
+            half_t* const a_nxt = CUR ? sA0 : sA1;
+            half_t* const b_nxt = CUR ? sB0 : sB1;
+            static_for<0, NM>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                constexpr int ks = i / (TM * 2), r = i % (TM * 2), ti = r / 2, tj = r % 2;
+                if constexpr (r == 0 && ks + 1 < KS)
+                    read_frags(af[(ks + 1) & 1], bf[(ks + 1) & 1], a_cur, b_cur, ks + 1);
+                acc[ti][tj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks & 1][ti], bf[ks & 1][tj], acc[ti][tj], 0, 0, 0);
+                // (scale, zero) terms of the stage dequantized in this step, in the shadow of the step's first MFMA;
+                // SZ 1: the odd stage (CUR == 0) shares the group of the even stage before it
+                if constexpr (i == 0 && (SZ != 1 || CUR == 1)) prep = slab[CUR ^ 1].make_prep(c0);
+                // load l goes out in slot l*SLOTS/NL (rounded down), consumer q in slot q*SLOTS/NC (rounded up)
+                static_for<0, NL>([&](auto lc) {
+                    constexpr int l = decltype(lc)::value;
+                    if constexpr (l * SLOTS / NL == i) {
+                        if constexpr (l < NLS) slab[CUR].template load_part<l>(a, rs, red_next2);
+                        else areg[CUR][l - NLS] = buf_load128(rs_a, voff_a + (l - NLS) * astride, red_next2 * 2);
+                    }
+                });
+                constexpr int q_lo = i < SLOTS ? (i * NC + SLOTS - 1) / SLOTS : NC;
+                constexpr int q_hi = i < SLOTS ? ((i + 1) * NC + SLOTS - 1) / SLOTS : NC;
+                static_for<q_lo, q_hi>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    constexpr int na_before = q * NA / NC;                       // activation stores among items 0..q-1
+                    constexpr bool is_a = (q + 1) * NA / NC > na_before;
+                    if constexpr (is_a)
+                        *reinterpret_cast<uint4_t*>(a_nxt + (arow + APASS * na_before) * LDS_STRIDE + acol) = areg[CUR ^ 1][na_before];
+                    else
+                        slab[CUR ^ 1].template store_slice<q - na_before>(a, c0, red_next1, b_nxt, prep);
+                });
+                if constexpr (i == BAR) {
+                    // every wavefront has finished reading LDS[CUR] (the last fragments were fetched at
+                    // sub-step KS-2) and has written its share of LDS[CUR^1]
+                    __syncthreads();
+                    read_frags(af[0], bf[0], a_nxt, b_nxt, 0);
+                    if constexpr (SZ == 2) slab[CUR].fetch_tab(sz_tab, red_next2);   // for the slices of the next step
                 }
+                __builtin_amdgcn_sched_barrier(0);
             });
-            constexpr int q_lo = i < SLOTS ? (i * NC + SLOTS - 1) / SLOTS : NC;
-            constexpr int q_hi = i < SLOTS ? ((i + 1) * NC + SLOTS - 1) / SLOTS : NC;
-            static_for<q_lo, q_hi>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                constexpr int na_before = q * NA / NC;                       // activation stores among items 0..q-1
-                constexpr bool is_a = (q + 1) * NA / NC > na_before;
-                if constexpr (is_a)
-                    *reinterpret_cast<uint4_t*>(a_nxt + (arow + APASS * na_before) * LDS_STRIDE + acol) = areg[CUR ^ 1][na_before];
-                else
-                    slab[CUR ^ 1].template store_slice<q - na_before>(a, c0, red_next1, b_nxt, prep);
-            });
-            if constexpr (i == BAR) {
-                // every wavefront has finished reading LDS[CUR] (the last fragments were fetched at
-                // sub-step KS-2) and has written its share of LDS[CUR^1]
-                __syncthreads();
-                read_frags(af[0], bf[0], a_nxt, b_nxt, 0);
-                if constexpr (SZ == 2) slab[CUR].fetch_tab(sz_tab, red_next2);   // for the slices of the next step
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    };
+        };
 
-    // rank-R adapter step: activations [M, R] (columns beyond R are zero) and the adapter matrix go through the LDS
-    // buffers pa / pb like one more reduction step
-    auto stage_lora = [&](half_t* pa, half_t* pb) {
-        __syncthreads();
-        const rsrc_t rs_l = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
+        // rank-R adapter step: activations [M, R] (columns beyond R are zero) and the adapter matrix go through the LDS
+        // buffers pa / pb like one more reduction step
+        auto stage_lora = [&](half_t* pa, half_t* pb) {
+            __syncthreads();
+            const rsrc_t rs_l = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            uint4_t v = {0u, 0u, 0u, 0u};
-            if (acol < a.R) v = buf_load128(rs_l, ((arow + APASS * i) * a.R + acol) * 2, 0);
-            *reinterpret_cast<uint4_t*>(pa + (arow + APASS * i) * LDS_STRIDE + acol) = v;
-        }
-        slab[0].store_lora(a, c0, pb, t);
-        __syncthreads();
-    };
-    const bool lora_masked = lora_here && a.drop.thr15 != 0;              // uniform
+            for (int i = 0; i < NA; ++i) {
+                uint4_t v = {0u, 0u, 0u, 0u};
+                if (acol < a.R) v = buf_load128(rs_l, ((arow + APASS * i) * a.R + acol) * 2, 0);
+                *reinterpret_cast<uint4_t*>(pa + (arow + APASS * i) * LDS_STRIDE + acol) = v;
+            }
+            slab[0].store_lora(a, c0, pb, t);
+            __syncthreads();
+        };
+        const bool lora_masked = lora_here && a.drop.thr15 != 0;              // uniform
 
-    if (lora_masked) {
-        // Dropout on the adapter input: the adapter's share of out[m, c] exists only where the mask keeps (m, c).
-        // It is summed by itself, one 32 x 32 tile at a time, masked, and added to the accumulators (before
-        // anything of the main loop is live: with its loads in flight the registers would not do); the main loop adds
-        // the unmasked product on top.  The kept values carry 1/(1-p) through lb_scale.
-        stage_lora(sA1, sB1);
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float16_t term;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) term[r] = 0.f;
-                for (int ks = 0; ks < (a.R + 15) / 16; ++ks)
-                    term = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8_t*>(sA1 + a_off + 32 * i * LDS_STRIDE + 16 * ks),
-                                                                  *reinterpret_cast<const half8_t*>(sB1 + b_off + 32 * j * LDS_STRIDE + 16 * ks),
-                                                                  term, 0, 0, 0);
-                const int col = c0 + wn * 64 + 32 * j + (lane & 31);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + (lane >> 5) * 4 + (r & 3);
-                    const uint32_t w = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)col >> 1);
-                    acc[i][j][r] += ((w >> (16 * (col & 1))) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[r];
-                }
-                __builtin_amdgcn_sched_barrier(0);                // one tile's masks and term at a time
-            }
-    }
-    const int red0 = red_of(0, sr, phase), red1 = red_of(1, sr, phase);
-    // Same order as inside a step (weights, scale, zero, then the activations): the compiler's wait counts at the
-    // head of the main loop are the merge of this path and the loop's own, and with the activations of stage 1
-    // requested BEFORE its weights that merge makes every even step wait for ALL loads of the step before it.
-    slab[0].load(a, rs, c0, red0);
-    load_a(areg[0], red0);
-    slab[1].load(a, rs, c0, red1);
-    load_a(areg[1], red1);
-    if constexpr (SZ == 2) {
-        // table of the tile's group: per unit of 8 columns one 16-byte load of scales and one zero word in, four
-        // (s_a, s_b, zero_a, zero_b) entries out
-        const int g = c0 / a.groupsize;
-        for (int u = t; u < (a.N >> 3); u += NT) {
-            const uint4_t s8 = buf_load128(rs.s, u * 16, g * a.N * 2);
-            const uint32_t z8 = buf_load32(rs.z, u * 4, g * (a.N >> 3) * 4);
-            const uint32_t sw[4] = {s8.x, s8.y, s8.z, s8.w};
-            uint32_t e[8];
-#pragma unroll
-            for (int pp = 0; pp < 4; ++pp) {
-                e[2 * pp] = sw[pp];
-                e[2 * pp + 1] = as_u32(zero_term(as_half2(sw[pp]), (z8 >> (8 * pp)) & 0xFu, (z8 >> (8 * pp + 4)) & 0xFu));
-            }
-            *reinterpret_cast<uint4_t*>(sz_tab + u * 32) = uint4_t{e[0], e[1], e[2], e[3]};
-            *reinterpret_cast<uint4_t*>(sz_tab + u * 32 + 16) = uint4_t{e[4], e[5], e[6], e[7]};
-        }
-        __syncthreads();
-        slab[0].fetch_tab(sz_tab, red0);
-        slab[1].fetch_tab(sz_tab, red1);
-    }
-    store_a(areg[0], sA0);
-    prep = slab[0].make_prep(c0);
-    static_for<0, NSL>([&](auto jc) { slab[0].template store_slice<decltype(jc)::value>(a, c0, red0, sB0, prep); });
-    __syncthreads();
-    read_frags(af[0], bf[0], sA0, sB0, 0);
-    for (int s = 0; s + 1 < sr.cnt; s += 2) {
-        step(s, std::integral_constant<int, 0>{});
-        step(s + 1, std::integral_constant<int, 1>{});
-    }
-    if (sr.cnt & 1) step(sr.cnt - 1, std::integral_constant<int, 0>{});   // an even number of steps precedes it: LDS[0]
-    if (lora_here && !lora_masked) {
-        stage_lora(sA0, sB0);
-        for (int ks = 0; ks < (a.R + 15) / 16; ++ks) {
-            read_frags(af[0], bf[0], sA0, sB0, ks);
+        if (lora_masked) {
+            // Dropout on the adapter input: the adapter's share of out[m, c] exists only where the mask keeps (m, c).
+            // It is summed by itself, one 32 x 32 tile at a time, masked, and added to the accumulators (before
+            // anything of the main loop is live: with its loads in flight the registers would not do); the main loop adds
+            // the unmasked product on top.  The kept values carry 1/(1-p) through lb_scale.
+            stage_lora(sA1, sB1);
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0][i], bf[0][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) {
+                    float16_t term;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) term[r] = 0.f;
+                    for (int ks = 0; ks < (a.R + 15) / 16; ++ks)
+                        term = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8_t*>(sA1 + a_off + 32 * i * LDS_STRIDE + 16 * ks),
+                                                                      *reinterpret_cast<const half8_t*>(sB1 + b_off + 32 * j * LDS_STRIDE + 16 * ks),
+                                                                      term, 0, 0, 0);
+                    const int col = c0 + wn * 64 + 32 * j + (lane & 31);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + (lane >> 5) * 4 + (r & 3);
+                        const uint32_t w = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)col >> 1);
+                        acc[i][j][r] += ((w >> (16 * (col & 1))) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[r];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);                // one tile's masks and term at a time
+                }
         }
-    }
+        const int red0 = red_of(0, sr, phase), red1 = red_of(1, sr, phase);
+        // Same order as inside a step (weights, scale, zero, then the activations): the compiler's wait counts at the
+        // head of the main loop are the merge of this path and the loop's own, and with the activations of stage 1
+        // requested BEFORE its weights that merge makes every even step wait for ALL loads of the step before it.
+        slab[0].load(a, rs, c0, red0);
+        load_a(areg[0], red0);
+        slab[1].load(a, rs, c0, red1);
+        load_a(areg[1], red1);
+        if constexpr (SZ == 2) {
+            // table of the tile's group: per unit of 8 columns one 16-byte load of scales and one zero word in, four
+            // (s_a, s_b, zero_a, zero_b) entries out
+            const int g = c0 / a.groupsize;
+            for (int u = t; u < (a.N >> 3); u += NT) {
+                const uint4_t s8 = buf_load128(rs.s, u * 16, g * a.N * 2);
+                const uint32_t z8 = buf_load32(rs.z, u * 4, g * (a.N >> 3) * 4);
+                const uint32_t sw[4] = {s8.x, s8.y, s8.z, s8.w};
+                uint32_t e[8];
+#pragma unroll
+                for (int pp = 0; pp < 4; ++pp) {
+                    e[2 * pp] = sw[pp];
+                    e[2 * pp + 1] = as_u32(zero_term(as_half2(sw[pp]), (z8 >> (8 * pp)) & 0xFu, (z8 >> (8 * pp + 4)) & 0xFu));
+                }
+                *reinterpret_cast<uint4_t*>(sz_tab + u * 32) = uint4_t{e[0], e[1], e[2], e[3]};
+                *reinterpret_cast<uint4_t*>(sz_tab + u * 32 + 16) = uint4_t{e[4], e[5], e[6], e[7]};
+            }
+            __syncthreads();
+            slab[0].fetch_tab(sz_tab, red0);
+            slab[1].fetch_tab(sz_tab, red1);
+        }
+        store_a(areg[0], sA0);
+        prep = slab[0].make_prep(c0);
+        static_for<0, NSL>([&](auto jc) { slab[0].template store_slice<decltype(jc)::value>(a, c0, red0, sB0, prep); });
+        __syncthreads();
+        read_frags(af[0], bf[0], sA0, sB0, 0);
+        for (int s = 0; s + 1 < sr.cnt; s += 2) {
+            step(s, std::integral_constant<int, 0>{});
+            step(s + 1, std::integral_constant<int, 1>{});
+        }
+        if (sr.cnt & 1) step(sr.cnt - 1, std::integral_constant<int, 0>{});   // an even number of steps precedes it: LDS[0]
+        if (lora_here && !lora_masked) {
+            stage_lora(sA0, sB0);
+            for (int ks = 0; ks < (a.R + 15) / 16; ++ks) {
+                read_frags(af[0], bf[0], sA0, sB0, ks);
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0][i], bf[0][j], acc[i][j], 0, 0, 0);
+            }
+        }
     };  // run_layer
 
     if constexpr (MULTI) {
@@ -640,7 +639,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
     // epilogue: acc[i][j][r] is row 8*(r/4) + 4*(lane/32) + r%4, column lane%32 of its 32x32 tile.
     // Each wavefront transposes one 32 x 64 block at a time through its own 4.5 KB of LDS
     // (row stride 72 halves) and writes it as 16-byte pieces: 8 lanes cover one 128-byte row segment.
-    const int lc = lane & 31, lrow = (lane >> 5) * 4;
+    const int lc = lane0 & 31, lrow = (lane0 >> 5) * 4;
     if (nsplit > 1) {
         // split-K: fp32 partial sums straight from the accumulators (32 lanes cover one 128-byte row segment);
         // the bias rides with split 0, the reduction kernel adds the splits in order and rounds once
@@ -649,19 +648,19 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int col = c0 + wn * 64 + 32 * j + lc;
+                const int col = c0 + wn0 * 64 + 32 * j + lc;
                 const float bv = zsplit == 0 ? bias_v[j] : 0.f;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * WROWS + 32 * i + 8 * (r >> 2) + lrow + (r & 3);
+                    const int m = m0 + wm0 * WROWS + 32 * i + 8 * (r >> 2) + lrow + (r & 3);
                     if (m < a0.M) pz[(size_t)m * a0.part_cols + col] = acc[i][j][r] + bv;
                 }
             }
         return;
     }
     __syncthreads();
-    half_t* stage = sA0 + wave * (32 * LDS_STRIDE);
-    const int orow = lane >> 3, ocol = (lane & 7) * 8;
+    half_t* stage = sA0 + wave0 * (32 * LDS_STRIDE);
+    const int orow = lane0 >> 3, ocol = (lane0 & 7) * 8;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -679,9 +678,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs* layers, const int nlay
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             const int rr = orow + 8 * p;
-            const int m = m0 + wm * WROWS + 32 * i + rr;
+            const int m = m0 + wm0 * WROWS + 32 * i + rr;
             const uint4_t v = *reinterpret_cast<const uint4_t*>(stage + rr * LDS_STRIDE + ocol);
-            if (m < a0.M) *reinterpret_cast<uint4_t*>(a0.out + (size_t)m * NOUT + c0 + wn * 64 + ocol) = v;
+            if (m < a0.M) *reinterpret_cast<uint4_t*>(a0.out + (size_t)m * NOUT + c0 + wn0 * 64 + ocol) = v;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -799,7 +798,7 @@ static void launch_tail(GemmArgs a, int nout, int tail_cols, int tail_splits, hi
 }
 
 // 256 x 256 tiles (8 wavefronts of 128 x 64): half the activation traffic and 30 % less LDS traffic per MFMA than the
-// 256 x 128 tile; for outputs with enough such tiles to fill the CUs.  No split, no second launch; the tile buffers
+// 256 x 128 tile; for outputs with enough such tiles to fill the CUs.  Their reduction is not split; the tile buffers
 // take 144 KB of LDS, so the grad-input kernel keeps its per-step scale / zero loads.
 // tail_cols > 0: the last tail_cols tiles of 128 columns are left to a second launch of 256 x 128 tiles, with the
 // reduction split tail_splits ways (see wide_tail).
@@ -841,7 +840,7 @@ static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout
     switch (p.cfg) {
         case 0: return launch_gemm<128, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 128 x 128, 4 wavefronts of 64 x 64
         case 1: return launch_gemm<256, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 256 x 128, 4 wavefronts of 128 x 64
-        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, p.tail_cols, p.tail_splits, stream);                        // 256 x 256, 8 wavefronts of 128 x 64
+        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, p.tail_cols, p.tail_splits, stream);   // 256 x 256, 8 wavefronts of 128 x 64
         default: return launch_gemm<256, 4, FWD, GIDX>(a, nout, p.splits, p.tail_cols, p.tail_splits, stream);   // 256 x 128, 8 wavefronts of 64 x 64
     }
 }

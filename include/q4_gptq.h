@@ -262,14 +262,17 @@ Q4_API int q4_gemm_bwd_dx_f16(const void *dy, const int32_t *qweight, const int3
                        void *workspace, size_t workspace_bytes, void *stream);
 
 /* The two GEMMs for 2..4 layers that share M, K and the group size (q|k|v, gate|up of a decoder block), each on its
- * own tensors, in ONE launch.  Sequential groups only (no g_idx), every |scale| < 64, M > 128; otherwise, and for
- * shapes with too few tiles to fill the GPU, Q4_ERR_BAD_SHAPE: use the per-layer entry points.
+ * own tensors, in one product launch or two (whole rounds of the GPU, then the columns left over).  Sequential groups
+ * only (no g_idx), every |scale| < 64, M > 128; otherwise, and for a forward of fewer than 96 tiles of 256 x 128 outputs
+ * over all layers, Q4_ERR_BAD_SHAPE: use the per-layer entry points.
  *   q4_gemm_grouped_fwd_f16:     y_i [M, N_i] = x @ W_i (+ bias_i) (+ lb_scale_i * la_i @ Lb_i), la_i = xa_i [M, R_i];
  *                                act of every layer = x.  No workspace.
  *   q4_gemm_grouped_bwd_dx_f16:  dx [M, K] = sum_i ( dy_i @ W_i^T + mask_i * lb_scale_i * la_i @ Lb_i ), act = dy_i
  *                                [M, N_i], la_i = dyb_i [M, R_i], Lb_i = lora_A_i [R_i, K], mask_i the dropout mask of
- *                                drop_i (NULL: none).  The layers are the shares of one split reduction: fp32 partial
- *                                tiles in `workspace` (q4_gemm_grouped_workspace_bytes), added in a fixed order.
+ *                                drop_i (NULL: none).  One reduction over the layers' columns one after the other,
+ *                                summed in fp32; where the tiles are few it is split, with fp32 partial tiles in
+ *                                `workspace` (q4_gemm_grouped_workspace_bytes; 0: none, it may be NULL) that another
+ *                                launch adds in a fixed order.
  * They replace the per-projection recons + torch.matmul calls (matmul_utils_4bit.py:114-127) that the reference fuses
  * by concatenating the packed tensors (model_attn_mlp_patch.py:88-100, 180-190), and for the grad-input also the
  * additions with which autograd sums the per-projection results.  Lb_i[r, c] = lb[r*lb_r + c*lb_c], fp16 or fp32. */
@@ -286,7 +289,8 @@ typedef struct {
     int N;
     const q4_dropout_t *drop;     /* grad-input only */
 } q4_gemm_layer_t;
-/* 1 when the two entry points below take this shape (enough tiles for one launch), 0 otherwise. */
+/* 1 when the entry point takes this shape, 0 otherwise; not whether it is the faster choice.  A forward of at most 256 rows
+ * without adapters is often faster layer by layer where q4_gemm_route says Q4_ROUTE_STREAM for every layer. */
 Q4_API int q4_gemm_grouped_applicable(int fwd, int n_layers, int M, int K, const int *N);
 Q4_API size_t q4_gemm_grouped_workspace_bytes(int fwd, int n_layers, int M, int K, const int *N);
 Q4_API int q4_gemm_grouped_fwd_f16(const q4_gemm_layer_t *layers, int n_layers, int groupsize, int M, int K, void *stream);

@@ -17,7 +17,7 @@ def _t(a):
 @pytest.mark.parametrize("M,K,Ns,gs,lora", [
     (1024, 4096, (4096, 4096, 4096), 128, (8, 0, 8)),          # q|k|v of config 4: 192 wide tiles, adapters on q and v
     (1024, 4096, (11008, 11008), 128, (0, 0)),                 # gate|up of config 4
-    (600, 1024, (4096, 2048, 1024, 2048), 256, (16, 8, 0, 0)),  # four layers, ragged rows, one row tile's worth of narrow tiles in eight shares
+    (600, 1024, (4096, 2048, 1024, 2048), 256, (16, 8, 0, 0)),  # four layers, ragged rows, 24 narrow tiles in eight shares, some across layers
     (2048, 512, (4096, 4096), 64, (0, 8)),                     # groups of 64 rows
 ])
 def test_grouped_forward_and_grad_input(oracle, M, K, Ns, gs, lora):
@@ -295,7 +295,7 @@ def test_grouped_forward_remainder_launch(oracle):
 @pytest.mark.parametrize("M,red,nout,gs,act,tail_cols,splits", [
     (2000, 512, 11008, 128, False, 22, 1),      # 8 x 43 wide tiles: 11 columns left, one round of narrow tiles
     (2000, 512, 11008, 64, False, 22, 1),
-    (4500, 1536, 4096, 128, True, 4, 3),        # 18 x 16: 2 columns left (36 tiles), reduction split
+    (4500, 1536, 4096, 128, True, 4, 3),        # 18 x 32 narrow tiles (indexed groups): 4 columns left, reduction split
     (4096, 2048, 5120, 256, False, 8, 2),       # 16 x 20: 4 columns left (64 tiles)
 ])
 def test_wide_tiles_with_a_remainder_launch(oracle, M, red, nout, gs, act, tail_cols, splits):
