@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restri
 // tiles a wavefront).  As two problems of half the rank, each reading `in` and leaving partial tiles, both gradients of
 // 2048 rows of 13824 and 13824 features took 72 us at rank 64 (77.5 with dropout) where library products take 44; now 31
 // with dropout; 4096 x 4096 features 33.8 -> 20.5, 512 rows of 5120 and 13824 39 -> 17.  One block of 64 rows alone
-// takes longer (7.7 -> 10 us).
+// takes longer (7.8 -> 8.8 us).
 constexpr int kG2Waves = 4, kG2Cols = 128, kG2PadRows = 40;
 
 // One or two gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
@@ -316,7 +316,7 @@ struct GradArgs {
 };
 
 // Above 32 adapter rows a result whose adapter rows lie side by side (lora_B.weight's layout) goes out along them, partial
-// tiles included: 64-byte pieces instead of single words (64 rows of 4096 features at rank 64: 11.3 -> 10.6 us).
+// tiles included: 64-byte pieces instead of single words (64 rows of 4096 features at rank 64: 0.7 us).
 __device__ __forceinline__ bool grad_jfast(const GradProb& q) { return q.o_sr < q.o_sc; }
 
 template <int RB>
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(64 * kG2Waves, RB == 3 ? 2 : 1) void lora_grad_kern
         }
         __syncthreads();
         const int nj = min(16, R - 16 * b);
-        for (int o = threadIdx.x; o < nj * kG2Cols; o += 64 * kG2Waves) {
+        auto write = [&](int o) {
             int jl = o >> 7, cl = o & (kG2Cols - 1);
             if (jfast) {                                                              // nj is 8 or 16
                 jl = o & (nj - 1);
@@ -481,6 +481,14 @@ __global__ __launch_bounds__(64 * kG2Waves, RB == 3 ? 2 : 1) void lora_grad_kern
             } else {
                 tile[jfast ? cl * R + j : j * kG2Cols + cl] = v;
             }
+        };
+        if constexpr (PV) {                    // nj is 8 or 16; four LDS sums under way at a time: 0.3-0.5 us of 7 to 16
+            for (int o = threadIdx.x; o < nj * kG2Cols; o += 4 * 64 * kG2Waves) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) write(o + u * 64 * kG2Waves);
+            }
+        } else {
+            for (int o = threadIdx.x; o < nj * kG2Cols; o += 64 * kG2Waves) write(o);
         }
     }
 }
