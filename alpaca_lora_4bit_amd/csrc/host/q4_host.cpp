@@ -497,7 +497,11 @@ void lora_update(const at::Tensor& x, const at::Tensor& a, const at::Tensor& b, 
     TORCH_CHECK_VALUE(b.dim() == 2 && b.size(0) == y.size(1) && b.size(1) == a.size(0) && b.device() == y.device(),
                       "b must be an [N, R] view on the same device");
     TORCH_CHECK_VALUE(b.scalar_type() == at::kHalf || b.scalar_type() == at::kFloat, "b must be float16 or float32");
-    TORCH_CHECK_VALUE(b.stride(0) >= 1 && b.stride(1) >= 1, "b must have positive strides");
+    if (b.stride(0) < 1 || b.stride(1) < 1 || b.stride(0) > INT32_MAX || b.stride(1) > INT32_MAX) {     // an expanded view
+        const at::Tensor copy = at::empty({b.size(0), b.size(1)}, b.options());
+        copy.copy_(b);
+        return lora_update(x, a, copy, y, alpha);
+    }
     const at::Tensor xa = lora_down(x, a, c10::nullopt);
     if (y.size(0) == 0) return;
     Launch L(y.device());

@@ -174,11 +174,10 @@ class Linear4bitLt(Autograd4bitQuantLinear, LoraLayer):
                 result = Autograd4bitQuantLinear.forward(self, x)
                 a, b = self.lora_A[name].weight, self.lora_B[name].weight
                 x2, out2 = x.reshape(-1, x.shape[-1]).to(torch.float16).contiguous(), result.view(-1, result.shape[-1])
-                if out2.dtype == torch.float16 and b.dtype in (torch.float16, torch.float32) and \
-                        0 < min(b.stride()) and max(b.stride()) < 1 << 31:
+                if out2.dtype == torch.float16 and b.dtype in (torch.float16, torch.float32):
                     autograd_4bit.quant_hip.lora_update(x2, a, b, out2, float(self.scaling[name]))
                     return result
-                # other types of lora_B, expanded ones and float32 results: through an fp16 copy of lora_B
+                # other types of lora_B and float32 results: through an fp16 copy of lora_B
                 xa = autograd_4bit.quant_hip.lora_down(x2, a)
                 if out2.dtype == torch.float16:
                     out2.addmm_(xa, self._half_lora_b(name), alpha=float(self.scaling[name]))

@@ -863,7 +863,7 @@ def lora_down(inp, w, dropout=None):
 
 def lora_update(x, a, b, y, alpha):
     """y fp16 [M, N] += alpha * (x @ a^T) @ b^T in place, for x fp16 [M, K], a = lora_A.weight [R, K] and
-    b = lora_B.weight [N, R] (fp16/fp32, any positive strides): the adapter of a few rows in two launches (models.py:66).
+    b = lora_B.weight [N, R] (fp16/fp32, any view; read in place unless a stride is 0): the adapter of a few rows in two launches (models.py:66).
     x @ a^T is rounded to fp16, the update once, onto y."""
     if _host is not None:
         return _host.lora_update(x, a, b, y, alpha)
@@ -872,7 +872,8 @@ def lora_update(x, a, b, y, alpha):
     _require(b.dim() == 2 and b.shape == (y.shape[1], a.shape[0]) and b.device == y.device, "b must be an [N, R] view on the same device")
     f32 = _adapter_dtype_flag(b, "b")
     sn, sr = b.stride()
-    _require(sn >= 1 and sr >= 1, "b must have positive strides")
+    if not (1 <= sn < 1 << 31 and 1 <= sr < 1 << 31):        # an expanded view
+        return lora_update(x, a, torch.empty(b.shape, dtype=b.dtype, device=b.device).copy_(b), y, alpha)
     xa = lora_down(x, a)
     if y.shape[0] == 0:
         return

@@ -200,7 +200,7 @@ def test_lora_layer_decode_path_matches_the_composition(oracle, rows, wdtype):
 @pytest.mark.parametrize("kind", ["transposed", "expanded", "bfloat16"])
 def test_decode_with_a_lora_b_of_another_layout_or_type(oracle, kind):
     """lora_B views with any positive strides are read in place; expanded ones (a stride of 0) and types the kernels do not
-    read go through an fp16 copy.  All give result + lora_B(lora_A(x)) * scaling."""
+    read go through a copy.  All give result + lora_B(lora_A(x)) * scaling."""
     import torch
     from alpaca_lora_4bit_amd import models
     K, N, r, rows = 256, 384, 8, 3
