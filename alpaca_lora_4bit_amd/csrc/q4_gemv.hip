@@ -1,11 +1,12 @@
 // Weight-streaming products for few activation rows:  y[M,N] = x[M,K] @ W   (HBM-bound).
-//   gemv_seq_kernel       1 <= M <= 16, sequential groups (also the v1 layout: one scale / zero per column)
+//   gemv_stream_kernel    1 <= M <= 16, sequential groups of 32, 64 or a multiple of 128 rows, K % 128 == 0 (q4_gemv_stream.hpp)
+//   gemv_seq_kernel       1 <= M <= 16, other sequential groups (also the v1 layout: one scale / zero per column)
 //   gemv_seq_perm_kernel  1 <= M <= 4, act-order layer with rows sorted by group: gathers x through the permutation
 //   gemv_gidx_kernel      1 <= M <= 16, act-order with per-row groups read through g_idx
 //   skinny_seq_kernel     17 <= M <= 64, sequential groups (fp32 partial rows + ordered reduction)
 //   skinny_dx_kernel      17 <= M <= 48, the transposed product dy @ W^T (grad-input), sequential groups
 //
-// Work split.  A workgroup owns a strip of 64 columns; its W wavefronts (W = blockDim.x / 64)
+// Work split of the kernels below but the first.  A workgroup owns a strip of 64 columns; its W wavefronts (W = blockDim.x / 64)
 // take consecutive chunks of 32*NSTEP rows, and gridDim.y workgroups share one strip when K is
 // longer than W chunks.  Lane l of a wavefront (kk = l / 16, c = l % 16) reads, per step of 32
 // rows, ONE 128-bit vector qweight[row/8 + kk, n0 + 4c .. 4c+3]: four packed words = 8
@@ -42,11 +43,13 @@
 #include <type_traits>
 
 #include "q4_gemv_core.hpp"
+#include "q4_gemv_plan.hpp"
+#include "q4_gemv_stream.hpp"
 
 namespace q4 {
 
 template <int NSTEP, int GSTEPS, bool V1 = false>
-__global__ __launch_bounds__(NSTEP >= 16 ? 512 : 1024) void gemv_seq_kernel(GemvArgs a) {
+__global__ __launch_bounds__(1024) void gemv_seq_kernel(GemvArgs a) {
     gemv_seq_body<NSTEP, GSTEPS, V1>(a, blockIdx.x * kColsPerWave, blockIdx.y, gridDim.y);
 }
 
@@ -59,6 +62,126 @@ struct GemvGroupArgs {
     GemvArgs layer[kMaxGroup];
     int strip_end[kMaxGroup];                     // running total of 64-column strips; unused entries = INT_MAX
 };
+
+// Chunks of 128 rows in 1, 2 or 4 groups: every launch whose K is a multiple of 128 and whose group size is 32, 64 or a multiple
+// of 128 (gemv_stream_takes).  Grid: strips of 64 columns of all layers x splits of the reduction, nb blocks of 8 chunks each.
+// A block is summed as the eight-wavefront kernels do, ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)), and blocks are added as
+// fixed-point integers, so a product has the same bits alone, in a group, however it is split, and in q4_mlp.hip.  Longer
+// shares leave the block sums of the wavefronts in LDS ([nb][wavefront][M][64] fp32 behind the tiles) and finish once.
+// GROUP: several layers, else one whose arguments sit where the first load finds them (0.2 us of a 4096 -> 4096 layer).
+struct StreamSplit {
+    uint32_t group_inv;
+    int nb, blocks;                               // blocks per workgroup, of the whole reduction
+};
+struct GemvStreamArgs {
+    GemvArgs layer;
+    StreamSplit split;
+};
+struct GemvStreamGroupArgs {
+    GemvGroupArgs g;
+    StreamSplit split;
+};
+
+// EB outputs per thread (EB * 256 >= M * 64, its own instantiation each: a launch pays for every line of code it passes over):
+// the reads, and the atomics, of all of them are under way together.
+template <bool ONE, int EB>
+__device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* slab, int n0, int nb, int blocks, int S) {
+    constexpr int T = 64 * kStreamWaves;
+    const int M = a.M, total = M * 64, ws = M << 6;              // ws: from one wavefront's sums to the next's
+    if (EB == 1 && (int)threadIdx.x >= total) return;
+    unsigned long long add[EB], old[EB];
+    float direct[EB];
+#pragma unroll
+    for (int i = 0; i < EB; ++i) add[i] = 1ull << 56;
+    constexpr int U = ONE ? 1 : 2;                               // blocks read together
+    for (int b = 0; b < nb; b += U) {
+        float p[EB][U][4];
+#pragma unroll
+        for (int i = 0; i < EB; ++i)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    p[i][u][w] = slab[((ONE ? 0 : min(b + u, nb - 1)) * kStreamWaves + w) * ws + (EB == 1 ? (int)threadIdx.x : min((int)threadIdx.x + i * T, total - 1))];
+#pragma unroll
+        for (int i = 0; i < EB; ++i)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float v = (p[i][u][0] + p[i][u][1]) + (p[i][u][2] + p[i][u][3]);
+                if (ONE) direct[i] = v;
+                if (u == 0 || b + u < nb) add[i] += fixed_biased(v);
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < EB; ++i) {
+        const int e = threadIdx.x + i * T;
+        old[i] = 0;
+        if (S > 1 && e < total)
+            old[i] = __hip_atomic_fetch_add(a.acc64 + (size_t)(e >> 6) * a.N + n0 + (e & 63), add[i], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // every reply first, then the stores: a reply that is looked at behind a store waits for that store as well
+    bool last[EB];
+    float out[EB];
+#pragma unroll
+    for (int i = 0; i < EB; ++i) {
+        const int e = threadIdx.x + i * T;
+        last[i] = e < total && (old[i] >> 56) == (unsigned long long)(S - 1);      // last of the S workgroups of the strip
+        out[i] = ONE && S == 1 ? direct[i] : fixed_sum(old[i] + add[i], blocks);
+        if (a.accumulate && last[i]) out[i] += (float)a.y[(size_t)(e >> 6) * a.N + n0 + (e & 63)];
+    }
+#pragma unroll
+    for (int i = 0; i < EB; ++i) {
+        const int e = threadIdx.x + i * T;
+        const size_t at = (size_t)(e >> 6) * a.N + n0 + (e & 63);
+        if (last[i]) {
+            a.y[at] = (half_t)out[i];
+            if (S > 1) __hip_atomic_store(a.acc64 + at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+template <int NG, bool ONE, int EB>
+__device__ __forceinline__ void gemv_stream_body(const GemvArgs& a, const StreamSplit& sa, int n0) {
+    extern __shared__ float red[];
+    const int M = a.M;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kk = lane >> 4, c = lane & 15;
+    const int block0 = blockIdx.y * sa.nb, nb = ONE ? 1 : min(sa.nb, sa.blocks - block0);
+    float* const slab = ONE ? red : red + kStreamLds / 4;         // ONE: over the tiles, behind a barrier
+    float4_t yacc[1][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) yacc[0][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const GemvArgs* const layers[1] = {&a};
+    stream_blocks<1, NG, ONE>(layers, sa.group_inv, n0, block0, nb, min(a.K >> 7, (block0 + nb) * 2 * kStreamWaves),
+                              reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc, [&](int b) {
+        if constexpr (ONE) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = 4 * kk + r;
+            if (m < M)
+                *reinterpret_cast<float4_t*>(slab + (((b * kStreamWaves + wave) * M + m) << 6) + 4 * c) =
+                    float4_t{yacc[0][0][r], yacc[0][1][r], yacc[0][2][r], yacc[0][3][r]};
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) yacc[0][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    });
+    __syncthreads();
+    stream_finish<ONE, EB>(a, slab, n0, nb, sa.blocks, gridDim.y);
+}
+
+template <int NG, bool ONE, int EB>
+__global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_kernel(GemvStreamArgs sa) {
+    gemv_stream_body<NG, ONE, EB>(sa.layer, sa.split, blockIdx.x * kColsPerWave);
+}
+template <int NG, bool ONE, int EB>
+__global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_group_kernel(GemvStreamGroupArgs sa) {
+    const GemvGroupArgs& g = sa.g;
+    const int bx = blockIdx.x;
+    const int li = (bx >= g.strip_end[0]) + (bx >= g.strip_end[1]) + (bx >= g.strip_end[2]);      // uniform
+    gemv_stream_body<NG, ONE, EB>(g.layer[li], sa.split, (bx - (li == 0 ? 0 : g.strip_end[li - 1])) * kColsPerWave);
+}
 
 template <int NSTEP, int GSTEPS>
 __global__ __launch_bounds__(1024) void gemv_seq_group_kernel(GemvGroupArgs g) {
@@ -1004,10 +1127,42 @@ static void launch_seq(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds,
     switch (p.gsteps) {
         case 0: hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0>), grid, block, lds, stream, a); break;
         case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 1>), grid, block, lds, stream, a); break;
-        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 2>), grid, block, lds, stream, a); break;
-        case 4: if constexpr (NSTEP > 4) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 4>), grid, block, lds, stream, a); break;
-        case 8: if constexpr (NSTEP > 8) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 8>), grid, block, lds, stream, a); break;
     }
+}
+
+static bool gemv_stream_takes(int K, int groupsize) {
+    return K % 128 == 0 && (groupsize % 128 == 0 || groupsize == 64 || groupsize == 32);
+}
+template <int NG, bool ONE, int EB>
+static void launch_stream_eb(const q4::GemvGroupArgs& g, int n, const q4::StreamSplit& split, dim3 grid, size_t lds, hipStream_t stream) {
+    using namespace q4;
+    const dim3 block(64 * kStreamWaves);
+    if (n == 1) hipLaunchKernelGGL((gemv_stream_kernel<NG, ONE, EB>), grid, block, lds, stream, GemvStreamArgs{g.layer[0], split});
+    else hipLaunchKernelGGL((gemv_stream_group_kernel<NG, ONE, EB>), grid, block, lds, stream, GemvStreamGroupArgs{g, split});
+}
+template <int NG, bool ONE>
+static void launch_stream_one(const q4::GemvGroupArgs& g, int n, const q4::StreamSplit& split, dim3 grid, size_t lds, hipStream_t stream) {
+    const int M = g.layer[0].M;
+    if (M <= 4) launch_stream_eb<NG, ONE, 1>(g, n, split, grid, lds, stream);
+    else if (M <= 8) launch_stream_eb<NG, ONE, 2>(g, n, split, grid, lds, stream);
+    else launch_stream_eb<NG, ONE, 4>(g, n, split, grid, lds, stream);
+}
+// n layers (g.layer[0] .. [n - 1]) of `strips` strips in all.  Groups of 64 and 32 rows have one block per workgroup
+// (plan_stream_blocks) but for reductions beyond the arrival count.
+static int launch_stream(const q4::GemvGroupArgs& g, int n, int strips, hipStream_t stream) {
+    using namespace q4;
+    const GemvArgs& a = g.layer[0];
+    StreamSplit sp;
+    sp.group_inv = stream_group_inv(a.groupsize);
+    sp.blocks = (a.K + 1023) / 1024;
+    sp.nb = plan_stream_blocks(a.M, sp.blocks, strips, a.groupsize);
+    const dim3 grid(strips, (sp.blocks + sp.nb - 1) / sp.nb);
+    const size_t lds = kStreamLds + (sp.nb == 1 ? 0 : stream_slab_bytes(a.M, sp.nb));
+    const bool one = sp.nb == 1;
+    if (a.groupsize == 32) one ? launch_stream_one<4, true>(g, n, sp, grid, lds, stream) : launch_stream_one<4, false>(g, n, sp, grid, lds, stream);
+    else if (a.groupsize == 64) one ? launch_stream_one<2, true>(g, n, sp, grid, lds, stream) : launch_stream_one<2, false>(g, n, sp, grid, lds, stream);
+    else one ? launch_stream_one<1, true>(g, n, sp, grid, lds, stream) : launch_stream_one<1, false>(g, n, sp, grid, lds, stream);
+    return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
 // Shapes q4_gemv_sorted_f16 takes: up to 4 rows whose activations (plus 4 KB per row of staging) fit in 64 KB of LDS.
@@ -1046,6 +1201,11 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
     a.v1_zeros = nullptr;
 
     const bool seq = (g_idx == nullptr);
+    if (seq && !perm && gemv_stream_takes(K, groupsize)) {
+        GemvGroupArgs g;
+        g.layer[0] = a;
+        return launch_stream(g, 1, N / kColsPerWave, stream);
+    }
     const GemvPlan p = plan_gemv(K, N, groupsize, seq, 4);
     const dim3 grid(N / kColsPerWave, p.splits);
     const dim3 block(64 * p.waves);
@@ -1061,10 +1221,7 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
         }
     } else if (seq) {
         switch (p.nstep) {
-            case 16: launch_seq<16>(p, grid, block, lds, stream, a); break;
-            case 8: launch_seq<8>(p, grid, block, lds, stream, a); break;
-            case 4: launch_seq<4>(p, grid, block, lds, stream, a); break;
-            case 2: launch_seq<2>(p, grid, block, lds, stream, a); break;
+            case 2: launch_seq<2>(p, grid, block, lds, stream, a); break;      // four steps: gemv_stream_takes
             default: launch_seq<1>(p, grid, block, lds, stream, a); break;
         }
     } else {
@@ -1085,7 +1242,6 @@ static void launch_seq_group(const q4::GemvPlan& p, dim3 grid, dim3 block, size_
     switch (p.gsteps) {
         case 0: hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 0>), grid, block, lds, stream, g); break;
         case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 1>), grid, block, lds, stream, g); break;
-        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 2>), grid, block, lds, stream, g); break;
     }
 }
 
@@ -1122,11 +1278,11 @@ extern "C" int q4_launch_gemv_group(int n, const void* const* x, const int32_t* 
             g.strip_end[i] = 0x7fffffff;
         }
     }
+    if (gemv_stream_takes(K, groupsize)) return launch_stream(g, n, strips, stream);
     const GemvPlan p = plan_gemv(K, N[0], groupsize, true, 4);      // the plan does not depend on N
     const dim3 grid(strips, p.splits), block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);
     switch (p.nstep) {
-        case 4: launch_seq_group<4>(p, grid, block, lds, stream, g); break;
         case 2: launch_seq_group<2>(p, grid, block, lds, stream, g); break;
         default: launch_seq_group<1>(p, grid, block, lds, stream, g); break;
     }

@@ -9,8 +9,11 @@
 namespace q4 {
 
 constexpr int kColsPerWave = 64;
+constexpr int kStreamWaves = 4;               // wavefronts of the kernels of q4_gemv_stream.hpp
 constexpr int kFracBits = 24;
 constexpr long long kBias = 1ll << 47;
+constexpr double kGrid = 402653184.0;         // 1.5 * 2^28: doubles about it are multiples of 2^-24
+constexpr unsigned long long kGridBits = 0x41B8000000000000ull;
 constexpr float kClamp = 4194304.0f;          // 2^22: |partial| beyond this saturates (fp16 max is 65504)
 
 struct GemvArgs {
@@ -31,6 +34,17 @@ struct GemvArgs {
 __device__ __forceinline__ half8_t make_half8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
     uint4_t v = {a, b, c, d};
     return __builtin_bit_cast(half8_t, v);
+}
+
+// v on the grid of 2^-24 as an integer plus kBias: adding 1.5 * 2^28 leaves it in the low bits of a double's mantissa.
+__device__ __forceinline__ unsigned long long fixed_biased(float v) {
+    const double d = (double)fminf(fmaxf(v, -kClamp), kClamp) + kGrid;
+    return (unsigned long long)__double_as_longlong(d) + (kBias - kGridBits);
+}
+// The sum of n such values, whatever the top 8 bits (the arrival count) hold.
+__device__ __forceinline__ float fixed_sum(unsigned long long sum, int n) {
+    const long long tot = (long long)(sum & ((1ull << 56) - 1)) - (long long)n * kBias;
+    return (float)((double)tot * (1.0 / (double)(1 << kFracBits)));
 }
 
 // Finishes EB outputs per thread (e0, e0 + blockDim.x, ...): all LDS reads of the batch are issued before
@@ -81,26 +95,31 @@ __device__ __forceinline__ void gemv_finish_batch(const GemvArgs& a, const float
 #pragma unroll
     for (int i = 0; i < EB; ++i) {
         const int e = e0 + i * blockDim.x;
-        const float c = fminf(fmaxf(v[i], -kClamp), kClamp);
-        const long long fx = __float2ll_rn(c * (float)(1 << kFracBits));
-        add[i] = (1ull << 56) + (unsigned long long)(fx + kBias);
+        add[i] = (1ull << 56) + fixed_biased(v[i]);
         old[i] = 0;
         if (e < total)
             old[i] = __hip_atomic_fetch_add(a.acc64 + (size_t)(e >> 6) * a.N + n0 + (e & 63), add[i],
                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    // every reply first, then the stores: a reply that is looked at behind a store waits for that store as well
+    bool last[EB];
+    half_t h[EB];
 #pragma unroll
     for (int i = 0; i < EB; ++i) {
         const int e = e0 + i * blockDim.x;
-        if (e < total && (old[i] >> 56) == (unsigned long long)(S - 1)) {      // last of the S workgroups of the strip
+        last[i] = e < total && (old[i] >> 56) == (unsigned long long)(S - 1);      // last of the S workgroups of the strip
+        float out = fixed_sum(old[i] + add[i], S);
+        if (a.accumulate && last[i]) out += (float)a.y[(size_t)(e >> 6) * a.N + n0 + (e & 63)];
+        h[i] = (half_t)out;
+    }
+#pragma unroll
+    for (int i = 0; i < EB; ++i) {
+        const int e = e0 + i * blockDim.x;
+        if (last[i]) {
             const size_t at = (size_t)(e >> 6) * a.N + n0 + (e & 63);
-            const long long tot = (long long)((old[i] + add[i]) & ((1ull << 56) - 1)) - (long long)S * kBias;
-            float out = (float)((double)tot * (1.0 / (double)(1 << kFracBits)));
-            if (a.accumulate) out += (float)a.y[at];
-            const half_t h = (half_t)out;
-            if (!hand || a.y) a.y[at] = h;
+            if (!hand || a.y) a.y[at] = h[i];
             if (hand)
-                __hip_atomic_store(hand + at, (uint32_t)__builtin_bit_cast(unsigned short, h) | (tag << 16),
+                __hip_atomic_store(hand + at, (uint32_t)__builtin_bit_cast(unsigned short, h[i]) | (tag << 16),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(a.acc64 + at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -199,9 +218,21 @@ struct SeqChunk {
         // B operands of the two extra MFMAs: per-position offsets (1024 | 64) and all ones
         const half8_t offs = make_half8(0x64006400u, 0x54005400u, 0x64006400u, 0x54005400u);
         const half8_t ones = make_half8(0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u);
-        // pass 1 (needs the activations only): A operands and the two weight-independent products
+        // pass 1 (needs the activations, scales and zeros only): A operands, the two weight-independent products, and
+        // from them what the sums of pass 2 start from, so that those end as sum x*(q - z - 1)
         half8_t av[NSTEP];
-        float4_t acco_g[NG], accx_g[NG];
+        float4_t acco_g[NG], accx_g[NG], acc[4];
+        auto start = [&](int gi) {
+            const uint32_t zw = V1 ? 0u : zv[gi] >> ((c & 1) * 16);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
+                acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)             // uniform: accumulator rows past M are unused
+                    if (r < a.M) acc[j][r] = V1 ? -acco_g[gi][r] : fmaf(-zf, accx_g[gi][r], -acco_g[gi][r]);
+            }
+        };
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
             acco_g[gi] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -217,13 +248,17 @@ struct SeqChunk {
                 accx_g[gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], ones, accx_g[gi], 0, 0, 0);
             }
         }
+        if constexpr (NG == 1) start(0);                // with several groups later: their sums would only hold registers
+        // mask (scalar register) and magic number (vector register) as opaque values: with two literals the compiler
+        // emits an AND and an OR, with register operands the single three-operand and-or instruction (128 -> 64 of the
+        // 144 instructions that build the operands of a chunk)
+        uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, g_lo = 0x64006400u, g_hi = 0x54005400u;
+        asm volatile("" : "+s"(m_lo), "+s"(m_hi));
+        asm volatile("" : "+v"(g_lo), "+v"(g_hi));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
-            float4_t acc[4];
-            const float4_t acco = acco_g[gi], accx = accx_g[gi];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (NG > 1) start(gi);
 #pragma unroll
             for (int tt = 0; tt < GS; ++tt) {
                 const int t = gi * GS + tt;
@@ -231,36 +266,26 @@ struct SeqChunk {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t hi = w[j] >> 8;
-                    const half8_t bv = make_half8((w[j] & 0x000F000Fu) | 0x64006400u, (w[j] & 0x00F000F0u) | 0x54005400u,
-                                                  (hi & 0x000F000Fu) | 0x64006400u, (hi & 0x00F000F0u) | 0x54005400u);
+                    const half8_t bv = make_half8((w[j] & m_lo) | g_lo, (w[j] & m_hi) | g_hi, (hi & m_lo) | g_lo, (hi & m_hi) | g_hi);
                     acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bv, acc[j], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);      // consume the loads in the order they return
             }
             const half2_t s01 = as_half2(sv[gi].x), s23 = as_half2(sv[gi].y);
             const float sf[4] = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
+            float zf[4] = {0.f, 0.f, 0.f, 0.f};
             if constexpr (V1) {
-                // y += s * (sum x*(off+q) - sum x*off) - zero * sum x
                 const half2_t z01 = as_half2(zh.x), z23 = as_half2(zh.y);
-                const float zf[4] = {(float)z01[0], (float)z01[1], (float)z23[0], (float)z23[1]};
+                zf[0] = (float)z01[0]; zf[1] = (float)z01[1]; zf[2] = (float)z23[0]; zf[3] = (float)z23[1];
+            }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (r < a.M) {
+            for (int r = 0; r < 4; ++r) {
+                if (r < a.M) {                          // uniform: with M <= 3 the other accumulator rows are unused
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) yacc[j][r] += sf[j] * (acc[j][r] - acco[r]) - zf[j] * accx[r];
-                    }
-                }
-            } else {
-                // group epilogue: y += s * ((sum x*(off+q) - sum x*off) - (z+1) * sum x)
-                const uint32_t zw = zv[gi] >> ((c & 1) * 16);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (r < a.M) {                      // uniform: with M <= 3 the other accumulator rows are unused
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
-                            yacc[j][r] += sf[j] * ((acc[j][r] - acco[r]) - zf * accx[r]);
-                        }
+                    for (int j = 0; j < 4; ++j) {
+                        // y += s * sum x*(q - z - 1);  V1: s * sum x*q - zero * sum x
+                        yacc[j][r] = fmaf(sf[j], acc[j][r], yacc[j][r]);
+                        if constexpr (V1) yacc[j][r] = fmaf(-zf[j], accx_g[gi][r], yacc[j][r]);
                     }
                 }
             }

@@ -181,3 +181,38 @@ def test_gemv_grouped_rejects_act_order_and_mismatched_layers(oracle):
         quant_hip.gemv_grouped(x, [(c["qweight"], c["qzeros"], c["scales"]), (b["qweight"], b["qzeros"], b["scales"])], 128)
     with pytest.raises(ValueError):
         quant_hip.gemv_grouped(x, [(c["qweight"], c["qzeros"], c["scales"])] * 5, 128)
+
+
+@pytest.mark.parametrize("K,Ns,gs", [(128, (64, 128), 128), (1152, (64, 192), 128), (1152, (128, 64), 2048), (2176, (64, 64), 64),
+                                     (1408, (64, 128), 32), (5120, (1024, 5120, 5120, 4096), 128), (11008, (2048, 2048), 128)])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+def test_gemv_same_bits_however_the_reduction_is_split(oracle, K, Ns, gs, M):
+    """Edges of the streaming kernel: one chunk of 128 rows, a last block with fewer than 8 chunks, groups of 32 and 64 rows, a group
+    beyond K, and groups of layers that take longer shares of the reduction than each of them alone.  Blocks are added as
+    integers, so the split never shows; rows past M (1..16 of the 16 of an operand) and neighbouring strips stay untouched."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    layers = [oracle.make_layer(K, N, gs, seed=K + 3 * N + i) for i, N in enumerate(Ns)]
+    ts = [to_cuda_layer(l) for l in layers]
+    xh = oracle.make_activations(M, K, seed=M + 7)
+    x = torch.from_numpy(xh).cuda()
+    outs = quant_hip.gemv_grouped(x, [(t["qweight"], t["qzeros"], t["scales"]) for t in ts], gs)
+    for lay, t, y in zip(layers, ts, outs):
+        assert torch.equal(y, quant_hip.gemv(x, t["qweight"], t["qzeros"], t["scales"], None, gs))
+    ref = oracle.matmul_recons(xh, layers[0]["qweight"], layers[0]["qzeros"], layers[0]["scales"], layers[0]["g_idx"])
+    assert rel_err(outs[0].cpu().numpy(), ref) <= 2e-3
+    assert quant_hip.workspaces_are_zero()
+
+
+def test_gemv_longest_reduction(oracle):
+    """More than 255 blocks of 1024 rows: shares of several blocks keep the arrival count within 8 bits."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    K, N, gs, M = 262144 + 128, 64, 128, 3
+    layer = oracle.make_layer(K, N, gs, seed=5)
+    t = to_cuda_layer(layer)
+    x = oracle.make_activations(M, K, seed=5)
+    y = quant_hip.gemv(torch.from_numpy(x).cuda(), t["qweight"], t["qzeros"], t["scales"], None, gs)
+    ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
+    assert rel_err(y.cpu().numpy(), ref) <= 2e-3
+    assert quant_hip.workspaces_are_zero()
