@@ -6,7 +6,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libq4gptq.so")
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 _lib = None
 
@@ -60,6 +60,9 @@ SIGNATURES["q4_mlp_decode_workspace_bytes"] = (_sz, [_i, _i, _i])
 SIGNATURES["q4_mlp_decode_status_offset"] = (_sz, [_i, _i, _i])
 SIGNATURES["q4_mlp_decode_f16"] = (_i, [_vp, ctypes.POINTER(Layer), ctypes.POINTER(Layer), ctypes.POINTER(Layer), _i, _vp, _vp, _vp,
                                         _i, _i, _i, _vp, _sz, _vp])
+SIGNATURES["q4_mlp_gate_up_f16"] = (_i, [_vp, ctypes.POINTER(Layer), ctypes.POINTER(Layer), _i, _vp, _i, _i, _i, _vp])
+
+
 class GemmLayer(ctypes.Structure):
     """q4_gemm_layer_t of include/q4_gptq.h."""
     _fields_ = [("act", _vp), ("qweight", _vp), ("qzeros", _vp), ("scales", _vp), ("bias", _vp), ("la", _vp), ("lb", _vp),

@@ -40,6 +40,7 @@ int q4_launch_gemm_group(int, int, const void* const*, const int32_t* const*, co
 int q4_mlp_applicable(int, int, int, int);
 size_t q4_mlp_plan_workspace(int, int, int);
 size_t q4_mlp_status_offset(int, int, int);
+int q4_launch_gate_up(const void*, const int32_t* const*, const int32_t* const*, const void* const*, int, void*, int, int, int, hipStream_t);
 int q4_launch_mlp(const void*, const int32_t* const*, const int32_t* const*, const void* const*, int, void*, void*, void*, int, int,
                   int, void*, int, hipStream_t);
 int q4_stream_fwd_applicable(int, int, int, int, int);
@@ -78,7 +79,7 @@ int check_layer(const void* qweight, const void* qzeros, const void* scales, con
 }
 }  // namespace
 
-extern "C" int q4_abi_version(void) { return 15; }
+extern "C" int q4_abi_version(void) { return 16; }
 
 extern "C" const char* q4_error_string(int code) {
     switch (code) {
@@ -244,6 +245,22 @@ extern "C" int q4_mlp_decode_f16(const void* x, const q4_layer_t* gate, const q4
     if (!workspace || workspace_bytes < q4_mlp_plan_workspace(M, H, I)) return Q4_ERR_WORKSPACE;
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return Q4_ERR_MISALIGNED;
     return q4_launch_mlp(x, qw, qz, sc, groupsize, gate_out, up_out, y, M, H, I, workspace, 0, (hipStream_t)stream);
+}
+
+extern "C" int q4_mlp_gate_up_f16(const void* x, const q4_layer_t* gate, const q4_layer_t* up, int groupsize, void* h, int M,
+                                  int H, int I, void* stream) {
+    if (!x || !h || !gate || !up) return Q4_ERR_NULL_POINTER;
+    if (M < 1 || M > 16 || H < 128 || (H % 128) != 0 || I < 64 || (I % 64) != 0) return Q4_ERR_BAD_SHAPE;
+    if (groupsize < 128 || (groupsize % 128) != 0) return Q4_ERR_BAD_SHAPE;
+    const q4_layer_t* ls[2] = {gate, up};
+    const int32_t* qw[2]; const int32_t* qz[2]; const void* sc[2];
+    for (int i = 0; i < 2; ++i) {
+        const int rc = gemv_check(x, ls[i]->qweight, ls[i]->qzeros, ls[i]->scales, nullptr, groupsize, h, M, 16, H, I,
+                                  (H + groupsize - 1) / groupsize);
+        if (rc != Q4_OK) return rc;
+        qw[i] = ls[i]->qweight; qz[i] = ls[i]->qzeros; sc[i] = ls[i]->scales;
+    }
+    return q4_launch_gate_up(x, qw, qz, sc, groupsize, h, M, H, I, (hipStream_t)stream);
 }
 
 extern "C" size_t q4_gemv_noalloc_max_outputs(void) { return q4_noalloc_scratch_bytes() / 8; }

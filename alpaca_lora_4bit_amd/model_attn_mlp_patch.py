@@ -9,7 +9,7 @@ classes.  Two ways here, both leaving the host model's own attention / MLP code 
   (quant_hip.gemv_grouped -> q4_gemv_grouped_f16) and the others pick their result up.  No second copy of the
   weights, the state dict keeps its keys, and members may be LoRA layers (Linear4bitLt): the grouped launch does the
   base products, each member adds its own adapter.  make_fused_mlp also routes the block's forward, at decode sizes,
-  through quant_hip.mlp_decode: gate, up, silu(gate) * up and down in one launch.
+  through quant_hip.mlp_decode (gate, up, silu(gate) * up and down in one launch) or quant_hip.mlp_rows (two launches).
 * `concatenate=True`: the reference's layout.  One new layer holds the N-concatenated tensors and each projection is
   replaced by a slice view of its output (one wider GEMM at prefill sizes as well); `inject_lora_layers(model,
   lora_path)` (model_attn_mlp_patch.py:283-335) then puts a saved q/v adapter onto the fused qkv layer as ONE
@@ -266,6 +266,7 @@ def ungroup(model):
             del m.__dict__['_q4_mlp_forward']
             del m.__dict__['forward']
             m.__dict__.pop('_q4_mlp_args', None)
+            m.__dict__.pop('_q4_mlp_gated', None)
     return count
 
 
@@ -289,9 +290,41 @@ def make_quant_attn(model, is_v1_model=False, concatenate=False):
     return count
 
 
-# The one-launch MLP step re-reads the intermediate once per output strip of the down projection, which grows with the
-# number of rows: measured against grouped gate|up + two elementwise launches + down it wins up to about 4 rows.
+# Up to so many rows the MLP step runs on the block's three layers directly, whatever the block's own forward looks like
+# (make_fused_mlp's premise); more rows only where that forward is known to compute the same.
 mlp_decode_max_rows = 4
+
+
+class _GatedForward:
+    """The forwards of a gated MLP block whose steps may run fused at any number of rows: compared by their code."""
+
+    def returned(self, x):
+        return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+
+    def assigned(self, x):
+        down_proj = self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+        return down_proj
+
+
+def _is_gated_forward(forward):
+    """True when `forward` (a bound method) is down_proj(act_fn(gate_proj(x)) * up_proj(x)) and nothing else."""
+    code = getattr(getattr(forward, '__func__', None), '__code__', None)
+    if code is None:
+        return False
+
+    def key(c):
+        return (c.co_code, c.co_names, c.co_consts[1:], c.co_argcount, c.co_kwonlyargcount, c.co_flags & 0x0F, c.co_freevars)
+    return any(key(code) == key(f.__code__) for f in (_GatedForward.returned, _GatedForward.assigned))
+
+
+def _steps_unobserved(mlp):
+    """No hook and no replaced forward on the block's four steps, which a fused step would pass by."""
+    mods = mlp._modules
+    for name in ('gate_proj', 'up_proj', 'down_proj', 'act_fn'):
+        m = mods.get(name)
+        if m is None or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or 'forward' in m.__dict__:
+            return False
+    return _is_silu(mods['act_fn']) and not torch.nn.modules.module._has_any_global_hook()
 
 
 def _is_silu(act):
@@ -325,9 +358,9 @@ def _mlp_decode_args(mlp):
 
 
 def _mlp_decode_forward(mlp, x):
-    """LlamaMLP.forward with the decode step (a few rows, no grad, fp16) as ONE launch: gate, up, silu(gate) * up and
-    down (quant_hip.mlp_decode); everything else goes to the block's own forward.  What the step needs of the three
-    layers is looked up once and kept while their buffers, adapters and bias switches stay the same objects / values."""
+    """LlamaMLP.forward with the decode step (up to 16 rows, no grad, fp16) as one launch (quant_hip.mlp_decode: gate, up,
+    silu(gate) * up and down) or two (quant_hip.mlp_rows); everything else goes to the block's own forward.  What the step
+    needs of the three layers is looked up once and kept while their buffers, adapters and bias switches stay the same objects / values."""
     from . import autograd_4bit, quant_hip
     d = mlp.__dict__
     if (not torch.is_grad_enabled() and x.dtype == torch.float16 and x.is_cuda and autograd_4bit.backend == 'cuda'
@@ -345,9 +378,12 @@ def _mlp_decode_forward(mlp, x):
         args = cached[1]
         if args is not None and x.shape[-1] == args[4]:
             rows = x.numel() // args[4]
-            if (1 <= rows <= min(int(matmul_utils_4bit.auto_switch_thd), quant_hip.MAX_GEMV_ROWS, mlp_decode_max_rows)
-                    and quant_hip.mlp_decode_applicable(rows, args[4], args[5], args[3])):
-                return quant_hip.mlp_decode_prepared(x, args[0], args[1], args[2], args[3], tuple(x.shape[:-1]) + (args[6],))
+            if (1 <= rows <= min(int(matmul_utils_4bit.auto_switch_thd), quant_hip.MAX_GEMV_ROWS)
+                    and quant_hip.mlp_decode_applicable(rows, args[4], args[5], args[3])
+                    and (rows <= mlp_decode_max_rows or (d['_q4_mlp_gated'] and _steps_unobserved(mlp)))):
+                faster = quant_hip.mlp_rows_is_faster(rows, args[4], args[5])
+                step = quant_hip.mlp_rows_prepared if faster or rows > mlp_decode_max_rows else quant_hip.mlp_decode_prepared
+                return step(x, args[0], args[1], args[2], args[3], tuple(x.shape[:-1]) + (args[6],))
     return d['_q4_mlp_forward'](x)
 
 
@@ -373,6 +409,7 @@ def make_fused_mlp(model, is_v1_model=False, concatenate=False, fuse_decode_step
                     and down.groupsize == m.gate_proj.groupsize and down.in_features == m.gate_proj.out_features
                     and down.out_features == m.gate_proj.in_features and '_q4_mlp_forward' not in m.__dict__):
                 import types
+                m.__dict__['_q4_mlp_gated'] = _is_gated_forward(m.forward)
                 m.__dict__['_q4_mlp_forward'] = m.forward                # the block's own (bound) forward
                 m.__dict__['forward'] = types.MethodType(_mlp_decode_forward, m)
     if concatenate and torch.cuda.is_available():

@@ -621,6 +621,18 @@ def mlp_decode_prepared(x, gate, up, down, groupsize, out_shape):
     return _host.mlp_decode(x, gate, up, down, groupsize, False, out_shape)[0]
 
 
+def mlp_rows_is_faster(M, H, I):
+    """Whether `mlp_rows` beats `mlp_decode` by more than its second launch costs a host-bound caller.  mlp_decode reads the
+    intermediate again for every 64 outputs of down.  us, mlp_decode / mlp_rows: 4096 -> 11008 21.7 / 20.7 at 4 rows, 24.7 / 21.5
+    at 6, 37.8 / 24.1 at 16; 5120 -> 13824 27.2 / 25.8 at 2 rows, 28.7 / 26.1 at 3, 50.3 / 30.8 at 16; 2048 -> 5632 12.5 / 12.6 at 6."""
+    return M * H * I > 200_000_000
+
+
+def mlp_rows_prepared(x, gate, up, down, groupsize, out_shape):
+    """The same step as two launches (q4_mlp_gate_up_f16, then down), under the same premise."""
+    return _host.mlp_rows(x, gate, up, down, groupsize, out_shape)
+
+
 def mlp_decode_gave_up():
     """True when a device-side wait of some `mlp_decode` launch ran into its poll limit (synchronises)."""
     return bool(_host is not None and _host.mlp_decode_gave_up())

@@ -156,6 +156,13 @@ Q4_API int q4_mlp_decode_f16(const void *x, const q4_layer_t *gate, const q4_lay
                              int groupsize, void *gate_out, void *up_out, void *y, int M, int H, int I,
                              void *workspace, size_t workspace_bytes, void *stream);
 
+/* Gate, up and the activation of a gated MLP block in one launch:  h fp16 [M, I] = silu(gate(x)) * up(x), 1 <= M <= 16, with
+ * the roundings of the separate modules (gate, up, silu(gate) and the product to fp16).  What q4_mlp_decode_f16 does up to the
+ * down projection, for callers that run that as a launch of its own (q4_gemv_f16): faster from two rows on
+ * (model_attn_mlp_patch.py:224-228).  groupsize % 128 == 0, H % 128 == 0, I % 64 == 0; no workspace. */
+Q4_API int q4_mlp_gate_up_f16(const void *x, const q4_layer_t *gate, const q4_layer_t *up, int groupsize, void *h,
+                              int M, int H, int I, void *stream);
+
 /* q4_gemv_f16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same product, same arguments
  * minus the workspace: the split-K accumulators live in a device array inside the library (4 MiB per device that

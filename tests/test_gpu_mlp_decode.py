@@ -140,3 +140,105 @@ def test_mlp_decode_through_the_c_abi_and_in_a_hip_graph(oracle):
                                None, None, y.data_ptr(), M, H, I, ws.data_ptr(), need, None) == -2
     assert L.q4_mlp_decode_f16(None, ctypes.byref(desc[0]), ctypes.byref(desc[1]), ctypes.byref(desc[2]), gs,
                                None, None, y.data_ptr(), M, H, I, ws.data_ptr(), need, None) == -1
+
+
+@pytest.mark.parametrize("H,I,gs", [(128, 128, 128), (256, 384, 128), (1152, 640, 128), (1024, 2816, 256), (640, 1024, 1024), (4096, 11008, 128)])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+def test_gate_up_launch_and_two_launch_step(oracle, H, I, gs, M):
+    """q4_mlp_gate_up_f16 at the edges of its range (one chunk of the reduction, a last block of less than 8 chunks, a group
+    beyond H, every number of outputs per thread) and quant_hip.mlp_rows_prepared, the step with down as its second launch."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    gate, up, down = _layers(oracle, H, I, gs, seed=H + I + M)
+    tg, tu, td = (to_cuda_layer(l) for l in (gate, up, down))
+    x = oracle.make_activations(M, H, seed=M + 5)
+    xt = torch.from_numpy(x).cuda()
+    _, _, inter_ref, y_ref = _reference(oracle, x, gate, up, down)
+    h = torch.full((M + 1, I), 7.0, dtype=torch.float16, device="cuda")            # one row beyond: stays as it is
+    desc = [_lib.Layer(t["qweight"].data_ptr(), t["qzeros"].data_ptr(), t["scales"].data_ptr()) for t in (tg, tu)]
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    assert L.q4_mlp_gate_up_f16(xt.data_ptr(), ctypes.byref(desc[0]), ctypes.byref(desc[1]), gs, h.data_ptr(), M, H, I, stream) == 0
+    assert bool((h[M] == 7.0).all())
+    # gate and up are within one fp16 rounding (2^-11) of the reference's, |silu'| <= 1.1 and two more roundings follow
+    assert rel_err(h[:M].cpu().numpy(), inter_ref.astype(np.float64)) <= 4.2 * 2.0 ** -11
+    y = quant_hip.mlp_rows_prepared(xt, _tuple(tg), _tuple(tu), _tuple(td), gs, (1, M, H))
+    assert y.shape == (1, M, H)
+    assert rel_err(y[0].cpu().numpy(), y_ref) <= 3e-3
+    assert torch.equal(y, quant_hip.mlp_rows_prepared(xt, _tuple(tg), _tuple(tu), _tuple(td), gs, (1, M, H)))
+    assert quant_hip.workspaces_are_zero()
+    for args, rc in (((xt.data_ptr(), 64, h.data_ptr(), M, H, I), -2), ((xt.data_ptr(), gs, h.data_ptr(), 17, H, I), -2),
+                     ((None, gs, h.data_ptr(), M, H, I), -1), ((xt.data_ptr() + 2, gs, h.data_ptr(), M, H, I), -5)):
+        assert L.q4_mlp_gate_up_f16(args[0], ctypes.byref(desc[0]), ctypes.byref(desc[1]), *args[1:], None) == rc
+
+
+def test_mlp_block_above_four_rows_keeps_its_own_forward_where_it_must(oracle, monkeypatch):
+    """5..16 rows take the fused step only when the block's forward is the gated expression and nobody watches its steps;
+    replayed as a graph the step gives what it gives eagerly."""
+    import torch
+    import torch.nn as nn
+    from alpaca_lora_4bit_amd import quant_hip
+    from alpaca_lora_4bit_amd.autograd_4bit import Autograd4bitQuantLinear
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_fused_mlp, ungroup
+
+    class Gated(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.act_fn = nn.SiLU()
+
+        def forward(self, x):
+            return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+
+    class Clamped(Gated):
+        def forward(self, x):
+            return self.down_proj(self.act_fn(self.gate_proj(x)).clamp(max=0.0) * self.up_proj(x))
+
+    H, I, gs = 256, 384, 128
+    layers = _layers(oracle, H, I, gs, seed=3)
+    calls = []
+    real = quant_hip.mlp_rows_prepared
+    monkeypatch.setattr(quant_hip, "mlp_rows_prepared", lambda *a: (calls.append(1), real(*a))[1])
+
+    def block(cls):
+        m = cls()
+        for name, layer in zip(("gate_proj", "up_proj", "down_proj"), layers):
+            lin = Autograd4bitQuantLinear(layer["qweight"].shape[0] * 8, layer["qweight"].shape[1], groupsize=gs)
+            for k, v in to_cuda_layer(layer).items():
+                if isinstance(v, torch.Tensor):
+                    setattr(lin, k, v)
+            lin.bias = torch.zeros(lin.out_features, dtype=torch.float16, device="cuda")
+            setattr(m, name, lin)
+        return m
+
+    with torch.no_grad():
+        for M in (5, 16):
+            x = torch.from_numpy(oracle.make_activations(M, H, seed=M)).cuda()
+            for cls in (Gated, Clamped):
+                m = block(cls)
+                want = m(x)
+                assert make_fused_mlp(m) == 1
+                calls.clear()
+                got = m(x)
+                assert len(calls) == (cls is Gated)
+                assert rel_err(got.cpu().numpy(), want.double().cpu().numpy()) <= 3e-3
+                seen = []
+                handle = m.act_fn.register_forward_hook(lambda *a: seen.append(1))
+                m(x)
+                handle.remove()
+                assert len(seen) == 1 and len(calls) == (cls is Gated)
+                if cls is Gated:
+                    side = torch.cuda.Stream()
+                    graph = torch.cuda.CUDAGraph()
+                    with torch.cuda.stream(side):
+                        m(x)
+                        side.synchronize()
+                        with torch.cuda.graph(graph, stream=side):
+                            y = m(x)
+                    for rep in range(4):
+                        y.fill_(float("nan"))
+                        (x.float() @ x.float().t()).sum().item()
+                        torch.cuda.synchronize()
+                        graph.replay()
+                        torch.cuda.synchronize()
+                        assert torch.equal(y, got)
+                assert ungroup(m) == 1 and "_q4_mlp_gated" not in m.__dict__
+    assert quant_hip.workspaces_are_zero()
