@@ -6,7 +6,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libq4gptq.so")
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 _lib = None
 
@@ -36,6 +36,8 @@ SIGNATURES = {
     "q4_lora_grad_workspace_bytes": (_sz, [_i, _i, _i]),
     "q4_lora_grad_f32": (_i, [_vp, _vp, _vp, _i, _i, _f, _i, _i, _i, _vp, _vp, _sz, _vp]),
     "q4_lora_grad_pair_f32": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _i, _i, _i, _f, _i, _i, _vp, _vp, _sz, _vp]),
+    "q4_silu_mul_f16": (_i, [_vp, _vp, _vp, ctypes.c_longlong, _vp]),
+    "q4_silu_mul_bwd_f16": (_i, [_vp, _vp, _vp, _vp, _vp, ctypes.c_longlong, _vp]),
     "q4_dropout_scale": (_f, [_f]),
     "q4_dropout_keep_u8": (_i, [_vp, _i, _i, _vp, _vp]),
 }

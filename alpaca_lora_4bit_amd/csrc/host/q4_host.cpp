@@ -327,6 +327,30 @@ at::Tensor mlp_rows(const at::Tensor& x, const std::tuple<at::Tensor, at::Tensor
     return y;
 }
 
+void check_act(const at::Tensor& t, const at::Tensor& like) {
+    TORCH_CHECK_VALUE(t.is_cuda() && t.scalar_type() == at::kHalf && t.is_contiguous() && t.device() == like.device() &&
+                      t.sizes() == like.sizes() && t.numel() > 0, "contiguous float16 CUDA tensors of one shape are expected");
+}
+at::Tensor silu_mul(const at::Tensor& gate, const at::Tensor& up) {
+    check_act(gate, gate);
+    check_act(up, gate);
+    at::Tensor out = at::empty_like(gate);
+    Launch L(gate.device());
+    const int rc = q4_silu_mul_f16(gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.numel(), L.stream);
+    if (rc != Q4_OK) raise_q4(rc, "q4_silu_mul_f16");
+    return out;
+}
+std::pair<at::Tensor, at::Tensor> silu_mul_bwd(const at::Tensor& dout, const at::Tensor& gate, const at::Tensor& up) {
+    check_act(gate, gate);
+    check_act(up, gate);
+    check_act(dout, gate);
+    at::Tensor dgate = at::empty_like(gate), dup = at::empty_like(gate);
+    Launch L(gate.device());
+    const int rc = q4_silu_mul_bwd_f16(dout.data_ptr(), gate.data_ptr(), up.data_ptr(), dgate.data_ptr(), dup.data_ptr(), gate.numel(), L.stream);
+    if (rc != Q4_OK) raise_q4(rc, "q4_silu_mul_bwd_f16");
+    return {dgate, dup};
+}
+
 // 1 when a wait inside some fused MLP launch on this device hit its poll limit (synchronises; for tests).
 bool mlp_decode_gave_up() {
     std::vector<std::pair<at::Tensor, size_t>> all;
@@ -630,6 +654,8 @@ PYBIND11_MODULE(_q4_host, m) {
           py::arg("intermediates") = false, py::arg("out_shape") = py::none());
     m.def("mlp_rows", &mlp_rows, py::arg("x"), py::arg("gate"), py::arg("up"), py::arg("down"), py::arg("groupsize"),
           py::arg("out_shape") = py::none());
+    m.def("silu_mul", &silu_mul, py::arg("gate"), py::arg("up"));
+    m.def("silu_mul_bwd", &silu_mul_bwd, py::arg("dout"), py::arg("gate"), py::arg("up"));
     m.def("mlp_decode_gave_up", &mlp_decode_gave_up);
     m.def("reset_workspaces", &reset_workspaces);
     m.def("workspaces_are_zero", &workspaces_are_zero);

@@ -40,6 +40,8 @@ int q4_launch_gemm_group(int, int, const void* const*, const int32_t* const*, co
 int q4_mlp_applicable(int, int, int, int);
 size_t q4_mlp_plan_workspace(int, int, int);
 size_t q4_mlp_status_offset(int, int, int);
+int q4_launch_silu_mul(const void*, const void*, void*, long, hipStream_t);
+int q4_launch_silu_mul_bwd(const void*, const void*, const void*, void*, void*, long, hipStream_t);
 int q4_launch_gate_up(const void*, const int32_t* const*, const int32_t* const*, const void* const*, int, void*, int, int, int, hipStream_t);
 int q4_launch_mlp(const void*, const int32_t* const*, const int32_t* const*, const void* const*, int, void*, void*, void*, int, int,
                   int, void*, int, hipStream_t);
@@ -79,7 +81,7 @@ int check_layer(const void* qweight, const void* qzeros, const void* scales, con
 }
 }  // namespace
 
-extern "C" int q4_abi_version(void) { return 16; }
+extern "C" int q4_abi_version(void) { return 17; }
 
 extern "C" const char* q4_error_string(int code) {
     switch (code) {
@@ -261,6 +263,22 @@ extern "C" int q4_mlp_gate_up_f16(const void* x, const q4_layer_t* gate, const q
         qw[i] = ls[i]->qweight; qz[i] = ls[i]->qzeros; sc[i] = ls[i]->scales;
     }
     return q4_launch_gate_up(x, qw, qz, sc, groupsize, h, M, H, I, (hipStream_t)stream);
+}
+
+static bool act_size(long long n) { return n >= 1 && n < (1ll << 38); }          /* 2^31 workgroups of 256 x 8 elements */
+
+extern "C" int q4_silu_mul_f16(const void* gate, const void* up, void* out, long long n, void* stream) {
+    if (!gate || !up || !out) return Q4_ERR_NULL_POINTER;
+    if (!act_size(n)) return Q4_ERR_BAD_SHAPE;
+    if (misaligned(gate) || misaligned(up) || misaligned(out)) return Q4_ERR_MISALIGNED;
+    return q4_launch_silu_mul(gate, up, out, (long)n, (hipStream_t)stream);
+}
+
+extern "C" int q4_silu_mul_bwd_f16(const void* dout, const void* gate, const void* up, void* dgate, void* dup, long long n, void* stream) {
+    if (!dout || !gate || !up || !dgate || !dup) return Q4_ERR_NULL_POINTER;
+    if (!act_size(n)) return Q4_ERR_BAD_SHAPE;
+    if (misaligned(dout) || misaligned(gate) || misaligned(up) || misaligned(dgate) || misaligned(dup)) return Q4_ERR_MISALIGNED;
+    return q4_launch_silu_mul_bwd(dout, gate, up, dgate, dup, (long)n, (hipStream_t)stream);
 }
 
 extern "C" size_t q4_gemv_noalloc_max_outputs(void) { return q4_noalloc_scratch_bytes() / 8; }

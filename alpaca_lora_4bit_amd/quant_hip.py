@@ -638,6 +638,23 @@ def mlp_decode_gave_up():
     return bool(_host is not None and _host.mlp_decode_gave_up())
 
 
+def silu_mul_takes(gate, up):
+    """Whether `silu_mul` takes these tensors (plain contiguous float16 CUDA tensors of one shape)."""
+    return (_host is not None and type(gate) is torch.Tensor and type(up) is torch.Tensor and gate.is_cuda and gate.device == up.device
+            and gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape and gate.numel() > 0
+            and gate.is_contiguous() and up.is_contiguous() and (gate.data_ptr() | up.data_ptr()) % 16 == 0)
+
+
+def silu_mul(gate, up):
+    """silu(gate) * up in one pass, with the fp16 roundings of the two operations."""
+    return _host.silu_mul(gate, up)
+
+
+def silu_mul_bwd(dout, gate, up):
+    """(dgate, dup) of silu_mul in one pass."""
+    return _host.silu_mul_bwd(dout, gate, up)
+
+
 def _adapter_dtype_flag(w, what):
     _require(w.dtype in (torch.float16, torch.float32), f"{what} must be float16 or float32")
     return int(w.dtype == torch.float32)

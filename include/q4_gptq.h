@@ -163,6 +163,12 @@ Q4_API int q4_mlp_decode_f16(const void *x, const q4_layer_t *gate, const q4_lay
 Q4_API int q4_mlp_gate_up_f16(const void *x, const q4_layer_t *gate, const q4_layer_t *up, int groupsize, void *h,
                               int M, int H, int I, void *stream);
 
+/* out fp16 [n] = silu(gate) * up, and its backward dgate = dout * up * silu'(gate), dup = dout * silu(gate), element by element
+ * with the fp16 roundings of the separate operations (model_attn_mlp_patch.py:224-228 above the decode sizes).  All pointers
+ * 16-byte aligned; the outputs overlap no input. */
+Q4_API int q4_silu_mul_f16(const void *gate, const void *up, void *out, long long n, void *stream);
+Q4_API int q4_silu_mul_bwd_f16(const void *dout, const void *gate, const void *up, void *dgate, void *dup, long long n, void *stream);
+
 /* q4_gemv_f16 for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same product, same arguments
  * minus the workspace: the split-K accumulators live in a device array inside the library (4 MiB per device that
