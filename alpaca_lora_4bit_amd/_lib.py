@@ -6,7 +6,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libq4gptq.so")
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 _lib = None
 
@@ -58,6 +58,28 @@ class Layer(ctypes.Structure):
     _fields_ = [("qweight", _vp), ("qzeros", _vp), ("scales", _vp)]
 
 
+class LoraDown(ctypes.Structure):
+    """q4_lora_down_t of include/q4_gptq.h."""
+    _fields_ = [("inp", _vp), ("w", _vp), ("out", _vp), ("w_sr", _i), ("w_sc", _i), ("w_is_f32", _i), ("C", _i), ("R", _i),
+                ("drop", ctypes.POINTER(Dropout))]
+
+
+class LoraUpdate(ctypes.Structure):
+    """q4_lora_update_t of include/q4_gptq.h."""
+    _fields_ = [("a", _vp), ("b", _vp), ("y", _vp), ("a_sr", _i), ("a_sc", _i), ("a_is_f32", _i), ("b_sn", _i), ("b_sr", _i),
+                ("b_is_f32", _i), ("N", _i), ("R", _i), ("alpha", _f)]
+
+
+class LoraGrad(ctypes.Structure):
+    """q4_lora_grad_t of include/q4_gptq.h."""
+    _fields_ = [("p", _vp), ("inp", _vp), ("out", _vp), ("o_sr", _i), ("o_sc", _i), ("C", _i), ("alpha", _f),
+                ("drop", ctypes.POINTER(Dropout))]
+
+
+SIGNATURES["q4_lora_down_grouped_f16"] = (_i, [ctypes.POINTER(LoraDown), _i, _i, _vp])
+SIGNATURES["q4_lora_update_fits"] = (_i, [ctypes.POINTER(LoraUpdate), _i, _i])
+SIGNATURES["q4_lora_update_grouped_f16"] = (_i, [ctypes.POINTER(LoraUpdate), _i, _vp, _i, _i, _vp])
+SIGNATURES["q4_lora_grad_grouped_f32"] = (_i, [ctypes.POINTER(LoraGrad), _i, _i, _i, _vp, _sz, _vp])
 SIGNATURES["q4_mlp_decode_workspace_bytes"] = (_sz, [_i, _i, _i])
 SIGNATURES["q4_mlp_decode_status_offset"] = (_sz, [_i, _i, _i])
 SIGNATURES["q4_mlp_decode_f16"] = (_i, [_vp, ctypes.POINTER(Layer), ctypes.POINTER(Layer), ctypes.POINTER(Layer), _i, _vp, _vp, _vp,

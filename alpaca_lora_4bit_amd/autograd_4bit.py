@@ -153,6 +153,20 @@ def _is_all_zero(bias):
     return verdict
 
 
+def _has_bias(layer):
+    return not layer.disable_bias and not _is_all_zero(layer.bias)
+
+
+def _decode_call(layer, x):
+    """Whether layer(x) goes straight to the decode kernel: fp16, a handful of rows, nothing to differentiate."""
+    if not (layer.bits == 4 and not layer.is_v1_model and x.dtype == torch.float16 and backend == 'cuda'
+            and not torch.is_grad_enabled() and mm4b.use_new and mm4b.auto_switch):
+        return False
+    K = layer.in_features
+    rows = x.numel() // K if K else 0
+    return 1 <= rows <= min(int(mm4b.auto_switch_thd), quant_hip.MAX_GEMV_ROWS) and x.shape[-1] == K
+
+
 class Autograd4bitQuantLinear(nn.Module):
     """GPTQ 4-bit linear layer; buffers as registered at autograd_4bit.py:166-189."""
 
@@ -179,22 +193,19 @@ class Autograd4bitQuantLinear(nn.Module):
         self.register_buffer('qweight', torch.empty((in_features * bits // 32, out_features), dtype=torch.int32))
 
     def forward(self, x):
-        if (self.bits == 4 and not self.is_v1_model and x.dtype == torch.float16 and backend == 'cuda'
-                and not torch.is_grad_enabled() and mm4b.use_new and mm4b.auto_switch):
-            # decode: the same call matmul4bit -> _matmul4bit_v2 would end in, without the stops on the way
-            rows = x.numel() // self.in_features if self.in_features else 0
-            if 1 <= rows <= min(int(mm4b.auto_switch_thd), quant_hip.MAX_GEMV_ROWS) and x.shape[-1] == self.in_features:
+        if _decode_call(self, x):
+            # the same call matmul4bit -> _matmul4bit_v2 would end in, without the stops on the way
+            # a member of a group made by model_attn_mlp_patch (q|k|v, gate|up): the first member called runs ONE
+            # launch over every member's own tensors and the others pick their result up
+            group = self.__dict__.get('_q4_group')
+            out = group.run(self, x) if group is not None else None
+            if out is None:
                 scales = self.scales
-                # a member of a group made by model_attn_mlp_patch (q|k|v, gate|up): the first member called runs ONE
-                # launch over every member's own tensors and the others pick their result up
-                group = self.__dict__.get('_q4_group')
-                out = group.run(self, x) if group is not None else None
-                if out is None:
-                    out = quant_hip.gemv(x, self.qweight, self.qzeros, scales if scales.dtype == torch.float16 else scales.half(),
-                                         self.g_idx, self.groupsize, out_shape=x.shape[:-1] + (self.out_features,))
-                if not self.disable_bias and not _is_all_zero(self.bias):
-                    out += self.bias
-                return out
+                out = quant_hip.gemv(x, self.qweight, self.qzeros, scales if scales.dtype == torch.float16 else scales.half(),
+                                     self.g_idx, self.groupsize, out_shape=x.shape[:-1] + (self.out_features,))
+            if not self.disable_bias and not _is_all_zero(self.bias):
+                out += self.bias
+            return out
         group = self.__dict__.get('_q4_group')
         if group is not None and self.bits == 4 and not self.is_v1_model and backend == 'cuda':
             # a member of a group made by model_attn_mlp_patch, above the decode sizes: one grouped GEMM launch for
@@ -428,6 +439,13 @@ class AutogradMatmul4bitGroup(torch.autograd.Function):
     Returns one output per layer."""
 
     @staticmethod
+    def _down(specs):
+        """The rank-r products of the layers that have an adapter, together; None stays None."""
+        todo = [s for s in specs if s is not None]
+        outs = iter(quant_hip.lora_down_grouped(todo) if todo else ())
+        return [None if s is None else next(outs) for s in specs]
+
+    @staticmethod
     @custom_fwd(device_type='cuda', cast_inputs=None)
     def forward(ctx, x, groupsize, specs, *tensors):
         n = len(specs)
@@ -437,20 +455,19 @@ class AutogradMatmul4bitGroup(torch.autograd.Function):
         if x2.dtype != torch.float16:
             x2 = x2.half()
         x2 = x2.contiguous()
-        fwd, xas, adapters, dropouts = [], [], [], []
+        fwd, biases, adapters, dropouts = [], [], [], []
         for (qweight, scales, zeros, bias, lora_a, lora_b), (scaling, drop_p, drop_seed) in zip(lay, specs):
             if bias is not None and bias.dtype != torch.float16:
                 bias = bias.half()
             dropout = (int(drop_seed), float(drop_p)) if drop_p and drop_p > 0.0 else None
+            a = b = None
             if lora_a is not None:
                 a = AutogradMatmul4bitLora._kernel_dtype(lora_a.detach())
                 b = AutogradMatmul4bitLora._kernel_dtype(lora_b.detach())
-                xa = quant_hip.lora_down(x2, a, dropout=dropout)
-                fwd.append((qweight, zeros, scales, bias, xa, b.t(), scaling))
-            else:
-                a = b = xa = None
-                fwd.append((qweight, zeros, scales, bias, None, None, 1.0))
-            xas.append(xa); adapters.append((a, b)); dropouts.append(dropout)
+            biases.append(bias); adapters.append((a, b)); dropouts.append(dropout)
+        xas = AutogradMatmul4bitGroup._down([None if a is None else (x2, a, d) for (a, _), d in zip(adapters, dropouts)])
+        for (qweight, scales, zeros, _, _, _), bias, xa, (a, b), spec in zip(lay, biases, xas, adapters, specs):
+            fwd.append((qweight, zeros, scales, bias, xa, None if b is None else b.t(), 1.0 if b is None else spec[0]))
         ys = quant_hip.gemm_grouped_fwd(x2, fwd, groupsize)
         lead = tuple(x.shape[:-1])
         saved = [x2]
@@ -486,21 +503,32 @@ class AutogradMatmul4bitGroup(torch.autograd.Function):
                 if dy.dtype != torch.float16:
                     dy = dy.half()
                 dy = dy.contiguous()
-            dyb = quant_hip.lora_down(dy, b.t()) if a is not None else None
             dys.append(dy)
-            layers.append((qweight, zeros, scales, dyb, a, ctx.specs[i][0] if a is not None else 1.0, ctx.dropouts[i]))
-            per_layer.append((xa, dyb, dy))
+            per_layer.append((qweight, zeros, scales, xa, a, b))
+        dybs = AutogradMatmul4bitGroup._down([None if b is None else (dy, b.t(), None) for dy, (*_, b) in zip(dys, per_layer)])
+        for (qweight, zeros, scales, _, a, _), dyb, spec, dropout in zip(per_layer, dybs, ctx.specs, ctx.dropouts):
+            layers.append((qweight, zeros, scales, dyb, a, spec[0] if a is not None else 1.0, dropout))
         dx = None
         if ctx.needs_input_grad[0]:
             lead = next((tuple(g.shape[:-1]) for g in grad_outputs if g is not None), (x2.shape[0],))
             dx = quant_hip.gemm_grouped_bwd_dx(dys, layers, ctx.groupsize, out_shape=lead + (x2.shape[1],))
+        together = []                                    # layers whose two gradients go out with those of the others
         for i in range(n):
-            if ctx.has_adapter[i]:
-                xa, dyb, dy = per_layer[i]
-                need_a, need_b = ctx.needs_input_grad[3 + 6 * i + 4], ctx.needs_input_grad[3 + 6 * i + 5]
-                if need_a or need_b:
-                    grads[6 * i + 4], grads[6 * i + 5] = AutogradMatmul4bitLora._adapter_grads(
-                        dyb, x2, xa, dy, ctx.specs[i][0], ctx.dropouts[i], need_a, need_b, ctx.ab_dtypes[i])
+            if not ctx.has_adapter[i]:
+                continue
+            xa, dyb, dy = per_layer[i][3], dybs[i], dys[i]
+            need_a, need_b = ctx.needs_input_grad[3 + 6 * i + 4], ctx.needs_input_grad[3 + 6 * i + 5]
+            if (need_a and need_b and quant_hip.lora_grad_pair_takes(x2.shape[0], x2.shape[1], dy.shape[1], dyb.shape[1])
+                    and (not together or dybs[together[0]].shape == dyb.shape)):
+                together.append(i)
+            elif need_a or need_b:
+                grads[6 * i + 4], grads[6 * i + 5] = AutogradMatmul4bitLora._adapter_grads(
+                    dyb, x2, xa, dy, ctx.specs[i][0], ctx.dropouts[i], need_a, need_b, ctx.ab_dtypes[i])
+        if together:
+            pairs = quant_hip.lora_grad_grouped([(dybs[i], x2, per_layer[i][3], dys[i], ctx.specs[i][0], ctx.dropouts[i])
+                                                 for i in together])
+            for i, (da, db) in zip(together, pairs):
+                grads[6 * i + 4], grads[6 * i + 5] = da.to(ctx.ab_dtypes[i][0]), db.to(ctx.ab_dtypes[i][1])
         return (dx, None, None) + tuple(grads)
 
 

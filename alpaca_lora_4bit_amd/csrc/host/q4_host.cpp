@@ -525,75 +525,153 @@ at::Tensor gemm_grouped_bwd_dx(const std::vector<at::Tensor>& dys, const std::ve
     return dx;
 }
 
-at::Tensor lora_down(const at::Tensor& inp, const at::Tensor& w, const c10::optional<std::pair<int64_t, double>>& dropout) {
-    TORCH_CHECK_VALUE(inp.is_cuda() && inp.scalar_type() == at::kHalf && inp.dim() == 2 && inp.is_contiguous(),
-                      "inp must be a contiguous float16 [M, C] CUDA tensor");
-    const int64_t M = inp.size(0), C = inp.size(1);
-    TORCH_CHECK_VALUE(w.dim() == 2 && w.size(1) == C && w.device() == inp.device(), "w must be an [R, C] view on the same device");
-    TORCH_CHECK_VALUE(w.scalar_type() == at::kHalf || w.scalar_type() == at::kFloat, "w must be float16 or float32");
-    const int64_t R = w.size(0);
-    at::Tensor o = at::empty({M, R}, inp.options());
-    if (M == 0) return o;
-    TORCH_CHECK_VALUE(R >= 1 && R <= 64 && C % 32 == 0, "lora_down needs 1 <= R <= 64 and C % 32 == 0");
-    TORCH_CHECK_VALUE(w.stride(0) >= 1 && w.stride(1) >= 1, "w must have positive strides");
-    q4_dropout_t d;
-    const bool has_drop = fill_drop(dropout, &d);
-    Launch L(inp.device());
-    const int rc = q4_lora_down_f16(inp.data_ptr(), w.data_ptr(), (int)w.stride(0), (int)w.stride(1), w.scalar_type() == at::kFloat,
-                                    o.data_ptr(), (int)M, (int)C, (int)R, has_drop ? &d : nullptr, L.stream);
-    if (rc != Q4_OK) raise_q4(rc, "q4_lora_down_f16");
-    return o;
+using DropOpt = c10::optional<std::pair<int64_t, double>>;
+// (input, adapter matrix view, dropout) of one down projection
+using DownSpec = std::tuple<at::Tensor, at::Tensor, DropOpt>;
+
+// the products of 1..4 adapters with the same number of rows, in as few launches as their layouts allow
+std::vector<at::Tensor> lora_down_grouped(const std::vector<DownSpec>& specs) {
+    const size_t n = specs.size();
+    TORCH_CHECK_VALUE(n >= 1 && n <= 4, "lora_down_grouped takes 1..4 products");
+    std::vector<at::Tensor> outs;
+    q4_lora_down_t probs[4];
+    q4_dropout_t drops[4];
+    const at::Tensor& first = std::get<0>(specs[0]);
+    for (size_t i = 0; i < n; ++i) {
+        const at::Tensor& inp = std::get<0>(specs[i]);
+        const at::Tensor& w = std::get<1>(specs[i]);
+        TORCH_CHECK_VALUE(inp.is_cuda() && inp.scalar_type() == at::kHalf && inp.dim() == 2 && inp.is_contiguous(),
+                          "inp must be a contiguous float16 [M, C] CUDA tensor");
+        TORCH_CHECK_VALUE(inp.device() == first.device() && inp.size(0) == first.size(0), "the inputs must share rows and device");
+        const int64_t M = inp.size(0), C = inp.size(1);
+        TORCH_CHECK_VALUE(w.dim() == 2 && w.size(1) == C && w.device() == inp.device(), "w must be an [R, C] view on the same device");
+        TORCH_CHECK_VALUE(w.scalar_type() == at::kHalf || w.scalar_type() == at::kFloat, "w must be float16 or float32");
+        const int64_t R = w.size(0);
+        outs.push_back(at::empty({M, R}, inp.options()));
+        if (M == 0) continue;
+        TORCH_CHECK_VALUE(R >= 1 && R <= 64 && C % 32 == 0, "lora_down needs 1 <= R <= 64 and C % 32 == 0");
+        TORCH_CHECK_VALUE(w.stride(0) >= 1 && w.stride(1) >= 1, "w must have positive strides");
+        const bool has_drop = fill_drop(std::get<2>(specs[i]), &drops[i]);
+        probs[i] = {inp.data_ptr(), w.data_ptr(), outs[i].data_ptr(), (int)w.stride(0), (int)w.stride(1),
+                    w.scalar_type() == at::kFloat, (int)C, (int)R, has_drop ? &drops[i] : nullptr};
+    }
+    if (first.size(0) == 0) return outs;
+    Launch L(first.device());
+    const int rc = q4_lora_down_grouped_f16(probs, (int)n, (int)first.size(0), L.stream);
+    if (rc != Q4_OK) raise_q4(rc, n == 1 ? "q4_lora_down_f16" : "q4_lora_down_grouped_f16");
+    return outs;
 }
 
-// y += alpha * (x @ a^T) @ b^T in place (x @ a^T in fp16), two launches
-void lora_update(const at::Tensor& x, const at::Tensor& a, const at::Tensor& b, const at::Tensor& y, double alpha) {
-    TORCH_CHECK_VALUE(y.is_cuda() && y.scalar_type() == at::kHalf && y.dim() == 2 && y.is_contiguous() && y.device() == x.device() &&
-                      x.dim() == 2 && y.size(0) == x.size(0), "y must be a contiguous float16 [M, N] tensor beside x [M, K]");
-    TORCH_CHECK_VALUE(b.dim() == 2 && b.size(0) == y.size(1) && b.size(1) == a.size(0) && b.device() == y.device(),
-                      "b must be an [N, R] view on the same device");
-    TORCH_CHECK_VALUE(b.scalar_type() == at::kHalf || b.scalar_type() == at::kFloat, "b must be float16 or float32");
-    if (b.stride(0) < 1 || b.stride(1) < 1 || b.stride(0) > INT32_MAX || b.stride(1) > INT32_MAX) {     // an expanded view
-        const at::Tensor copy = at::empty({b.size(0), b.size(1)}, b.options());
-        copy.copy_(b);
-        return lora_update(x, a, copy, y, alpha);
+at::Tensor lora_down(const at::Tensor& inp, const at::Tensor& w, const DropOpt& dropout) {
+    return lora_down_grouped({DownSpec(inp, w, dropout)})[0];
+}
+
+// (lora_A [R, K], lora_B [N, R], result [M, N] to update in place, scale) of one adapter
+using UpdateSpec = std::tuple<at::Tensor, at::Tensor, at::Tensor, double>;
+
+// y_i += alpha_i * (x @ a_i^T) @ b_i^T in place (x @ a^T in fp16): one launch where it takes all of them, else two per adapter
+void lora_update_grouped(const at::Tensor& x, const std::vector<UpdateSpec>& specs) {
+    const size_t n = specs.size();
+    TORCH_CHECK_VALUE(n >= 1 && n <= 4, "lora_update_grouped takes 1..4 adapters");
+    TORCH_CHECK_VALUE(x.is_cuda() && x.scalar_type() == at::kHalf && x.dim() == 2 && x.is_contiguous(),
+                      "inp must be a contiguous float16 [M, C] CUDA tensor");
+    const int64_t M = x.size(0), K = x.size(1);
+    q4_lora_update_t probs[4];
+    std::vector<at::Tensor> copies;
+    for (size_t i = 0; i < n; ++i) {
+        const at::Tensor& a = std::get<0>(specs[i]);
+        at::Tensor b = std::get<1>(specs[i]);
+        const at::Tensor& y = std::get<2>(specs[i]);
+        TORCH_CHECK_VALUE(y.is_cuda() && y.scalar_type() == at::kHalf && y.dim() == 2 && y.is_contiguous() && y.device() == x.device() &&
+                          y.size(0) == M, "y must be a contiguous float16 [M, N] tensor beside x [M, K]");
+        TORCH_CHECK_VALUE(a.dim() == 2 && a.size(1) == K && a.device() == x.device(), "w must be an [R, C] view on the same device");
+        TORCH_CHECK_VALUE(a.scalar_type() == at::kHalf || a.scalar_type() == at::kFloat, "w must be float16 or float32");
+        TORCH_CHECK_VALUE(b.dim() == 2 && b.size(0) == y.size(1) && b.size(1) == a.size(0) && b.device() == y.device(),
+                          "b must be an [N, R] view on the same device");
+        TORCH_CHECK_VALUE(b.scalar_type() == at::kHalf || b.scalar_type() == at::kFloat, "b must be float16 or float32");
+        if (M == 0) continue;
+        const int64_t R = a.size(0);
+        TORCH_CHECK_VALUE(R >= 1 && R <= 64 && K % 32 == 0, "lora_down needs 1 <= R <= 64 and C % 32 == 0");
+        TORCH_CHECK_VALUE(a.stride(0) >= 1 && a.stride(1) >= 1, "w must have positive strides");
+        if (b.stride(0) < 1 || b.stride(1) < 1 || b.stride(0) > INT32_MAX || b.stride(1) > INT32_MAX) {     // an expanded view
+            copies.push_back(at::empty({b.size(0), b.size(1)}, b.options()).copy_(b));
+            b = copies.back();
+        }
+        probs[i] = {a.data_ptr(), b.data_ptr(), y.data_ptr(), (int)a.stride(0), (int)a.stride(1), a.scalar_type() == at::kFloat,
+                    (int)b.stride(0), (int)b.stride(1), b.scalar_type() == at::kFloat, (int)y.size(1), (int)R,
+                    (float)std::get<3>(specs[i])};
     }
-    const at::Tensor xa = lora_down(x, a, c10::nullopt);
-    if (y.size(0) == 0) return;
-    Launch L(y.device());
-    const int rc = q4_lora_up_f16(xa.data_ptr(), b.data_ptr(), (int)b.stride(0), (int)b.stride(1), b.scalar_type() == at::kFloat,
-                                  y.data_ptr(), (float)alpha, (int)y.size(0), (int)y.size(1), (int)a.size(0), L.stream);
-    if (rc != Q4_OK) raise_q4(rc, "q4_lora_up_f16");
+    if (M == 0) return;
+    Launch L(x.device());
+    if (M <= INT32_MAX && q4_lora_update_fits(probs, (int)n, (int)M)) {
+        const int rc = q4_lora_update_grouped_f16(probs, (int)n, x.data_ptr(), (int)M, (int)K, L.stream);
+        if (rc != Q4_OK) raise_q4(rc, "q4_lora_update_grouped_f16");
+        return;
+    }
+    for (size_t i = 0; i < n; ++i) {
+        const q4_lora_update_t& p = probs[i];
+        const at::Tensor xa = lora_down(x, std::get<0>(specs[i]), c10::nullopt);
+        const int rc = q4_lora_up_f16(xa.data_ptr(), p.b, p.b_sn, p.b_sr, p.b_is_f32, p.y, p.alpha, (int)M, p.N, p.R, L.stream);
+        if (rc != Q4_OK) raise_q4(rc, "q4_lora_up_f16");
+    }
+}
+
+void lora_update(const at::Tensor& x, const at::Tensor& a, const at::Tensor& b, const at::Tensor& y, double alpha) {
+    lora_update_grouped(x, {UpdateSpec(a, b, y, alpha)});
+}
+
+// (p1, inp1, p2, inp2, alpha, dropout of inp1) of one layer's two adapter gradients
+using GradSpec = std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, double, DropOpt>;
+
+// both gradients of 1..4 layers whose rank-R operands share their shape: one launch and one for the reductions
+std::vector<std::pair<at::Tensor, at::Tensor>> lora_grad_grouped(const std::vector<GradSpec>& specs) {
+    const size_t n = specs.size();
+    TORCH_CHECK_VALUE(n >= 1 && n <= 4, "lora_grad_grouped takes 1..4 layers");
+    const at::Tensor& first = std::get<0>(specs[0]);
+    std::vector<std::pair<at::Tensor, at::Tensor>> outs;
+    q4_lora_grad_t probs[8];
+    q4_dropout_t drops[4];
+    size_t need = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const at::Tensor &p1 = std::get<0>(specs[i]), &in1 = std::get<1>(specs[i]), &p2 = std::get<2>(specs[i]), &in2 = std::get<3>(specs[i]);
+        for (const auto& pr : {std::make_pair(&p1, &in1), std::make_pair(&p2, &in2)}) {
+            const at::Tensor& p = *pr.first;
+            const at::Tensor& in = *pr.second;
+            TORCH_CHECK_VALUE(p.is_cuda() && p.scalar_type() == at::kHalf && p.dim() == 2 && p.is_contiguous(),
+                              "p must be a contiguous float16 [M, R] CUDA tensor");
+            TORCH_CHECK_VALUE(in.scalar_type() == at::kHalf && in.dim() == 2 && in.is_contiguous() && in.device() == p.device() &&
+                              in.size(0) == p.size(0), "inp must be a contiguous float16 [M, C] tensor on the same device");
+            TORCH_CHECK_VALUE(p.sizes() == first.sizes() && p.device() == first.device(),
+                              "the rank-R operands must share shape and device");
+        }
+        const int64_t M = p1.size(0), R = p1.size(1), C1 = in1.size(1), C2 = in2.size(1);
+        TORCH_CHECK_VALUE(((R >= 2 && R <= 32 && R % 2 == 0) || (R > 32 && R <= 64 && R % 8 == 0)) && C1 % 8 == 0 && C2 % 8 == 0,
+                          "lora_grad_pair needs an even R in 2..32 or a multiple of 8 up to 64, and C % 8 == 0");
+        const auto opt = at::TensorOptions().dtype(at::kFloat).device(p1.device());
+        if (M == 0) {
+            outs.emplace_back(at::zeros({R, C1}, opt), at::zeros({C2, R}, opt));
+            continue;
+        }
+        outs.emplace_back(at::empty({R, C1}, opt), at::empty({C2, R}, opt));
+        const bool has_drop = fill_drop(std::get<5>(specs[i]), &drops[i]);
+        const float alpha = (float)std::get<4>(specs[i]);
+        probs[2 * i] = {p1.data_ptr(), in1.data_ptr(), outs[i].first.data_ptr<float>(), (int)C1, 1, (int)C1, alpha,
+                        has_drop ? &drops[i] : nullptr};                       // the mask applies to inp1 only
+        probs[2 * i + 1] = {p2.data_ptr(), in2.data_ptr(), outs[i].second.data_ptr<float>(), 1, (int)R, (int)C2, alpha, nullptr};
+        need += q4_lora_grad_workspace_bytes((int)M, (int)C1, (int)R) + q4_lora_grad_workspace_bytes((int)M, (int)C2, (int)R);
+    }
+    if (first.size(0) == 0) return outs;
+    Launch L(first.device());
+    size_t have = 0;
+    void* ws = scratch_workspace(first.device(), L.stream, need, &have);
+    const int rc = q4_lora_grad_grouped_f32(probs, (int)(2 * n), (int)first.size(0), (int)first.size(1), ws, have, L.stream);
+    if (rc != Q4_OK) raise_q4(rc, n == 1 ? "q4_lora_grad_pair_f32" : "q4_lora_grad_grouped_f32");
+    return outs;
 }
 
 std::pair<at::Tensor, at::Tensor> lora_grad_pair(const at::Tensor& p1, const at::Tensor& in1, const at::Tensor& p2,
-                                                 const at::Tensor& in2, double alpha,
-                                                 const c10::optional<std::pair<int64_t, double>>& dropout) {
-    for (const auto& pr : {std::make_pair(&p1, &in1), std::make_pair(&p2, &in2)}) {
-        const at::Tensor& p = *pr.first;
-        const at::Tensor& in = *pr.second;
-        TORCH_CHECK_VALUE(p.is_cuda() && p.scalar_type() == at::kHalf && p.dim() == 2 && p.is_contiguous(),
-                          "p must be a contiguous float16 [M, R] CUDA tensor");
-        TORCH_CHECK_VALUE(in.scalar_type() == at::kHalf && in.dim() == 2 && in.is_contiguous() && in.device() == p.device() &&
-                          in.size(0) == p.size(0), "inp must be a contiguous float16 [M, C] tensor on the same device");
-    }
-    TORCH_CHECK_VALUE(p1.sizes() == p2.sizes() && p1.device() == p2.device(), "the two rank-R operands must share shape and device");
-    const int64_t M = p1.size(0), R = p1.size(1), C1 = in1.size(1), C2 = in2.size(1);
-    TORCH_CHECK_VALUE(((R >= 2 && R <= 32 && R % 2 == 0) || (R > 32 && R <= 64 && R % 8 == 0)) && C1 % 8 == 0 && C2 % 8 == 0,
-                      "lora_grad_pair needs an even R in 2..32 or a multiple of 8 up to 64, and C % 8 == 0");
-    const auto opt = at::TensorOptions().dtype(at::kFloat).device(p1.device());
-    if (M == 0) return {at::zeros({R, C1}, opt), at::zeros({C2, R}, opt)};
-    at::Tensor o1 = at::empty({R, C1}, opt), o2 = at::empty({C2, R}, opt);
-    q4_dropout_t d;
-    const bool has_drop = fill_drop(dropout, &d);
-    Launch L(p1.device());
-    size_t have = 0;
-    const size_t need = q4_lora_grad_workspace_bytes((int)M, (int)C1, (int)R) + q4_lora_grad_workspace_bytes((int)M, (int)C2, (int)R);
-    void* ws = scratch_workspace(p1.device(), L.stream, need, &have);
-    const int rc = q4_lora_grad_pair_f32(p1.data_ptr(), in1.data_ptr(), o1.data_ptr<float>(), (int)C1, 1, (int)C1,
-                                         p2.data_ptr(), in2.data_ptr(), o2.data_ptr<float>(), 1, (int)R, (int)C2,
-                                         (float)alpha, (int)M, (int)R, has_drop ? &d : nullptr, ws, have, L.stream);
-    if (rc != Q4_OK) raise_q4(rc, "q4_lora_grad_pair_f32");
-    return {o1, o2};
+                                                 const at::Tensor& in2, double alpha, const DropOpt& dropout) {
+    return lora_grad_grouped({GradSpec(p1, in1, p2, in2, alpha, dropout)})[0];
 }
 
 // Clears the cached GEMV accumulators of every stream (after an aborted run, or when a caller is unsure).
@@ -647,6 +725,9 @@ PYBIND11_MODULE(_q4_host, m) {
     m.def("gemm_grouped_bwd_dx", &gemm_grouped_bwd_dx, py::arg("dys"), py::arg("layers"), py::arg("groupsize"),
           py::arg("out_shape") = py::none());
     m.def("lora_down", &lora_down, py::arg("inp"), py::arg("w"), py::arg("dropout") = py::none());
+    m.def("lora_down_grouped", &lora_down_grouped, py::arg("specs"));
+    m.def("lora_update_grouped", &lora_update_grouped, py::arg("x"), py::arg("specs"));
+    m.def("lora_grad_grouped", &lora_grad_grouped, py::arg("specs"));
     m.def("lora_update", &lora_update, py::arg("x"), py::arg("a"), py::arg("b"), py::arg("y"), py::arg("alpha"));
     m.def("lora_grad_pair", &lora_grad_pair, py::arg("p1"), py::arg("inp1"), py::arg("p2"), py::arg("inp2"), py::arg("alpha"),
           py::arg("dropout") = py::none());

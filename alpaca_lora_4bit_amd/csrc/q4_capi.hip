@@ -19,11 +19,9 @@ int q4_launch_dropout_keep(uint8_t*, int, int, const q4_drop_args*, hipStream_t)
 size_t q4_gemm_plan_workspace(int, int, int, int);
 int q4_gemv_sorted_applicable(int, int);
 int q4_launch_gemv_v1(const void*, const int32_t*, const void*, const void*, void*, int, int, int, int, void*, hipStream_t);
-int q4_launch_lora_down(const void*, const void*, int, int, int, void*, int, int, int, const q4_drop_args*, hipStream_t);
-int q4_launch_lora_grad(const void*, const void*, float*, int, int, float, int, int, int, const q4_drop_args*, void*,
-                        hipStream_t);
-int q4_launch_lora_grad_pair(const void*, const void*, float*, int, int, int, const void*, const void*, float*, int, int, int,
-                             float, int, int, const q4_drop_args*, void*, hipStream_t);
+int q4_launch_lora_down(const q4_lora_down_t*, const q4_drop_args* const*, int, int, hipStream_t);
+int q4_launch_lora_update(const q4_lora_update_t*, int, const void*, int, int, hipStream_t);
+int q4_launch_lora_grad(const q4_lora_grad_t*, const q4_drop_args* const*, int, int, int, void*, hipStream_t);
 int q4_launch_lora_up(const void*, const void*, int, int, int, void*, float, int, int, int, hipStream_t);
 size_t q4_lora_grad_workspace(int, int, int);
 int q4_launch_gemv_group(int, const void* const*, const int32_t* const*, const int32_t* const*, const void* const*,
@@ -81,7 +79,7 @@ int check_layer(const void* qweight, const void* qzeros, const void* scales, con
 }
 }  // namespace
 
-extern "C" int q4_abi_version(void) { return 17; }
+extern "C" int q4_abi_version(void) { return 18; }
 
 extern "C" const char* q4_error_string(int code) {
     switch (code) {
@@ -449,19 +447,46 @@ extern "C" int q4_gemm_grouped_bwd_dx_f16(const q4_gemm_layer_t* layers, int n_l
     return gemm_grouped_common(0, layers, n_layers, groupsize, dx, M, K, workspace, workspace_bytes, stream);
 }
 
+extern "C" int q4_lora_down_grouped_f16(const q4_lora_down_t* probs, int n, int M, void* stream) {
+    if (!probs) return Q4_ERR_NULL_POINTER;
+    if (n < 1 || n > 4) return Q4_ERR_BAD_SHAPE;
+    q4_drop_args das[4];
+    const q4_drop_args* dps[4];
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_down_t& p = probs[i];
+        if (!p.in || !p.w || !p.out) return Q4_ERR_NULL_POINTER;
+        if (!make_drop(p.drop, &das[i], &dps[i])) return Q4_ERR_BAD_SHAPE;
+        if (M < 1 || p.C < 32 || (p.C % 32) != 0 || p.R < 1 || p.R > 64 || p.w_sr < 1 || p.w_sc < 1) return Q4_ERR_BAD_SHAPE;
+        /* 32-bit buffer offsets: the 16-row block of `in` and the span of the adapter matrix */
+        if ((long long)p.C * 32 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;
+        if (((long long)(p.R - 1) * p.w_sr + (long long)(p.C - 1) * p.w_sc + 1) * (p.w_is_f32 ? 4 : 2) >= 0x70000000ll)
+            return Q4_ERR_BAD_SHAPE;
+        if (misaligned(p.in) || (reinterpret_cast<uintptr_t>(p.out) & 1u) ||
+            (reinterpret_cast<uintptr_t>(p.w) & (p.w_is_f32 ? 3u : 1u))) return Q4_ERR_MISALIGNED;
+    }
+    return q4_launch_lora_down(probs, dps, n, M, (hipStream_t)stream);
+}
+
 extern "C" int q4_lora_down_f16(const void* in, const void* w, int w_sr, int w_sc, int w_is_f32, void* out,
                                 int M, int C, int R, const q4_dropout_t* drop, void* stream) {
-    if (!in || !w || !out) return Q4_ERR_NULL_POINTER;
-    q4_drop_args da;
-    const q4_drop_args* dp;
-    if (!make_drop(drop, &da, &dp)) return Q4_ERR_BAD_SHAPE;
-    if (M < 1 || C < 32 || (C % 32) != 0 || R < 1 || R > 64 || w_sr < 1 || w_sc < 1) return Q4_ERR_BAD_SHAPE;
-    /* 32-bit buffer offsets: the 16-row block of `in` and the span of the adapter matrix */
-    if ((long long)C * 32 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;
-    if (((long long)(R - 1) * w_sr + (long long)(C - 1) * w_sc + 1) * (w_is_f32 ? 4 : 2) >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;
-    if (misaligned(in) || (reinterpret_cast<uintptr_t>(out) & 1u) || (reinterpret_cast<uintptr_t>(w) & (w_is_f32 ? 3u : 1u)))
-        return Q4_ERR_MISALIGNED;
-    return q4_launch_lora_down(in, w, w_sr, w_sc, w_is_f32, out, M, C, R, dp, (hipStream_t)stream);
+    const q4_lora_down_t p = {in, w, out, w_sr, w_sc, w_is_f32, C, R, drop};
+    return q4_lora_down_grouped_f16(&p, 1, M, stream);
+}
+
+extern "C" int q4_lora_update_grouped_f16(const q4_lora_update_t* probs, int n, const void* x, int M, int K, void* stream) {
+    if (!probs || !x) return Q4_ERR_NULL_POINTER;
+    if (n < 1 || n > 4 || M < 1 || K < 32 || (K % 32) != 0) return Q4_ERR_BAD_SHAPE;
+    if ((long long)K * 32 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;                              /* 32-bit buffer offsets */
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_update_t& p = probs[i];
+        if (!p.a || !p.b || !p.y) return Q4_ERR_NULL_POINTER;
+        if (p.N < 1 || p.R < 1 || p.R > 64 || p.a_sr < 1 || p.a_sc < 1 || p.b_sn < 1 || p.b_sr < 1) return Q4_ERR_BAD_SHAPE;
+        if (((long long)(p.R - 1) * p.a_sr + K) * (p.a_is_f32 ? 4 : 2) >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;
+        if (reinterpret_cast<uintptr_t>(p.y) & 1u) return Q4_ERR_MISALIGNED;
+    }
+    if (misaligned(x)) return Q4_ERR_MISALIGNED;
+    if (!q4_lora_update_fits(probs, n, M)) return Q4_ERR_BAD_SHAPE;
+    return q4_launch_lora_update(probs, n, x, M, K, (hipStream_t)stream);
 }
 
 extern "C" int q4_lora_up_f16(const void* xa, const void* w, int w_sn, int w_sr, int w_is_f32, void* y, float alpha,
@@ -481,50 +506,48 @@ extern "C" size_t q4_lora_grad_workspace_bytes(int M, int C, int R) {
     return q4_lora_grad_workspace(M, C, R);
 }
 
-extern "C" int q4_lora_grad_f32(const void* p, const void* in, float* out, int o_sr, int o_sc, float alpha,
-                                int M, int C, int R, const q4_dropout_t* drop,
-                                void* workspace, size_t workspace_bytes, void* stream) {
-    if (!p || !in || !out) return Q4_ERR_NULL_POINTER;
-    q4_drop_args da;
-    const q4_drop_args* dp;
-    if (!make_drop(drop, &da, &dp)) return Q4_ERR_BAD_SHAPE;
-    if (M < 1 || C < 8 || (C % 8) != 0 || R < 2 || R > 32 || (R & 1) || o_sr < 1 || o_sc < 1) return Q4_ERR_BAD_SHAPE;
-    if ((long long)M * C * 2 >= 0x70000000ll || C > (1 << 20)) return Q4_ERR_BAD_SHAPE;     /* 32-bit buffer offsets */
-    if (misaligned(p) || misaligned(in) || (reinterpret_cast<uintptr_t>(out) & 3u)) return Q4_ERR_MISALIGNED;
-    const size_t need = q4_lora_grad_workspace(M, C, R);
+extern "C" int q4_lora_grad_grouped_f32(const q4_lora_grad_t* probs, int n, int M, int R, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+    if (!probs) return Q4_ERR_NULL_POINTER;
+    if (n < 1 || n > 8) return Q4_ERR_BAD_SHAPE;
+    q4_drop_args das[8];
+    const q4_drop_args* dps[8];
+    for (int i = 0; i < n; ++i)
+        if (!probs[i].p || !probs[i].in || !probs[i].out) return Q4_ERR_NULL_POINTER;
+    if (M < 1 || !lora_grad_pair_rank(R)) return Q4_ERR_BAD_SHAPE;
+    if (R > 32 && (long long)M * R * 2 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;          /* 32-bit buffer offsets of p */
+    bool aligned = true;
+    size_t need = 0;
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_grad_t& p = probs[i];
+        if (!make_drop(p.drop, &das[i], &dps[i])) return Q4_ERR_BAD_SHAPE;
+        if (p.C < 8 || (p.C % 8) != 0 || p.C > (1 << 20) || p.o_sr < 1 || p.o_sc < 1) return Q4_ERR_BAD_SHAPE;
+        if ((long long)M * p.C * 2 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;              /* 32-bit buffer offsets */
+        aligned = aligned && !misaligned(p.p) && !misaligned(p.in) && (reinterpret_cast<uintptr_t>(p.out) & 3u) == 0;
+        need += q4_lora_grad_workspace(M, p.C, R);
+    }
+    if (!aligned) return Q4_ERR_MISALIGNED;
     if (need > 0) {
         if (!workspace || workspace_bytes < need) return Q4_ERR_WORKSPACE;
         if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return Q4_ERR_MISALIGNED;
     }
-    return q4_launch_lora_grad(p, in, out, o_sr, o_sc, alpha, M, C, R, dp, workspace, (hipStream_t)stream);
+    return q4_launch_lora_grad(probs, dps, n, M, R, workspace, (hipStream_t)stream);
+}
+
+extern "C" int q4_lora_grad_f32(const void* p, const void* in, float* out, int o_sr, int o_sc, float alpha,
+                                int M, int C, int R, const q4_dropout_t* drop,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+    if (p && in && out && !lora_grad_rank(R)) return Q4_ERR_BAD_SHAPE;
+    const q4_lora_grad_t g = {p, in, out, o_sr, o_sc, C, alpha, drop};
+    return q4_lora_grad_grouped_f32(&g, 1, M, R, workspace, workspace_bytes, stream);
 }
 
 extern "C" int q4_lora_grad_pair_f32(const void* p1, const void* in1, float* out1, int o1_sr, int o1_sc, int C1,
                                      const void* p2, const void* in2, float* out2, int o2_sr, int o2_sc, int C2,
                                      float alpha, int M, int R, const q4_dropout_t* drop1,
                                      void* workspace, size_t workspace_bytes, void* stream) {
-    if (!p1 || !in1 || !out1 || !p2 || !in2 || !out2) return Q4_ERR_NULL_POINTER;
-    q4_drop_args da;
-    const q4_drop_args* dp;
-    if (!make_drop(drop1, &da, &dp)) return Q4_ERR_BAD_SHAPE;
-    if (M < 1 || !lora_grad_pair_rank(R)) return Q4_ERR_BAD_SHAPE;
-    if (R > 32 && (long long)M * R * 2 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;          /* 32-bit buffer offsets of p */
-    const int Cs[2] = {C1, C2};
-    const int strides[4] = {o1_sr, o1_sc, o2_sr, o2_sc};
-    for (int i = 0; i < 2; ++i) {
-        if (Cs[i] < 8 || (Cs[i] % 8) != 0 || Cs[i] > (1 << 20) || strides[2 * i] < 1 || strides[2 * i + 1] < 1) return Q4_ERR_BAD_SHAPE;
-        if ((long long)M * Cs[i] * 2 >= 0x70000000ll) return Q4_ERR_BAD_SHAPE;               /* 32-bit buffer offsets */
-    }
-    if (misaligned(p1) || misaligned(in1) || misaligned(p2) || misaligned(in2) ||
-        (reinterpret_cast<uintptr_t>(out1) & 3u) || (reinterpret_cast<uintptr_t>(out2) & 3u))
-        return Q4_ERR_MISALIGNED;
-    const size_t need = q4_lora_grad_workspace(M, C1, R) + q4_lora_grad_workspace(M, C2, R);
-    if (need > 0) {
-        if (!workspace || workspace_bytes < need) return Q4_ERR_WORKSPACE;
-        if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return Q4_ERR_MISALIGNED;
-    }
-    return q4_launch_lora_grad_pair(p1, in1, out1, o1_sr, o1_sc, C1, p2, in2, out2, o2_sr, o2_sc, C2, alpha, M, R,
-                                    dp, workspace, (hipStream_t)stream);
+    const q4_lora_grad_t g[2] = {{p1, in1, out1, o1_sr, o1_sc, C1, alpha, drop1}, {p2, in2, out2, o2_sr, o2_sc, C2, alpha, nullptr}};
+    return q4_lora_grad_grouped_f32(g, 2, M, R, workspace, workspace_bytes, stream);
 }
 
 extern "C" float q4_dropout_scale(float p) {

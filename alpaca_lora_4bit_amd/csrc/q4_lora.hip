@@ -10,7 +10,8 @@
 // W is read in place with strides and in its own dtype (fp32 or fp16): no cast or transpose
 // kernels around the adapter.
 #include "q4_common.hpp"
-#include <stdlib.h>
+#include "q4_gptq.h"
+#include <algorithm>
 
 namespace q4 {
 
@@ -41,22 +42,40 @@ __device__ __forceinline__ half8_t to_half8(float4_t a, float4_t b) {
 enum WLayout { kRows = 0, kCols = 1, kAny = 2, kRowsT = 3 };
 constexpr int kDownWaves = 16;
 
+// The adapters of layers that run together (q | v) go out side by side, blockIdx.y = the problem: a single one of a few hundred
+// rows fills a fifth of the chip and its time is the latency of one burst of loads.  us for q and v of 4096 features at rank 8
+// with dropout, one launch each -> one launch: 200 rows
+// 12.1 -> 6.4, 1024 13.5 -> 7.1 (dy @ B without: 8.6 -> 4.6, 9.5 -> 5.8), 4096 of 5120 features 25.1 -> 23.4.  2048 rows at rank 64: 98 -> 50.
+constexpr int kDownProbs = 4;
+struct DownProb {
+    const half_t* in;         // [M, C]
+    const void* w;            // [R, C] through w_sr, w_sc
+    half_t* out;              // [M, R]
+    int w_sr, w_sc, C;
+    DropArgs drop;
+};
+struct DownArgs { DownProb p[kDownProbs]; };
+
+// LDS of a workgroup: the partial products, and the transposition tile of the staged layouts
+template <int RB, int WL> struct DownLds {
+    static constexpr bool kStaged = WL == kCols || WL == kRowsT;
+    static constexpr int UN = WL == kAny ? (RB == 1 ? 4 : RB == 2 ? 2 : 1) : (RB == 1 ? 8 : 4);   // steps whose loads are issued together
+    static constexpr int TRW = UN * 32 + 8;                     // padded row of the transposition tile (halves)
+    float red[kDownWaves][RB][256];
+    __attribute__((aligned(16))) half_t tr[kStaged ? kDownWaves : 1][16][kStaged ? TRW : 8];
+};
+
+// Leaves the wavefronts' partial 16 x 16 products of rows m0 .. m0 + rows - 1 in lds.red (no barrier after the last write).
 template <int RB, int WL, bool F32, int RQ>   // RQ: ceil(R/4) for kCols / kRowsT, else unused
-__global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(const half_t* __restrict__ in,
-                                                                    const void* __restrict__ w, int w_sr, int w_sc,
-                                                                    half_t* __restrict__ out, int M, int C, int R,
-                                                                    int rows, DropArgs drop) {
-    constexpr int NW = kDownWaves;
-    constexpr int UN = WL == kAny ? (RB == 1 ? 4 : RB == 2 ? 2 : 1) : (RB == 1 ? 8 : 4);   // steps whose loads are issued together
+__device__ __forceinline__ void lora_down_rows(DownLds<RB, WL>& lds, const half_t* __restrict__ in, const void* __restrict__ w,
+                                               int w_sr, int w_sc, int m0, int M, int C, int R, int rows, const DropArgs& drop) {
+    constexpr int NW = kDownWaves, UN = DownLds<RB, WL>::UN;
     constexpr int ES = F32 ? 4 : 2;
-    constexpr int TRW = UN * 32 + 8;                            // padded row of the transposition tile (halves)
-    __shared__ float red[NW][RB][256];
-    constexpr bool kStaged = WL == kCols || WL == kRowsT;
-    __shared__ __attribute__((aligned(16))) half_t tr[kStaged ? NW : 1][16][kStaged ? TRW : 8];
+    constexpr bool kStaged = DownLds<RB, WL>::kStaged;
+    auto& tr = lds.tr;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kk = lane >> 4, c = lane & 15;
-    const int m0 = blockIdx.x * rows;                           // rows = 16, 8 or 4: operand rows past it read as zero
     const int steps = C / 32;                                   // C is a multiple of 32
     const int s_begin = (steps * wave) / NW, s_end = (steps * (wave + 1)) / NW;
     const rsrc_t rs_in = make_rsrc(in + (size_t)m0 * C, (unsigned)min(rows, M - m0) * (unsigned)C * 2u);
@@ -215,15 +234,30 @@ __global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(const half_t
 #pragma unroll
     for (int b = 0; b < RB; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[wave][b][(4 * kk + r) * 16 + c] = acc[b][r];
-    __syncthreads();
-    for (int e = threadIdx.x; e < RB * 256; e += 64 * NW) {
-        const int b = e >> 8, i = e & 255;
-        float v = 0.f;
+        for (int r = 0; r < 4; ++r) lds.red[wave][b][(4 * kk + r) * 16 + c] = acc[b][r];
+}
+
+template <int RB, int WL>
+__device__ __forceinline__ float lora_down_sum(const DownLds<RB, WL>& lds, int b, int i) {     // element i of column block b
+    float v = 0.f;
 #pragma unroll
-        for (int wv = 0; wv < NW; ++wv) v += red[wv][b][i];
+    for (int wv = 0; wv < kDownWaves; ++wv) v += lds.red[wv][b][i];
+    return v;
+}
+
+template <int RB, int WL, bool F32, int RQ>
+__global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(DownArgs da, int M, int R, int rows) {
+    __shared__ DownLds<RB, WL> lds;
+    const DownProb& p = da.p[blockIdx.y];
+    const int m0 = blockIdx.x * rows;                           // rows = 16, 8 or 4: operand rows past it read as zero
+    const DropArgs drop = p.drop;
+    lora_down_rows<RB, WL, F32, RQ>(lds, p.in, p.w, p.w_sr, p.w_sc, m0, M, p.C, R, rows, drop);
+    __syncthreads();
+    for (int e = threadIdx.x; e < RB * 256; e += 64 * kDownWaves) {
+        const int b = e >> 8, i = e & 255;
+        const float v = lora_down_sum(lds, b, i);
         const int m = m0 + (i >> 4), j = 16 * b + (i & 15);
-        if ((i >> 4) < rows && m < M && j < R) out[(size_t)m * R + j] = (half_t)(v * drop.scale);
+        if ((i >> 4) < rows && m < M && j < R) p.out[(size_t)m * R + j] = (half_t)(v * drop.scale);
     }
 }
 
@@ -279,6 +313,70 @@ __global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restri
         if (m < rows) y[(size_t)(m0 + m) * N + n] = (half_t)fmaf(alpha, acc[m], old[m]);
 }
 
+// ---- the whole adapter of up to 16 rows in one launch ----------------------------------------
+// y += alpha * fp16(x @ A^T) @ B^T for the adapters of layers that share x.  Every workgroup forms x @ A^T for itself, exactly as
+// lora_down_kernel does (whose grid is one to four workgroups here: A comes from L2 either way, R * K * 4 bytes a workgroup),
+// and then updates 256 columns with lora_up_kernel's products in its order: the results are the two kernels' to the bit.  B and y
+// are on their way while x @ A^T is formed.  us for q and v of 4096 features at rank 8,
+// four launches -> one: 11.8 -> 4.5 at 1 row, 13.6 -> 5.4 at 4, 14.0 -> 7.9 at 16; rank 16 15.3 -> 9.2 at 16 rows.
+constexpr int kUpdCols = 256, kUpdRows = 16;
+struct UpdProb {
+    const void* a;            // [R, K], rows a_sr apart, contiguous and 16-byte aligned
+    const void* b;            // [N, R], rows b_sn apart, contiguous and 4 values aligned
+    half_t* y;                // [M, N]
+    int a_sr, b_sn, N;
+    float alpha;
+};
+struct UpdArgs { UpdProb p[kDownProbs]; };
+
+template <bool F32, int RQ>             // R == 4 * RQ
+__global__ __launch_bounds__(64 * kDownWaves) void lora_update_kernel(UpdArgs ua, const half_t* __restrict__ x, int M, int K) {
+    constexpr int R = 4 * RQ, RG = 64 * kDownWaves / kUpdCols, MR = kUpdRows / RG;    // RG groups of up to MR rows
+    __shared__ DownLds<1, kRowsT> lds;
+    __shared__ float sx[kUpdRows][R];
+    const UpdProb& p = ua.p[blockIdx.y];
+    if ((int)blockIdx.x * kUpdCols >= p.N) return;              // uniform: past a narrower layer of the launch
+    const int n = blockIdx.x * kUpdCols + (threadIdx.x & (kUpdCols - 1));
+    const int per = (M + RG - 1) / RG, m0 = (threadIdx.x / kUpdCols) * per, rows = n < p.N ? min(per, M - m0) : 0;
+    constexpr bool kLate = F32 && RQ > 3;                       // 16 more fp32 values would spill beside the loads of the products
+    float bv[R], old[MR];
+    auto load_b = [&] {
+#pragma unroll
+        for (int r = 0; r < R; r += 4) {
+            if constexpr (F32) {
+                float4_t b = {0.f, 0.f, 0.f, 0.f};
+                if (rows > 0) b = *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(p.b) + (size_t)n * p.b_sn + r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv[r + e] = b[e];
+            } else {
+                half4_t b = {(half_t)0.f, (half_t)0.f, (half_t)0.f, (half_t)0.f};
+                if (rows > 0) b = *reinterpret_cast<const half4_t*>(reinterpret_cast<const half_t*>(p.b) + (size_t)n * p.b_sn + r);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv[r + e] = (float)b[e];
+            }
+        }
+    };
+    if constexpr (!kLate) load_b();
+#pragma unroll
+    for (int m = 0; m < MR; ++m) old[m] = m < rows ? (float)p.y[(size_t)(m0 + m) * p.N + n] : 0.f;
+    const DropArgs none{0u, 0u, 0u, 1.0f};
+    lora_down_rows<1, kRowsT, F32, RQ>(lds, x, p.a, p.a_sr, 1, 0, M, K, R, kUpdRows, none);
+    if constexpr (kLate) load_b();
+    __syncthreads();
+    if (threadIdx.x < 256 && (threadIdx.x & 15) < R)
+        sx[threadIdx.x >> 4][threadIdx.x & 15] = (float)(half_t)lora_down_sum(lds, 0, threadIdx.x);
+    __syncthreads();
+    const float alpha = p.alpha;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+        if (m >= rows) break;
+        float acc = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc = fmaf(sx[m0 + m][r], bv[r], acc);
+        p.y[(size_t)(m0 + m) * p.N + n] = (half_t)fmaf(alpha, acc, old[m]);
+    }
+}
+
 // ---- gradient of an adapter matrix --------------------------------------------------------
 // out[j, c] = alpha * sum_m P[m, j] * in[m, c] as v_mfma_f32_16x16x32_f16 products whose reduction index is the ROW m:
 //   A operand  P^T: lane (j = l % 16, kk = l / 16) holds P[mb + 8*kk .. + 7][j]   (rows j >= R are zero)
@@ -299,19 +397,22 @@ __global__ __launch_bounds__(kUpCols) void lora_up_kernel(const half_t* __restri
 // takes longer (7.8 -> 8.8 us).
 constexpr int kG2Waves = 4, kG2Cols = 128, kG2PadRows = 40;
 
-// One or two gradients per launch (blockIdx.z): the two adapter gradients of a layer share M, R and alpha and are
-// independent, so they go out side by side.  Workgroups beyond a problem's own grid leave at once.
+// Up to kGradProbs gradients per launch (blockIdx.z): the two adapter gradients of a layer, and those of the layers that run
+// together, share M and R and are independent, so they go out side by side.  Workgroups beyond a problem's own grid leave at
+// once.  us, gradients and reduction of q and v of 4096 features at rank 8 with dropout, two launches each -> two together:
+// 200 rows 13.5 -> 7.4, 1024 15.2 -> 12.6, 4096 of 5120 features 36.2 -> 29.4.
+constexpr int kGradProbs = 8;
 struct GradProb {
     const half_t* P;          // [M, R]
     const half_t* in;         // [M, C]
     float* out;               // through o_sr, o_sc
     float* part;              // partial tiles [splits][col_blocks][R][128]
     int o_sr, o_sc, C, col_blocks, splits, rows_per_wg;
+    float alpha;
     DropArgs drop;            // dropout mask applied to `in` (thr15 == 0: none); the result carries drop.scale
 };
 struct GradArgs {
-    GradProb p[2];
-    float alpha;
+    GradProb p[kGradProbs];
     int M;
 };
 
@@ -453,7 +554,7 @@ __global__ __launch_bounds__(64 * kG2Waves, RB == 3 ? 2 : 1) void lora_grad_kern
     }
     const bool direct = q.splits == 1;
     const bool jfast = PV && grad_jfast(q);
-    const float alpha = ga.alpha * drop.scale;
+    const float alpha = q.alpha * drop.scale;
     float* tile = q.part + ((size_t)blockIdx.y * q.col_blocks + blockIdx.x) * (size_t)(R * kG2Cols);
 #pragma unroll
     for (int b = 0; b < RB; ++b) {
@@ -518,7 +619,7 @@ __global__ __launch_bounds__(256) void lora_grad_reduce_kernel(GradArgs ga, int 
         j = o - cl * R;
     }
     const int cc = bx * kG2Cols + cl;
-    if (cc < q.C) q.out[(size_t)j * q.o_sr + (size_t)cc * q.o_sc] = ga.alpha * q.drop.scale * v;
+    if (cc < q.C) q.out[(size_t)j * q.o_sr + (size_t)cc * q.o_sc] = q.alpha * q.drop.scale * v;
 }
 
 // keep[m, c] = 1 where dropout keeps element (m, c), else 0: the mask the kernels above regenerate, written out
@@ -554,59 +655,114 @@ inline GradPlan plan_grad(int M, int C, int R) {
 }  // namespace q4
 
 template <int RB, int WL, bool F32, int RQ>
-static void launch_down_kernel(const q4::half_t* ip, const void* w, int w_sr, int w_sc, q4::half_t* op,
-                               int M, int C, int R, const q4::DropArgs& drop, hipStream_t stream) {
+static void launch_down_kernel(const q4::DownArgs& da, int n, int M, int R, hipStream_t stream) {
     // rows of `in` per workgroup: 16 fill the MFMA operand, but with few rows that leaves compute units idle and
     // the kernel is bound by the latency of its single burst of loads, so smaller blocks spread it out
     int rows = 16;
-    while (rows > 4 && (M + rows - 1) / rows < 256) rows >>= 1;
-    hipLaunchKernelGGL((q4::lora_down_kernel<RB, WL, F32, RQ>), dim3((M + rows - 1) / rows), dim3(64 * q4::kDownWaves), 0,
-                       stream, ip, w, w_sr, w_sc, op, M, C, R, rows, drop);
+    while (rows > 4 && (M + rows - 1) / rows * n < 256) rows >>= 1;
+    hipLaunchKernelGGL((q4::lora_down_kernel<RB, WL, F32, RQ>), dim3((M + rows - 1) / rows, n), dim3(64 * q4::kDownWaves), 0,
+                       stream, da, M, R, rows);
 }
 
 template <int WL, bool F32>
-static void launch_down_rb(const q4::half_t* ip, const void* w, int w_sr, int w_sc, q4::half_t* op,
-                           int M, int C, int R, const q4::DropArgs& drop, hipStream_t stream) {
+static void launch_down_rb(const q4::DownArgs& da, int n, int M, int R, hipStream_t stream) {
     switch ((R + 15) / 16) {
-        case 1: launch_down_kernel<1, WL, F32, 0>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        case 2: launch_down_kernel<2, WL, F32, 0>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        case 3: launch_down_kernel<3, WL, F32, 0>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        default: launch_down_kernel<4, WL, F32, 0>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
+        case 1: launch_down_kernel<1, WL, F32, 0>(da, n, M, R, stream); break;
+        case 2: launch_down_kernel<2, WL, F32, 0>(da, n, M, R, stream); break;
+        case 3: launch_down_kernel<3, WL, F32, 0>(da, n, M, R, stream); break;
+        default: launch_down_kernel<4, WL, F32, 0>(da, n, M, R, stream); break;
     }
 }
 
 template <int WL, bool F32>
-static void launch_down_staged(const q4::half_t* ip, const void* w, int w_sr, int w_sc, q4::half_t* op,
-                             int M, int C, int R, const q4::DropArgs& drop, hipStream_t stream) {
+static void launch_down_staged(const q4::DownArgs& da, int n, int M, int R, hipStream_t stream) {
     switch ((R + 3) / 4) {
-        case 1: launch_down_kernel<1, WL, F32, 1>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        case 2: launch_down_kernel<1, WL, F32, 2>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        case 3: launch_down_kernel<1, WL, F32, 3>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
-        default: launch_down_kernel<1, WL, F32, 4>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream); break;
+        case 1: launch_down_kernel<1, WL, F32, 1>(da, n, M, R, stream); break;
+        case 2: launch_down_kernel<1, WL, F32, 2>(da, n, M, R, stream); break;
+        case 3: launch_down_kernel<1, WL, F32, 3>(da, n, M, R, stream); break;
+        default: launch_down_kernel<1, WL, F32, 4>(da, n, M, R, stream); break;
     }
 }
 
-extern "C" int q4_launch_lora_down(const void* in, const void* w, int w_sr, int w_sc, int w_is_f32, void* out,
-                                   int M, int C, int R, const q4::DropArgs* dropp, hipStream_t stream) {
+static q4::WLayout down_layout(const void* w, int w_sr, int w_sc, int w_is_f32, int R) {
     using namespace q4;
-    const DropArgs drop = dropp ? *dropp : DropArgs{0u, 0u, 0u, 1.0f};
-    const half_t* ip = reinterpret_cast<const half_t*>(in);
-    half_t* op = reinterpret_cast<half_t*>(out);
     const bool base16 = (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
     const int vec = w_is_f32 ? 4 : 8;                       // elements per 16 bytes
-    if (w_sc == 1 && base16 && w_sr % 4 == 0 && R <= 16) {
-        if (w_is_f32) launch_down_staged<kRowsT, true>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-        else launch_down_staged<kRowsT, false>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-    } else if (w_sc == 1 && base16 && w_sr % vec == 0) {
-        if (w_is_f32) launch_down_rb<kRows, true>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-        else launch_down_rb<kRows, false>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-    } else if (w_sr == 1 && base16 && w_sc % 4 == 0 && R % 4 == 0 && R <= 16 && w_sc >= R) {
-        if (w_is_f32) launch_down_staged<kCols, true>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-        else launch_down_staged<kCols, false>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-    } else {
-        if (w_is_f32) launch_down_rb<kAny, true>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
-        else launch_down_rb<kAny, false>(ip, w, w_sr, w_sc, op, M, C, R, drop, stream);
+    if (w_sc == 1 && base16 && w_sr % 4 == 0 && R <= 16) return kRowsT;
+    if (w_sc == 1 && base16 && w_sr % vec == 0) return kRows;
+    if (w_sr == 1 && base16 && w_sc % 4 == 0 && R % 4 == 0 && R <= 16 && w_sc >= R) return kCols;
+    return kAny;
+}
+
+template <bool F32>
+static void launch_down(q4::WLayout layout, const q4::DownArgs& da, int n, int M, int R, hipStream_t stream) {
+    using namespace q4;
+    switch (layout) {
+        case kRowsT: launch_down_staged<kRowsT, F32>(da, n, M, R, stream); break;
+        case kRows: launch_down_rb<kRows, F32>(da, n, M, R, stream); break;
+        case kCols: launch_down_staged<kCols, F32>(da, n, M, R, stream); break;
+        default: launch_down_rb<kAny, F32>(da, n, M, R, stream); break;
     }
+}
+
+// `n` products of M rows; neighbours of the same rank, type and layout of w share a launch.  drops[i] null: no dropout.
+extern "C" int q4_launch_lora_down(const q4_lora_down_t* probs, const q4::DropArgs* const* drops, int n, int M, hipStream_t stream) {
+    using namespace q4;
+    for (int i = 0; i < n;) {
+        const q4_lora_down_t& f = probs[i];
+        const WLayout layout = down_layout(f.w, f.w_sr, f.w_sc, f.w_is_f32, f.R);
+        DownArgs da;
+        int k = 0;
+        for (; i + k < n && k < kDownProbs; ++k) {
+            const q4_lora_down_t& g = probs[i + k];
+            if (g.R != f.R || g.w_is_f32 != f.w_is_f32 || down_layout(g.w, g.w_sr, g.w_sc, g.w_is_f32, g.R) != layout) break;
+            da.p[k] = {reinterpret_cast<const half_t*>(g.in), g.w, reinterpret_cast<half_t*>(g.out), g.w_sr, g.w_sc, g.C,
+                       drops[i + k] ? *drops[i + k] : DropArgs{0u, 0u, 0u, 1.0f}};
+        }
+        if (f.w_is_f32) launch_down<true>(layout, da, k, M, f.R, stream);
+        else launch_down<false>(layout, da, k, M, f.R, stream);
+        i += k;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+// One launch takes up to 16 rows, ranks 4, 8, 12 and 16, and matrices of one type read in whole vectors.  A single adapter above
+// eight rows stays with the two launches, whose first spreads the rows: us, 4096 features at rank 8, two launches -> one: 5.9 -> 4.4
+// at 1 row, 6.9 -> 6.0 at 8, 7.1 -> 7.8 at 16; 13824 features 13.7 -> 12.7 at 4, 13.9 -> 20.6 at 16 (two adapters 27.5 -> 20.8).
+extern "C" int q4_lora_update_fits(const q4_lora_update_t* probs, int n, int M) {
+    if (n < 1 || n > q4::kDownProbs || M > (n == 1 ? q4::kUpdRows / 2 : q4::kUpdRows)) return 0;
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_update_t& g = probs[i];
+        if (g.R != probs[0].R || g.a_is_f32 != probs[0].a_is_f32 || g.b_is_f32 != g.a_is_f32 || g.R % 4 != 0 || g.R > 16) return 0;
+        if (down_layout(g.a, g.a_sr, g.a_sc, g.a_is_f32, g.R) != q4::kRowsT) return 0;
+        if (g.b_sr != 1 || g.b_sn % 4 != 0 || (reinterpret_cast<uintptr_t>(g.b) & (g.b_is_f32 ? 15u : 7u)) != 0) return 0;
+    }
+    return 1;
+}
+
+template <bool F32>
+static void launch_update(const q4::UpdArgs& ua, int R, const q4::half_t* x, int M, int K, dim3 grid, hipStream_t stream) {
+    const dim3 block(64 * q4::kDownWaves);
+    switch (R / 4) {
+        case 1: hipLaunchKernelGGL((q4::lora_update_kernel<F32, 1>), grid, block, 0, stream, ua, x, M, K); break;
+        case 2: hipLaunchKernelGGL((q4::lora_update_kernel<F32, 2>), grid, block, 0, stream, ua, x, M, K); break;
+        case 3: hipLaunchKernelGGL((q4::lora_update_kernel<F32, 3>), grid, block, 0, stream, ua, x, M, K); break;
+        default: hipLaunchKernelGGL((q4::lora_update_kernel<F32, 4>), grid, block, 0, stream, ua, x, M, K); break;
+    }
+}
+
+extern "C" int q4_launch_lora_update(const q4_lora_update_t* probs, int n, const void* x, int M, int K, hipStream_t stream) {
+    using namespace q4;
+    UpdArgs ua;
+    int gx = 1;
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_update_t& g = probs[i];
+        ua.p[i] = {g.a, g.b, reinterpret_cast<half_t*>(g.y), g.a_sr, g.b_sn, g.N, g.alpha};
+        gx = std::max(gx, (g.N + kUpdCols - 1) / kUpdCols);
+    }
+    const half_t* xp = reinterpret_cast<const half_t*>(x);
+    if (probs[0].a_is_f32) launch_update<true>(ua, probs[0].R, xp, M, K, dim3(gx, n), stream);
+    else launch_update<false>(ua, probs[0].R, xp, M, K, dim3(gx, n), stream);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -627,20 +783,6 @@ extern "C" int q4_launch_lora_up(const void* xa, const void* w, int w_sn, int w_
 extern "C" size_t q4_lora_grad_workspace(int M, int C, int R) {
     const q4::GradPlan g = q4::plan_grad(M, C, R);
     return g.splits == 1 ? 0 : (size_t)g.splits * g.col_blocks * R * q4::kG2Cols * sizeof(float);
-}
-
-static q4::GradProb make_grad_prob(const void* P, const void* in, float* out, int o_sr, int o_sc, int M, int C, int R,
-                                   float* part, const q4::DropArgs* drop = nullptr) {
-    const q4::GradPlan g = q4::plan_grad(M, C, R);
-    q4::GradProb q;
-    q.P = reinterpret_cast<const q4::half_t*>(P);
-    q.in = reinterpret_cast<const q4::half_t*>(in);
-    q.out = out;
-    q.part = part;
-    q.o_sr = o_sr; q.o_sc = o_sc; q.C = C;
-    q.col_blocks = g.col_blocks; q.splits = g.splits; q.rows_per_wg = g.rows_per_wg;
-    q.drop = drop ? *drop : q4::DropArgs{0u, 0u, 0u, 1.0f};
-    return q;
 }
 
 template <int RB>
@@ -674,34 +816,26 @@ static int launch_grad(const q4::GradArgs& ga, int nprob, int R, hipStream_t str
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-extern "C" int q4_launch_lora_grad(const void* P, const void* in, float* out, int o_sr, int o_sc, float alpha,
-                                   int M, int C, int R, const q4::DropArgs* drop, void* workspace, hipStream_t stream) {
-    q4::GradArgs ga;
-    ga.p[0] = make_grad_prob(P, in, out, o_sr, o_sc, M, C, R, reinterpret_cast<float*>(workspace), drop);
-    ga.p[1] = ga.p[0];
-    ga.alpha = alpha;
-    ga.M = M;
-    return launch_grad(ga, 1, R, stream);
-}
-
 extern "C" int q4_launch_dropout_keep(uint8_t* keep, int M, int C, const q4::DropArgs* drop, hipStream_t stream) {
     const long pairs = (long)M * (C / 2);
     hipLaunchKernelGGL(q4::dropout_keep_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, keep, M, C, *drop);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-// Two gradients with the same M, R and alpha in one launch (plus one launch for both reductions); the workspace
-// holds the partial tiles of the first problem followed by those of the second.
-extern "C" int q4_launch_lora_grad_pair(const void* P1, const void* in1, float* out1, int o1_sr, int o1_sc, int C1,
-                                        const void* P2, const void* in2, float* out2, int o2_sr, int o2_sc, int C2,
-                                        float alpha, int M, int R, const q4::DropArgs* drop1, void* workspace,
-                                        hipStream_t stream) {
-    q4::GradArgs ga;
+// Up to kGradProbs gradients with the same M and R in one launch (plus one launch for their reductions); the workspace holds
+// the partial tiles of one problem after the other.
+extern "C" int q4_launch_lora_grad(const q4_lora_grad_t* probs, const q4::DropArgs* const* drops, int n, int M, int R,
+                                   void* workspace, hipStream_t stream) {
+    using namespace q4;
+    GradArgs ga;
     float* ws = reinterpret_cast<float*>(workspace);
-    ga.p[0] = make_grad_prob(P1, in1, out1, o1_sr, o1_sc, M, C1, R, ws, drop1);      // the mask applies to in1 only
-    ga.p[1] = make_grad_prob(P2, in2, out2, o2_sr, o2_sc, M, C2, R,
-                             ws ? ws + q4_lora_grad_workspace(M, C1, R) / sizeof(float) : nullptr);
-    ga.alpha = alpha;
+    for (int i = 0; i < n; ++i) {
+        const q4_lora_grad_t& p = probs[i];
+        const GradPlan g = plan_grad(M, p.C, R);
+        ga.p[i] = {reinterpret_cast<const half_t*>(p.p), reinterpret_cast<const half_t*>(p.in), p.out, ws, p.o_sr, p.o_sc, p.C,
+                   g.col_blocks, g.splits, g.rows_per_wg, p.alpha, drops[i] ? *drops[i] : DropArgs{0u, 0u, 0u, 1.0f}};
+        if (ws) ws += q4_lora_grad_workspace(M, p.C, R) / sizeof(float);
+    }
     ga.M = M;
-    return launch_grad(ga, 2, R, stream);
+    return launch_grad(ga, n, R, stream);
 }

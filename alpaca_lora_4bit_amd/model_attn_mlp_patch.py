@@ -23,7 +23,7 @@ import torch
 import torch.nn as nn
 
 from . import matmul_utils_4bit
-from .autograd_4bit import Autograd4bitQuantLinear, fuse_quant_linears
+from .autograd_4bit import Autograd4bitQuantLinear, _has_bias, fuse_quant_linears
 
 
 class FusedProjectionSlice(nn.Module):
@@ -71,6 +71,13 @@ class _FusedGroup:
         self._served = 0
 
 
+_ADAPTER_TYPES = (torch.float16, torch.float32)
+
+
+def _same_adapter(p, q):
+    return p[0] is q[0] and p[2] is q[2] and (p[1], p[3], p[4]) == (q[1], q[3], q[4])
+
+
 class _MemberGroup:
     """Projections that share their input (q|k|v, gate|up), each on its own tensors.  `run(member, x)` is called from
     Autograd4bitQuantLinear.forward at decode sizes: the first call for an input runs one grouped launch for all
@@ -114,17 +121,71 @@ class _MemberGroup:
         if layers is None:
             return None
         i = self.index[id(member)]
-        if self._x is not x or self._version != x._version or self._outs[i] is None:
-            from . import quant_hip
-            # the compiled binding checks shapes, dtypes and devices; sequential groups were established by _check()
-            outs = quant_hip.gemv_grouped_prepared(x, layers, self.groupsize)
+        if not self._current(i, x) or self._adapted[i] is not None:
+            self._launch(x, layers)
+        return self._take(i)
+
+    def _current(self, i, x):
+        return self._x is x and self._version == x._version and self._outs[i] is not None
+
+    def _launch(self, x, layers):
+        # the compiled binding checks shapes, dtypes and devices; sequential groups were established by _check()
+        outs = matmul_utils_4bit.quant_hip.gemv_grouped_prepared(x, layers, self.groupsize)
+        if x.dim() != 2:
             lead = tuple(x.shape[:-1])
-            self._outs = [o.view(lead + (o.shape[-1],)) for o in outs]
-            self._x, self._version = x, x._version
-        y, self._outs[i] = self._outs[i], None
+            outs = [o.view(lead + (o.shape[-1],)) for o in outs]
+        self._outs = outs
+        self._adapted = [None] * len(self.members)
+        self._x, self._version = x, x._version
+
+    def _take(self, i):
+        y, self._outs[i], self._adapted[i] = self._outs[i], None, None
         if all(o is None for o in self._outs):
             self._x = None
         return y
+
+    def run_adapted(self, member, x, name):
+        """`run` for a member whose adapter `name` is to be added (decode sizes): the products of all members in one launch and
+        the adapters of all members in the next, each member picks its finished output up.  None when the group does not take
+        this call.  An output that was finished with another adapter than the member now asks for is not handed out."""
+        layers = self._layers()
+        adapter = self._adapter(member, name, x)
+        if layers is None or adapter is None:
+            return None
+        i = self.index[id(member)]
+        if not self._current(i, x) or (self._adapted[i] is not None and not _same_adapter(self._adapted[i], adapter)):
+            self._launch(x, layers)
+        if self._adapted[i] is None:
+            todo = {i: adapter}
+            for j, m in enumerate(self.members):
+                if j != i and self._outs[j] is not None and self._adapted[j] is None and type(m) is type(member) and not m.disable_adapters:
+                    other = m._decode_adapter(x)
+                    ad = None if other is None else self._adapter(m, other, x)
+                    if ad is not None:
+                        todo[j] = ad
+            try:
+                flat = x.dim() == 2
+                matmul_utils_4bit.quant_hip.lora_update_grouped(
+                    x if flat and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous(),
+                    [(ad[0], ad[2], self._outs[j] if flat else self._outs[j].view(-1, self._outs[j].shape[-1]), ad[4]) for j, ad in todo.items()])
+            except BaseException:
+                self.clear()                                 # some outputs may have been updated
+                raise
+            for j, ad in todo.items():
+                self._adapted[j] = ad
+        return self._take(i)
+
+    @staticmethod
+    def _adapter(m, name, x):
+        """(A, its version, B, its version, scaling) of member m's adapter as the grouped update takes it, or None."""
+        if _has_bias(m):
+            return None                                      # the bias comes between the product and the update
+        a, b, dev = m.lora_A[name].weight, m.lora_B[name].weight, x.get_device()
+        for w in (a, b):
+            if w.get_device() != dev or w.dtype not in _ADAPTER_TYPES or w.is_inference():
+                return None
+        scaling = float(m.scaling[name])
+        return a, a._version, b, b._version, scaling
 
     def _gemm_spec(self, m, x):
         """How member `m` enters a grouped GEMM for input x: (bias | None, lora_A | None, lora_B | None, scaling, drop_p)."""
@@ -194,6 +255,7 @@ class _MemberGroup:
         self._x = None
         self._version = -1
         self._outs = [None] * len(self.members)
+        self._adapted = [None] * len(self.members)
         self._gx = None
         self._gkey = None
         self._gouts = [None] * len(self.members)

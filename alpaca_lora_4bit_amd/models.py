@@ -169,8 +169,13 @@ class Linear4bitLt(Autograd4bitQuantLinear, LoraLayer):
         if not self.disable_adapters:
             name = self._decode_adapter(x)
             if name is not None:
-                # decode: base product (GEMV), x @ A^T and the rank-r update in place with the adapter read where it is:
-                # three launches instead of the seven of the composition below, same values up to fp16 rounding
+                # decode: the base product and the adapter in place, read where it is, in two launches instead of the seven of the
+                # composition below, same values up to fp16 rounding; members of a group share both launches
+                group = self.__dict__.get('_q4_group')
+                if group is not None and autograd_4bit._decode_call(self, x):
+                    result = group.run_adapted(self, x, name)
+                    if result is not None:
+                        return result
                 result = Autograd4bitQuantLinear.forward(self, x)
                 a, b = self.lora_A[name].weight, self.lora_B[name].weight
                 x2, out2 = x.reshape(-1, x.shape[-1]).to(torch.float16).contiguous(), result.view(-1, result.shape[-1])

@@ -890,6 +890,35 @@ def lora_down(inp, w, dropout=None):
     return out
 
 
+def _drop_pair(dropout):
+    return None if dropout is None else (int(dropout[0]), float(dropout[1]))
+
+
+def lora_down_grouped(specs):
+    """[lora_down(inp, w, dropout) for (inp, w, dropout) in specs] for up to four adapters of the same number of rows, as one
+    launch where they agree in rank, type and layout."""
+    if _host is None:
+        return [lora_down(inp, w, dropout) for inp, w, dropout in specs]
+    return _host.lora_down_grouped([(inp, w, _drop_pair(dropout)) for inp, w, dropout in specs])
+
+
+def lora_update_grouped(x, specs):
+    """lora_update(x, a, b, y, alpha) for every (a, b, y, alpha) of up to four adapters, as one launch where that takes them."""
+    if _host is None:
+        for a, b, y, alpha in specs:
+            lora_update(x, a, b, y, alpha)
+    else:
+        _host.lora_update_grouped(x, specs)
+
+
+def lora_grad_grouped(specs):
+    """[lora_grad_pair(p1, inp1, p2, inp2, alpha, dropout), ...] for up to four layers whose rank-R operands share their shape, as
+    one launch and one for the reductions."""
+    if _host is None:
+        return [lora_grad_pair(p1, in1, p2, in2, alpha, dropout=dropout) for p1, in1, p2, in2, alpha, dropout in specs]
+    return _host.lora_grad_grouped([(p1, in1, p2, in2, float(alpha), _drop_pair(dropout)) for p1, in1, p2, in2, alpha, dropout in specs])
+
+
 def lora_update(x, a, b, y, alpha):
     """y fp16 [M, N] += alpha * (x @ a^T) @ b^T in place, for x fp16 [M, K], a = lora_A.weight [R, K] and
     b = lora_B.weight [N, R] (fp16/fp32, any view; read in place unless a stride is 0): the adapter of a few rows in two launches (models.py:66).

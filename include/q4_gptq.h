@@ -318,6 +318,20 @@ Q4_API int q4_gemm_grouped_bwd_dx_f16(const q4_gemm_layer_t *layers, int n_layer
 Q4_API int q4_lora_down_f16(const void *in, const void *w, int w_sr, int w_sc, int w_is_f32, void *out,
                      int M, int C, int R, const q4_dropout_t *drop, void *stream);
 
+/* `n` (1..4) such products with the same M, each on its own operands, masks and outputs, in as few launches as their ranks,
+ * types and layouts allow (one where these agree): the adapters of layers that run together (q|v of an attention block). */
+typedef struct { const void *in, *w; void *out; int w_sr, w_sc, w_is_f32, C, R; const q4_dropout_t *drop; } q4_lora_down_t;
+Q4_API int q4_lora_down_grouped_f16(const q4_lora_down_t *probs, int n, int M, void *stream);
+
+/* y_i fp16 [M, N_i] += alpha_i * fp16(x @ A_i^T) @ B_i^T in place for `n` (1..4) adapters of layers that share x fp16 [M, K], as
+ * ONE launch with the values of q4_lora_down_f16 + q4_lora_up_f16.  A (element (r, k) at a[r*a_sr + k*a_sc]) and B as there.
+ * Takes what q4_lora_update_fits says: M <= 16 (8 with n == 1), R in {4, 8, 12, 16}, one R and one type of all matrices, A and B with contiguous
+ * rows a multiple of 4 values apart, A 16-byte and B 4-value aligned; anything else is Q4_ERR_BAD_SHAPE and goes to the two
+ * calls above.  The y_i must not overlap each other or x. */
+typedef struct { const void *a, *b; void *y; int a_sr, a_sc, a_is_f32, b_sn, b_sr, b_is_f32, N, R; float alpha; } q4_lora_update_t;
+Q4_API int q4_lora_update_fits(const q4_lora_update_t *probs, int n, int M);
+Q4_API int q4_lora_update_grouped_f16(const q4_lora_update_t *probs, int n, const void *x, int M, int K, void *stream);
+
 /* y fp16 [M, N] += alpha * xa fp16 [M, R] @ B^T in place, one rounding; B (element (n, r) at w[n*w_sn + r*w_sr], fp16 or
  * fp32) is lora_B.weight: the second half of the adapter at decode sizes (models.py:66).  R <= 64; sums in fp32. */
 Q4_API int q4_lora_up_f16(const void *xa, const void *w, int w_sn, int w_sr, int w_is_f32, void *y, float alpha,
@@ -345,6 +359,12 @@ Q4_API int q4_lora_grad_pair_f32(const void *p1, const void *in1, float *out1, i
                           const void *p2, const void *in2, float *out2, int o2_sr, int o2_sc, int C2,
                           float alpha, int M, int R, const q4_dropout_t *drop1,
                           void *workspace, size_t workspace_bytes, void *stream);
+
+/* `n` (1..8) gradients that share M and R in one launch (plus one for their reductions): the pairs of layers that run together.
+ * R as for the pair; `workspace`: the sum of q4_lora_grad_workspace_bytes(M, C_i, R), 256-byte aligned, contents irrelevant. */
+typedef struct { const void *p, *in; float *out; int o_sr, o_sc, C; float alpha; const q4_dropout_t *drop; } q4_lora_grad_t;
+Q4_API int q4_lora_grad_grouped_f32(const q4_lora_grad_t *probs, int n, int M, int R, void *workspace, size_t workspace_bytes,
+                                    void *stream);
 
 #ifdef __cplusplus
 }
