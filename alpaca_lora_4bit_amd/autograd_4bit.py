@@ -153,8 +153,19 @@ def _is_all_zero(bias):
     return verdict
 
 
+def _buffer(layer, name):
+    """layer.<name> without nn.Module.__getattr__ where it is a buffer, as it is unless somebody replaced it."""
+    t = layer._buffers.get(name)
+    return t if t is not None else getattr(layer, name)
+
+
+def _weight(linear):
+    w = linear._parameters.get('weight')
+    return w if w is not None else linear.weight             # parametrized
+
+
 def _has_bias(layer):
-    return not layer.disable_bias and not _is_all_zero(layer.bias)
+    return not layer.disable_bias and not _is_all_zero(_buffer(layer, 'bias'))
 
 
 def _decode_call(layer, x):
@@ -200,10 +211,11 @@ class Autograd4bitQuantLinear(nn.Module):
             group = self.__dict__.get('_q4_group')
             out = group.run(self, x) if group is not None else None
             if out is None:
-                scales = self.scales
-                out = quant_hip.gemv(x, self.qweight, self.qzeros, scales if scales.dtype == torch.float16 else scales.half(),
-                                     self.g_idx, self.groupsize, out_shape=x.shape[:-1] + (self.out_features,))
-            if not self.disable_bias and not _is_all_zero(self.bias):
+                scales = _buffer(self, 'scales')
+                out = quant_hip.gemv(x, _buffer(self, 'qweight'), _buffer(self, 'qzeros'),
+                                     scales if scales.dtype == torch.float16 else scales.half(),
+                                     _buffer(self, 'g_idx'), self.groupsize, out_shape=x.shape[:-1] + (self.out_features,))
+            if _has_bias(self):
                 out += self.bias
             return out
         group = self.__dict__.get('_q4_group')
@@ -213,18 +225,18 @@ class Autograd4bitQuantLinear(nn.Module):
             out = group.run_gemm(self, x)
             if out is not None:
                 return out
-        zeros = self.zeros if self.is_v1_model else self.qzeros
+        zeros = _buffer(self, 'zeros' if self.is_v1_model else 'qzeros')
         if self.bits == 4:
+            qweight, scales, g_idx = _buffer(self, 'qweight'), _buffer(self, 'scales'), _buffer(self, 'g_idx')
             if torch.is_grad_enabled():
-                out = AutogradMatmul4bit.apply(x, self.qweight, self.scales, zeros, self.g_idx, self.bits, self.maxq)
+                out = AutogradMatmul4bit.apply(x, qweight, scales, zeros, g_idx, self.bits, self.maxq)
             else:
-                out = matmul4bit_with_backend(x, self.qweight, self.scales, zeros, self.g_idx, self.bits, self.maxq,
-                                              self.groupsize)
+                out = matmul4bit_with_backend(x, qweight, scales, zeros, g_idx, self.bits, self.maxq, self.groupsize)
         elif self.bits == 2:
             out = AutogradMatmul2bit.apply(x, self.qweight, self.scales, self.qzeros, self.g_idx, self.bits, self.maxq)
         else:
             raise ValueError('Unsupported bitwidth.')
-        if not self.disable_bias and not _is_all_zero(self.bias):
+        if _has_bias(self):
             out += self.bias
         return out
 

@@ -183,11 +183,14 @@ at::Tensor dequant(const at::Tensor& qweight, const at::Tensor& qzeros, const at
 
 at::Tensor gemv(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& qzeros, const at::Tensor& scales,
                 const c10::optional<at::Tensor>& g_idx, int64_t groupsize, c10::optional<at::Tensor> out, bool accumulate,
-                const c10::optional<std::vector<int64_t>>& out_shape) {
+                const c10::optional<std::vector<int64_t>>& out_shape, const c10::optional<at::Tensor>& in_perm) {
     const Layer l = check_layer(qweight, qzeros, scales, g_idx, groupsize);
     const at::Tensor x2 = flat_half(x, l.K, l.device, "x");
     const int64_t M = x2.size(0);
     if (M == 0 && !out.has_value()) return at::empty(out_sizes(out_shape, 0, l.N), x2.options());
+    TORCH_CHECK_VALUE(!in_perm.has_value() || (in_perm->scalar_type() == at::kInt && in_perm->dim() == 1 && in_perm->size(0) == l.K &&
+                                               in_perm->is_contiguous() && in_perm->device() == l.device && !l.g_idx),
+                      "the column index must be a contiguous int32 [K] tensor on the same device, beside sequential groups");
     TORCH_CHECK_VALUE(M >= 1 && M <= 16, "gemv handles 1..16 rows, got ", M);
     TORCH_CHECK_VALUE(out.has_value() || !accumulate, "accumulate needs an output tensor");
     at::Tensor o = out.has_value() ? *out : at::empty(out_sizes(out_shape, M, l.N), x2.options());
@@ -197,11 +200,14 @@ at::Tensor gemv(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor
     Launch L(l.device);
     size_t have = 0;
     void* ws = zeroed_workspace(l.device, L.stream, q4_gemv_workspace_bytes((int)M, l.K, l.N), &have);
-    const int rc = q4_gemv_f16(x2.data_ptr(), l.qweight, l.qzeros, l.scales, l.g_idx, l.groupsize, o.data_ptr(),
-                               accumulate ? 1 : 0, (int)M, l.K, l.N, l.G, ws, have, L.stream);
+    const int rc = in_perm.has_value()             // act-order: sorted rows of `qweight`, x gathered by the kernel
+        ? q4_gemv_sorted_f16(x2.data_ptr(), l.qweight, l.qzeros, l.scales, in_perm->data_ptr<int32_t>(), l.groupsize, o.data_ptr(),
+                             accumulate ? 1 : 0, (int)M, l.K, l.N, l.G, ws, have, L.stream)
+        : q4_gemv_f16(x2.data_ptr(), l.qweight, l.qzeros, l.scales, l.g_idx, l.groupsize, o.data_ptr(),
+                      accumulate ? 1 : 0, (int)M, l.K, l.N, l.G, ws, have, L.stream);
     if (rc != Q4_OK) {
         if (rc == Q4_ERR_LAUNCH) reset_zeroed_workspace(l.device, L.stream);
-        raise_q4(rc, "q4_gemv_f16");
+        raise_q4(rc, in_perm.has_value() ? "q4_gemv_sorted_f16" : "q4_gemv_f16");
     }
     return o;
 }
@@ -712,7 +718,8 @@ PYBIND11_MODULE(_q4_host, m) {
     m.def("dequant", &dequant, py::arg("qweight"), py::arg("qzeros"), py::arg("scales"), py::arg("g_idx"), py::arg("groupsize"),
           py::arg("out") = py::none());
     m.def("gemv", &gemv, py::arg("x"), py::arg("qweight"), py::arg("qzeros"), py::arg("scales"), py::arg("g_idx"),
-          py::arg("groupsize"), py::arg("out") = py::none(), py::arg("accumulate") = false, py::arg("out_shape") = py::none());
+          py::arg("groupsize"), py::arg("out") = py::none(), py::arg("accumulate") = false, py::arg("out_shape") = py::none(),
+          py::arg("in_perm") = py::none());
     m.def("gemv_grouped", &gemv_grouped, py::arg("xs"), py::arg("layers"), py::arg("groupsize"), py::arg("outs") = py::none(),
           py::arg("accumulate") = false);
     m.def("gemm_fwd", &gemm_fwd, py::arg("x"), py::arg("qweight"), py::arg("qzeros"), py::arg("scales"), py::arg("g_idx"),

@@ -22,8 +22,8 @@ import re
 import torch
 import torch.nn as nn
 
-from . import matmul_utils_4bit
-from .autograd_4bit import Autograd4bitQuantLinear, _has_bias, fuse_quant_linears
+from . import autograd_4bit, matmul_utils_4bit
+from .autograd_4bit import Autograd4bitQuantLinear, _buffer, _has_bias, _weight, fuse_quant_linears
 
 
 class FusedProjectionSlice(nn.Module):
@@ -108,9 +108,13 @@ class _MemberGroup:
     def _layers(self):
         """(qweight, qzeros, scales) of every member, rebuilt when a member's buffers were replaced (a cast, a reload)."""
         cached = self._layer_cache
-        if cached is not None and all(m._buffers.get('qweight') is c[0] and m._buffers.get('scales') is c[2]
-                                      for m, c in zip(self.members, cached)):
-            return cached
+        if cached is not None:
+            for m, c in zip(self.members, cached):
+                b = m._buffers
+                if b.get('qweight') is not c[0] or b.get('scales') is not c[2]:
+                    break
+            else:
+                return cached
         self.usable = self._check()
         self._gemm_ok = None
         self._layer_cache = [(m.qweight, m.qzeros, m.scales) for m in self.members] if self.usable else None
@@ -180,7 +184,8 @@ class _MemberGroup:
         """(A, its version, B, its version, scaling) of member m's adapter as the grouped update takes it, or None."""
         if _has_bias(m):
             return None                                      # the bias comes between the product and the update
-        a, b, dev = m.lora_A[name].weight, m.lora_B[name].weight, x.get_device()
+        mods = m._modules
+        a, b, dev = _weight(mods['lora_A']._modules[name]), _weight(mods['lora_B']._modules[name]), x.get_device()
         for w in (a, b):
             if w.get_device() != dev or w.dtype not in _ADAPTER_TYPES or w.is_inference():
                 return None
@@ -189,16 +194,13 @@ class _MemberGroup:
 
     def _gemm_spec(self, m, x):
         """How member `m` enters a grouped GEMM for input x: (bias | None, lora_A | None, lora_B | None, scaling, drop_p)."""
-        from .autograd_4bit import _is_all_zero
-        bias = None
-        if not m.disable_bias and not _is_all_zero(m.bias):
-            bias = m.bias
+        bias = _buffer(m, 'bias') if _has_bias(m) else None
         name = None
         if type(m) is not Autograd4bitQuantLinear and not getattr(m, 'disable_adapters', False):
             name = m._fusable_adapter(x)                     # the adapter rides in the launch; otherwise the layer adds it
         if name is None:
             return (bias, None, None, None, 0.0)
-        return (bias, m.lora_A[name].weight, m.lora_B[name].weight, float(m.scaling[name]), m._dropout_p(name))
+        return (bias, _weight(m._modules['lora_A']._modules[name]), _weight(m._modules['lora_B']._modules[name]), float(m.scaling[name]), m._dropout_p(name))
 
     def run_gemm(self, member, x):
         """Above the decode sizes: ONE grouped GEMM launch for all members (under autograd one node, whose backward is
@@ -211,7 +213,7 @@ class _MemberGroup:
             if all(o is None for o in self._gouts):
                 self._gx = None
             return y
-        from . import autograd_4bit, quant_hip
+        from . import quant_hip
         layers = self._layers()
         if layers is None or not x.is_cuda or x.shape[-1] != member.in_features:
             return None
@@ -461,11 +463,15 @@ def _mlp_decode_args(mlp):
             (down.qweight, down.qzeros, down.scales), int(gate.groupsize), gate.in_features, gate.out_features, down.out_features)
 
 
+def _adapters_off(layer):
+    return None if type(layer) is Autograd4bitQuantLinear else getattr(layer, 'disable_adapters', None)
+
+
 def _mlp_decode_forward(mlp, x):
     """LlamaMLP.forward with the decode step (up to 16 rows, no grad, fp16) as one launch (quant_hip.mlp_decode: gate, up,
     silu(gate) * up and down) or two (quant_hip.mlp_rows); everything else goes to the block's own forward.  What the step
     needs of the three layers is looked up once and kept while their buffers, adapters and bias switches stay the same objects / values."""
-    from . import autograd_4bit, quant_hip
+    quant_hip = matmul_utils_4bit.quant_hip
     d = mlp.__dict__
     if (not torch.is_grad_enabled() and x.dtype == torch.float16 and x.is_cuda and autograd_4bit.backend == 'cuda'
             and matmul_utils_4bit.use_new and matmul_utils_4bit.auto_switch):
@@ -476,7 +482,7 @@ def _mlp_decode_forward(mlp, x):
         key = (gate._buffers.get('qweight'), up._buffers.get('qweight'), down._buffers.get('qweight'),
                gate._buffers.get('scales'), bias[0], bias[1], bias[2],
                tuple(-1 if b is None else b._version for b in bias), gate.disable_bias, up.disable_bias, down.disable_bias,
-               getattr(gate, 'disable_adapters', None), getattr(up, 'disable_adapters', None), getattr(down, 'disable_adapters', None))
+               _adapters_off(gate), _adapters_off(up), _adapters_off(down))
         if cached is None or not (all(a is b for a, b in zip(cached[0][:7], key[:7])) and cached[0][7:] == key[7:]):
             cached = d['_q4_mlp_args'] = (key, _mlp_decode_args(mlp))
         args = cached[1]

@@ -114,14 +114,16 @@ class Linear4bitLt(Autograd4bitQuantLinear, LoraLayer):
             return None
         if autograd_4bit.backend != 'cuda':
             return None
-        active = [a for a in self.active_adapters if a in self.lora_A.keys()]
+        adapters = self._modules['lora_A']._modules
+        active = [a for a in self.active_adapters if a in adapters]
         if len(active) != 1:
             return None
         name = active[0]
-        r = self.lora_A[name].weight.shape[0]
+        r = autograd_4bit._weight(adapters[name]).shape[0]
         if r % 8 != 0 or not (8 <= r <= 64):
             return None
-        if self._dropout_p(name) >= 1.0 or (self._dropout_p(name) > 0.0 and torch.cuda.is_current_stream_capturing()):
+        p = self._dropout_p(name)
+        if p >= 1.0 or (p > 0.0 and torch.cuda.is_current_stream_capturing()):
             return None                                   # the mask's seed is a launch argument: a replayed graph would repeat it
         rows = x.numel() // x.shape[-1]
         if rows <= autograd_4bit.quant_hip.MAX_GEMV_ROWS:
@@ -134,7 +136,7 @@ class Linear4bitLt(Autograd4bitQuantLinear, LoraLayer):
 
     def _dropout_p(self, name):
         """Probability of the adapter's dropout as it applies to this call (0 in eval mode / without dropout)."""
-        drop = self.lora_dropout[name]
+        drop = self._modules['lora_dropout']._modules[name]
         if isinstance(drop, nn.Dropout) and drop.p > 0.0 and self.training:
             return float(drop.p)
         return 0.0
@@ -145,12 +147,14 @@ class Linear4bitLt(Autograd4bitQuantLinear, LoraLayer):
             return None
         if x.numel() // x.shape[-1] > autograd_4bit.quant_hip.MAX_GEMV_ROWS:
             return None
-        active = [a for a in self.active_adapters if a in self.lora_A.keys()]
+        mods = self._modules                                 # direct: nn.Module's attribute lookup costs a decode step microseconds
+        adapters = mods['lora_A']._modules
+        active = [a for a in self.active_adapters if a in adapters]
         if len(active) != 1:
             return None
         name = active[0]
-        r = self.lora_A[name].weight.shape[0]
-        drop = self.lora_dropout[name]
+        r = autograd_4bit._weight(adapters[name]).shape[0]
+        drop = mods['lora_dropout']._modules[name]
         if r < 1 or r > 64 or self.in_features % 32 or (isinstance(drop, nn.Dropout) and drop.p > 0.0 and self.training):
             return None
         return name

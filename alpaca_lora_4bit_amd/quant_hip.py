@@ -482,6 +482,11 @@ def dequant2(qweight, qzeros, scales, g_idx=None, groupsize=None, out=None):
     return out
 
 
+def _sorted_rows_fit(M, K):
+    """The act-order decode kernel keeps the gathered rows in LDS."""
+    return 1 <= M <= MAX_GEMV_SORTED_ROWS and K >= 1024 and M * (2 * K + 4096) <= 65536
+
+
 def gemv(x, qweight, qzeros, scales, g_idx=None, groupsize=None, out=None, accumulate=False, out_shape=None):
     """y fp16 [M, N] = x [M, K] @ W for M <= 16 (decode).  `out_shape` (same number of elements)
     lets the result be allocated with the caller's leading dimensions instead of being a view."""
@@ -490,6 +495,10 @@ def gemv(x, qweight, qzeros, scales, g_idx=None, groupsize=None, out=None, accum
         if info.plan is None:
             return _host.gemv(x, qweight, qzeros, scales, info.gemv_gidx, info.gemv_gs, out, bool(accumulate),
                               _shape_arg(out_shape))
+        if x.shape[-1] == info.K and _sorted_rows_fit(x.numel() // info.K, info.K):
+            # sorted copy of the packed rows; the kernel gathers x through the permutation itself
+            perm, _, qsorted, gs_sorted = info.plan
+            return _host.gemv(x, qsorted, qzeros, scales, None, gs_sorted, out, bool(accumulate), _shape_arg(out_shape), perm)
     dev, K, N, G = _check_layer(qweight, qzeros, scales, g_idx, groupsize)
     x2 = _flat_half(x, K, dev, "x")
     M = x2.shape[0]
@@ -504,7 +513,7 @@ def gemv(x, qweight, qzeros, scales, g_idx=None, groupsize=None, out=None, accum
     L = _lib.lib()
     nbytes = L.q4_gemv_workspace_bytes(M, K, N)
     plan = _actorder_plan(qweight, scales, g_idx, groupsize, G)
-    if plan is not None and M <= MAX_GEMV_SORTED_ROWS and K >= 1024 and M * (2 * K + 4096) <= 65536:     # rows fit in LDS
+    if plan is not None and _sorted_rows_fit(M, K):
         # sorted copy of the packed rows; the kernel gathers x through the permutation itself
         perm, _, qweight, gs_sorted = plan
         with _device_ctx(dev):
