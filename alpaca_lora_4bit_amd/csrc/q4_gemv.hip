@@ -1206,7 +1206,7 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
         g.layer[0] = a;
         return launch_stream(g, 1, N / kColsPerWave, stream);
     }
-    const GemvPlan p = plan_gemv(K, N, groupsize, seq, 4);
+    const GemvPlan p = plan_gemv(K, groupsize, seq);
     const dim3 grid(N / kColsPerWave, p.splits);
     const dim3 block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);
@@ -1279,7 +1279,7 @@ extern "C" int q4_launch_gemv_group(int n, const void* const* x, const int32_t* 
         }
     }
     if (gemv_stream_takes(K, groupsize)) return launch_stream(g, n, strips, stream);
-    const GemvPlan p = plan_gemv(K, N[0], groupsize, true, 4);      // the plan does not depend on N
+    const GemvPlan p = plan_gemv(K, groupsize, true);
     const dim3 grid(strips, p.splits), block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);
     switch (p.nstep) {
@@ -1306,7 +1306,7 @@ extern "C" int q4_launch_gemv_v1(const void* x, const int32_t* qweight, const vo
     a.acc64 = reinterpret_cast<unsigned long long*>(workspace);
     a.perm = nullptr;
     a.v1_zeros = reinterpret_cast<const half_t*>(zeros);
-    const GemvPlan p = plan_gemv(K, N, K, true, 4);
+    const GemvPlan p = plan_gemv(K, K, true);
     const dim3 grid(N / kColsPerWave, p.splits), block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);
     switch (p.nstep) {                                       // one group: gsteps is always 0

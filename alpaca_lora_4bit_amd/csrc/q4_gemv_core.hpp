@@ -326,29 +326,27 @@ struct GemvPlan {
 
 inline bool group_compatible(int gs32, int nstep, int* gsteps) {
     if (gs32 % nstep == 0) { *gsteps = 0; return true; }
-    if (gs32 < nstep && nstep % gs32 == 0 && (gs32 == 1 || gs32 == 2 || gs32 == 4 || gs32 == 8)) { *gsteps = gs32; return true; }
+    if (gs32 < nstep && nstep % gs32 == 0) { *gsteps = gs32; return true; }
     return false;
 }
 
-// Largest chunk (<= max_nstep steps) that divides K and is compatible with the grouping; 8 waves
+// Largest chunk (4, 2 or 1 steps of 32 rows) that divides K and is compatible with the grouping; 8 waves
 // per workgroup reduce through LDS, the rest of K goes to gridDim.y (measured best on MI355X:
 // ~700 workgroups of 512 threads for the LLaMA-7B MLP shapes).
-inline GemvPlan plan_gemv(int K, int N, int groupsize, bool seq, int max_nstep) {
+inline GemvPlan plan_gemv(int K, int groupsize, bool seq) {
     const int steps = K / 32;
     const int gs32 = seq ? groupsize / 32 : 1;
     GemvPlan p{1, 0, 1, 1};
-    for (int ns : {16, 8, 4, 2, 1}) {
-        if (ns > max_nstep || steps % ns) continue;
+    for (int ns : {4, 2, 1}) {
+        if (steps % ns) continue;
         int gst = 0;
         if (seq && !group_compatible(gs32, ns, &gst)) continue;
         p.nstep = ns; p.gsteps = gst;
         break;
     }
     const int chunks = steps / p.nstep;
-    const int strips = N / kColsPerWave;
-    (void)strips;
     int waves = 8;
-    const int max_waves = (!seq || p.nstep >= 16) ? 8 : 16;      // register budget of the kernels' launch bounds
+    const int max_waves = seq ? 16 : 8;                          // register budget of the kernels' launch bounds
     if (waves > chunks) waves = chunks;
     if (waves > max_waves) waves = max_waves;
     if (waves < 1) waves = 1;

@@ -666,9 +666,9 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(head["gate_up"]["gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(head["gate_up"]["gbs"] / HBM_PEAK_GBS, 4), "traffic": GEMV_TRAFFIC_BYTES,
                      "traffic_source": GEMV_TRAFFIC_SOURCE,
-                     "kernel": "q4::gemv_seq_group_kernel<4, 0> (gate|up, N = 2 x 11008)",
+                     "kernel": "q4::gemv_stream_group_kernel<1, true, 1> (gate|up, N = 2 x 11008)",
                      "bytes_per_launch": head["gate_up"]["bytes"], "avg_launch_us": round(head["gate_up"]["us"], 3),
-                     "other_kernel": {"kernel": "q4::gemv_seq_kernel<4, 0, false> (down, 11008 -> 4096)",
+                     "other_kernel": {"kernel": "q4::gemv_stream_kernel<1, true, 1> (down, 11008 -> 4096)",
                                       "bytes_per_launch": head["down"]["bytes"],
                                       "avg_launch_us": round(head["down"]["us"], 3),
                                       "frac": round(head["down"]["gbs"] / HBM_PEAK_GBS, 4)},
