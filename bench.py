@@ -27,8 +27,8 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, GB/s
 MFMA_FP16_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 MFMA
 # HBM bytes per launch of the headline kernel (the grouped gate|up GEMV), measured in two rocprofv3 --pmc runs
 # (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for a 256 MiB copy (--calibrate-copy):
-# 2 x 23 470.3 KiB read + 903.0 KiB written.  Not re-measured by a bench run: the file named below holds the commands.
-GEMV_TRAFFIC_BYTES = 48991000
+# 2 x 23 472.5 KiB read + 903.0 KiB written.  Not re-measured by a bench run: the file named below holds the commands.
+GEMV_TRAFFIC_BYTES = 48996000
 GEMV_TRAFFIC_SOURCE = "profiles/gemv_mlp_decode_M1_gate_up_grouped_and_down.md"
 
 
