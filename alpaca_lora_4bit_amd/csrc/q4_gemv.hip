@@ -198,7 +198,12 @@ __global__ __launch_bounds__(1024) void gemv_seq_group_kernel(GemvGroupArgs g) {
 // entries of its K range from there into the operand tile and continues as the kernel above.  The
 // permutation entries are requested first and the weights right after, so everything is in flight together.
 // LDS: reduction buffer [nwaves][M][64] fp32, operand tile [M][span] fp16, activation rows [M][K] fp16.
-template <int NSTEP, int GSTEPS>
+// XT pieces of 16 bytes of x per thread (2, 4 or 8), MR >= M rows: as few as the call needs.  With eight pieces and four rows for every
+// call the kernel took 66 registers, three workgroups a compute unit instead of four, and the 1080 workgroups of 5120 -> 13824 went in a
+// round and a half; the smaller forms take 62 or 63 and leave out loads and LDS reads that return nothing.  us, one form ->
+// these: 5120 -> 13824 10.9 -> 9.5 at 1 row, 11.5 -> 10.5 at 2, 11.9 -> 11.3 at 3; 4096 -> 4096 4.8 -> 4.0, 5.1 -> 4.3, 5.3 -> 4.7;
+// 11008 -> 4096 8.0 -> 7.4 at 1 row, level at 2 (eight pieces).
+template <int NSTEP, int GSTEPS, int XT, int MR>
 __global__ __launch_bounds__(1024) void gemv_seq_perm_kernel(GemvArgs a) {
     extern __shared__ float red[];
     const int lane = threadIdx.x & 63;
@@ -220,7 +225,6 @@ __global__ __launch_bounds__(1024) void gemv_seq_perm_kernel(GemvArgs a) {
     // No branch sits between the loads below (out-of-range pieces come back as zeros), so the compiler's wait
     // before the first use of the early ones does not include the weights.
     constexpr int PT = 2;                          // reduction rows per thread: span <= 2 * blockDim.x
-    constexpr int XT = 8;                          // 16-byte pieces of x per thread: M*K*2 <= 64 KB with 512 threads
     const rsrc_t rp = make_rsrc(a.perm, (unsigned)a.K * 4u);
     const rsrc_t rx = make_rsrc(a.x, (unsigned)(a.M * a.K) * 2u);
     int src[PT];
@@ -240,17 +244,17 @@ __global__ __launch_bounds__(1024) void gemv_seq_perm_kernel(GemvArgs a) {
     }
     __syncthreads();
     {
-        half_t got[PT][4];                         // all LDS reads first, then the writes: one LDS latency, not 2*M
+        half_t got[PT][MR];                        // all LDS reads first, then the writes: one LDS latency, not 2*M
 #pragma unroll
         for (int u = 0; u < PT; ++u)
 #pragma unroll
-            for (int m = 0; m < 4; ++m) got[u][m] = xfull[min(m, a.M - 1) * a.K + src[u]];
+            for (int m = 0; m < MR; ++m) got[u][m] = xfull[min(m, a.M - 1) * a.K + src[u]];
 #pragma unroll
         for (int u = 0; u < PT; ++u) {
             const int i = threadIdx.x + u * blockDim.x;
             if (i < span && kbase + i < a.K) {
 #pragma unroll
-                for (int m = 0; m < 4; ++m)
+                for (int m = 0; m < MR; ++m)
                     if (m < a.M) xs[m * span + i] = got[u][m];
             }
         }
@@ -1170,13 +1174,13 @@ extern "C" int q4_gemv_sorted_applicable(int M, int K) {
     return M >= 1 && M <= 4 && K >= 1024 && (size_t)M * ((size_t)K * 2 + 4096) <= 65536;   // K >= 1024: 8 wavefronts
 }
 
-template <int NSTEP>
+template <int NSTEP, int XT, int MR>
 static void launch_seq_perm(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvArgs& a) {
     using namespace q4;
     switch (p.gsteps) {
-        case 0: hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 0>), grid, block, lds, stream, a); break;
-        case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 1>), grid, block, lds, stream, a); break;
-        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 2>), grid, block, lds, stream, a); break;
+        case 0: hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 0, XT, MR>), grid, block, lds, stream, a); break;
+        case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 1, XT, MR>), grid, block, lds, stream, a); break;
+        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_perm_kernel<NSTEP, 2, XT, MR>), grid, block, lds, stream, a); break;
     }
 }
 
@@ -1213,11 +1217,18 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
     if (perm) {
         // + the operand tile and the activation rows; q4_gemv_sorted_applicable() keeps this within 64 KB
         const size_t lds_x = lds + (size_t)M * p.waves * 32 * p.nstep * sizeof(half_t) + (size_t)M * K * sizeof(half_t);
-        if (!seq || M > 4 || lds_x > 65536 || (size_t)M * K / 8 > (size_t)8 * block.x) return -2;
+        const size_t pieces = (size_t)M * K / 8;             // 16-byte pieces of x, up to XT per thread
+        if (!seq || M > 4 || lds_x > 65536 || pieces > (size_t)8 * block.x) return -2;
         switch (p.nstep) {
-            case 4: launch_seq_perm<4>(p, grid, block, lds_x, stream, a); break;
-            case 2: launch_seq_perm<2>(p, grid, block, lds_x, stream, a); break;
-            default: launch_seq_perm<1>(p, grid, block, lds_x, stream, a); break;
+            case 4:
+                if (M == 1 && pieces <= 2 * block.x) launch_seq_perm<4, 2, 1>(p, grid, block, lds_x, stream, a);
+                else if (M == 1 && pieces <= 4 * block.x) launch_seq_perm<4, 4, 1>(p, grid, block, lds_x, stream, a);
+                else if (M == 2 && pieces <= 4 * block.x) launch_seq_perm<4, 4, 2>(p, grid, block, lds_x, stream, a);
+                else if (pieces <= 4 * block.x) launch_seq_perm<4, 4, 4>(p, grid, block, lds_x, stream, a);
+                else launch_seq_perm<4, 8, 4>(p, grid, block, lds_x, stream, a);
+                break;
+            case 2: launch_seq_perm<2, 8, 4>(p, grid, block, lds_x, stream, a); break;
+            default: launch_seq_perm<1, 8, 4>(p, grid, block, lds_x, stream, a); break;
         }
     } else if (seq) {
         switch (p.nstep) {

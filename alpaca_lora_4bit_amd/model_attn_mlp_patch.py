@@ -81,7 +81,8 @@ def _same_adapter(p, q):
 class _MemberGroup:
     """Projections that share their input (q|k|v, gate|up), each on its own tensors.  `run(member, x)` is called from
     Autograd4bitQuantLinear.forward at decode sizes: the first call for an input runs one grouped launch for all
-    members, every member takes its own output tensor exactly once (callers add bias and adapter in place)."""
+    members, every member takes its own output tensor exactly once (callers add bias and adapter in place; `run_adapted`
+    adds the adapters of all members in one more launch)."""
 
     def __init__(self, members):
         self.members = list(members)
@@ -490,11 +491,11 @@ def _mlp_decode_forward(mlp, x):
             rows = x.numel() // args[4]
             if (1 <= rows <= min(int(matmul_utils_4bit.auto_switch_thd), quant_hip.MAX_GEMV_ROWS)
                     and quant_hip.mlp_decode_applicable(rows, args[4], args[5], args[3])
-                    and (rows <= mlp_decode_max_rows or (d['_q4_mlp_gated'] and _steps_unobserved(mlp)))):
+                    and (rows <= mlp_decode_max_rows or (d.get('_q4_mlp_gated') and _steps_unobserved(mlp)))):
                 faster = quant_hip.mlp_rows_is_faster(rows, args[4], args[5])
                 step = quant_hip.mlp_rows_prepared if faster or rows > mlp_decode_max_rows else quant_hip.mlp_decode_prepared
                 return step(x, args[0], args[1], args[2], args[3], tuple(x.shape[:-1]) + (args[6],))
-    if x.is_cuda and d['_q4_mlp_gated'] and _act_unobserved(mlp):
+    if x.is_cuda and d.get('_q4_mlp_gated') and _act_unobserved(mlp):
         return _gated_rows_forward(mlp, x)
     return d['_q4_mlp_forward'](x)
 

@@ -34,6 +34,29 @@ def test_permute_rows_bit_exact(oracle):
     assert _lib.lib().q4_permute_rows(qw.data_ptr(), qw.data_ptr(), qw.data_ptr(), K, N, None) == -2   # in place refused
 
 
+@pytest.mark.parametrize("M,K", [(1, 1024), (1, 8192), (1, 8320), (1, 16384), (1, 16512), (2, 8192), (2, 8320), (3, 5376), (3, 5504), (3, 1024)])
+@pytest.mark.parametrize("gs", [128, 64, 32])
+def test_gathering_product_has_the_bits_of_gather_and_product(M, K, gs):
+    """q4_gemv_sorted_f16 on both sides of the sizes where it changes the number of pieces of x a thread loads, against the
+    product of the gathered activations: the same operands in the same order of sums."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    N, G = 128, K // gs
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=g)
+    qz = torch.randint(-2 ** 31, 2 ** 31 - 1, (G, N // 8), device="cuda", dtype=torch.int32, generator=g)
+    sc = (torch.rand((G, N), device="cuda", generator=g) * 0.02).half()
+    x = torch.randn((M, K), device="cuda", generator=g).half()
+    perm = torch.randperm(K, device="cuda", generator=g).int()
+    want = quant_hip.gemv(x[:, perm.long()].contiguous(), qw, qz, sc, None, gs)
+    L = _lib.lib()
+    ws = torch.zeros(L.q4_gemv_workspace_bytes(M, K, N), device="cuda", dtype=torch.uint8)
+    guard = torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.float16)
+    _lib.check(L.q4_gemv_sorted_f16(x.data_ptr(), qw.data_ptr(), qz.data_ptr(), sc.data_ptr(), perm.data_ptr(), gs, guard.data_ptr(), 0,
+                                    M, K, N, G, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "q4_gemv_sorted_f16")
+    assert torch.equal(guard[:M], want) and bool((guard[M] == 7.0).all()) and not bool(ws.any())
+
+
 @pytest.mark.parametrize("M,K", [(1, 128), (7, 4096), (64, 4096), (300, 11008), (2049, 5120), (33, 32768), (1000, 256)])
 def test_permute_cols_bit_exact(M, K):
     """q4_permute_cols_f16 through the C ABI: out[m, p] = in[m, idx[p]] for a permutation and for an index vector with
