@@ -263,7 +263,7 @@ __global__ __launch_bounds__(1024) void gemv_seq_perm_kernel(GemvArgs a) {
     if (active) {
         ch.load_x(xs + min(c, a.M - 1) * span + (k0 - kbase) + 8 * kk);
         __builtin_amdgcn_sched_barrier(0);
-        ch.multiply(a, yacc, c);
+        ch.template multiply<MR>(a, yacc, c);
     }
     gemv_finish(a, yacc, n0, wave, nwaves, kk, c, gridDim.y);
 }
@@ -1224,6 +1224,7 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
                 if (M == 1 && pieces <= 2 * block.x) launch_seq_perm<4, 2, 1>(p, grid, block, lds_x, stream, a);
                 else if (M == 1 && pieces <= 4 * block.x) launch_seq_perm<4, 4, 1>(p, grid, block, lds_x, stream, a);
                 else if (M == 2 && pieces <= 4 * block.x) launch_seq_perm<4, 4, 2>(p, grid, block, lds_x, stream, a);
+                else if (M == 3 && pieces <= 4 * block.x) launch_seq_perm<4, 4, 3>(p, grid, block, lds_x, stream, a);
                 else if (pieces <= 4 * block.x) launch_seq_perm<4, 4, 4>(p, grid, block, lds_x, stream, a);
                 else launch_seq_perm<4, 8, 4>(p, grid, block, lds_x, stream, a);
                 break;

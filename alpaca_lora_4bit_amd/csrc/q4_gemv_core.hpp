@@ -214,25 +214,15 @@ struct SeqChunk {
         for (int t = 0; t < NSTEP; ++t) xv[t] = *reinterpret_cast<const uint4_t*>(row_chunk + 32 * t);
     }
 
+    // ROWS < 4: the caller has at most that many rows of x, the accumulators of the others hold no registers
+    template <int ROWS = 4>
     __device__ __forceinline__ void multiply(const GemvArgs& a, float4_t yacc[4], int c) const {
         // B operands of the two extra MFMAs: per-position offsets (1024 | 64) and all ones
         const half8_t offs = make_half8(0x64006400u, 0x54005400u, 0x64006400u, 0x54005400u);
         const half8_t ones = make_half8(0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u);
-        // pass 1 (needs the activations, scales and zeros only): A operands, the two weight-independent products, and
-        // from them what the sums of pass 2 start from, so that those end as sum x*(q - z - 1)
+        // pass 1 (needs the activations only): A operands and the two weight-independent products
         half8_t av[NSTEP];
-        float4_t acco_g[NG], accx_g[NG], acc[4];
-        auto start = [&](int gi) {
-            const uint32_t zw = V1 ? 0u : zv[gi] >> ((c & 1) * 16);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
-                acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int r = 0; r < 4; ++r)             // uniform: accumulator rows past M are unused
-                    if (r < a.M) acc[j][r] = V1 ? -acco_g[gi][r] : fmaf(-zf, accx_g[gi][r], -acco_g[gi][r]);
-            }
-        };
+        float4_t acco_g[NG], accx_g[NG];
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
             acco_g[gi] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -248,17 +238,16 @@ struct SeqChunk {
                 accx_g[gi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], ones, accx_g[gi], 0, 0, 0);
             }
         }
-        if constexpr (NG == 1) start(0);                // with several groups later: their sums would only hold registers
-        // mask (scalar register) and magic number (vector register) as opaque values: with two literals the compiler
-        // emits an AND and an OR, with register operands the single three-operand and-or instruction (128 -> 64 of the
-        // 144 instructions that build the operands of a chunk)
-        uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, g_lo = 0x64006400u, g_hi = 0x54005400u;
-        asm volatile("" : "+s"(m_lo), "+s"(m_hi));
-        asm volatile("" : "+v"(g_lo), "+v"(g_hi));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
-            if constexpr (NG > 1) start(gi);
+            // The sums with the codes start from zero and the offset and zero terms come off at the end: the sums with and
+            // without the codes round alike, which cancels.  Letting them start from -(sum x*off + (z + 1) * sum x) saves
+            // these operations and made the fp32 error 1.5 times as large (rms, groups of 128 rows).
+            float4_t acc[4];
+            const float4_t acco = acco_g[gi], accx = accx_g[gi];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int tt = 0; tt < GS; ++tt) {
                 const int t = gi * GS + tt;
@@ -266,26 +255,36 @@ struct SeqChunk {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t hi = w[j] >> 8;
-                    const half8_t bv = make_half8((w[j] & m_lo) | g_lo, (w[j] & m_hi) | g_hi, (hi & m_lo) | g_lo, (hi & m_hi) | g_hi);
+                    const half8_t bv = make_half8((w[j] & 0x000F000Fu) | 0x64006400u, (w[j] & 0x00F000F0u) | 0x54005400u,
+                                                  (hi & 0x000F000Fu) | 0x64006400u, (hi & 0x00F000F0u) | 0x54005400u);
                     acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bv, acc[j], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);      // consume the loads in the order they return
             }
             const half2_t s01 = as_half2(sv[gi].x), s23 = as_half2(sv[gi].y);
             const float sf[4] = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
-            float zf[4] = {0.f, 0.f, 0.f, 0.f};
             if constexpr (V1) {
+                // y += s * (sum x*(off+q) - sum x*off) - zero * sum x
                 const half2_t z01 = as_half2(zh.x), z23 = as_half2(zh.y);
-                zf[0] = (float)z01[0]; zf[1] = (float)z01[1]; zf[2] = (float)z23[0]; zf[3] = (float)z23[1];
-            }
+                const float zf[4] = {(float)z01[0], (float)z01[1], (float)z23[0], (float)z23[1]};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (r < a.M) {                          // uniform: with M <= 3 the other accumulator rows are unused
+                for (int r = 0; r < ROWS; ++r) {
+                    if (r < a.M) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // y += s * sum x*(q - z - 1);  V1: s * sum x*q - zero * sum x
-                        yacc[j][r] = fmaf(sf[j], acc[j][r], yacc[j][r]);
-                        if constexpr (V1) yacc[j][r] = fmaf(-zf[j], accx_g[gi][r], yacc[j][r]);
+                        for (int j = 0; j < 4; ++j) yacc[j][r] += sf[j] * (acc[j][r] - acco[r]) - zf[j] * accx[r];
+                    }
+                }
+            } else {
+                // group epilogue: y += s * ((sum x*(off+q) - sum x*off) - (z+1) * sum x)
+                const uint32_t zw = zv[gi] >> ((c & 1) * 16);
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    if (r < a.M) {                      // uniform: with M <= 3 the other accumulator rows are unused
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
+                            yacc[j][r] += sf[j] * ((acc[j][r] - acco[r]) - zf * accx[r]);
+                        }
                     }
                 }
             }

@@ -33,8 +33,8 @@ inline uint32_t stream_group_inv(int groupsize) {
 // n0 + 4 * (lane % 16) + j.  Chunks from `end` on are left out.  The layers share x, M, K, N and the group size.
 // NG groups per chunk (1, 2, 4; 1: groupsize % 128 == 0).  `tile`: this wavefront's two activation tiles in LDS.  ONE: a single
 // block, in straight line and with nothing requested past it.
-// The operands are built as in gemv_core: codes as 1024 + q or 64 + q, and per group sum x*(q - z - 1) by letting the sums
-// start from -(sum x*offset + (z + 1) * sum x).
+// The operands are built as in gemv_core: codes as 1024 + q or 64 + q, and per group (sum x*(offset + q) - sum x*offset) -
+// (z + 1) * sum x in the same order.
 template <int NL, int NG, bool ONE, typename Flush>
 __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], uint32_t inv, int n0, int block0, int nb, int end,
                                               half_t* tile, float4_t (&yacc)[NL][4], Flush&& flush) {
@@ -137,13 +137,8 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
 #pragma unroll
             for (int e = 0; e < NG; ++e) {
                 float4_t acc[4];
-                const uint32_t zw = zv[S][q][e] >> ((c & 1) * 16);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(-zf, accx[e][r], -acco[e][r]);
-                }
+                for (int j = 0; j < 4; ++j) acc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int t = e * GS; t < (e + 1) * GS; ++t) {
                     const uint32_t ww[4] = {w[S][q][t].x, w[S][q][t].y, w[S][q][t].z, w[S][q][t].w};
@@ -157,10 +152,16 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
                 }
                 const half2_t s01 = as_half2(sv[S][q][e].x), s23 = as_half2(sv[S][q][e].y);
                 const float sf[4] = {(float)s01[0], (float)s01[1], (float)s23[0], (float)s23[1]};
+                const uint32_t zw = zv[S][q][e] >> ((c & 1) * 16);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < 4; ++j) {
+                    const float zf = (float)(((zw >> (4 * j)) & 0xFu) + 1u);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) p[j][r] = e == 0 ? sf[j] * acc[j][r] : fmaf(sf[j], acc[j][r], p[j][r]);
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = sf[j] * ((acc[j][r] - acco[e][r]) - zf * accx[e][r]);
+                        p[j][r] = e == 0 ? v : p[j][r] + v;
+                    }
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll

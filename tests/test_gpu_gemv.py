@@ -216,3 +216,60 @@ def test_gemv_longest_reduction(oracle):
     ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
     assert rel_err(y.cpu().numpy(), ref) <= 2e-3
     assert quant_hip.workspaces_are_zero()
+
+
+def _offset_heavy(M, K, gs, gen):
+    """Activations whose plain sums are exact in fp32 in any order (multiples of 2^-9, partial sums below 2^14) while their sums
+    with the operand offsets (1024 on even rows, 64 on odd ones) need more than 24 bits, and their sum per group."""
+    import torch
+    G = K // gs
+    x = torch.zeros((M, G, gs), dtype=torch.float64)
+    big = torch.randint(256, 512, (M, G, gs // 4), generator=gen).double()
+    x[:, :, 0:gs // 2:2] = big
+    x[:, :, gs // 2::2] = -big.flip(-1)
+    x[:, :, 1::2] = torch.randint(-500, 500, (M, G, gs // 2), generator=gen).double() / 512
+    return x.view(M, K), x.sum(-1)
+
+
+@pytest.mark.parametrize("route,K,gs", [("stream", 4096, 128), ("stream", 1152, 64), ("stream", 1152, 32), ("grouped", 2176, 128),
+                                        ("burst", 2080, 32), ("burst", 2112, 64), ("sorted", 2048, 128), ("sorted", 2048, 32), ("v1", 2048, 2048)])
+@pytest.mark.parametrize("M", [1, 2, 3, 7, 16])
+def test_gemv_offsets_of_the_operands_cancel_exactly(route, K, gs, M):
+    """With all codes 0 the sum with the codes and the sum of the offsets are the same operations, so what is left is
+    -s * (z + 1) * sum x, exact in fp32 here: nothing of the rounding of the offset products may stay in the result."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    if route == "sorted" and M > 3:
+        pytest.skip("the gathering kernel takes up to three rows")
+    gen = torch.Generator().manual_seed(K + gs + M)
+    N, G = 128, K // gs
+    x, sums = _offset_heavy(M, K, min(gs, 128), gen)
+    qw = torch.zeros((K // 8, N), dtype=torch.int32, device="cuda")
+    z = torch.randint(0, 16, (G, N), generator=gen)
+    qz = torch.zeros((G, N // 8), dtype=torch.int64)
+    for b in range(8):
+        qz |= z[:, b::8] << (4 * b)
+    qz = torch.where(qz >= 2 ** 31, qz - 2 ** 32, qz).int().cuda()
+    sc = torch.full((G, N), 0.125, dtype=torch.float16, device="cuda")
+    want = (-0.125 * (sums @ (z + 1).double())).half().cuda() if route != "v1" else None
+    xt = x.half().cuda()
+    assert torch.equal(xt.double().cpu(), x)
+    if route == "grouped":
+        got = quant_hip.gemv_grouped(xt, [(qw, qz, sc)] * 2, gs)[1]
+    elif route == "v1":
+        zeros = torch.full((N, 1), 0.75, dtype=torch.float16, device="cuda")
+        got = quant_hip.gemv_v1(xt, qw, torch.ones_like(zeros), zeros)
+        want = (-0.75 * sums.sum(1, keepdim=True)).half().expand(M, N).cuda()
+    elif route == "sorted":
+        perm = torch.randperm(K, generator=gen)
+        inverse = torch.empty_like(perm)
+        inverse[perm] = torch.arange(K)
+        xt = xt[:, inverse.cuda()].contiguous()              # gathered through perm it is x again
+        got = torch.empty((M, N), dtype=torch.float16, device="cuda")
+        ws = torch.zeros(_lib.lib().q4_gemv_workspace_bytes(M, K, N), device="cuda", dtype=torch.uint8)
+        perm = perm.int().cuda()
+        _lib.check(_lib.lib().q4_gemv_sorted_f16(xt.data_ptr(), qw.data_ptr(), qz.data_ptr(), sc.data_ptr(), perm.data_ptr(), gs, got.data_ptr(),
+                                                 0, M, K, N, G, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "sorted")
+    else:
+        got = quant_hip.gemv(xt, qw, qz, sc, None, gs)
+    assert torch.equal(got, want)
