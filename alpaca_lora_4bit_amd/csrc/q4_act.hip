@@ -1,16 +1,15 @@
 // silu(gate) * up of a gated MLP block above the decode sizes, forward and backward (HBM-bound): the two elementwise kernels of
 // the block's forward (src/alpaca_lora_4bit/model_attn_mlp_patch.py:224-228) and the three of its backward in one pass each.
-// The roundings are those of the separate kernels: silu(gate), the product and, backward, the gradient of silu(gate) go to fp16
-// as they do on tensors between them.  Bytes moved per element: 6 instead of 10 forward, 10 instead of 18
-// backward; 8 elements a thread, one 16-byte load per operand.  us forward / backward, separate kernels -> here: 200 x 11008
-// 8.6 / 17.5 -> 4.3 / 6.1, 1024 x 11008 24.7 / 37.3 -> 12.7 / 20.5, 4096 x 13824 93 / 175 -> 56 / 104 (6.0 and 5.4 TB/s).
+// The results have the bits of the separate kernels: the same fp32 expressions with the exact expf, and silu(gate), the product
+// and, backward, the gradient of silu(gate) go to fp16 as they do on tensors between them.  Bytes moved per element: 6 instead of 10 forward, 10 instead of 18
+// backward; 8 elements a thread, one 16-byte load per operand.  us forward / backward, separate kernels -> here, over operands that
+// come from HBM: 200 x 11008 7.7 / 12.1 -> 5.4 / 7.8, 1024 x 11008 23.9 / 37.4 -> 15.6 / 24.0, 4096 x 13824 93.6 / 176 -> 60.7 / 105
+// (5.6 and 5.4 TB/s); the exact exponential is 0.5 us of the first and nothing of the last.
 #include "q4_common.hpp"
 
 namespace q4 {
 
 constexpr int kActThreads = 256;
-
-__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 template <int V>
 struct Halves { half_t v[V]; };
@@ -32,7 +31,7 @@ __device__ __forceinline__ void silu_mul_item(const half_t* gate, const half_t* 
 #pragma unroll
     for (int e = 0; e < V; ++e) {
         const float x = (float)g.v[e];
-        const half_t s = (half_t)(x / (1.0f + __expf(-x)));
+        const half_t s = (half_t)(x / (1.0f + expf(-x)));
         o.v[e] = (half_t)((float)s * (float)u.v[e]);
     }
     store_halves<V>(out, i, o);
@@ -52,11 +51,11 @@ __device__ __forceinline__ void silu_mul_bwd_item(const half_t* dout, const half
     Halves<V> dg, du;
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-        const float x = (float)g.v[e], dy = (float)d.v[e], sig = sigmoid_f32(x);
-        const half_t s = (half_t)(x / (1.0f + __expf(-x)));
+        const float x = (float)g.v[e], dy = (float)d.v[e], den = 1.0f + expf(-x), sig = 1.0f / den;
+        const half_t s = (half_t)(x / den);
         const half_t ds = (half_t)(dy * (float)u.v[e]);
         du.v[e] = (half_t)(dy * (float)s);
-        dg.v[e] = (half_t)((float)ds * sig * (1.0f + x * (1.0f - sig)));
+        dg.v[e] = (half_t)((float)ds * sig * fmaf(x, 1.0f - sig, 1.0f));
     }
     store_halves<V>(dgate, i, dg);
     store_halves<V>(dup, i, du);

@@ -431,7 +431,7 @@ class _SiluMul(torch.autograd.Function):
 
 def _gated_rows_forward(mlp, x):
     """The block's forward above the decode sizes: its own three layers, silu(gate) * up in one pass (us, forward / backward, 1024 x
-    11008: 25 / 37 as five elementwise kernels, 13 / 21 as two).  Only for forwards known to be this expression."""
+    11008: 24 / 37 as five elementwise kernels, 16 / 24 as two).  Only for forwards known to be this expression."""
     from . import quant_hip
     gate, up = mlp.gate_proj(x), mlp.up_proj(x)
     if not quant_hip.silu_mul_takes(gate, up):

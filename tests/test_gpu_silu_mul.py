@@ -114,3 +114,22 @@ def test_gated_block_trains_like_its_own_forward(oracle):
             assert torch.equal(a, b)
     finally:
         quant_hip.silu_mul = real
+
+
+def test_silu_mul_has_the_bits_of_the_separate_operations():
+    """Every fp16 value of gate with some of up and of the output gradient: the one pass forms the same fp32 expressions as torch's
+    silu, silu_backward and products, so nothing but the sign and payload of a NaN may differ."""
+    import torch
+    import torch.nn.functional as F
+    from alpaca_lora_4bit_amd import quant_hip
+    gate = torch.arange(-2 ** 15, 2 ** 15, device="cuda", dtype=torch.int32).to(torch.int16).view(torch.float16).repeat(8, 1)
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    up, dout = (torch.randn(gate.shape, device="cuda", generator=gen).half() for _ in range(2))
+    dout *= 0.01
+    g, u = gate.clone().requires_grad_(True), up.clone().requires_grad_(True)
+    want = F.silu(g) * u
+    want.backward(dout)
+    dg, du = quant_hip.silu_mul_bwd(dout, gate, up)
+    for got, ref in ((quant_hip.silu_mul(gate, up), want.detach()), (dg, g.grad), (du, u.grad)):
+        num = ~torch.isnan(ref)
+        assert torch.equal(torch.isnan(got), ~num) and torch.equal(got.view(torch.int16)[num], ref.view(torch.int16)[num])
