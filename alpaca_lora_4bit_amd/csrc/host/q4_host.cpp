@@ -302,7 +302,7 @@ std::vector<at::Tensor> mlp_decode(const at::Tensor& x, const std::tuple<at::Ten
     return {y};
 }
 
-// The same step as two launches: gate, up and the activation, then down; the faster way from two rows on.
+// The same step as two launches: gate, up and the activation, then down (quant_hip.mlp_rows_is_faster: when).
 at::Tensor mlp_rows(const at::Tensor& x, const std::tuple<at::Tensor, at::Tensor, at::Tensor>& gate,
                     const std::tuple<at::Tensor, at::Tensor, at::Tensor>& up,
                     const std::tuple<at::Tensor, at::Tensor, at::Tensor>& down, int64_t groupsize,

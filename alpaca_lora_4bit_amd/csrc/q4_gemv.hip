@@ -151,8 +151,6 @@ __device__ __forceinline__ void gemv_stream_body(const GemvArgs& a, const Stream
     const int block0 = blockIdx.y * sa.nb, nb = ONE ? 1 : min(sa.nb, sa.blocks - block0);
     float* const slab = ONE ? red : red + kStreamLds / 4;         // ONE: over the tiles, behind a barrier
     float4_t yacc[1][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) yacc[0][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     const GemvArgs* const layers[1] = {&a};
     stream_blocks<1, NG, ONE>(layers, sa.group_inv, n0, block0, nb, min(a.K >> 7, (block0 + nb) * 2 * kStreamWaves),
                               reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc, [&](int b) {
@@ -164,8 +162,6 @@ __device__ __forceinline__ void gemv_stream_body(const GemvArgs& a, const Stream
                 *reinterpret_cast<float4_t*>(slab + (((b * kStreamWaves + wave) * M + m) << 6) + 4 * c) =
                     float4_t{yacc[0][0][r], yacc[0][1][r], yacc[0][2][r], yacc[0][3][r]};
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) yacc[0][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     });
     __syncthreads();
     stream_finish<ONE, EB>(a, slab, n0, nb, sa.blocks, gridDim.y);

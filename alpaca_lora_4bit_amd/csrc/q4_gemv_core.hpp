@@ -36,15 +36,16 @@ __device__ __forceinline__ half8_t make_half8(uint32_t a, uint32_t b, uint32_t c
     return __builtin_bit_cast(half8_t, v);
 }
 
-// v on the grid of 2^-24 as an integer plus kBias: adding 1.5 * 2^28 leaves it in the low bits of a double's mantissa.
-__device__ __forceinline__ unsigned long long fixed_biased(float v) {
+// v on the grid of 2^-24 as an integer: adding 1.5 * 2^28 leaves it in the low bits of a double's mantissa.
+__device__ __forceinline__ long long fixed_signed(float v) {
     const double d = (double)fminf(fmaxf(v, -kClamp), kClamp) + kGrid;
-    return (unsigned long long)__double_as_longlong(d) + (kBias - kGridBits);
+    return __double_as_longlong(d) - (long long)kGridBits;
 }
-// The sum of n such values, whatever the top 8 bits (the arrival count) hold.
+__device__ __forceinline__ unsigned long long fixed_biased(float v) { return (unsigned long long)(fixed_signed(v) + kBias); }
+__device__ __forceinline__ float fixed_value(long long tot) { return (float)((double)tot * (1.0 / (double)(1 << kFracBits))); }
+// The sum of n biased values, whatever the top 8 bits (the arrival count) hold.
 __device__ __forceinline__ float fixed_sum(unsigned long long sum, int n) {
-    const long long tot = (long long)(sum & ((1ull << 56) - 1)) - (long long)n * kBias;
-    return (float)((double)tot * (1.0 / (double)(1 << kFracBits)));
+    return fixed_value((long long)(sum & ((1ull << 56) - 1)) - (long long)n * kBias);
 }
 
 // Finishes EB outputs per thread (e0, e0 + blockDim.x, ...): all LDS reads of the batch are issued before

@@ -29,7 +29,7 @@ inline uint32_t stream_group_inv(int groupsize) {
 }
 
 // The reduction goes in blocks of 8 chunks, two neighbouring chunks per wavefront; `flush(b)` follows block b of the nb blocks
-// from `block0` on with sums of this wavefront's two chunks added to yacc[layer][j][r]: row 4 * (lane / 16) + r, column
+// from `block0` on with the sums of this wavefront's two chunks in yacc[layer][j][r]: row 4 * (lane / 16) + r, column
 // n0 + 4 * (lane % 16) + j.  Chunks from `end` on are left out.  The layers share x, M, K, N and the group size.
 // NG groups per chunk (1, 2, 4; 1: groupsize % 128 == 0).  `tile`: this wavefront's two activation tiles in LDS.  ONE: a single
 // block, in straight line and with nothing requested past it.
@@ -100,7 +100,7 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
 
     // multiplies a chunk (words and activations in `slot`), chunk `next` requested on the way; without a branch
     // around the requests (past the end: no traffic), or every wait below would have to assume the shorter queue
-    auto step = [&](auto slot, auto more, int next) {
+    auto step = [&](auto slot, auto more, int next) {              // slot 0: the first chunk of a block
         constexpr int S = decltype(slot)::value;
         // the chunk's activations have landed: of everything requested, only what was asked for behind them may be missing
         __builtin_amdgcn_s_waitcnt(0x0F70 | (kBehind & 15) | ((kBehind >> 4) << 14));
@@ -166,7 +166,7 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                yacc[q][j] += p[j];
+                yacc[q][j] = S == 0 ? p[j] : yacc[q][j] + p[j];
                 asm volatile("" : "+v"(yacc[q][j]));       // added here: left to itself the compiler keeps every chunk's sums to the end
             }
             __builtin_amdgcn_sched_barrier(0);

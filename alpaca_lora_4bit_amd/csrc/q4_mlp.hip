@@ -66,14 +66,11 @@ __device__ __forceinline__ uint32_t load_word_agent(const uint32_t* p) {
 
 // silu(g) * u with the roundings of the unfused modules: act_fn on an fp16 tensor evaluates in fp32 and rounds to
 // fp16, the product with up is one more fp16 rounding.
-__device__ __forceinline__ half_t silu_mul(half_t g16, half_t u16) {
-    const float g = (float)g16;
-    const half_t h = (half_t)(g / (1.0f + __expf(-g)));
-    return (half_t)((float)h * (float)u16);
-}
 __device__ __forceinline__ uint32_t silu_mul_bits(uint32_t g_word, uint32_t u_word) {
-    const half_t r = silu_mul(__builtin_bit_cast(half_t, (unsigned short)(g_word & 0xFFFFu)),
-                              __builtin_bit_cast(half_t, (unsigned short)(u_word & 0xFFFFu)));
+    const float g = (float)__builtin_bit_cast(half_t, (unsigned short)(g_word & 0xFFFFu));
+    const float u = (float)__builtin_bit_cast(half_t, (unsigned short)(u_word & 0xFFFFu));
+    const half_t h = (half_t)(g / (1.0f + __expf(-g)));
+    const half_t r = (half_t)((float)h * u);
     return (uint32_t)__builtin_bit_cast(unsigned short, r);
 }
 
@@ -214,57 +211,92 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 }
 
 // ---- gate, up and the activation:  h fp16 [M, I] = silu(gate(x)) * up(x), 1 <= M <= 16 -------------------------------------
-// The first half of the step above for callers that run down as a launch of its own, from two rows on the faster way: the
-// launch above re-reads the intermediate once per output strip of down.  A workgroup owns the same 64 columns of gate and up
-// for the whole reduction (q4_gemv_stream.hpp), so it holds both finished sums and applies the activation itself: no
-// atomics, no workspace, and neither projection leaves the kernel.  A wavefront multiplies each chunk of activations with
-// both layers.  4096 -> 2 x 11008 at 1 / 4 / 16 rows 12.0 / 12.5 / 14.1 us; grouped product, silu and multiply 16 / 18 / 21 us.
+// The first half of the step above for callers that run down as a launch of its own: the launch above re-reads the intermediate
+// once per output strip of down (quant_hip.mlp_rows_is_faster has the rule and both sides measured).  A workgroup owns the same
+// 64 columns of gate and up for the whole reduction (q4_gemv_stream.hpp), so it holds both finished sums and applies the
+// activation itself: no atomics, no workspace, and neither projection leaves the kernel.  A wavefront multiplies each chunk of
+// activations with both layers.  The sums are gemv_stream_kernel's, block by block of 1024 rows in fp32 and from block to block as
+// fixed-point integers, and the activation is the separate module's: h has the bits of the three calls it stands for.  Bound by
+// the instructions of one wavefront per SIMD; the sums of a block therefore go to LDS in the accumulators' own order (row by row
+// they took 0.6 to 1.9 us more, added up block by block behind barriers 1 to 2 us more).  4096 -> 2 x 11008 at 1 / 4 / 16 rows 13.2 / 13.3 / 15.2 us
+// (12.0 / 12.6 / 14.1 with sums carried in fp32 over the whole reduction, which rounds more often); grouped product, silu and multiply 16 / 17 / 21 us.
 struct GateUpArgs {
     GemvArgs gate, up;
     half_t* h;
     uint32_t group_inv;
+    int slots;                                        // blocks whose sums are kept in LDS behind the tiles
 };
+// floats of one block's sums for RG groups of four rows: [wavefront][layer][column 4c + j: j][lane < 16 * RG][row 4 kk + r: r],
+// the order of the accumulators, so that a wavefront writes them as they are
+constexpr int gate_up_slot(int RG) { return kStreamWaves * 2 * 4 * 64 * RG; }
 
-template <int EB>                                     // outputs per thread: EB * 256 >= M * 64
+// silu(g) * u as act_fn and the product with up give it on fp16 tensors
+__device__ __forceinline__ half_t silu_mul_exact(half_t g16, half_t u16) {
+    const float g = (float)g16;
+    const half_t h = (half_t)(g / (1.0f + expf(-g)));
+    return (half_t)((float)h * (float)u16);
+}
+
+template <int RG>                                     // 4 * RG >= M
 __global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(2))) void gate_up_kernel(GateUpArgs a) {
     extern __shared__ float red[];
     const GemvArgs* const layers[2] = {&a.gate, &a.up};
-    const int M = a.gate.M, N = a.gate.N, n0 = blockIdx.x * kColsPerWave;
+    const int n0 = blockIdx.x * kColsPerWave;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int kk = lane >> 4, c = lane & 15;
+    constexpr int kSlot = gate_up_slot(RG);
+    float* const slab = red + kStreamLds / 4;
     float4_t yacc[2][4];
+    const int chunks = a.gate.K >> 7, blocks = (chunks + 2 * kStreamWaves - 1) / (2 * kStreamWaves);
+    // this thread finishes rows 4 i + lane % 4, i < RG, of column n0 + 4 * (lane / 4) + wave
+    long long sum[RG][2];
+    float v[RG][2];                                   // the latest block
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int i = 0; i < RG; ++i) sum[i][0] = sum[i][1] = 0;
+    auto put = [&](float* at) {                       // this wavefront's sums of one block
+        if (lane < 16 * RG)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) yacc[q][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-    const int chunks = a.gate.K >> 7;
-    stream_blocks<2, 1, false>(layers, a.group_inv, n0, 0, (chunks + 2 * kStreamWaves - 1) / (2 * kStreamWaves), chunks,
-                               reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc, [](int) {});
-    __syncthreads();                                  // the tiles become the buffer of the sums: [layer][wavefront][M][64]
+            for (int q = 0; q < 2; ++q)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<float4_t*>(at + wave * (8 * 64 * RG) + (q * 4 + j) * (64 * RG) + 4 * lane) = yacc[q][j];
+    };
+    auto collect = [&](const float* at) {
+        const float* const p = at + wave * (64 * RG) + lane;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = 4 * kk + r;
-            if (m < M)
-                *reinterpret_cast<float4_t*>(red + (((q * kStreamWaves + wave) * M + m) << 6) + 4 * c) =
-                    float4_t{yacc[q][0][r], yacc[q][1][r], yacc[q][2][r], yacc[q][3][r]};
+        for (int i = 0; i < RG; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                float t[kStreamWaves];
+#pragma unroll
+                for (int w = 0; w < kStreamWaves; ++w) t[w] = p[(w * 8 + q * 4) * (64 * RG) + 64 * i];
+                v[i][q] = (t[0] + t[1]) + (t[2] + t[3]);
+                sum[i][q] += fixed_signed(v[i][q]);
+            }
+    };
+    int used = 0;
+    stream_blocks<2, 1, false>(layers, a.group_inv, n0, 0, blocks, chunks, reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc,
+                               [&](int b) {
+        if (b == blocks - 1) return;                  // stays in the registers
+        if (used == a.slots) {                        // uniform: more blocks than LDS
+            __syncthreads();
+            for (int s = 0; s < used; ++s) collect(slab + s * kSlot);
+            __syncthreads();
+            used = 0;
         }
+        put(slab + used * kSlot);
+        ++used;
+    });
     __syncthreads();
-    const int total = M * 64, ws = M << 6;
-    float s[EB][2];
+    put(red);                                         // the last block's over the tiles
+    __syncthreads();
+    for (int s = 0; s < used; ++s) collect(slab + s * kSlot);
+    collect(red);
 #pragma unroll
-    for (int i = 0; i < EB; ++i) {
-        const float* p = red + min((int)threadIdx.x + i * 64 * kStreamWaves, total - 1);
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-            s[i][q] = (p[4 * q * ws] + p[(4 * q + 1) * ws]) + (p[(4 * q + 2) * ws] + p[(4 * q + 3) * ws]);
-    }
-#pragma unroll
-    for (int i = 0; i < EB; ++i) {
-        const int e = threadIdx.x + i * 64 * kStreamWaves;
-        if (e < total) a.h[(size_t)(e >> 6) * N + n0 + (e & 63)] = silu_mul((half_t)s[i][0], (half_t)s[i][1]);
+    for (int i = 0; i < RG; ++i) {
+        const int m = 4 * i + (lane & 3);
+        const half_t g = (half_t)(blocks == 1 ? v[i][0] : fixed_value(sum[i][0])), u = (half_t)(blocks == 1 ? v[i][1] : fixed_value(sum[i][1]));
+        if (m < a.gate.M) a.h[(size_t)m * a.gate.N + n0 + (lane & ~3) + wave] = silu_mul_exact(g, u);
     }
 }
 
@@ -354,10 +386,16 @@ extern "C" int q4_launch_gate_up(const void* x, const int32_t* const* qweight, c
     }
     a.h = reinterpret_cast<half_t*>(h);
     a.group_inv = stream_group_inv(groupsize);
-    const dim3 grid(I / kColsPerWave), block(64 * kStreamWaves);          // kStreamLds also holds 2 x 4 x 16 x 64 sums
-    if (M <= 4) hipLaunchKernelGGL(gate_up_kernel<1>, grid, block, kStreamLds, stream, a);
-    else if (M <= 8) hipLaunchKernelGGL(gate_up_kernel<2>, grid, block, kStreamLds, stream, a);
-    else hipLaunchKernelGGL(gate_up_kernel<4>, grid, block, kStreamLds, stream, a);
+    const dim3 grid(I / kColsPerWave), block(64 * kStreamWaves);
+    // every block but the last where the LDS holds them; with more strips than compute units half of it, for a second workgroup
+    // every block but the last where the LDS holds them; with more strips than compute units half of it, for a second workgroup
+    const int RG = M <= 4 ? 1 : M <= 8 ? 2 : 4, slot = gate_up_slot(RG) * (int)sizeof(float);
+    const int room = (grid.x <= 256 ? 160 : 80) * 1024 - kStreamLds, blocks = (H + 1023) / 1024;
+    a.slots = blocks - 1 < room / slot ? blocks - 1 : room / slot;
+    const size_t lds = kStreamLds + (size_t)a.slots * slot;
+    if (RG == 1) hipLaunchKernelGGL(gate_up_kernel<1>, grid, block, lds, stream, a);
+    else if (RG == 2) hipLaunchKernelGGL(gate_up_kernel<2>, grid, block, lds, stream, a);
+    else hipLaunchKernelGGL(gate_up_kernel<4>, grid, block, lds, stream, a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 

@@ -631,9 +631,10 @@ def mlp_decode_prepared(x, gate, up, down, groupsize, out_shape):
 
 
 def mlp_rows_is_faster(M, H, I):
-    """Whether `mlp_rows` beats `mlp_decode` by more than its second launch costs a host-bound caller.  mlp_decode reads the
-    intermediate again for every 64 outputs of down.  us, mlp_decode / mlp_rows: 4096 -> 11008 21.7 / 20.7 at 4 rows, 24.7 / 21.5
-    at 6, 37.8 / 24.1 at 16; 5120 -> 13824 27.2 / 25.8 at 2 rows, 28.7 / 26.1 at 3, 50.3 / 30.8 at 16; 2048 -> 5632 12.5 / 12.6 at 6."""
+    """Whether a step of 1..4 rows goes out as `mlp_rows` (more rows always do): where that beats `mlp_decode` by more than its
+    second launch costs a host-bound caller.  mlp_decode reads the intermediate again for every 64 outputs of down.  us on the
+    device, mlp_decode / mlp_rows: 4096 -> 11008 18.5 / 20.9 at 1 row, 21.8 / 21.3 at 3, 23.3 / 21.7 at 4, 39.2 / 25.0 at 16; 5120 -> 13824
+    25.8 / 26.5 at 1 row, 28.5 / 27.0 at 2, 31.1 / 27.5 at 3, 52.2 / 32.3 at 16; 2048 -> 5632 11.8 / 12.9 at 4, 12.6 / 13.3 at 6, 17.5 / 15.1 at 16."""
     return M * H * I > 200_000_000
 
 

@@ -157,9 +157,9 @@ Q4_API int q4_mlp_decode_f16(const void *x, const q4_layer_t *gate, const q4_lay
                              void *workspace, size_t workspace_bytes, void *stream);
 
 /* Gate, up and the activation of a gated MLP block in one launch:  h fp16 [M, I] = silu(gate(x)) * up(x), 1 <= M <= 16, with
- * the roundings of the separate modules (gate, up, silu(gate) and the product to fp16).  What q4_mlp_decode_f16 does up to the
- * down projection, for callers that run that as a launch of its own (q4_gemv_f16): faster above four rows, or
- * from about 2e8 of M * H * I on (model_attn_mlp_patch.py:224-228).  groupsize % 128 == 0, H % 128 == 0, I % 64 == 0; no workspace. */
+ * the bits of q4_gemv_f16 on either layer and of silu and the product on fp16 tensors.  What q4_mlp_decode_f16 does up to the
+ * down projection, for callers that run that as a launch of its own (q4_gemv_f16): on the device the faster way from about 1.5e8
+ * of M * H * I on (model_attn_mlp_patch.py:224-228).  groupsize % 128 == 0, H % 128 == 0, I % 64 == 0; no workspace. */
 Q4_API int q4_mlp_gate_up_f16(const void *x, const q4_layer_t *gate, const q4_layer_t *up, int groupsize, void *h,
                               int M, int H, int I, void *stream);
 

@@ -242,3 +242,29 @@ def test_mlp_block_above_four_rows_keeps_its_own_forward_where_it_must(oracle, m
                         assert torch.equal(y, got)
                 assert ungroup(m) == 1 and "_q4_mlp_gated" not in m.__dict__
     assert quant_hip.workspaces_are_zero()
+
+
+@pytest.mark.parametrize("H,I,gs", [(256, 192, 128), (1024, 128, 128), (1152, 192, 384), (4096, 11008, 128), (5120, 13824, 128), (9216, 128, 1024),
+                                    (2048, 16640, 128)])
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9, 16])
+def test_gate_up_launch_has_the_bits_of_the_separate_calls(oracle, H, I, gs, M):
+    """silu(gate) * up out of one launch against the two projections by themselves and torch's activation and product: one block
+    of the reduction, a last block of one chunk, as many blocks as fit in LDS together and more, more strips than compute units."""
+    import torch
+    import torch.nn.functional as F
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    gen = torch.Generator(device="cuda").manual_seed(H + I + M)
+    layers = []
+    for _ in range(2):
+        G = -(-H // gs)
+        qweight = torch.randint(-2 ** 31, 2 ** 31 - 1, (H // 8, I), device="cuda", dtype=torch.int32, generator=gen)
+        qzeros = torch.randint(-2 ** 31, 2 ** 31 - 1, (G, I // 8), device="cuda", dtype=torch.int32, generator=gen)
+        layers.append((qweight, qzeros, (0.02 * torch.rand((G, I), device="cuda", generator=gen)).half()))
+    x = torch.randn((M, H), device="cuda", generator=gen).half()
+    gate, up = (quant_hip.gemv(x, *l, None, gs) for l in layers)
+    h = torch.empty_like(gate)
+    desc = [_lib.Layer(*(t.data_ptr() for t in l)) for l in layers]
+    _lib.check(_lib.lib().q4_mlp_gate_up_f16(x.data_ptr(), ctypes.byref(desc[0]), ctypes.byref(desc[1]), gs, h.data_ptr(), M, H, I,
+                                             torch.cuda.current_stream().cuda_stream), "q4_mlp_gate_up_f16")
+    assert bool(torch.isfinite(gate).all()) and float(gate.abs().max()) > 1.0
+    assert torch.equal(h, F.silu(gate) * up)
