@@ -1,6 +1,7 @@
 // Weight-streaming products for few activation rows:  y[M,N] = x[M,K] @ W   (HBM-bound).
 //   gemv_stream_kernel    1 <= M <= 16, sequential groups of 32, 64 or a multiple of 128 rows, K % 128 == 0 (q4_gemv_stream.hpp)
-//   gemv_seq_kernel       1 <= M <= 16, other sequential groups (also the v1 layout: one scale / zero per column)
+//   gemv_seq_kernel       most of these at one row (plan_stream_takes); 1 <= M <= 16, other sequential groups (also the v1
+//                         layout: one scale / zero per column)
 //   gemv_seq_perm_kernel  1 <= M <= 4, act-order layer with rows sorted by group: gathers x through the permutation
 //   gemv_gidx_kernel      1 <= M <= 16, act-order with per-row groups read through g_idx
 //   skinny_seq_kernel     17 <= M <= 64, sequential groups (fp32 partial rows + ordered reduction)
@@ -64,7 +65,7 @@ struct GemvGroupArgs {
 };
 
 // Chunks of 128 rows in 1, 2 or 4 groups: every launch whose K is a multiple of 128 and whose group size is 32, 64 or a multiple
-// of 128 (gemv_stream_takes).  Grid: strips of 64 columns of all layers x splits of the reduction, nb blocks of 8 chunks each.
+// of 128 (whole_chunks).  Grid: strips of 64 columns of all layers x splits of the reduction, nb blocks of 8 chunks each.
 // A block is summed as the eight-wavefront kernels do, ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)), and blocks are added as
 // fixed-point integers, so a product has the same bits alone, in a group, however it is split, and in q4_mlp.hip.  Longer
 // shares leave the block sums of the wavefronts in LDS ([nb][wavefront][M][64] fp32 behind the tiles) and finish once.
@@ -1127,10 +1128,11 @@ static void launch_seq(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds,
     switch (p.gsteps) {
         case 0: hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0>), grid, block, lds, stream, a); break;
         case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 1>), grid, block, lds, stream, a); break;
+        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 2>), grid, block, lds, stream, a); break;
     }
 }
 
-static bool gemv_stream_takes(int K, int groupsize) {
+static bool whole_chunks(int K, int groupsize) {
     return K % 128 == 0 && (groupsize % 128 == 0 || groupsize == 64 || groupsize == 32);
 }
 template <int NG, bool ONE, int EB>
@@ -1147,14 +1149,31 @@ static void launch_stream_one(const q4::GemvGroupArgs& g, int n, const q4::Strea
     else if (M <= 8) launch_stream_eb<NG, ONE, 2>(g, n, split, grid, lds, stream);
     else launch_stream_eb<NG, ONE, 4>(g, n, split, grid, lds, stream);
 }
+template <int NSTEP>
+static void launch_seq_group(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvGroupArgs& g) {
+    using namespace q4;
+    switch (p.gsteps) {
+        case 0: hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 0>), grid, block, lds, stream, g); break;
+        case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 1>), grid, block, lds, stream, g); break;
+        case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 2>), grid, block, lds, stream, g); break;
+    }
+}
 // n layers (g.layer[0] .. [n - 1]) of `strips` strips in all.  Groups of 64 and 32 rows have one block per workgroup
 // (plan_stream_blocks) but for reductions beyond the arrival count.
-static int launch_stream(const q4::GemvGroupArgs& g, int n, int strips, hipStream_t stream) {
+static int launch_chunks(const q4::GemvGroupArgs& g, int n, int strips, hipStream_t stream) {
     using namespace q4;
     const GemvArgs& a = g.layer[0];
     StreamSplit sp;
     sp.group_inv = stream_group_inv(a.groupsize);
     sp.blocks = (a.K + 1023) / 1024;
+    if (!plan_stream_takes(a.M, sp.blocks, strips, a.groupsize)) {
+        const GemvPlan p{4, a.groupsize % 128 == 0 ? 0 : a.groupsize / 32, 8, sp.blocks};
+        const dim3 grid(strips, p.splits), block(64 * p.waves);
+        const size_t lds = (size_t)p.waves * a.M * 64 * sizeof(float);
+        if (n == 1) launch_seq<4>(p, grid, block, lds, stream, a);
+        else launch_seq_group<4>(p, grid, block, lds, stream, g);
+        return hipGetLastError() == hipSuccess ? 0 : -4;
+    }
     sp.nb = plan_stream_blocks(a.M, sp.blocks, strips, a.groupsize);
     const dim3 grid(strips, (sp.blocks + sp.nb - 1) / sp.nb);
     const size_t lds = kStreamLds + (sp.nb == 1 ? 0 : stream_slab_bytes(a.M, sp.nb));
@@ -1201,10 +1220,10 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
     a.v1_zeros = nullptr;
 
     const bool seq = (g_idx == nullptr);
-    if (seq && !perm && gemv_stream_takes(K, groupsize)) {
+    if (seq && !perm && whole_chunks(K, groupsize)) {
         GemvGroupArgs g;
         g.layer[0] = a;
-        return launch_stream(g, 1, N / kColsPerWave, stream);
+        return launch_chunks(g, 1, N / kColsPerWave, stream);
     }
     const GemvPlan p = plan_gemv(K, groupsize, seq);
     const dim3 grid(N / kColsPerWave, p.splits);
@@ -1229,7 +1248,7 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
         }
     } else if (seq) {
         switch (p.nstep) {
-            case 2: launch_seq<2>(p, grid, block, lds, stream, a); break;      // four steps: gemv_stream_takes
+            case 2: launch_seq<2>(p, grid, block, lds, stream, a); break;      // four steps: whole_chunks
             default: launch_seq<1>(p, grid, block, lds, stream, a); break;
         }
     } else {
@@ -1242,16 +1261,6 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-
-template <int NSTEP>
-static void launch_seq_group(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream,
-                             const q4::GemvGroupArgs& g) {
-    using namespace q4;
-    switch (p.gsteps) {
-        case 0: hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 0>), grid, block, lds, stream, g); break;
-        case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 1>), grid, block, lds, stream, g); break;
-    }
-}
 
 // n layers (1..4) sharing M, K and the group size (sequential groups); layer i: x[i], packed tensors, y[i], N[i];
 // its accumulators start at workspace + 8*M*(N[0] + .. + N[i-1]).
@@ -1286,7 +1295,7 @@ extern "C" int q4_launch_gemv_group(int n, const void* const* x, const int32_t* 
             g.strip_end[i] = 0x7fffffff;
         }
     }
-    if (gemv_stream_takes(K, groupsize)) return launch_stream(g, n, strips, stream);
+    if (whole_chunks(K, groupsize)) return launch_chunks(g, n, strips, stream);
     const GemvPlan p = plan_gemv(K, groupsize, true);
     const dim3 grid(strips, p.splits), block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);

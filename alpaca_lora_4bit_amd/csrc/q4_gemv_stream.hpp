@@ -8,11 +8,12 @@
 // with the activations straight into the operand registers, touched 16 cache lines per activation load and summed twice
 // as many wavefronts per KB of weights.  Here the next chunk's words and activations are on their way while one is multiplied,
 // and the activations come row-contiguous into the wavefront's own LDS tile by the loads themselves (buffer_load ... lds).
-// us at one row / 4 / 16 rows, launches replayed as a graph over cold weights, burst -> stream: 4096 -> 4096 5.0 / 5.4 / 6.6 ->
-// 4.6 / 4.9 / 6.3, 11008 -> 4096 7.9 / 8.4 / 10.5 -> 7.7 / 8.0 / 9.7, q|k|v of 4096 features 8.0 / 8.6 / 10.2 -> 7.9 / 8.3 / 10.0
-// and in groups of 32 rows 9.9 / 11.3 / 13.7 -> 9.1 / 9.4 / 11.3, q|k|v of 5120 features 10.6 / 11.7 / 15.2 -> 10.6 / 11.3 / 12.8,
-// 5120 -> 13824 10.4 / 11.4 / 15.0 -> 10.3 / 10.9 / 12.5.  Eight wavefronts of half the length time the same, words two chunks
-// ahead 0.3 us more, both chunks requested at once 0.2 us more.
+// us at 2 / 4 / 16 rows, launches replayed as a graph over cold weights, burst -> stream: 4096 -> 4096 4.8 / 5.1 / 6.3 ->
+// 4.7 / 4.8 / 6.2, 11008 -> 4096 7.5 / 7.9 / 10.1 -> 7.6 / 7.8 / 9.5, q|k|v of 4096 features 8.2 / 8.5 / 10.3 -> 8.1 / 8.3 / 10.2, in groups
+// of 64 rows at 4 / 16 rows 9.1 / 10.9 -> 9.1 / 11.3, of 32 rows 11.3 / 13.9 -> 10.4 / 12.6, q|k|v of 5120 features 11.1 / 12.1 / 15.7 ->
+// 11.0 / 11.3 / 12.9, 5120 -> 13824 10.2 / 10.9 / 14.9 -> 10.3 / 10.7 / 12.2; one row and small groups: plan_stream_takes.  Eight wavefronts of half
+// the length time the same, words two chunks ahead 0.3 us more, both chunks requested at once 0.2 us more, rows below four skipped by
+// a uniform branch in the scaling 0.1 to 0.6 us more.
 #pragma once
 #include "q4_gemv_core.hpp"
 #include <type_traits>

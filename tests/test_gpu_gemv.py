@@ -273,3 +273,25 @@ def test_gemv_offsets_of_the_operands_cancel_exactly(route, K, gs, M):
     else:
         got = quant_hip.gemv(xt, qw, qz, sc, None, gs)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("K,Ns,gs", [(128, (64,), 128), (384, (64, 128), 128), (896, (192,), 32), (1152, (64, 64), 64), (4096, (4096,), 128),
+                                     (4096, (8192,), 128), (4096, (4096, 4096, 64), 128), (5120, (128,), 64), (2048, (8192, 64), 32), (3200, (13824,), 640)])
+def test_one_and_two_rows_have_the_bits_of_the_first_of_three(K, Ns, gs):
+    """One and two rows go through eight wavefronts of one chunk or through the stream, by groups and number of workgroups; three
+    rows through the stream: the same sums in the same order, alone and in a group."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    gen = torch.Generator(device="cuda").manual_seed(K + sum(Ns))
+    G = -(-K // gs)
+    layers = [(torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=gen),
+               torch.randint(-2 ** 31, 2 ** 31 - 1, (G, N // 8), device="cuda", dtype=torch.int32, generator=gen),
+               torch.rand((G, N), device="cuda", generator=gen).half()) for N in Ns]
+    x = torch.randn((3, K), device="cuda", generator=gen).half()
+    three = [quant_hip.gemv(x, *l, None, gs) for l in layers]
+    for M in (1, 2):
+        grouped = quant_hip.gemv_grouped(x[:M].contiguous(), layers, gs)
+        for l, want, got in zip(layers, three, grouped):
+            assert bool(torch.isfinite(want).all())
+            assert torch.equal(quant_hip.gemv(x[:M].contiguous(), *l, None, gs), want[:M]) and torch.equal(got, want[:M])
+    assert quant_hip.workspaces_are_zero()
