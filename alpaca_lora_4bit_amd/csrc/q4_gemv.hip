@@ -84,16 +84,20 @@ struct GemvStreamGroupArgs {
 };
 
 // EB outputs per thread (EB * 256 >= M * 64, its own instantiation each: a launch pays for every line of code it passes over):
-// the reads, and the atomics, of all of them are under way together.
+// the reads, and the atomics, of all of them are under way together.  A workgroup adds its blocks as signed integers and one
+// bias, the largest its share can be: `per` blocks of at most 2^46 (a block saturates at 2^22).  S * per of these, twice, fit in the
+// 56 bits below the arrival count up to 511; above, a share beyond +-2^23 saturates there, and S <= 255 of them fit.
 template <bool ONE, int EB>
-__device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* slab, int n0, int nb, int blocks, int S) {
+__device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* slab, int n0, int nb, int per, int S) {
     constexpr int T = 64 * kStreamWaves;
     const int M = a.M, total = M * 64, ws = M << 6;              // ws: from one wavefront's sums to the next's
     if (EB == 1 && (int)threadIdx.x >= total) return;
     unsigned long long add[EB], old[EB];
+    const long long bias = ONE || S * per > 511 ? kBias : (long long)per << 46;
+    long long share[EB];
     float direct[EB];
 #pragma unroll
-    for (int i = 0; i < EB; ++i) add[i] = 1ull << 56;
+    for (int i = 0; i < EB; ++i) share[i] = 0;
     constexpr int U = ONE ? 1 : 2;                               // blocks read together
     for (int b = 0; b < nb; b += U) {
         float p[EB][U][4];
@@ -110,12 +114,13 @@ __device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* sl
             for (int u = 0; u < U; ++u) {
                 const float v = (p[i][u][0] + p[i][u][1]) + (p[i][u][2] + p[i][u][3]);
                 if (ONE) direct[i] = v;
-                if (u == 0 || b + u < nb) add[i] += fixed_biased(v);
+                if (u == 0 || b + u < nb) share[i] += fixed_signed(v);
             }
     }
 #pragma unroll
     for (int i = 0; i < EB; ++i) {
         const int e = threadIdx.x + i * T;
+        add[i] = (1ull << 56) + (unsigned long long)((ONE ? share[i] : min(max(share[i], -bias), bias)) + bias);
         old[i] = 0;
         if (S > 1 && e < total)
             old[i] = __hip_atomic_fetch_add(a.acc64 + (size_t)(e >> 6) * a.N + n0 + (e & 63), add[i], __ATOMIC_RELAXED,
@@ -128,7 +133,7 @@ __device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* sl
     for (int i = 0; i < EB; ++i) {
         const int e = threadIdx.x + i * T;
         last[i] = e < total && (old[i] >> 56) == (unsigned long long)(S - 1);      // last of the S workgroups of the strip
-        out[i] = ONE && S == 1 ? direct[i] : fixed_sum(old[i] + add[i], blocks);
+        out[i] = S > 1 ? fixed_sum(old[i] + add[i], S, bias) : ONE ? direct[i] : fixed_value(share[i]);
         if (a.accumulate && last[i]) out[i] += (float)a.y[(size_t)(e >> 6) * a.N + n0 + (e & 63)];
     }
 #pragma unroll
@@ -165,7 +170,7 @@ __device__ __forceinline__ void gemv_stream_body(const GemvArgs& a, const Stream
         }
     });
     __syncthreads();
-    stream_finish<ONE, EB>(a, slab, n0, nb, sa.blocks, gridDim.y);
+    stream_finish<ONE, EB>(a, slab, n0, nb, sa.nb, gridDim.y);
 }
 
 template <int NG, bool ONE, int EB>

@@ -44,8 +44,8 @@ __device__ __forceinline__ long long fixed_signed(float v) {
 __device__ __forceinline__ unsigned long long fixed_biased(float v) { return (unsigned long long)(fixed_signed(v) + kBias); }
 __device__ __forceinline__ float fixed_value(long long tot) { return (float)((double)tot * (1.0 / (double)(1 << kFracBits))); }
 // The sum of n biased values, whatever the top 8 bits (the arrival count) hold.
-__device__ __forceinline__ float fixed_sum(unsigned long long sum, int n) {
-    return fixed_value((long long)(sum & ((1ull << 56) - 1)) - (long long)n * kBias);
+__device__ __forceinline__ float fixed_sum(unsigned long long sum, int n, long long bias = kBias) {
+    return fixed_value((long long)(sum & ((1ull << 56) - 1)) - (long long)n * bias);
 }
 
 // Finishes EB outputs per thread (e0, e0 + blockDim.x, ...): all LDS reads of the batch are issued before

@@ -12,6 +12,7 @@ WRAPPER = r"""
 extern "C" int blocks_per_workgroup(int M, int blocks, int strips, int groupsize) {
     return q4::plan_stream_blocks(M, blocks, strips, groupsize);
 }
+extern "C" int stream_takes(int M, int blocks, int strips, int groupsize) { return q4::plan_stream_takes(M, blocks, strips, groupsize); }
 extern "C" long slab(int M, int nb) { return (long)q4::stream_slab_bytes(M, nb); }
 """
 
@@ -38,3 +39,8 @@ def test_every_split_fits_the_arrival_count_and_the_lds(plan, groupsize):
                 # beside the activation tiles (32 KB) within the 160 KB of a compute unit
                 assert nb == 1 or plan.slab(M, nb) <= 128 * 1024
                 assert nb == 1 or blocks > 255 or (strips * splits <= 256 and groupsize % 128 == 0 and M >= 5)
+                # the fixed-point exchange below the arrival count: a workgroup adds up to twice its bias
+                if plan.stream_takes(M, blocks, strips, groupsize):
+                    assert splits * 2 * (nb << 46 if nb > 1 and splits * nb <= 511 else 1 << 47) < 2 ** 56
+                else:
+                    assert blocks * 2 ** 48 < 2 ** 56

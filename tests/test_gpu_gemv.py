@@ -295,3 +295,33 @@ def test_one_and_two_rows_have_the_bits_of_the_first_of_three(K, Ns, gs):
             assert bool(torch.isfinite(want).all())
             assert torch.equal(quant_hip.gemv(x[:M].contiguous(), *l, None, gs), want[:M]) and torch.equal(got, want[:M])
     assert quant_hip.workspaces_are_zero()
+
+
+@pytest.mark.parametrize("blocks,gs,M", [(257, 64, 2), (300, 32, 5), (600, 128, 1), (600, 1024, 16), (1020, 128, 3), (1020, 32, 9)])
+def test_gemv_of_more_blocks_than_arrivals(oracle, blocks, gs, M):
+    """Shares of several blocks, up to the longest reduction that is taken, for every number of groups per chunk and of outputs per
+    thread: the exchange holds them, the result is the sum and the accumulators are left zero.  The last block has one chunk."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    K, N = blocks * 1024 - 896, 64
+    layer = oracle.make_layer(K, N, gs, seed=blocks)
+    t = to_cuda_layer(layer)
+    x = oracle.make_activations(M, K, seed=M)
+    y = quant_hip.gemv(torch.from_numpy(x).cuda(), t["qweight"], t["qzeros"], t["scales"], None, gs)
+    ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
+    assert rel_err(y.cpu().numpy(), ref) <= 2e-3
+    assert quant_hip.workspaces_are_zero()
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_gemv_shares_beyond_the_exchange_saturate(sign):
+    """1020 blocks of sums beyond 2^22 in 255 workgroups: the most the exchange can be asked to hold, in either direction."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    K, N = 1020 * 1024, 64
+    qw = torch.full((K // 8, N), -1, dtype=torch.int32, device="cuda")                # codes 15, zero points 1
+    qz = torch.zeros((K // 128, N // 8), dtype=torch.int32, device="cuda")
+    x = torch.full((1, K), sign * 60000.0, dtype=torch.float16, device="cuda")
+    y = quant_hip.gemv(x, qw, qz, torch.full((K // 128, N), 2.0, dtype=torch.float16, device="cuda"), None, 128)
+    assert torch.equal(y, torch.full_like(y, sign * float("inf")))
+    assert quant_hip.workspaces_are_zero()
