@@ -21,6 +21,7 @@ import re
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 
 from . import autograd_4bit, matmul_utils_4bit
 from .autograd_4bit import Autograd4bitQuantLinear, _buffer, _has_bias, _weight, fuse_quant_linears
@@ -377,9 +378,7 @@ def _is_gated_forward(forward):
     if code is None:
         return False
 
-    def key(c):
-        return (c.co_code, c.co_names, c.co_consts[1:], c.co_argcount, c.co_kwonlyargcount, c.co_flags & 0x0F, c.co_freevars)
-    return any(key(code) == key(f.__code__) for f in (_GatedForward.returned, _GatedForward.assigned))
+    return any(_code_key(code) == _code_key(f.__code__) for f in (_GatedForward.returned, _GatedForward.assigned))
 
 
 def _steps_unobserved(mlp):
@@ -392,8 +391,43 @@ def _steps_unobserved(mlp):
     return _is_silu(mods['act_fn']) and not torch.nn.modules.module._has_any_global_hook()
 
 
+def _code_key(c):
+    return (c.co_code, c.co_names, c.co_consts[1:], c.co_argcount, c.co_kwonlyargcount, c.co_flags & 0x0F, c.co_freevars)
+
+
+class _SiluForward:
+    """The forwards of activation modules that are silu and nothing else: compared by their code."""
+
+    def functional(self, input):
+        return nn.functional.silu(input)
+
+    def short(self, input):
+        return F.silu(input)
+
+
+_SILU, _SILU_MODULE = F.silu, nn.SiLU.forward
+
+
 def _is_silu(act):
-    return isinstance(act, nn.SiLU) or type(act).__name__.lower() in ("silu", "siluactivation") or act is torch.nn.functional.silu
+    """True for silu itself and for a module whose class runs exactly that: nn.SiLU and classes with its forward, or with one that is
+    `return nn.functional.silu(input)` (transformers' SiLUActivation).  The class's name or base says nothing about its forward."""
+    if F.silu is not _SILU:
+        return False                                         # somebody replaced it
+    if act is _SILU:
+        return True
+    if not isinstance(act, nn.Module) or 'forward' in act.__dict__ or type(act).__call__ is not nn.Module.__call__:
+        return False
+    forward = type(act).forward
+    if forward is _SILU_MODULE:
+        return True
+    code = getattr(forward, '__code__', None)
+    if code is None:
+        return False
+    names = forward.__globals__
+    return (code.co_code == _SiluForward.functional.__code__.co_code and _code_key(code) == _code_key(_SiluForward.functional.__code__)
+            and names.get('nn') is nn
+            or code.co_code == _SiluForward.short.__code__.co_code and _code_key(code) == _code_key(_SiluForward.short.__code__)
+            and names.get('F') is F)
 
 
 def _plain_no_bias(layer):
@@ -490,7 +524,7 @@ def _mlp_decode_forward(mlp, x):
         if args is not None and x.shape[-1] == args[4]:
             rows = x.numel() // args[4]
             if (1 <= rows <= min(int(matmul_utils_4bit.auto_switch_thd), quant_hip.MAX_GEMV_ROWS)
-                    and quant_hip.mlp_decode_applicable(rows, args[4], args[5], args[3])
+                    and quant_hip.mlp_decode_applicable(rows, args[4], args[5], args[3]) and _is_silu(mods.get('act_fn') if 'act_fn' in mods else getattr(mlp, 'act_fn', None))
                     and (rows <= mlp_decode_max_rows or (d.get('_q4_mlp_gated') and _steps_unobserved(mlp)))):
                 faster = quant_hip.mlp_rows_is_faster(rows, args[4], args[5])
                 step = quant_hip.mlp_rows_prepared if faster or rows > mlp_decode_max_rows else quant_hip.mlp_decode_prepared
