@@ -79,6 +79,23 @@ def _same_adapter(p, q):
     return p[0] is q[0] and p[2] is q[2] and (p[1], p[3], p[4]) == (q[1], q[3], q[4])
 
 
+def _layer_key(m):
+    """What is kept about layer `m` rests on: its buffers, their contents as the version counters show them, and the count of
+    quant_hip.invalidate calls, which stand for writes that the counters do not show."""
+    b = m._buffers
+    q, z, s, g = b.get('qweight'), b.get('qzeros'), b.get('scales'), b.get('g_idx')
+    return (q, z, s, g, q._version, z._version, s._version, -1 if g is None else g._version, matmul_utils_4bit.quant_hip.invalidations)
+
+
+def _same_layer(m, k):
+    """_layer_key(m) is `k`, without building it."""
+    b = m._buffers
+    g = b.get('g_idx')
+    return (b.get('qweight') is k[0] and b.get('qzeros') is k[1] and b.get('scales') is k[2] and g is k[3] and k[0]._version == k[4]
+            and k[1]._version == k[5] and k[2]._version == k[6] and (g is None or g._version == k[7])
+            and matmul_utils_4bit.quant_hip.invalidations == k[8])
+
+
 class _MemberGroup:
     """Projections that share their input (q|k|v, gate|up), each on its own tensors.  `run(member, x)` is called from
     Autograd4bitQuantLinear.forward at decode sizes: the first call for an input runs one grouped launch for all
@@ -90,7 +107,7 @@ class _MemberGroup:
         self.index = {id(m): i for i, m in enumerate(self.members)}
         self.groupsize = self.members[0].groupsize
         self.usable = None                                   # decided at the first call (needs the tensors on the GPU)
-        self._layer_cache = None
+        self._layer_cache = self._keys = None
         self._gemm_ok = None                                 # sequential groups AND scales below 64 (the tiled kernels' fused form)
         self.hook = None
         self.clear()
@@ -108,31 +125,34 @@ class _MemberGroup:
         return all(m.scales.dtype == torch.float16 for m in self.members)
 
     def _layers(self):
-        """(qweight, qzeros, scales) of every member, rebuilt when a member's buffers were replaced (a cast, a reload)."""
-        cached = self._layer_cache
-        if cached is not None:
-            for m, c in zip(self.members, cached):
-                b = m._buffers
-                if b.get('qweight') is not c[0] or b.get('scales') is not c[2]:
+        """(qweight, qzeros, scales) of every member, rebuilt when a member's buffers were replaced (a cast, a reload) or written in
+        place, or `quant_hip.invalidate` was called."""
+        if self._layer_cache is not None:
+            for m, k in zip(self.members, self._keys):
+                if not _same_layer(m, k):
                     break
             else:
-                return cached
+                return self._layer_cache
+        self.clear()                                         # outputs of the tensors as they were
         self.usable = self._check()
         self._gemm_ok = None
         self._layer_cache = [(m.qweight, m.qzeros, m.scales) for m in self.members] if self.usable else None
+        self._keys = [_layer_key(m) for m in self.members] if self.usable else None
         return self._layer_cache
 
     def run(self, member, x):
-        layers = self._layers()
-        if layers is None:
-            return None
         i = self.index[id(member)]
-        if not self._current(i, x) or self._adapted[i] is not None:
+        if not self._held(i, x) or self._adapted[i] is not None:
+            layers = self._layers()
+            if layers is None:
+                return None
             self._launch(x, layers)
         return self._take(i)
 
-    def _current(self, i, x):
-        return self._x is x and self._version == x._version and self._outs[i] is not None
+    def _held(self, i, x):
+        """Member i's output for x is there, of the tensors that the member has now."""
+        return (self._x is x and self._version == x._version and self._outs[i] is not None
+                and _same_layer(self.members[i], self._keys[i]))
 
     def _launch(self, x, layers):
         # the compiled binding checks shapes, dtypes and devices; sequential groups were established by _check()
@@ -154,12 +174,14 @@ class _MemberGroup:
         """`run` for a member whose adapter `name` is to be added (decode sizes): the products of all members in one launch and
         the adapters of all members in the next, each member picks its finished output up.  None when the group does not take
         this call.  An output that was finished with another adapter than the member now asks for is not handed out."""
-        layers = self._layers()
         adapter = self._adapter(member, name, x)
-        if layers is None or adapter is None:
+        if adapter is None:
             return None
         i = self.index[id(member)]
-        if not self._current(i, x) or (self._adapted[i] is not None and not _same_adapter(self._adapted[i], adapter)):
+        if not self._held(i, x) or (self._adapted[i] is not None and not _same_adapter(self._adapted[i], adapter)):
+            layers = self._layers()
+            if layers is None:
+                return None
             self._launch(x, layers)
         if self._adapted[i] is None:
             todo = {i: adapter}
@@ -210,7 +232,7 @@ class _MemberGroup:
         the group does not take this call (the member then runs by itself)."""
         i = self.index[id(member)]
         key = (x._version, torch.is_grad_enabled())
-        if self._gx is x and self._gkey == key and self._gouts[i] is not None:
+        if self._gx is x and self._gkey == key and self._gouts[i] is not None and _same_layer(member, self._keys[i]):
             y, self._gouts[i] = self._gouts[i], None
             if all(o is None for o in self._gouts):
                 self._gx = None
@@ -272,7 +294,7 @@ class _MemberGroup:
         self.index[id(new)] = i
         new.__dict__['_q4_group'] = self
         self.usable = None
-        self._layer_cache = None
+        self._layer_cache = self._keys = None
         self.clear()
 
 
@@ -513,13 +535,16 @@ def _mlp_decode_forward(mlp, x):
         cached = d.get('_q4_mlp_args')
         mods = mlp._modules
         gate, up, down = mods['gate_proj'], mods['up_proj'], mods['down_proj']
+        group = gate.__dict__.get('_q4_group')
+        layers = None if group is None else group._layers()  # the same list as long as nothing about gate and up changed
         bias = [l._buffers.get('bias') for l in (gate, up, down)]
-        key = (gate._buffers.get('qweight'), up._buffers.get('qweight'), down._buffers.get('qweight'),
-               gate._buffers.get('scales'), bias[0], bias[1], bias[2],
+        key = (layers, bias[0], bias[1], bias[2], down._buffers.get('qweight'),
                tuple(-1 if b is None else b._version for b in bias), gate.disable_bias, up.disable_bias, down.disable_bias,
                _adapters_off(gate), _adapters_off(up), _adapters_off(down))
-        if cached is None or not (all(a is b for a, b in zip(cached[0][:7], key[:7])) and cached[0][7:] == key[7:]):
-            cached = d['_q4_mlp_args'] = (key, _mlp_decode_args(mlp))
+        if (cached is None or not (all(a is b for a, b in zip(cached[0][:5], key[:5])) and cached[0][5:] == key[5:])
+                or (cached[1] is not None and not _same_layer(down, cached[2]))):
+            args = _mlp_decode_args(mlp)
+            cached = d['_q4_mlp_args'] = (key, args, None if args is None else _layer_key(down))
         args = cached[1]
         if args is not None and x.shape[-1] == args[4]:
             rows = x.numel() // args[4]

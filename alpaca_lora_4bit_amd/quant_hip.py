@@ -255,10 +255,15 @@ def _layer_info(qweight, qzeros, scales, g_idx, groupsize):
     return info
 
 
+invalidations = 0                                       # calls of `invalidate` so far: verdicts kept elsewhere compare it
+
+
 def invalidate(*tensors_or_modules):
     """Forget what was cached about these tensors (or about every tensor of these modules): the layer verdicts,
     the g_idx classification, the scale-range check and the sorted copy of an act-order layer.  Needed only after
     writing packed tensors through `.data` (which does not bump the version counter the caches are keyed on)."""
+    global invalidations
+    invalidations += 1
     for obj in tensors_or_modules:
         items = [obj] if isinstance(obj, torch.Tensor) else [t for _, t in obj.named_buffers()] + list(obj.parameters())
         for t in items:

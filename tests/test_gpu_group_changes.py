@@ -1,0 +1,101 @@
+"""Grouped projections and fused MLP blocks whose layers change between calls give what the same layers give ungrouped: what the
+group and the block keep from one call to the next follows the tensors."""
+import copy
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(a, b):
+    """The same products, in groups or with the rows of an act-order layer sorted: sums in another order, one fp16 rounding apart."""
+    from conftest import rel_err
+    assert rel_err(a.float().cpu().numpy(), b.double().cpu().numpy()) <= 3e-3
+
+
+def _mlp(oracle, H, I, gs):
+    import torch
+    import torch.nn as nn
+    from conftest import to_cuda_layer
+    from alpaca_lora_4bit_amd.autograd_4bit import Autograd4bitQuantLinear
+
+    class Gated(nn.Module):
+        def forward(self, x):
+            return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+
+    m = Gated()
+    m.act_fn = nn.SiLU()
+    for i, (name, k, n) in enumerate((("gate_proj", H, I), ("up_proj", H, I), ("down_proj", I, H))):
+        lin = Autograd4bitQuantLinear(k, n, groupsize=gs)
+        for key, v in to_cuda_layer(oracle.make_layer(k, n, gs, seed=50 + i)).items():
+            if isinstance(v, torch.Tensor):
+                setattr(lin, key, v)
+        lin.bias = torch.zeros(n, dtype=torch.float16, device="cuda")
+        setattr(m, name, lin)
+    return m
+
+
+def _shuffled(g_idx):
+    import torch
+    return g_idx[torch.randperm(g_idx.numel(), generator=torch.Generator().manual_seed(9)).to(g_idx.device)]
+
+
+def _change(block, what):
+    """One change of one of the block's layers, the same for the grouped and the ungrouped block."""
+    from alpaca_lora_4bit_amd import quant_hip
+    layer, buffer, how = what
+    m = getattr(block, layer)
+    t = getattr(m, buffer)
+    new = _shuffled(t) if buffer == "g_idx" else t * 0.5 if t.is_floating_point() else t.roll(1, -1)
+    if how == "replaced":
+        setattr(m, buffer, new)
+    elif how == "written":
+        t.copy_(new)
+    else:                                                    # behind the version counter's back, and said so
+        t.data.copy_(new)
+        quant_hip.invalidate(m)
+
+
+CHANGES = [(layer, buffer, how) for how in ("replaced", "written", "invalidated") for layer, buffer in
+           (("down", "scales"), ("up", "qzeros"), ("gate", "scales"), ("down", "qweight"), ("up", "g_idx"), ("down", "g_idx"))]
+
+
+@pytest.mark.parametrize("rows", [1, 8, 40])
+@pytest.mark.parametrize("layer,buffer,how", CHANGES)
+def test_mlp_step_follows_its_layers(oracle, rows, layer, buffer, how):
+    import torch
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_fused_mlp
+    own = _mlp(oracle, 256, 384, 128)
+    fused = copy.deepcopy(own)
+    assert make_fused_mlp(fused) == 1
+    x = torch.from_numpy(oracle.make_activations(rows, 256, seed=rows)).cuda()
+    with torch.no_grad():
+        before = own(x)
+        _close(fused(x), before)
+        for m in (own, fused):
+            _change(m, (layer + "_proj", buffer, how))
+        want = own(x)
+        assert not torch.equal(want, before)
+        _close(fused(x), want)
+
+
+@pytest.mark.parametrize("rows,N", [(3, 512), (200, 4096)])
+@pytest.mark.parametrize("layer,buffer,how", [("k", "qzeros", "replaced"), ("k", "qweight", "written"), ("v", "scales", "written"), ("q", "g_idx", "written"), ("v", "g_idx", "replaced"),
+                                              ("k", "g_idx", "invalidated")])
+def test_grouped_projections_follow_their_layers(oracle, rows, N, layer, buffer, how):
+    """Also when a member changes after another of the group was called for the same input."""
+    import torch
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_quant_attn
+    from test_gpu_gemm_grouped import _Block
+    grouped, plain = (_Block(oracle, 1024, N, 128, 0.0, 70).eval() for _ in range(2))
+    assert make_quant_attn(grouped) == 1
+    x = torch.from_numpy(oracle.make_activations(rows, 1024, seed=rows)).cuda()
+    others = [n for n in ("q_proj", "k_proj", "v_proj") if n != layer + "_proj"]
+    with torch.no_grad():
+        for a, b in zip(grouped(x), plain(x)):
+            _close(a, b)
+        _close(getattr(grouped, others[0])(x), getattr(plain, others[0])(x))
+        for b in (grouped, plain):
+            _change(b, (layer + "_proj", buffer, how))
+        for name in (layer + "_proj", others[1], others[0]):
+            _close(getattr(grouped, name)(x), getattr(plain, name)(x))
