@@ -76,7 +76,7 @@ _ADAPTER_TYPES = (torch.float16, torch.float32)
 
 
 def _same_adapter(p, q):
-    return p[0] is q[0] and p[2] is q[2] and (p[1], p[3], p[4]) == (q[1], q[3], q[4])
+    return p[0] is q[0] and p[1] is q[1] and p[2:] == q[2:]
 
 
 def _layer_key(m):
@@ -173,7 +173,8 @@ class _MemberGroup:
     def run_adapted(self, member, x, name):
         """`run` for a member whose adapter `name` is to be added (decode sizes): the products of all members in one launch and
         the adapters of all members in the next, each member picks its finished output up.  None when the group does not take
-        this call.  An output that was finished with another adapter than the member now asks for is not handed out."""
+        this call.  An output that was finished with another adapter than the member now asks for is not handed out: other matrices,
+        other storage, a write that the version counters show or that quant_hip.invalidate was told of."""
         adapter = self._adapter(member, name, x)
         if adapter is None:
             return None
@@ -195,7 +196,7 @@ class _MemberGroup:
                 flat = x.dim() == 2
                 matmul_utils_4bit.quant_hip.lora_update_grouped(
                     x if flat and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous(),
-                    [(ad[0], ad[2], self._outs[j] if flat else self._outs[j].view(-1, self._outs[j].shape[-1]), ad[4]) for j, ad in todo.items()])
+                    [(ad[0], ad[1], self._outs[j] if flat else self._outs[j].view(-1, self._outs[j].shape[-1]), ad[2]) for j, ad in todo.items()])
             except BaseException:
                 self.clear()                                 # some outputs may have been updated
                 raise
@@ -205,7 +206,7 @@ class _MemberGroup:
 
     @staticmethod
     def _adapter(m, name, x):
-        """(A, its version, B, its version, scaling) of member m's adapter as the grouped update takes it, or None."""
+        """(A, B, scaling, what their contents are known by) of member m's adapter as the grouped update takes it, or None."""
         if _has_bias(m):
             return None                                      # the bias comes between the product and the update
         mods = m._modules
@@ -213,8 +214,7 @@ class _MemberGroup:
         for w in (a, b):
             if w.get_device() != dev or w.dtype not in _ADAPTER_TYPES or w.is_inference():
                 return None
-        scaling = float(m.scaling[name])
-        return a, a._version, b, b._version, scaling
+        return a, b, float(m.scaling[name]), (a._version, b._version, a.data_ptr(), b.data_ptr(), matmul_utils_4bit.quant_hip.invalidations)
 
     def _gemm_spec(self, m, x):
         """How member `m` enters a grouped GEMM for input x: (bias | None, lora_A | None, lora_B | None, scaling, drop_p)."""

@@ -99,3 +99,30 @@ def test_grouped_projections_follow_their_layers(oracle, rows, N, layer, buffer,
             _change(b, (layer + "_proj", buffer, how))
         for name in (layer + "_proj", others[1], others[0]):
             _close(getattr(grouped, name)(x), getattr(plain, name)(x))
+
+
+@pytest.mark.parametrize("matrix", ["lora_A", "lora_B"])
+@pytest.mark.parametrize("how", ["storage", "invalidated", "version"])
+def test_adapter_changed_between_two_members(oracle, matrix, how):
+    """v's adapter is added together with q's; a change of it in between is followed."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_quant_attn
+    from test_gpu_gemm_grouped import _Block
+    grouped, plain = (_Block(oracle, 1024, 512, 128, 0.0, 80).eval() for _ in range(2))
+    for b in (grouped, plain):
+        b.v_proj.bias.zero_()
+    assert make_quant_attn(grouped) == 1
+    x = torch.from_numpy(oracle.make_activations(2, 1024, seed=8)).cuda()
+    with torch.no_grad():
+        _close(grouped.q_proj(x), plain.q_proj(x))
+        for b in (grouped, plain):
+            w = getattr(b.v_proj, matrix)["default"].weight
+            if how == "storage":
+                w.data = w.data * -3.0
+            elif how == "version":
+                w.mul_(-3.0)
+            else:
+                w.data.mul_(-3.0)
+                quant_hip.invalidate(b.v_proj)
+        _close(grouped.v_proj(x), plain.v_proj(x))
