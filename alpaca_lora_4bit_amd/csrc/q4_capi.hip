@@ -263,7 +263,8 @@ extern "C" int q4_mlp_gate_up_f16(const void* x, const q4_layer_t* gate, const q
     return q4_launch_gate_up(x, qw, qz, sc, groupsize, h, M, H, I, (hipStream_t)stream);
 }
 
-static bool act_size(long long n) { return n >= 1 && n < (1ll << 38); }          /* 2^31 workgroups of 256 x 8 elements */
+/* a grid has less than 2^32 threads, here 256 more than n / 8 at most */
+static bool act_size(long long n) { return n >= 1 && n < (1ll << 35) - 2048; }
 
 extern "C" int q4_silu_mul_f16(const void* gate, const void* up, void* out, long long n, void* stream) {
     if (!gate || !up || !out) return Q4_ERR_NULL_POINTER;

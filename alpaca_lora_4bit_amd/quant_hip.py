@@ -653,10 +653,13 @@ def mlp_decode_gave_up():
     return bool(_host is not None and _host.mlp_decode_gave_up())
 
 
+MAX_SILU_MUL = 2 ** 35 - 2048                          # elements one grid covers (q4_silu_mul_f16)
+
+
 def silu_mul_takes(gate, up):
     """Whether `silu_mul` takes these tensors (plain contiguous float16 CUDA tensors of one shape)."""
     return (_host is not None and type(gate) is torch.Tensor and type(up) is torch.Tensor and gate.is_cuda and gate.device == up.device
-            and gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape and gate.numel() > 0
+            and gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape and 0 < gate.numel() < MAX_SILU_MUL
             and gate.is_contiguous() and up.is_contiguous() and (gate.data_ptr() | up.data_ptr()) % 16 == 0)
 
 

@@ -164,8 +164,8 @@ Q4_API int q4_mlp_gate_up_f16(const void *x, const q4_layer_t *gate, const q4_la
                               int M, int H, int I, void *stream);
 
 /* out fp16 [n] = silu(gate) * up, and its backward dgate = dout * up * silu'(gate), dup = dout * silu(gate), element by element
- * with the fp16 roundings of the separate operations (model_attn_mlp_patch.py:224-228 above the decode sizes).  All pointers
- * 16-byte aligned; the outputs overlap no input. */
+ * with the bits of the separate operations (model_attn_mlp_patch.py:224-228 above the decode sizes).  1 <= n < 2^35 - 2048, what
+ * one grid covers; all pointers 16-byte aligned; the outputs overlap no input. */
 Q4_API int q4_silu_mul_f16(const void *gate, const void *up, void *out, long long n, void *stream);
 Q4_API int q4_silu_mul_bwd_f16(const void *dout, const void *gate, const void *up, void *dgate, void *dup, long long n, void *stream);
 

@@ -408,3 +408,16 @@ def test_bench_refuses_more_than_one_gpu():
     import sys
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0 and "--gpus must be 1" in r.stderr
+
+
+def test_silu_mul_refuses_what_one_grid_does_not_cover():
+    """From the size on that quant_hip leaves to torch's own operations; a grid has less than 2^32 threads of 8 elements, 256 to a
+    workgroup and the last of these for what is left over."""
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    L = _lib.lib()
+    fake = ctypes.c_void_p(0x1000)           # never dereferenced: refused by the size
+    most = quant_hip.MAX_SILU_MUL - 1
+    assert (most // 8 + 256) // 256 * 256 < 2 ** 32 <= ((most + 1) // 8 + 256) // 256 * 256
+    for n in (0, -1, most + 1, 2 ** 35, 2 ** 38 - 1, 2 ** 38):
+        assert L.q4_silu_mul_f16(fake, fake, fake, n, None) == -2
+        assert L.q4_silu_mul_bwd_f16(fake, fake, fake, fake, fake, n, None) == -2
