@@ -56,6 +56,8 @@ class _FusedGroup:
         self.clear()
 
     def run(self, x):
+        if x.is_inference():
+            return self.layer(x)                             # no version counter to hold a result by
         key = (x._version, torch.is_grad_enabled())
         if self._x is not x or self._key != key:
             self._y = self.layer(x)
@@ -141,6 +143,8 @@ class _MemberGroup:
         return self._layer_cache
 
     def run(self, member, x):
+        if x.is_inference():
+            return None                                      # writes to x cannot be told from its version: nothing is held for it
         i = self.index[id(member)]
         if not self._held(i, x) or self._adapted[i] is not None:
             layers = self._layers()
@@ -175,7 +179,7 @@ class _MemberGroup:
         the adapters of all members in the next, each member picks its finished output up.  None when the group does not take
         this call.  An output that was finished with another adapter than the member now asks for is not handed out: other matrices,
         other storage, a write that the version counters show or that quant_hip.invalidate was told of."""
-        adapter = self._adapter(member, name, x)
+        adapter = None if x.is_inference() else self._adapter(member, name, x)
         if adapter is None:
             return None
         i = self.index[id(member)]
@@ -230,6 +234,8 @@ class _MemberGroup:
         """Above the decode sizes: ONE grouped GEMM launch for all members (under autograd one node, whose backward is
         one grouped grad-input launch).  Returns the member's output, bias and fused adapter included, or None when
         the group does not take this call (the member then runs by itself)."""
+        if x.is_inference():
+            return None
         i = self.index[id(member)]
         key = (x._version, torch.is_grad_enabled())
         if self._gx is x and self._gkey == key and self._gouts[i] is not None and _same_layer(member, self._keys[i]):

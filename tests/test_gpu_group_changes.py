@@ -126,3 +126,29 @@ def test_adapter_changed_between_two_members(oracle, matrix, how):
                 w.data.mul_(-3.0)
                 quant_hip.invalidate(b.v_proj)
         _close(grouped.v_proj(x), plain.v_proj(x))
+
+
+@pytest.mark.parametrize("rows,N", [(1, 512), (3, 512), (200, 4096)])
+def test_grouped_blocks_under_inference_mode(oracle, rows, N):
+    """Inference tensors have no version counter: members run by themselves, and a write to the input between them is followed."""
+    import torch
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_fused_mlp, make_quant_attn
+    from test_gpu_gemm_grouped import _Block
+    grouped, plain = (_Block(oracle, 1024, N, 128, 0.0, 90).eval() for _ in range(2))
+    mlp = _mlp(oracle, 256, 384, 128)
+    fused = copy.deepcopy(mlp)
+    assert make_quant_attn(grouped) == 1 and make_fused_mlp(fused) == 1
+    wide = copy.deepcopy(mlp)
+    assert make_fused_mlp(wide, concatenate=True) == 1
+    with torch.inference_mode():
+        x = torch.from_numpy(oracle.make_activations(rows, 1024, seed=rows)).cuda()
+        assert x.is_inference()
+        for a, b in zip(grouped(x), plain(x)):
+            _close(a, b)
+        _close(grouped.q_proj(x), plain.q_proj(x))
+        x.mul_(-2.0)
+        _close(grouped.v_proj(x), plain.v_proj(x))
+        _close(grouped.k_proj(x), plain.k_proj(x))
+        y = x[:, :256].contiguous()
+        _close(fused(y), mlp(y))
+        _close(wide(y), mlp(y))
