@@ -49,9 +49,9 @@
 
 namespace q4 {
 
-template <int NSTEP, int GSTEPS, bool V1 = false>
+template <int NSTEP, int GSTEPS, bool V1 = false, bool TURNS = false>
 __global__ __launch_bounds__(1024) void gemv_seq_kernel(GemvArgs a) {
-    gemv_seq_body<NSTEP, GSTEPS, V1>(a, blockIdx.x * kColsPerWave, blockIdx.y, gridDim.y);
+    gemv_seq_body<NSTEP, GSTEPS, V1, TURNS>(a, blockIdx.x * kColsPerWave, blockIdx.y, gridDim.y);
 }
 
 // Up to kMaxGroup layers with the same K, group size and row count M in ONE grid (q|k|v or gate|up of a decoder
@@ -185,12 +185,12 @@ __global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_
     gemv_stream_body<NG, ONE, EB>(g.layer[li], sa.split, (bx - (li == 0 ? 0 : g.strip_end[li - 1])) * kColsPerWave);
 }
 
-template <int NSTEP, int GSTEPS>
+template <int NSTEP, int GSTEPS, bool TURNS = false>
 __global__ __launch_bounds__(1024) void gemv_seq_group_kernel(GemvGroupArgs g) {
     const int bx = blockIdx.x;
     const int li = (bx >= g.strip_end[0]) + (bx >= g.strip_end[1]) + (bx >= g.strip_end[2]);      // uniform
     const int first = li == 0 ? 0 : g.strip_end[li - 1];
-    gemv_seq_body<NSTEP, GSTEPS, false>(g.layer[li], (bx - first) * kColsPerWave, blockIdx.y, gridDim.y);
+    gemv_seq_body<NSTEP, GSTEPS, false, TURNS>(g.layer[li], (bx - first) * kColsPerWave, blockIdx.y, gridDim.y);
 }
 
 // The same for an act-order layer whose packed rows were sorted by group (q4_permute_rows): row p of the
@@ -1052,20 +1052,20 @@ void stream_dx_kernel(SkinnyDxArgs a) {
 }
 
 // ------------------------------------------------------------------ act-order (per-row groups)
-template <int NSTEP>
+template <int NSTEP, bool TURNS>
 __global__ __launch_bounds__(512) void gemv_gidx_kernel(GemvArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
     const int kk = lane >> 4, c = lane & 15;
     const int n0 = blockIdx.x * kColsPerWave;
-    const int k0 = (blockIdx.y * nwaves + wave) * (32 * NSTEP);
 
     float4_t yacc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) yacc[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    if (k0 < a.K) {
+    int k0 = (blockIdx.y * nwaves + wave) * (32 * NSTEP);
+    auto chunk = [&] {
         const int ncol8 = a.N >> 3;
         const int col = n0 + 4 * c;
         const int zshift = (c & 1) * 16;
@@ -1115,7 +1115,13 @@ __global__ __launch_bounds__(512) void gemv_gidx_kernel(GemvArgs a) {
                 yacc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, make_half8(b[0], b[1], b[2], b[3]), yacc[j], 0, 0, 0);
             }
         }
+    };
+    if constexpr (TURNS) {
+        for (; k0 < a.K; k0 += gridDim.y * nwaves * (32 * NSTEP)) chunk();
+    } else {
+        if (k0 < a.K) chunk();
     }
+
     gemv_finish(a, yacc, n0, wave, nwaves, kk, c, gridDim.y);
 }
 
@@ -1130,11 +1136,31 @@ extern "C" size_t q4_gemv_workspace_bytes(int M, int K, int N) {
 template <int NSTEP>
 static void launch_seq(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvArgs& a) {
     using namespace q4;
+    if constexpr (NSTEP <= 2) {                              // chunks of four steps in such numbers: the stream
+        if (p.turns) {
+            if (p.gsteps == 0) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0, false, true>), grid, block, lds, stream, a);
+            else if constexpr (NSTEP == 2) hipLaunchKernelGGL((gemv_seq_kernel<2, 1, false, true>), grid, block, lds, stream, a);
+            return;
+        }
+    }
     switch (p.gsteps) {
         case 0: hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0>), grid, block, lds, stream, a); break;
         case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 1>), grid, block, lds, stream, a); break;
         case 2: if constexpr (NSTEP > 2) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 2>), grid, block, lds, stream, a); break;
     }
+}
+
+template <int NSTEP>
+static void launch_v1(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvArgs& a) {
+    using namespace q4;
+    if (p.turns) hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0, true, true>), grid, block, lds, stream, a);
+    else hipLaunchKernelGGL((gemv_seq_kernel<NSTEP, 0, true>), grid, block, lds, stream, a);
+}
+template <int NSTEP>
+static void launch_gidx(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvArgs& a) {
+    using namespace q4;
+    if (p.turns) hipLaunchKernelGGL((gemv_gidx_kernel<NSTEP, true>), grid, block, lds, stream, a);
+    else hipLaunchKernelGGL((gemv_gidx_kernel<NSTEP, false>), grid, block, lds, stream, a);
 }
 
 static bool whole_chunks(int K, int groupsize) {
@@ -1157,6 +1183,13 @@ static void launch_stream_one(const q4::GemvGroupArgs& g, int n, const q4::Strea
 template <int NSTEP>
 static void launch_seq_group(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvGroupArgs& g) {
     using namespace q4;
+    if constexpr (NSTEP <= 2) {
+        if (p.turns) {
+            if (p.gsteps == 0) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 0, true>), grid, block, lds, stream, g);
+            else if constexpr (NSTEP == 2) hipLaunchKernelGGL((gemv_seq_group_kernel<2, 1, true>), grid, block, lds, stream, g);
+            return;
+        }
+    }
     switch (p.gsteps) {
         case 0: hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 0>), grid, block, lds, stream, g); break;
         case 1: if constexpr (NSTEP > 1) hipLaunchKernelGGL((gemv_seq_group_kernel<NSTEP, 1>), grid, block, lds, stream, g); break;
@@ -1172,7 +1205,7 @@ static int launch_chunks(const q4::GemvGroupArgs& g, int n, int strips, hipStrea
     sp.group_inv = stream_group_inv(a.groupsize);
     sp.blocks = (a.K + 1023) / 1024;
     if (!plan_stream_takes(a.M, sp.blocks, strips, a.groupsize)) {
-        const GemvPlan p{4, a.groupsize % 128 == 0 ? 0 : a.groupsize / 32, 8, sp.blocks};
+        const GemvPlan p{4, a.groupsize % 128 == 0 ? 0 : a.groupsize / 32, 8, sp.blocks, false};
         const dim3 grid(strips, p.splits), block(64 * p.waves);
         const size_t lds = (size_t)p.waves * a.M * 64 * sizeof(float);
         if (n == 1) launch_seq<4>(p, grid, block, lds, stream, a);
@@ -1258,9 +1291,9 @@ extern "C" int q4_launch_gemv(const void* x, const int32_t* qweight, const int32
         }
     } else {
         switch (p.nstep) {
-            case 4: hipLaunchKernelGGL(gemv_gidx_kernel<4>, grid, block, lds, stream, a); break;
-            case 2: hipLaunchKernelGGL(gemv_gidx_kernel<2>, grid, block, lds, stream, a); break;
-            default: hipLaunchKernelGGL(gemv_gidx_kernel<1>, grid, block, lds, stream, a); break;
+            case 4: launch_gidx<4>(p, grid, block, lds, stream, a); break;
+            case 2: launch_gidx<2>(p, grid, block, lds, stream, a); break;
+            default: launch_gidx<1>(p, grid, block, lds, stream, a); break;
         }
     }
     return hipGetLastError() == hipSuccess ? 0 : -4;
@@ -1332,9 +1365,9 @@ extern "C" int q4_launch_gemv_v1(const void* x, const int32_t* qweight, const vo
     const dim3 grid(N / kColsPerWave, p.splits), block(64 * p.waves);
     const size_t lds = (size_t)p.waves * M * 64 * sizeof(float);
     switch (p.nstep) {                                       // one group: gsteps is always 0
-        case 4: hipLaunchKernelGGL((gemv_seq_kernel<4, 0, true>), grid, block, lds, stream, a); break;
-        case 2: hipLaunchKernelGGL((gemv_seq_kernel<2, 0, true>), grid, block, lds, stream, a); break;
-        default: hipLaunchKernelGGL((gemv_seq_kernel<1, 0, true>), grid, block, lds, stream, a); break;
+        case 4: launch_v1<4>(p, grid, block, lds, stream, a); break;
+        case 2: launch_v1<2>(p, grid, block, lds, stream, a); break;
+        default: launch_v1<1>(p, grid, block, lds, stream, a); break;
     }
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }

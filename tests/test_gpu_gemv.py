@@ -325,3 +325,39 @@ def test_gemv_shares_beyond_the_exchange_saturate(sign):
     y = quant_hip.gemv(x, qw, qz, torch.full((K // 128, N), 2.0, dtype=torch.float16, device="cuda"), None, 128)
     assert torch.equal(y, torch.full_like(y, sign * float("inf")))
     assert quant_hip.workspaces_are_zero()
+
+
+@pytest.mark.parametrize("route,K,gs", [("burst", 131104, 32), ("burst", 131136, 96), ("grouped", 262208, 64), ("gidx", 65312, 32), ("gidx", 524352, 64),
+                                        ("v1", 131104, 131104), ("v1", 524416, 524416)])
+@pytest.mark.parametrize("M", [1, 6])
+def test_long_reductions_of_odd_chunks(oracle, route, K, gs, M):
+    """Reductions of more chunks than 255 workgroups of one chunk per wavefront hold, by every kernel that takes such sizes."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    N = 64
+    layer = oracle.make_layer(K, N, gs, act_order=route == "gidx", seed=M)
+    t = to_cuda_layer(layer)
+    x = oracle.make_activations(M, K, seed=M)
+    xt = torch.from_numpy(x).cuda()
+    if route == "grouped":
+        y = quant_hip.gemv_grouped(xt, [(t["qweight"], t["qzeros"], t["scales"])] * 2, gs)[1]
+    elif route == "v1":
+        zeros = torch.from_numpy(layer["scales"] * (layer["zcodes"] + 1).astype("float16")).cuda()      # scale * (q - z - 1)
+        y = torch.empty((M, N), dtype=torch.float16, device="cuda")
+        ws = torch.zeros(M * N * 8 + 256, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        _lib.check(_lib.lib().q4_gemv_v1_f16(xt.data_ptr(), t["qweight"].data_ptr(), t["scales"].data_ptr(), zeros.data_ptr(), y.data_ptr(), 0,
+                                             M, K, N, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "q4_gemv_v1_f16")
+        assert not bool(ws.any())
+        weights = layer["codes"].astype("float64") * layer["scales"].astype("float64") - zeros.cpu().numpy().astype("float64")
+        assert rel_err(y.cpu().numpy(), x.astype("float64") @ weights) <= 2e-3
+        return
+    else:
+        try:
+            quant_hip.actorder_repack = False
+            y = quant_hip.gemv(xt, t["qweight"], t["qzeros"], t["scales"], t["g_idx"] if route == "gidx" else None, gs)
+        finally:
+            quant_hip.actorder_repack = True
+    ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
+    assert rel_err(y.cpu().numpy(), ref) <= 3e-3             # the gathering kernel multiplies fp16 weights
+    assert quant_hip.workspaces_are_zero()
