@@ -82,20 +82,19 @@ def _same_adapter(p, q):
 
 
 def _layer_key(m):
-    """What is kept about layer `m` rests on: its buffers, their contents as the version counters show them, and the count of
-    quant_hip.invalidate calls, which stand for writes that the counters do not show."""
+    """What is kept about layer `m` rests on: its buffers and their contents as the version counters show them.  Writes that these
+    do not show are what quant_hip.invalidate is for; its count is compared beside this."""
     b = m._buffers
     q, z, s, g = b.get('qweight'), b.get('qzeros'), b.get('scales'), b.get('g_idx')
-    return (q, z, s, g, q._version, z._version, s._version, -1 if g is None else g._version, matmul_utils_4bit.quant_hip.invalidations)
+    return q, z, s, g, q._version, z._version, s._version, -1 if g is None else g._version
 
 
 def _same_layer(m, k):
     """_layer_key(m) is `k`, without building it."""
     b = m._buffers
-    g = b.get('g_idx')
-    return (b.get('qweight') is k[0] and b.get('qzeros') is k[1] and b.get('scales') is k[2] and g is k[3] and k[0]._version == k[4]
-            and k[1]._version == k[5] and k[2]._version == k[6] and (g is None or g._version == k[7])
-            and matmul_utils_4bit.quant_hip.invalidations == k[8])
+    q, z, s, g, vq, vz, vs, vg = k
+    return (b.get('qweight') is q and b.get('qzeros') is z and b.get('scales') is s and b.get('g_idx') is g and s._version == vs
+            and q._version == vq and z._version == vz and (g is None or g._version == vg))
 
 
 class _MemberGroup:
@@ -110,6 +109,7 @@ class _MemberGroup:
         self.groupsize = self.members[0].groupsize
         self.usable = None                                   # decided at the first call (needs the tensors on the GPU)
         self._layer_cache = self._keys = None
+        self._invalidations = -1
         self._gemm_ok = None                                 # sequential groups AND scales below 64 (the tiled kernels' fused form)
         self.hook = None
         self.clear()
@@ -129,9 +129,11 @@ class _MemberGroup:
     def _layers(self):
         """(qweight, qzeros, scales) of every member, rebuilt when a member's buffers were replaced (a cast, a reload) or written in
         place, or `quant_hip.invalidate` was called."""
-        if self._layer_cache is not None:
-            for m, k in zip(self.members, self._keys):
-                if not _same_layer(m, k):
+        if self._layer_cache is not None and self._invalidations == matmul_utils_4bit.quant_hip.invalidations:
+            for m, (q, z, s, g, vq, vz, vs, vg) in zip(self.members, self._keys):
+                b = m._buffers                               # _same_layer, without a call per member
+                if (b.get('qweight') is not q or b.get('qzeros') is not z or b.get('scales') is not s or b.get('g_idx') is not g
+                        or s._version != vs or q._version != vq or z._version != vz or (g is not None and g._version != vg)):
                     break
             else:
                 return self._layer_cache
@@ -140,6 +142,7 @@ class _MemberGroup:
         self._gemm_ok = None
         self._layer_cache = [(m.qweight, m.qzeros, m.scales) for m in self.members] if self.usable else None
         self._keys = [_layer_key(m) for m in self.members] if self.usable else None
+        self._invalidations = matmul_utils_4bit.quant_hip.invalidations
         return self._layer_cache
 
     def run(self, member, x):
@@ -155,8 +158,10 @@ class _MemberGroup:
 
     def _held(self, i, x):
         """Member i's output for x is there, of the tensors that the member has now."""
-        return (self._x is x and self._version == x._version and self._outs[i] is not None
-                and _same_layer(self.members[i], self._keys[i]))
+        return self._x is x and self._version == x._version and self._outs[i] is not None and self._same(i)
+
+    def _same(self, i):
+        return self._invalidations == matmul_utils_4bit.quant_hip.invalidations and _same_layer(self.members[i], self._keys[i])
 
     def _launch(self, x, layers):
         # the compiled binding checks shapes, dtypes and devices; sequential groups were established by _check()
@@ -165,12 +170,14 @@ class _MemberGroup:
             lead = tuple(x.shape[:-1])
             outs = [o.view(lead + (o.shape[-1],)) for o in outs]
         self._outs = outs
-        self._adapted = [None] * len(self.members)
+        self._adapted = [None] * len(outs)
+        self._left = len(outs)
         self._x, self._version = x, x._version
 
     def _take(self, i):
         y, self._outs[i], self._adapted[i] = self._outs[i], None, None
-        if all(o is None for o in self._outs):
+        self._left -= 1
+        if not self._left:
             self._x = None
         return y
 
@@ -238,7 +245,7 @@ class _MemberGroup:
             return None
         i = self.index[id(member)]
         key = (x._version, torch.is_grad_enabled())
-        if self._gx is x and self._gkey == key and self._gouts[i] is not None and _same_layer(member, self._keys[i]):
+        if self._gx is x and self._gkey == key and self._gouts[i] is not None and self._same(i):
             y, self._gouts[i] = self._gouts[i], None
             if all(o is None for o in self._gouts):
                 self._gx = None
@@ -434,6 +441,7 @@ class _SiluForward:
 
 
 _SILU, _SILU_MODULE = F.silu, nn.SiLU.forward
+_SILU_FUNCTIONAL, _SILU_SHORT = _code_key(_SiluForward.functional.__code__), _code_key(_SiluForward.short.__code__)
 
 
 def _is_silu(act):
@@ -451,11 +459,8 @@ def _is_silu(act):
     code = getattr(forward, '__code__', None)
     if code is None:
         return False
-    names = forward.__globals__
-    return (code.co_code == _SiluForward.functional.__code__.co_code and _code_key(code) == _code_key(_SiluForward.functional.__code__)
-            and names.get('nn') is nn
-            or code.co_code == _SiluForward.short.__code__.co_code and _code_key(code) == _code_key(_SiluForward.short.__code__)
-            and names.get('F') is F)
+    key = _code_key(code)
+    return (key == _SILU_FUNCTIONAL and forward.__globals__.get('nn') is nn) or (key == _SILU_SHORT and forward.__globals__.get('F') is F)
 
 
 def _plain_no_bias(layer):
@@ -543,15 +548,14 @@ def _mlp_decode_forward(mlp, x):
         gate, up, down = mods['gate_proj'], mods['up_proj'], mods['down_proj']
         group = gate.__dict__.get('_q4_group')
         layers = None if group is None else group._layers()  # the same list as long as nothing about gate and up changed
-        bias = [l._buffers.get('bias') for l in (gate, up, down)]
-        key = (layers, bias[0], bias[1], bias[2], down._buffers.get('qweight'),
-               tuple(-1 if b is None else b._version for b in bias), gate.disable_bias, up.disable_bias, down.disable_bias,
-               _adapters_off(gate), _adapters_off(up), _adapters_off(down))
-        if (cached is None or not (all(a is b for a, b in zip(cached[0][:5], key[:5])) and cached[0][5:] == key[5:])
-                or (cached[1] is not None and not _same_layer(down, cached[2]))):
+        b0, b1, b2 = gate._buffers.get('bias'), up._buffers.get('bias'), down._buffers.get('bias')
+        flags = (-1 if b0 is None else b0._version, -1 if b1 is None else b1._version, -1 if b2 is None else b2._version,
+                 gate.disable_bias, up.disable_bias, down.disable_bias, _adapters_off(gate), _adapters_off(up), _adapters_off(down))
+        if (cached is None or cached[0] is not layers or cached[1] is not b0 or cached[2] is not b1 or cached[3] is not b2
+                or cached[4] != flags or (cached[5] is not None and not _same_layer(down, cached[6]))):
             args = _mlp_decode_args(mlp)
-            cached = d['_q4_mlp_args'] = (key, args, None if args is None else _layer_key(down))
-        args = cached[1]
+            cached = d['_q4_mlp_args'] = (layers, b0, b1, b2, flags, args, None if args is None else _layer_key(down))
+        args = cached[5]
         if args is not None and x.shape[-1] == args[4]:
             rows = x.numel() // args[4]
             if (1 <= rows <= min(int(matmul_utils_4bit.auto_switch_thd), quant_hip.MAX_GEMV_ROWS)
