@@ -297,17 +297,21 @@ def test_one_and_two_rows_have_the_bits_of_the_first_of_three(K, Ns, gs):
     assert quant_hip.workspaces_are_zero()
 
 
-@pytest.mark.parametrize("blocks,gs,M", [(257, 64, 2), (300, 32, 5), (600, 128, 1), (600, 1024, 16), (1020, 128, 3), (1020, 32, 9)])
+@pytest.mark.parametrize("blocks,gs,M", [(257, 64, 2), (257, 64, 7), (258, 64, 16), (300, 32, 3), (300, 32, 5), (600, 128, 1), (600, 1024, 16), (1020, 128, 3),
+                                         (1020, 32, 9)])
 def test_gemv_of_more_blocks_than_arrivals(oracle, blocks, gs, M):
     """Shares of several blocks, up to the longest reduction that is taken, for every number of groups per chunk and of outputs per
-    thread: the exchange holds them, the result is the sum and the accumulators are left zero.  The last block has one chunk."""
+    thread, alone and in a group: the exchange holds them, the result is the sum and the accumulators are left zero.  The last
+    block has one chunk."""
     import torch
     from alpaca_lora_4bit_amd import quant_hip
     K, N = blocks * 1024 - 896, 64
     layer = oracle.make_layer(K, N, gs, seed=blocks)
     t = to_cuda_layer(layer)
     x = oracle.make_activations(M, K, seed=M)
-    y = quant_hip.gemv(torch.from_numpy(x).cuda(), t["qweight"], t["qzeros"], t["scales"], None, gs)
+    xt, packed = torch.from_numpy(x).cuda(), (t["qweight"], t["qzeros"], t["scales"])
+    y = quant_hip.gemv(xt, *packed, None, gs)
+    assert all(torch.equal(y, other) for other in quant_hip.gemv_grouped(xt, [packed] * 2, gs))
     ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
     assert rel_err(y.cpu().numpy(), ref) <= 2e-3
     assert quant_hip.workspaces_are_zero()
