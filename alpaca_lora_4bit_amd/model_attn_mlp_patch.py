@@ -573,7 +573,7 @@ def make_fused_mlp(model, is_v1_model=False, concatenate=False, fuse_decode_step
     """One launch for gate_proj / up_proj of every MLP block (model_attn_mlp_patch.py:163-247; the reference's Triton
     fused-MLP kernel is replaced by one launch over both projections followed by the block's own activation).  In place
     by default; then, with `fuse_decode_step` and a SiLU block of three 4-bit layers of the same group size, the block's
-    forward runs the whole decode step (gate, up, silu(gate) * up, down) as one launch."""
+    forward runs the whole decode step (gate, up, silu(gate) * up, down) as one launch or two."""
     if is_v1_model:
         raise NotImplementedError("v1 (fp zeros) layers are not fused")
     names = ("gate_proj", "up_proj")

@@ -260,8 +260,9 @@ invalidations = 0                                       # calls of `invalidate` 
 
 def invalidate(*tensors_or_modules):
     """Forget what was cached about these tensors (or about every tensor of these modules): the layer verdicts,
-    the g_idx classification, the scale-range check and the sorted copy of an act-order layer.  Needed only after
-    writing packed tensors through `.data` (which does not bump the version counter the caches are keyed on)."""
+    the g_idx classification, the scale-range check, the sorted copy of an act-order layer, and what grouped projections and fused
+    blocks hold.  Needed only after writing packed tensors or the adapters of grouped layers through `.data` (which does not
+    bump the version counter the caches are keyed on)."""
     global invalidations
     invalidations += 1
     for obj in tensors_or_modules:

@@ -27,7 +27,7 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, GB/s
 MFMA_FP16_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 MFMA
 # HBM bytes per launch of the headline kernel (the grouped gate|up GEMV), measured in two rocprofv3 --pmc runs
 # (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for a 256 MiB copy (--calibrate-copy):
-# 2 x 23 472.5 KiB read + 903.0 KiB written.  Not re-measured by a bench run: the file named below holds the commands.
+# 2 x 23 472.3 KiB read + 903.0 KiB written.  Not re-measured by a bench run: the file named below holds the commands.
 GEMV_TRAFFIC_BYTES = 48996000
 GEMV_TRAFFIC_SOURCE = "profiles/gemv_mlp_decode_M1_gate_up_grouped_and_down.md"
 
@@ -666,9 +666,9 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(head["gate_up"]["gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(head["gate_up"]["gbs"] / HBM_PEAK_GBS, 4), "traffic": GEMV_TRAFFIC_BYTES,
                      "traffic_source": GEMV_TRAFFIC_SOURCE,
-                     "kernel": "q4::gemv_stream_group_kernel<1, true, 1> (gate|up, N = 2 x 11008)",
+                     "kernel": "q4::gemv_seq_group_kernel<4, 0> (gate|up, N = 2 x 11008)",
                      "bytes_per_launch": head["gate_up"]["bytes"], "avg_launch_us": round(head["gate_up"]["us"], 3),
-                     "other_kernel": {"kernel": "q4::gemv_stream_kernel<1, true, 1> (down, 11008 -> 4096)",
+                     "other_kernel": {"kernel": "q4::gemv_seq_kernel<4, 0> (down, 11008 -> 4096)",
                                       "bytes_per_launch": head["down"]["bytes"],
                                       "avg_launch_us": round(head["down"]["us"], 3),
                                       "frac": round(head["down"]["gbs"] / HBM_PEAK_GBS, 4)},
