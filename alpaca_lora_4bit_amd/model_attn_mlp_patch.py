@@ -18,6 +18,7 @@ classes.  Two ways here, both leaving the host model's own attention / MLP code 
 import json
 import os
 import re
+import threading
 
 import torch
 import torch.nn as nn
@@ -25,6 +26,23 @@ import torch.nn.functional as F
 
 from . import autograd_4bit, matmul_utils_4bit
 from .autograd_4bit import Autograd4bitQuantLinear, _buffer, _has_bias, _weight, fuse_quant_linears
+
+
+def _where(x):
+    """The thread, the stream and whether it is being captured: what is queued here is there for callers of the same only."""
+    if not x.is_cuda:
+        return threading.get_ident(), 0, False
+    return threading.get_ident(), torch._C._cuda_getCurrentRawStream(x.get_device()), torch.cuda.is_current_stream_capturing()
+
+
+class _Held:
+    """Outputs for one input that members of a group have not called for yet, put in place by one assignment."""
+    __slots__ = ('x', 'key', 'where', 'outs', 'adapted', 'left', 'layers', 'invalidations')
+
+    def __init__(self, x, key, outs, left, layers=None):
+        self.x, self.key, self.where = x, key, _where(x)
+        self.outs, self.adapted, self.left = outs, [None] * len(outs), left
+        self.layers, self.invalidations = layers, matmul_utils_4bit.quant_hip.invalidations
 
 
 class FusedProjectionSlice(nn.Module):
@@ -47,7 +65,8 @@ class _FusedGroup:
     """Runs the fused layer once per input tensor and hands the result to every slice.  The result is kept for as
     long as the same tensor object comes back unmodified in the same grad mode (identity, in-place version counter),
     whatever the order in which the host block calls its projections, and dropped as soon as every slice has been
-    served or the block returns (forward hook installed by _fuse_children), so nothing stays pinned between forwards."""
+    served or the block returns (forward hook installed by _fuse_children), so nothing stays pinned between forwards.
+    Another thread, stream or capture than the one that ran the layer runs it again."""
 
     def __init__(self, layer, n_slices):
         self.layer = layer
@@ -58,20 +77,20 @@ class _FusedGroup:
     def run(self, x):
         if x.is_inference():
             return self.layer(x)                             # no version counter to hold a result by
-        key = (x._version, torch.is_grad_enabled())
-        if self._x is not x or self._key != key:
-            self._y = self.layer(x)
-            self._x, self._key, self._served = x, key, 0
-        y = self._y
-        self._served += 1
-        if self._served >= self.n_slices:
-            self.clear()
+        h = self._now
+        if h is None or h.x is not x or h.key != (x._version, torch.is_grad_enabled()) or h.where != _where(x):
+            h = self._now = _Held(x, (x._version, torch.is_grad_enabled()), [self.layer(x)], self.n_slices)
+        y = h.outs[0]
+        h.left -= 1
+        if not h.left and self._now is h:
+            self._now = None
         return y
 
+    _x = property(lambda self: None if self._now is None else self._now.x)
+    _y = property(lambda self: None if self._now is None else self._now.outs[0])
+
     def clear(self, *unused):
-        self._x = self._y = None
-        self._key = None
-        self._served = 0
+        self._now = None
 
 
 _ADAPTER_TYPES = (torch.float16, torch.float32)
@@ -140,28 +159,32 @@ class _MemberGroup:
         self.clear()                                         # outputs of the tensors as they were
         self.usable = self._check()
         self._gemm_ok = None
-        self._layer_cache = [(m.qweight, m.qzeros, m.scales) for m in self.members] if self.usable else None
         self._keys = [_layer_key(m) for m in self.members] if self.usable else None
         self._invalidations = matmul_utils_4bit.quant_hip.invalidations
-        return self._layer_cache
+        layers = self._layer_cache = [(m.qweight, m.qzeros, m.scales) for m in self.members] if self.usable else None
+        return layers                                        # last, so that another thread finds the keys of what it finds
 
     def run(self, member, x):
         if x.is_inference():
             return None                                      # writes to x cannot be told from its version: nothing is held for it
         i = self.index[id(member)]
-        if not self._held(i, x) or self._adapted[i] is not None:
+        h = self._held(i, x)
+        if h is None or h.adapted[i] is not None:
             layers = self._layers()
             if layers is None:
                 return None
-            self._launch(x, layers)
-        return self._take(i)
+            h = self._launch(x, layers)
+        return self._take(h, i)
 
     def _held(self, i, x):
-        """Member i's output for x is there, of the tensors that the member has now."""
-        return self._x is x and self._version == x._version and self._outs[i] is not None and self._same(i)
+        """Member i's output for x is there, of the tensors that the member has now and for this thread, stream and capture."""
+        h = self._now
+        if h is not None and h.x is x and h.key == x._version and h.outs[i] is not None and self._same(h, i) and h.where == _where(x):
+            return h
+        return None
 
-    def _same(self, i):
-        return self._invalidations == matmul_utils_4bit.quant_hip.invalidations and _same_layer(self.members[i], self._keys[i])
+    def _same(self, h, i):
+        return h.invalidations == matmul_utils_4bit.quant_hip.invalidations and _same_layer(self.members[i], h.layers[i])
 
     def _launch(self, x, layers):
         # the compiled binding checks shapes, dtypes and devices; sequential groups were established by _check()
@@ -169,16 +192,14 @@ class _MemberGroup:
         if x.dim() != 2:
             lead = tuple(x.shape[:-1])
             outs = [o.view(lead + (o.shape[-1],)) for o in outs]
-        self._outs = outs
-        self._adapted = [None] * len(outs)
-        self._left = len(outs)
-        self._x, self._version = x, x._version
+        h = self._now = _Held(x, x._version, outs, len(outs), self._keys)
+        return h
 
-    def _take(self, i):
-        y, self._outs[i], self._adapted[i] = self._outs[i], None, None
-        self._left -= 1
-        if not self._left:
-            self._x = None
+    def _take(self, h, i):
+        y, h.outs[i], h.adapted[i] = h.outs[i], None, None
+        h.left -= 1
+        if not h.left and self._now is h:
+            self._now = None
         return y
 
     def run_adapted(self, member, x, name):
@@ -190,15 +211,16 @@ class _MemberGroup:
         if adapter is None:
             return None
         i = self.index[id(member)]
-        if not self._held(i, x) or (self._adapted[i] is not None and not _same_adapter(self._adapted[i], adapter)):
+        h = self._held(i, x)
+        if h is None or (h.adapted[i] is not None and not _same_adapter(h.adapted[i], adapter)):
             layers = self._layers()
             if layers is None:
                 return None
-            self._launch(x, layers)
-        if self._adapted[i] is None:
+            h = self._launch(x, layers)
+        if h.adapted[i] is None:
             todo = {i: adapter}
             for j, m in enumerate(self.members):
-                if j != i and self._outs[j] is not None and self._adapted[j] is None and type(m) is type(member) and not m.disable_adapters:
+                if j != i and h.outs[j] is not None and h.adapted[j] is None and type(m) is type(member) and not m.disable_adapters:
                     other = m._decode_adapter(x)
                     ad = None if other is None else self._adapter(m, other, x)
                     if ad is not None:
@@ -207,13 +229,13 @@ class _MemberGroup:
                 flat = x.dim() == 2
                 matmul_utils_4bit.quant_hip.lora_update_grouped(
                     x if flat and x.is_contiguous() else x.reshape(-1, x.shape[-1]).contiguous(),
-                    [(ad[0], ad[1], self._outs[j] if flat else self._outs[j].view(-1, self._outs[j].shape[-1]), ad[2]) for j, ad in todo.items()])
+                    [(ad[0], ad[1], h.outs[j] if flat else h.outs[j].view(-1, h.outs[j].shape[-1]), ad[2]) for j, ad in todo.items()])
             except BaseException:
                 self.clear()                                 # some outputs may have been updated
                 raise
             for j, ad in todo.items():
-                self._adapted[j] = ad
-        return self._take(i)
+                h.adapted[j] = ad
+        return self._take(h, i)
 
     @staticmethod
     def _adapter(m, name, x):
@@ -245,10 +267,12 @@ class _MemberGroup:
             return None
         i = self.index[id(member)]
         key = (x._version, torch.is_grad_enabled())
-        if self._gx is x and self._gkey == key and self._gouts[i] is not None and self._same(i):
-            y, self._gouts[i] = self._gouts[i], None
-            if all(o is None for o in self._gouts):
-                self._gx = None
+        h = self._gemm_now
+        if h is not None and h.x is x and h.key == key and h.outs[i] is not None and self._same(h, i) and h.where == _where(x):
+            y, h.outs[i] = h.outs[i], None
+            h.left -= 1
+            if not h.left and self._gemm_now is h:
+                self._gemm_now = None
             return y
         from . import quant_hip
         layers = self._layers()
@@ -285,19 +309,15 @@ class _MemberGroup:
             specs.append((scaling, drop_p, seed))
             tensors += [qweight, scales, qzeros, bias, la, lb]
         outs = autograd_4bit.AutogradMatmul4bitGroup.apply(x, self.groupsize, tuple(specs), *tensors)
-        self._gouts = list(outs)
-        self._gx, self._gkey = x, key
-        y, self._gouts[i] = self._gouts[i], None
+        h = _Held(x, key, list(outs), len(outs) - 1, self._keys)
+        y, h.outs[i] = h.outs[i], None
+        self._gemm_now = h
         return y
 
+    _x = property(lambda self: None if self._now is None else self._now.x)
+
     def clear(self, *unused):
-        self._x = None
-        self._version = -1
-        self._outs = [None] * len(self.members)
-        self._adapted = [None] * len(self.members)
-        self._gx = None
-        self._gkey = None
-        self._gouts = [None] * len(self.members)
+        self._now = self._gemm_now = None
 
     def replace(self, old, new):
         """`new` (for instance a LoRA layer sharing `old`'s packed tensors) takes `old`'s place in the group."""

@@ -152,3 +152,92 @@ def test_grouped_blocks_under_inference_mode(oracle, rows, N):
         y = x[:, :256].contiguous()
         _close(fused(y), mlp(y))
         _close(wide(y), mlp(y))
+
+
+def _attention(oracle, rows, seed):
+    import torch
+    from alpaca_lora_4bit_amd.model_attn_mlp_patch import make_quant_attn
+    from test_gpu_gemm_grouped import _Block
+    grouped, plain = (_Block(oracle, 1024, 4096 if rows > 16 else 512, 128, 0.0, seed).eval() for _ in range(2))
+    for b in (grouped, plain):
+        b.v_proj.bias.zero_()
+    assert make_quant_attn(grouped) == 1
+    x = torch.from_numpy(oracle.make_activations(rows, 1024, seed=seed)).cuda()
+    with torch.no_grad():
+        want = plain(x)
+        for a, b in zip(grouped(x), want):
+            _close(a, b)
+    torch.cuda.synchronize()
+    return grouped, x, want
+
+
+@pytest.mark.parametrize("rows", [3, 200])
+def test_members_called_on_another_stream(oracle, rows):
+    """q is queued behind other work of one stream; k and v, called on another one meanwhile, do not take what is not there yet."""
+    import torch
+    grouped, x, want = _attention(oracle, rows, 110)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(100_000_000)                   # some tens of milliseconds
+            q = grouped.q_proj(x)
+        with torch.cuda.stream(second):
+            v, k = grouped.v_proj(x).clone(), grouped.k_proj(x).clone()
+            second.synchronize()
+            assert not first.query()
+        first.synchronize()
+        for a, b in zip((q, k, v), want):
+            _close(a, b)
+
+
+@pytest.mark.parametrize("rows", [3, 200])
+def test_members_called_after_a_capture_that_left_them(oracle, rows):
+    """What a capture queued was not computed: an eager call on the same stream and input computes its own."""
+    import torch
+    grouped, x, want = _attention(oracle, rows, 120)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.stream(stream):
+        grouped(x)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            q = grouped.q_proj(x)
+        k = grouped.k_proj(x)
+        stream.synchronize()
+        _close(k, want[1])
+        for _ in range(3):
+            q.fill_(float("nan"))
+            graph.replay()
+            stream.synchronize()
+            _close(q, want[0])
+
+
+@pytest.mark.parametrize("rows", [3, 200])
+def test_members_called_from_two_threads(oracle, rows):
+    """Two threads with inputs of their own, and one input, call the members of one group in turn."""
+    import threading
+    import torch
+    grouped, x, want = _attention(oracle, rows, 130)
+    other = torch.from_numpy(oracle.make_activations(rows, 1024, seed=131)).cuda()
+    with torch.no_grad():
+        want_other = grouped(other)
+    torch.cuda.synchronize()
+    failed, barrier = [], threading.Barrier(2, timeout=60)
+
+    def work(t, results):
+        try:
+            with torch.no_grad():
+                for rep in range(40):
+                    inp, ref = results[rep % len(results)]
+                    for name, r in zip(("q_proj", "k_proj", "v_proj"), ref):
+                        if rep % 2:
+                            barrier.wait()
+                        _close(getattr(grouped, name)(inp), r)
+        except BaseException as e:                           # noqa: B902
+            failed.append(e)
+            barrier.abort()
+    threads = [threading.Thread(target=work, args=(t, ((x, want), (other, want_other))[::1 - 2 * t])) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed[0]
