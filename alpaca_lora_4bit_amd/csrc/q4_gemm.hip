@@ -30,95 +30,14 @@
 // The LoRA term is one more reduction step whose A operand is the precomputed [M,R] rank-R
 // activation and whose B operand is the fp16 adapter matrix: no second pass over the output.
 // The epilogue transposes the accumulators through LDS so that y is written in 16-byte pieces.
-#include "q4_common.hpp"
-#include "q4_gemm_plan.hpp"
+#include "q4_gemm_args.hpp"
 #include <initializer_list>
 #include <stdlib.h>
-#include <type_traits>
 
 namespace q4 {
 
 constexpr int LDS_STRIDE = BK + 8;   // halves
 
-struct GemmArgs {
-    const half_t* a;          // fwd: x [M,K]      bwd: dy [M,N]
-    const uint32_t* qweight;  // [K/8, N]
-    const uint32_t* qzeros;   // [G, N/8]
-    const half_t* scales;     // [G, N]
-    const int32_t* g_idx;     // [K] or null
-    int groupsize;
-    uint32_t gs_inv31;        // ceil(2^31 / (groupsize / 64)): reduction offset -> group without a division
-    const half_t* bias;       // fwd only, [N] or null
-    const half_t* la;         // fwd: xa [M,R]     bwd: dyb [M,R]   (or null)
-    const void* lb;           // adapter matrix (fp16 or fp32), element (r, c) at lb[r*lb_sr + c*lb_sc]; fwd: c = n, bwd: c = k
-    int lb_sr, lb_sc, lb_is_f32;
-    float lb_scale;           // multiplied into the adapter matrix when it is staged in LDS
-    int R;
-    half_t* out;              // fwd: y [M,N]      bwd: dx [M,K]
-    int M, K, N, G;
-    int phase_step;           // bits 0-7: rotation of the reduction loop per row tile, in steps of 64; bits 8+: row tiles per group of the tile order
-    float* part;              // split-K: fp32 partial outputs [gridDim.z][M][part_cols] (gridDim.z > 1 only)
-    int col_tile0;            // first column tile of this launch (a launch may cover a range of column tiles)
-    int part_cols;            // columns held by `part`: those of this launch's column tiles
-    DropArgs drop;            // thr15 != 0: the adapter term of out[m, c] is kept only where dropout keeps (m, c)
-};
-
-// Which output tile a workgroup computes.  Workgroups are handed to the 8 XCDs round-robin in dispatch order.  The ids are
-// permuted so that one XCD owns a contiguous range of tiles, ordered in groups of `rg` row tiles: all column tiles of a
-// group, then the next group.  The 32 workgroups an XCD runs at a time then share 2 slabs of activations and 16 column
-// tiles of W (about 4 MB each at K = 4096, what its L2 holds) instead of every row tile of a few columns: with many row
-// tiles the activations would otherwise stream from HBM once per column tile (8192 x 4096 x 4096: 306 -> 260 us; no shape
-// slower).
-struct TileMap {
-    int tile_c, tile_r;
-};
-__device__ __forceinline__ TileMap map_tile(int phase_step, int col_tile0) {
-    const int nc = gridDim.x, nr = gridDim.y, total = nc * nr;
-    int id = blockIdx.y * nc + blockIdx.x;
-    if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
-    TileMap m;
-    const int rg = phase_step >> 8;                   // row tiles per group (0: column-major over all row tiles)
-    const int grouped = rg > 0 ? (nr / rg) * rg * nc : 0;
-    if (id < grouped) {
-        // groups of rg row tiles: all column tiles of a group, then the next group
-        const int gi = id / (rg * nc), rem = id - gi * rg * nc;
-        m.tile_c = rem / rg;
-        m.tile_r = gi * rg + (rem - m.tile_c * rg);
-    } else {
-        const int left = rg > 0 ? nr % rg : nr, base = nr - left, rem = id - grouped;
-        m.tile_c = rem / left;
-        m.tile_r = base + (rem - m.tile_c * left);
-    }
-    m.tile_c += col_tile0;
-    return m;
-}
-// Split-K: gridDim.z workgroups share an output tile; workgroup z owns `cnt` consecutive steps from `begin`.
-struct StepRange {
-    int begin, cnt;
-};
-__device__ __forceinline__ StepRange split_steps(int nsteps, int z, int S) {
-    const int base = nsteps / S, rem = nsteps - base * S;
-    StepRange r;
-    r.cnt = base + (z < rem ? 1 : 0);
-    r.begin = z * base + min(z, rem);
-    return r;
-}
-// reduction offset of pipeline stage `stage` (stages past the end repeat the last one: harmless reloads)
-__device__ __forceinline__ int red_of(int stage, StepRange sr, int phase) {
-    int v = min(stage, sr.cnt - 1) + phase;
-    if (v >= sr.cnt) v -= sr.cnt;
-    return (sr.begin + v) * BK;
-}
-
-// Group of reduction row k (a multiple of 64; sequential groups of a multiple of 64 rows):
-// floor((k/64) / (groupsize/64)) as a multiply-high, exact while k * groupsize < 2^40.
-__device__ __forceinline__ int group_of(const GemmArgs& a, int k) {
-    return (int)__umulhi((uint32_t)k >> 5, a.gs_inv31);
-}
-
-__device__ __forceinline__ float adapter_at(const GemmArgs& a, size_t idx) {
-    return a.lb_is_f32 ? reinterpret_cast<const float*>(a.lb)[idx] : (float)reinterpret_cast<const half_t*>(a.lb)[idx];
-}
 // rn16(rn16(s*q) - zero) for a pair of codes given as (0x6400 | q): one fused multiply-add
 // computes s*(1024+q) - 1024*s = s*q with a single rounding (1024*s is exact), i.e. exactly
 // rn16(s*q); the subtraction of the zero term is the third rounding.  Needs |s| < 64 so that
@@ -126,14 +45,6 @@ __device__ __forceinline__ float adapter_at(const GemmArgs& a, size_t idx) {
 __device__ __forceinline__ half2_t dequant_pair_magic(uint32_t codes_or_magic, half2_t s, half2_t s1024, half2_t zero) {
     const half2_t p = __builtin_elementwise_fma(as_half2(codes_or_magic), s, -s1024);
     return p - zero;
-}
-
-template <int I, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
 }
 
 struct SlabRsrc {
@@ -695,19 +606,6 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs a) {
     gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(&a, 1, map_tile(a.phase_step, a.col_tile0), sr, blockIdx.z, gridDim.z);
 }
 
-// Up to kGemmGroup layers that share M, K, the group size and (forward) the activations -- q|k|v, gate|up -- in ONE
-// grid, each on its own tensors.
-//   forward:    blockIdx.x walks the column tiles of layer 0, then of layer 1, ...; every workgroup computes one tile of
-//               one layer's own output, over the whole reduction (no split).
-//   grad-input: dx = sum_i dy_i @ W_i^T is ONE reduction over the layers' columns one after the other: a workgroup
-//               walks the layers (all of them, or its share of the concatenated steps where the tiles are few) with
-//               the sum in its accumulators, adapter term and dropout mask of each layer included.
-struct GemmGroupArgs {
-    GemmArgs layer[kGemmGroup];
-    int tile_end[kGemmGroup];          // forward: running total of column tiles (tile width of the launch)
-    int n;
-};
-
 template <int BM, int WGM, bool FWD, bool GIDX, int SZ = 0, int WGN = 2>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_group_kernel(GemmGroupArgs g) {
     TileMap tm = map_tile(g.layer[0].phase_step, g.layer[0].col_tile0);
@@ -797,23 +695,18 @@ static void launch_tail(GemmArgs a, int nout, int tail_cols, int tail_splits, hi
     if (tail_splits > 1) launch_reduce_cols(a, a.part_cols, nout, a.col_tile0 * BN, tail_splits, stream);
 }
 
-// 256 x 256 tiles (8 wavefronts of 128 x 64): half the activation traffic and 30 % less LDS traffic per MFMA than the
-// 256 x 128 tile; for outputs with enough such tiles to fill the CUs.  Their reduction is not split; the tile buffers
-// take 144 KB of LDS, so the grad-input kernel keeps its per-step scale / zero loads.
+// 256 x 256 tiles, for outputs with enough of them to fill the CUs: half the activation traffic of the 256 x 128 tile per MFMA.
+// Their reduction is not split.  Sequential groups: q4_gemm_wide.hip.  Per-row groups: 8 wavefronts of 128 x 64 of gemm_kernel.
 // tail_cols > 0: the last tail_cols tiles of 128 columns are left to a second launch of 256 x 128 tiles, with the
 // reduction split tail_splits ways (see wide_tail).
 template <bool FWD, bool GIDX>
 static hipError_t launch_gemm_wide(GemmArgs a, int nout, int tail_cols, int tail_splits, hipStream_t stream) {
     const int nr = (a.M + 255) / 256;
-    const dim3 grid((nout - tail_cols * BN) / 256, nr, 1), block(512);
+    const dim3 grid((nout - tail_cols * BN) / 256, nr, 1);
     a.col_tile0 = 0;
     a.part_cols = nout;
-    bool sz1 = false;
-    if constexpr (FWD && !GIDX) {
-        sz1 = a.groupsize % 128 == 0 && (a.K / BK) % 2 == 0 && ((a.phase_step & 0xff) % 2) == 0;
-        if (sz1) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 1, 4>), grid, block, 0, stream, a);
-    }
-    if (!sz1) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 0, 4>), grid, block, 0, stream, a);
+    if constexpr (GIDX) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 0, 4>), grid, dim3(512), 0, stream, a);
+    else launch_wide_tiles(FWD, a, grid, stream);
     if (tail_cols > 0) launch_tail<FWD, GIDX>(a, nout, tail_cols, tail_splits, stream);
     return hipGetLastError();
 }
@@ -923,29 +816,30 @@ extern "C" int q4_launch_gemm(int fwd, const void* act, const int32_t* qweight, 
 
 // ---- several layers in one launch (sequential groups only) ---------------------------------------------------------
 namespace q4 {
-template <int BM, int WGM, bool FWD, int WGN>
+// 256 x 128 tiles
+template <bool FWD>
 static void launch_group_tiles(const GemmGroupArgs& g, int n, dim3 grid, hipStream_t stream) {
     const GemmArgs& a = g.layer[0];
-    const dim3 block(64 * WGM * WGN);
+    const dim3 block(512);
     if (a.groupsize % 128 == 0) {
         if constexpr (FWD) {
             if ((a.K / BK) % 2 == 0 && ((a.phase_step & 0xff) % 2) == 0) {
-                hipLaunchKernelGGL((gemm_group_kernel<BM, WGM, FWD, false, 1, WGN>), grid, block, 0, stream, g);
+                hipLaunchKernelGGL((gemm_group_kernel<256, 4, FWD, false, 1>), grid, block, 0, stream, g);
                 return;
             }
-        } else if constexpr (WGN == 2) {
+        } else {
             int mx = 0;
             for (int i = 0; i < n; ++i) mx = g.layer[i].N > mx ? g.layer[i].N : mx;
             const size_t tab = (size_t)mx * 4;
-            static const bool attr_ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_group_kernel<BM, WGM, FWD, false, 2, WGN>),
+            static const bool attr_ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_group_kernel<256, 4, FWD, false, 2>),
                                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSzTableMax) == hipSuccess;
             if (attr_ok && tab <= kSzTableMax) {
-                hipLaunchKernelGGL((gemm_group_kernel<BM, WGM, FWD, false, 2, WGN>), grid, block, tab, stream, g);
+                hipLaunchKernelGGL((gemm_group_kernel<256, 4, FWD, false, 2>), grid, block, tab, stream, g);
                 return;
             }
         }
     }
-    hipLaunchKernelGGL((gemm_group_kernel<BM, WGM, FWD, false, 0, WGN>), grid, block, 0, stream, g);
+    hipLaunchKernelGGL((gemm_group_kernel<256, 4, FWD, false, 0>), grid, block, 0, stream, g);
 }
 }  // namespace q4
 
@@ -1011,10 +905,9 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
             g.tile_end[i] = ends[wide ? 0 : 1][i];
         }
         const dim3 grid(count, nr, splits);
-        if (fwd && wide) launch_group_tiles<256, 2, true, 4>(g, n, grid, stream);
-        else if (fwd) launch_group_tiles<256, 4, true, 2>(g, n, grid, stream);
-        else if (wide) launch_group_tiles<256, 2, false, 4>(g, n, grid, stream);
-        else launch_group_tiles<256, 4, false, 2>(g, n, grid, stream);
+        if (wide) launch_wide_group_tiles(fwd != 0, g, grid, stream);
+        else if (fwd) launch_group_tiles<true>(g, n, grid, stream);
+        else launch_group_tiles<false>(g, n, grid, stream);
         if (splits > 1) launch_reduce_cols(g.layer[0], part_cols, K, first * (wide ? 256 : BN), splits, stream);
     };
     const bool wide = p.cfg == 3;

@@ -1,0 +1,486 @@
+// Tiled GEMMs whose weight operands are built in registers (sequential groups of a multiple of 64 rows):
+//   forward   y [M,N] = x  [M,K] @ W      (+ bias) (+ xa  [M,R] @ lora_bt [R,N])
+//   backward  dx[M,K] = dy [M,N] @ W^T             (+ dyb [M,R] @ lora_a  [R,K])
+// the products of q4_gemm.hip for outputs that have enough large tiles (plan_gemm).
+//
+// What bounds them.  A full round of 256 x 256 tiles runs into the chip's power limit: products of normally distributed operands
+// from registers alone reach 1.64 PFLOP/s at 1.6-1.7 GHz (2.4 PFLOP/s at 2.4 GHz on zeros), with a 128-bit LDS fragment per two
+// MFMAs and two packed vector operations per MFMA beside them 1.50.  Speed is then energy per MFMA, not cycles: with parts of the
+// loop taken out, the activations' way from L2 into LDS is 11 % of it, the operand build 13 %, the fragment reads 6 %, the
+// packed words less than 1 %.
+//
+// Layout.  A workgroup computes 32*TM x 256 outputs with four wavefronts, one per SIMD, side by side: each has all rows of 64
+// columns as TM x 2 accumulators of v_mfma_f32_32x32x16_f16 (256 registers at TM = 8).  No two wavefronts share a column, so
+// every weight is decoded once per workgroup and its operand never goes through LDS: forward, a packed word IS the 8-deep
+// reduction slice of one column that a lane feeds to the MFMA.  Grad-input, a word holds eight output columns of one reduction
+// index; the workgroup turns each 8 x 8 block of codes around in registers (32 byte permutes and masks per thread and step) and
+// passes the turned words, still packed, through 8 KB of LDS.  LDS otherwise holds activations only: four tiles of 64 reduction
+// entries, written by the loads themselves (buffer_load ... lds) three steps ahead, units of 16 bytes swizzled by the row so
+// that the 128-bit fragment reads meet no bank twice.  Per 256 x 256 x 64 step 32 KB are written and 128 KB read, where staging
+// both operands (8 wavefronts of 128 x 64) writes 64 KB and reads 192.
+//
+// Operand build.  13 (forward) or 11 vector operations per word: masks, permutes, one conversion per pair (codes_of_bytes) and one
+// fused multiply-add, weight = rn16(scale * code - rn16(scale * (zero + 1))) -- one rounding less than the dense kernel, and
+// less energy than the magic-number form (16: and 1.5 % of the time).  The pieces sit one by one behind the MFMAs.
+//
+// us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 115 -> 108.5,
+// 4096 x (5120 -> 13824) 489 -> 468, 4096 x (13824 -> 5120) 480 -> 457; grad-input 115 -> 110, 488 -> 473, 490 -> 476; cycles per
+// step (2048 of them MFMAs) forward 2500, grad-input 2770, at 1.55 and 1.67 GHz.
+#include "q4_gemm_args.hpp"
+
+namespace q4 {
+
+// 16 bytes per lane from memory to LDS, lane l's at lds + 16 l
+__device__ __forceinline__ void load_lds128(rsrc_t r, half_t* lds, int voff, int soff) {
+    typedef __attribute__((address_space(3))) void lds_void;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, 0);
+}
+
+constexpr int kStages = 4;               // activation tiles in LDS: one being multiplied, three on their way
+constexpr int kWideCols = 256;
+constexpr int kFar = 0x70000000;         // beyond every buffer: reads as zero, without traffic
+
+// Codes in bytes 2H, 2H + 1 of `b` as two fp16 values.  The byte 0x0q read as an 8-bit float of 4 exponent and 3 mantissa bits
+// is q * 2^-9 for every q of 0..15 (the first binade continues the subnormals), so one conversion scaled by 2^9 yields the codes.
+template <int H>
+__device__ __forceinline__ half2_t codes_of_bytes(uint32_t b) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.f, H != 0));
+}
+__device__ __forceinline__ uint32_t bfi(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
+
+template <int TM, bool FWD, bool MULTI>
+__device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay, const TileMap tm, const StepRange share,
+                                          const int zsplit, const int nsplit) {
+    constexpr int BM = 32 * TM, KS = BK / 16, NMK = 2 * TM;       // NMK: MFMAs of a sub-step of 16
+    constexpr int kTile = BM * BK;                                // halves of an activation tile
+    constexpr int kOther = FWD ? KS + 2 : 4;                      // loads of a step beside its activations
+    constexpr int kLoads = TM + kOther;
+    __shared__ __attribute__((aligned(16))) half_t sA0[kTile];
+    __shared__ __attribute__((aligned(16))) half_t sA1[kTile];
+    __shared__ __attribute__((aligned(16))) half_t sA2[kTile];
+    __shared__ __attribute__((aligned(16))) half_t sA3[kTile];
+    // grad-input: codes of a step, nibbles along the reduction: [octet][column], and (scales, zero terms) of a wavefront's step
+    constexpr int kTw = kWideCols + 8;
+    __shared__ __attribute__((aligned(16))) uint32_t sT0[FWD ? 4 : 8 * kTw];
+    __shared__ __attribute__((aligned(16))) uint32_t sT1[FWD ? 4 : 8 * kTw];
+    __shared__ __attribute__((aligned(16))) half_t sZ[FWD ? 1 : 4][2][2][FWD ? 4 : BK];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lc = lane & 31, lg = lane >> 5;
+    const GemmArgs& a0 = layers[0];
+    const int NOUT = FWD ? a0.N : a0.K;
+    const int m0 = tm.tile_r * BM, c0 = tm.tile_c * kWideCols, cw = c0 + 64 * wave;
+    const int rows_valid = min(BM, a0.M - m0);
+
+    float bias_v[2] = {0.f, 0.f};
+    if (FWD && a0.bias) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bias_v[j] = (float)a0.bias[cw + 2 * lc + j];
+    }
+    float16_t acc[TM][2];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    auto run_layer = [&](const GemmArgs& a, const StepRange sr) {
+        const int RED = FWD ? a.K : a.N;
+        const int phase = (tm.tile_r * (a.phase_step & 0xff)) % sr.cnt;
+        const rsrc_t ra = make_rsrc(a.a + (size_t)m0 * RED, (unsigned)rows_valid * (unsigned)RED * 2u);
+        const rsrc_t rw = make_rsrc(a.qweight, (unsigned)(a.K >> 3) * (unsigned)a.N * 4u);
+        const rsrc_t rs = make_rsrc(a.scales, (unsigned)a.G * (unsigned)a.N * 2u);
+        const rsrc_t rz = make_rsrc(a.qzeros, (unsigned)a.G * (unsigned)(a.N >> 3) * 4u);
+
+        // activations: load q of a wavefront brings rows 8 (4q + wave) .. + 7, lane (row, slot); 16-byte unit u of row r sits
+        // in slot u ^ (r / 2 % 8)
+        int va[TM];
+#pragma unroll
+        for (int q = 0; q < TM; ++q)
+            va[q] = ((8 * (4 * q + wave) + (lane >> 3)) * RED + 8 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)))) * 2;
+        auto load_a = [&](half_t* dst, int q, int red) {
+            load_lds128(ra, dst + (4 * q + wave) * 512, va[q], red * 2);
+        };
+        auto stage_ptr = [&](auto st) -> half_t* {
+            constexpr int S = decltype(st)::value & 3;
+            if constexpr (S == 0) return sA0;
+            else if constexpr (S == 1) return sA1;
+            else if constexpr (S == 2) return sA2;
+            else return sA3;
+        };
+        int fo[KS];                                               // fragment of sub-step ks, halves from the tile's start
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) fo[ks] = lc * BK + 8 * ((2 * ks + lg) ^ ((lc >> 1) & 7));
+
+        // packed words.  Forward: word-row 2 ks + lg of the step, columns cw + 2 lc, + 1: the lane's own B operands.
+        // Grad-input: word-row t % 32 of the tile's 256 output columns, octet t / 32 of the step's 64 columns n.
+        uint2_t w[FWD ? kStages : 2][KS];                         // grad-input: read back from sT, turned around
+        uint4_t wr[FWD ? 1 : kStages][2];
+        uint32_t sraw[kStages], zraw[kStages];
+        const int twr = (threadIdx.x >> 3) & 31, toc = threadIdx.x & 7;
+        const int g_out = FWD ? 0 : cw / a.groupsize;
+        const int vw = FWD ? (lg * a.N + cw + 2 * lc) * 4 : (((c0 >> 3) + twr) * a.N + 8 * toc) * 4;
+        const int vs = FWD ? (cw + 2 * lc) * 2 : (g_out * a.N + lane) * 2;
+        const int vz = FWD ? ((cw + 2 * lc) >> 3) * 4 : (g_out * (a.N >> 3) + (lane >> 3)) * 4;
+        // load number l of the step that multiplies reduction offset red; `slot` its registers
+        auto load_other = [&](auto slot, auto lt, int red) {
+            constexpr int S = decltype(slot)::value & 3, l = decltype(lt)::value;
+            if constexpr (FWD) {
+                if constexpr (l < KS) w[S][l] = buf_load64(rw, vw, ((red >> 3) + 2 * l) * a.N * 4);
+                else if constexpr (l == KS) sraw[S] = buf_load32(rs, vs, group_of(a, red) * a.N * 2);
+                else zraw[S] = buf_load32(rz, vz, group_of(a, red) * (a.N >> 3) * 4);
+            } else {
+                if constexpr (l < 2) wr[S][l] = buf_load128(rw, vw, (red + 4 * l) * 4);
+                else if constexpr (l == 2) sraw[S] = buf_load16(rs, vs, red * 2);
+                else zraw[S] = buf_load32(rz, vz, (red >> 3) * 4);
+            }
+        };
+
+        // forward: (scale, zero term) of the lane's two columns
+        half2_t s2[2], z2[2];
+        auto prep = [&](uint32_t s, uint32_t z) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                s2[j] = as_half2(__builtin_amdgcn_perm(s, s, j ? 0x03020302u : 0x01000100u));
+                const uint32_t zz = (z >> (4 * ((2 * lc + j) & 7))) & 0xFu;
+                z2[j] = zero_term(s2[j], zz, zz);
+            }
+        };
+        // grad-input: scales and zero terms of the octet the lane multiplies in a sub-step
+        uint4_t so[2], zo[2];
+        uint32_t bo[2][2][4];                                     // B operands [sub-step parity][j][pair]
+        half8_t af[2][TM];
+        auto read_sz = [&](auto st, auto kt) {
+            constexpr int P = decltype(st)::value & 1, ks = decltype(kt)::value;
+            so[ks & 1] = *reinterpret_cast<const uint4_t*>(&sZ[FWD ? 0 : wave][P][0][FWD ? 0 : 8 * (2 * ks + lg)]);
+            zo[ks & 1] = *reinterpret_cast<const uint4_t*>(&sZ[FWD ? 0 : wave][P][1][FWD ? 0 : 8 * (2 * ks + lg)]);
+        };
+        // The operands of sub-step ks of a stage in 12 pieces for as many MFMAs' shadows: the codes of column j as bytes
+        // (pieces 0..3: the two halves of j = 0, of j = 1), then one pair of weights each.
+        uint32_t bt[2][2];
+        auto build = [&](auto st, auto kt, auto ut) {
+            constexpr int ks = decltype(kt)::value, u = decltype(ut)::value, S = decltype(st)::value & (FWD ? 3 : 1);
+            if constexpr (u % 6 < 2) {
+                constexpr int j = u / 6, h = u % 6;
+                const uint32_t c = j ? w[S][ks].y : w[S][ks].x;
+                if constexpr (!FWD) bt[j][h] = (h ? c >> 4 : c) & 0x0F0F0F0Fu;
+                else if constexpr (h == 0) { bt[j][0] = c & 0x0F0F0F0Fu; bt[j][1] = (c >> 4) & 0x0F0F0F0Fu; }
+                else {                                            // rows 0..3 and 4..7 in order
+                    const uint32_t lo = bt[j][0], hi = bt[j][1];
+                    bt[j][0] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+                    bt[j][1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+                }
+            } else {
+                constexpr int j = u / 6, p = u % 6 - 2;
+                const half2_t q = codes_of_bytes<p & 1>(bt[j][p >> 1]);
+                const half2_t sc = FWD ? s2[j] : as_half2(so[ks & 1][p]), zt = FWD ? z2[j] : as_half2(zo[ks & 1][p]);
+                bo[ks & 1][j][p] = as_u32(__builtin_elementwise_fma(q, sc, -zt));
+            }
+        };
+        auto build_all = [&](auto st, auto kt) {
+            static_for<0, 12>([&](auto ut) { build(st, kt, ut); });
+        };
+        // grad-input: the eight words of a thread turned around and stored, in pieces
+        uint32_t tx[8];
+        auto turn = [&](auto slot, auto par, auto it) {
+            constexpr int S = decltype(slot)::value & 3, P = decltype(par)::value & 1, I = decltype(it)::value;
+            if constexpr (!FWD) {
+                if constexpr (I == 0 || I == 1) {                 // 16-bit halves: rows 0-3 against 4-7
+                    const uint4_t lo = wr[S][0], hi = wr[S][1];
+                    const uint32_t x[8] = {lo.x, hi.x, lo.y, hi.y, lo.z, hi.z, lo.w, hi.w};      // nibble 2 c of a turned word is column c, 2 c + 1 column c + 4
+#pragma unroll
+                    for (int i = 2 * I; i < 2 * I + 2; ++i) {
+                        tx[i] = __builtin_amdgcn_perm(x[i + 4], x[i], 0x05040100u);
+                        tx[i + 4] = __builtin_amdgcn_perm(x[i + 4], x[i], 0x07060302u);
+                    }
+                } else if constexpr (I == 2 || I == 3) {          // bytes
+                    constexpr int b = 4 * (I - 2);
+#pragma unroll
+                    for (int i = b; i < b + 2; ++i) {
+                        const uint32_t u = tx[i], v = tx[i + 2];
+                        tx[i] = __builtin_amdgcn_perm(v, u, 0x06020400u);
+                        tx[i + 2] = __builtin_amdgcn_perm(v, u, 0x07030501u);
+                    }
+                } else if constexpr (I < 8) {                     // nibbles
+                    constexpr int i = 2 * (I - 4);
+                    const uint32_t u = tx[i], v = tx[i + 1];
+                    tx[i] = bfi(0x0F0F0F0Fu, u, v << 4);
+                    tx[i + 1] = bfi(0x0F0F0F0Fu, u >> 4, v);
+                } else if constexpr (I == 8) {
+                    uint32_t* d = (P ? sT1 : sT0) + toc * kTw + 8 * twr;
+                    *reinterpret_cast<uint4_t*>(d) = uint4_t{tx[0], tx[1], tx[2], tx[3]};
+                    *reinterpret_cast<uint4_t*>(d + 4) = uint4_t{tx[4], tx[5], tx[6], tx[7]};
+                } else {                                          // scale and zero term of column n = lane of the step
+                    const half_t s = __builtin_bit_cast(half_t, (unsigned short)sraw[S]);
+                    const half_t z = (half_t)(float)(((zraw[S] >> (4 * (lane & 7))) & 0xFu) + 1u);
+                    sZ[wave][P][0][FWD ? 0 : lane] = s;
+                    sZ[wave][P][1][FWD ? 0 : lane] = s * z;
+                }
+            }
+        };
+        constexpr int kTurns = 10;
+        auto read_t = [&](auto st) {
+            constexpr int P = decltype(st)::value & 1;
+            if constexpr (!FWD) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+                    w[P][ks] = *reinterpret_cast<const uint2_t*>((P ? sT1 : sT0) + (2 * ks + lg) * kTw + 64 * wave + 2 * lc);
+            }
+        };
+        constexpr int kAhead = FWD ? 3 : 4;                       // stage whose words, scales, zeros a step requests
+        constexpr int BAR = TM / 4;                               // slot of the last sub-step behind which the barrier sits
+
+        // multiplies stage s (ring position C = s % 4); on entry af[0] and bo[0] hold its sub-step 0
+        auto step = [&](int s, auto ct) {
+            constexpr int C = decltype(ct)::value;
+            const int red3 = red_of(s + 3, sr, phase), redx = red_of(s + kAhead, sr, phase);
+            static_for<0, KS>([&](auto kt) {
+                constexpr int ks = decltype(kt)::value, kn = (ks + 1) % KS;
+                constexpr int sn = ks + 1 == KS ? C + 1 : C;      // stage of the operands built in this sub-step
+                static_for<0, NMK>([&](auto it) {
+                    constexpr int i = decltype(it)::value, g = ks * NMK + i;
+                    acc[i / 2][i % 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks & 1][i / 2],
+                        __builtin_bit_cast(half8_t, uint4_t{bo[ks & 1][i % 2][0], bo[ks & 1][i % 2][1], bo[ks & 1][i % 2][2], bo[ks & 1][i % 2][3]}),
+                        acc[i / 2][i % 2], 0, 0, 0);
+                    // requests, one at a time over the first three sub-steps
+                    constexpr int SL = 3 * NMK;
+                    static_for<0, kLoads>([&](auto lt) {
+                        constexpr int l = decltype(lt)::value;
+                        if constexpr (l * SL / kLoads == g) {
+                            if constexpr (l < kOther) load_other(std::integral_constant<int, C + kAhead>{}, lt, redx);
+                            else load_a(stage_ptr(std::integral_constant<int, C + 3>{}), l - kOther, red3);
+                        }
+                    });
+                    // activation fragments of the next sub-step
+                    constexpr int first = ks + 1 == KS ? BAR + 1 : 0, span = NMK - 1 - first;
+                    if constexpr (ks + 1 == KS && i == BAR) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        __builtin_amdgcn_s_waitcnt(0x0070 | ((2 * kLoads) & 15) | (((2 * kLoads) >> 4) << 14));
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    static_for<0, TM>([&](auto rt) {
+                        constexpr int r = decltype(rt)::value;
+                        if constexpr (first + r * span / TM == i)
+                            af[kn & 1][r] = *reinterpret_cast<const half8_t*>(stage_ptr(std::integral_constant<int, sn>{}) + fo[kn] + r * 32 * BK);
+                    });
+                    // operands of the next sub-step
+                    if constexpr (FWD) {
+                        if constexpr (ks + 1 == KS && i == 0) prep(sraw[(C + 1) & 3], zraw[(C + 1) & 3]);
+                    } else {
+                        if constexpr (i == 0) read_sz(std::integral_constant<int, ks + 2 >= KS ? C + 1 : C>{}, std::integral_constant<int, (ks + 2) % KS>{});
+                        if constexpr (ks == KS - 2 && i == 1) read_t(std::integral_constant<int, C + 1>{});
+                        static_for<0, kTurns>([&](auto qt) {      // words of stage s + 2
+                            constexpr int q = decltype(qt)::value;
+                            if constexpr (NMK / 2 + q * 2 * NMK / kTurns == g) turn(std::integral_constant<int, C + 2>{}, std::integral_constant<int, C>{}, qt);
+                        });
+                    }
+                    static_for<0, 12>([&](auto ut) {
+                        constexpr int u = decltype(ut)::value;
+                        if constexpr (u * (NMK - 1) / 12 == i) build(std::integral_constant<int, sn>{}, std::integral_constant<int, kn>{}, ut);
+                    });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            });
+        };
+
+        // the first stages
+        static_for<0, kAhead>([&](auto st) {
+            constexpr int S = decltype(st)::value;
+            const int red = red_of(S, sr, phase);
+            static_for<0, kOther>([&](auto lt) { load_other(st, lt, red); });
+            if constexpr (S < 3) {
+#pragma unroll
+                for (int q = 0; q < TM; ++q) load_a(stage_ptr(st), q, red);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (!FWD) {
+            static_for<0, kTurns>([&](auto qt) { turn(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, qt); });
+            static_for<0, kTurns>([&](auto qt) { turn(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, qt); });
+        }
+        constexpr int kBehind = FWD ? 2 * kLoads : 2 * kLoads + kOther;     // requested behind stage 0
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kBehind & 15) | ((kBehind >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if constexpr (FWD) prep(sraw[0], zraw[0]);
+        else {
+            read_t(std::integral_constant<int, 0>{});
+            read_sz(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+            read_sz(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) af[0][i] = *reinterpret_cast<const half8_t*>(sA0 + fo[0] + i * 32 * BK);
+        build_all(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        int s = 0;
+        for (; s + 4 <= sr.cnt; s += 4) {
+            step(s, std::integral_constant<int, 0>{});
+            step(s + 1, std::integral_constant<int, 1>{});
+            step(s + 2, std::integral_constant<int, 2>{});
+            step(s + 3, std::integral_constant<int, 3>{});
+        }
+        if (s < sr.cnt) step(s, std::integral_constant<int, 0>{});
+        if (s + 1 < sr.cnt) step(s + 1, std::integral_constant<int, 1>{});
+        if (s + 2 < sr.cnt) step(s + 2, std::integral_constant<int, 2>{});
+        // nothing on its way into the tiles any more, and every wavefront done with them
+        __builtin_amdgcn_s_waitcnt(0x0070);
+        __syncthreads();
+    };
+
+    // Adapter term: its operands straight from memory, one block of 32 rows at a time, behind the main loop, where its
+    // registers are free.  Dropout on the adapter input: its share of out[m, c] exists only where the mask keeps (m, c); the kept
+    // values carry 1 / (1 - p) through lb_scale.
+    auto add_adapter = [&](const GemmArgs& a) {
+        const rsrc_t rl = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
+        const bool masked = a.drop.thr15 != 0;
+        half8_t lb[4][2];
+        uint4_t v[2][4];
+        auto load_rows = [&](uint4_t* d, int i) {
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)                    // columns past R and rows past M read as zero
+                d[ks] = buf_load128(rl, 16 * ks + 8 * lg < a.R ? ((32 * i + lc) * a.R + 16 * ks + 8 * lg) * 2 : kFar, 0);
+        };
+        load_rows(v[0], 0);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) lb[ks][j] = half8_t{};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int r0 = 16 * ks + 8 * lg;
+            if (r0 < a.R) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        lb[ks][j][e] = (half_t)(a.lb_scale * adapter_at(a, (size_t)(r0 + e) * a.lb_sr + (size_t)(cw + 2 * lc + j) * a.lb_sc));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            float16_t term[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) term[j][r] = 0.f;
+            if (i + 1 < TM) load_rows(v[(i + 1) & 1], i + 1);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                if (16 * ks < a.R) {                          // uniform
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        term[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, v[i & 1][ks]), lb[ks][j], term[j], 0, 0, 0);
+                }
+            if (masked) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
+                    const uint32_t dw = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)(cw + 2 * lc) >> 1);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) term[j][r] = ((dw >> (16 * j)) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[j][r];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] += term[j][r];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    if constexpr (MULTI) {
+        int base = 0;
+#pragma unroll 1
+        for (int li = 0; li < nlay; ++li) {
+            const int steps = (FWD ? layers[li].K : layers[li].N) / BK;
+            const int lo = max(share.begin, base) - base, hi = min(share.begin + share.cnt, base + steps) - base;
+            base += steps;
+            if (lo >= hi) continue;                               // uniform
+            run_layer(layers[li], StepRange{lo, hi - lo});
+        }
+        base = 0;
+#pragma unroll 1
+        for (int li = 0; li < nlay; ++li) {                       // with the share that holds a layer's first step
+            if (layers[li].R > 0 && share.begin <= base && base < share.begin + share.cnt) add_adapter(layers[li]);
+            base += (FWD ? layers[li].K : layers[li].N) / BK;
+        }
+    } else {
+        run_layer(a0, share);
+        if (a0.R > 0 && zsplit == 0) add_adapter(a0);
+    }
+
+    // acc[i][j][r]: row 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, column cw + 2 (lane % 32) + j
+    if (nsplit > 1) {
+        float* const pz = a0.part + (size_t)zsplit * a0.M * a0.part_cols - (size_t)a0.col_tile0 * kWideCols;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
+                typedef float float2_t __attribute__((ext_vector_type(2)));
+                const float2_t v = {acc[i][0][r] + (zsplit == 0 ? bias_v[0] : 0.f), acc[i][1][r] + (zsplit == 0 ? bias_v[1] : 0.f)};
+                if (m < a0.M) *reinterpret_cast<float2_t*>(pz + (size_t)m * a0.part_cols + cw + 2 * lc) = v;
+            }
+        return;
+    }
+    constexpr int kRow = 64 + 8;                                  // halves of a staged row of 64 outputs
+    half_t* stage = (wave < 2 ? sA0 : sA1) + (wave & 1) * (32 * kRow);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const half2_t h = {(half_t)(acc[i][0][r] + bias_v[0]), (half_t)(acc[i][1][r] + bias_v[1])};
+            *reinterpret_cast<half2_t*>(stage + (8 * (r >> 2) + 4 * lg + (r & 3)) * kRow + 2 * lc) = h;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int rr = (lane >> 3) + 8 * p, m = m0 + 32 * i + rr;
+            const uint4_t v = *reinterpret_cast<const uint4_t*>(stage + rr * kRow + 8 * (lane & 7));
+            if (m < a0.M) *reinterpret_cast<uint4_t*>(a0.out + (size_t)m * NOUT + cw + 8 * (lane & 7)) = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
+
+template <int TM, bool FWD>
+__global__ __launch_bounds__(256) void gemm_wide_kernel(GemmArgs a) {
+    const StepRange sr = split_steps((FWD ? a.K : a.N) / BK, blockIdx.z, gridDim.z);
+    wide_body<TM, FWD, false>(&a, 1, map_tile(a.phase_step, a.col_tile0), sr, blockIdx.z, gridDim.z);
+}
+
+// Several layers in one grid (see GemmGroupArgs).
+template <int TM, bool FWD>
+__global__ __launch_bounds__(256) void gemm_wide_group_kernel(GemmGroupArgs g) {
+    TileMap tm = map_tile(g.layer[0].phase_step, g.layer[0].col_tile0);
+    if constexpr (FWD) {
+        const int li = (tm.tile_c >= g.tile_end[0]) + (tm.tile_c >= g.tile_end[1]) + (tm.tile_c >= g.tile_end[2]);   // uniform
+        tm.tile_c -= li == 0 ? 0 : g.tile_end[li - 1];
+        const GemmArgs a = g.layer[li];
+        wide_body<TM, FWD, false>(&a, 1, tm, split_steps(a.K / BK, 0, 1), 0, 1);
+    } else {
+        int nsteps = 0;
+        for (int i = 0; i < g.n; ++i) nsteps += g.layer[i].N / BK;
+        wide_body<TM, FWD, true>(g.layer, g.n, tm, split_steps(nsteps, blockIdx.z, gridDim.z), (int)blockIdx.z, (int)gridDim.z);
+    }
+}
+
+void launch_wide_tiles(bool fwd, const GemmArgs& a, dim3 grid, hipStream_t stream) {
+    if (fwd) hipLaunchKernelGGL((gemm_wide_kernel<8, true>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((gemm_wide_kernel<8, false>), grid, dim3(256), 0, stream, a);
+}
+void launch_wide_group_tiles(bool fwd, const GemmGroupArgs& g, dim3 grid, hipStream_t stream) {
+    if (fwd) hipLaunchKernelGGL((gemm_wide_group_kernel<8, true>), grid, dim3(256), 0, stream, g);
+    else hipLaunchKernelGGL((gemm_wide_group_kernel<8, false>), grid, dim3(256), 0, stream, g);
+}
+
+}  // namespace q4
