@@ -652,6 +652,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_cols_kernel(const floa
     *reinterpret_cast<half4_t*>(out + m * out_cols + col0 + c) = h;
 }
 
+// What TileMap is told: row tile r starts its reduction loop kPhaseStep * r steps later; tiles are ordered in groups
+// of kRowTilesPerGroup row tiles (measured optimum over the benchmark shapes).
+constexpr int kPhaseStep = 2, kRowTilesPerGroup = 2;
+
 // One grid of tiles, with the cheapest way of feeding scale and zero that the problem allows (see gemm_kernel).
 constexpr size_t kSzTableMax = 48 * 1024;     // dynamic LDS left beside the 108 KB of tile buffers
 template <int BM, int WGM, bool FWD, bool GIDX>
@@ -686,11 +690,24 @@ static void launch_reduce_cols(const GemmArgs& a, int part_cols, int out_cols, i
                        a.part, a.out, a.M, part_cols, out_cols, col0, splits);
 }
 
+// Forward, sequential groups, an unsplit grid of 256 x 128 tiles over an even number of column tiles: the same area as
+// 128 x 256 tiles of q4_gemm_wide.hip.
+template <bool FWD, bool GIDX>
+static bool launch_low_tiles(GemmArgs a, int first, int cols, int splits, hipStream_t stream) {
+    if constexpr (!FWD || GIDX) return false;
+    if (splits > 1 || first % 2 != 0 || cols % 2 != 0) return false;
+    a.col_tile0 = first / 2;
+    a.phase_step = (a.phase_step & 0xff) | (2 * kRowTilesPerGroup << 8);
+    launch_wide_tiles(true, true, a, dim3(cols / 2, (a.M + 127) / 128), stream);
+    return true;
+}
+
 // The last tail_cols column tiles of 128 as a launch of 256 x 128 tiles whose reduction is split tail_splits ways.
 template <bool FWD, bool GIDX>
 static void launch_tail(GemmArgs a, int nout, int tail_cols, int tail_splits, hipStream_t stream) {
     a.col_tile0 = nout / BN - tail_cols;
     a.part_cols = tail_cols * BN;
+    if (launch_low_tiles<FWD, GIDX>(a, a.col_tile0, tail_cols, tail_splits, stream)) return;
     launch_tiles<256, 4, FWD, GIDX>(a, dim3(tail_cols, (a.M + 255) / 256, tail_splits), stream);
     if (tail_splits > 1) launch_reduce_cols(a, a.part_cols, nout, a.col_tile0 * BN, tail_splits, stream);
 }
@@ -706,7 +723,7 @@ static hipError_t launch_gemm_wide(GemmArgs a, int nout, int tail_cols, int tail
     a.col_tile0 = 0;
     a.part_cols = nout;
     if constexpr (GIDX) hipLaunchKernelGGL((gemm_kernel<256, 2, FWD, GIDX, 0, 4>), grid, dim3(512), 0, stream, a);
-    else launch_wide_tiles(FWD, a, grid, stream);
+    else launch_wide_tiles(FWD, false, a, grid, stream);
     if (tail_cols > 0) launch_tail<FWD, GIDX>(a, nout, tail_cols, tail_splits, stream);
     return hipGetLastError();
 }
@@ -718,7 +735,8 @@ static hipError_t launch_gemm(GemmArgs a, int nout, int splits, int tail_cols, i
     const int nc = nout / BN, nr = (a.M + BM - 1) / BM;
     a.col_tile0 = 0;
     a.part_cols = nout;
-    launch_tiles<BM, WGM, FWD, GIDX>(a, dim3(nc - tail_cols, nr, splits), stream);
+    const bool low = BM == 256 && launch_low_tiles<FWD, GIDX>(a, 0, nc - tail_cols, splits, stream);
+    if (!low) launch_tiles<BM, WGM, FWD, GIDX>(a, dim3(nc - tail_cols, nr, splits), stream);
     if (splits > 1) {
         const long total = (long)a.M * nout;
         hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream,
@@ -737,10 +755,6 @@ static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout
         default: return launch_gemm<256, 4, FWD, GIDX>(a, nout, p.splits, p.tail_cols, p.tail_splits, stream);   // 256 x 128, 8 wavefronts of 64 x 64
     }
 }
-
-// What TileMap is told: row tile r starts its reduction loop kPhaseStep * r steps later; tiles are ordered in groups
-// of kRowTilesPerGroup row tiles (measured optimum over the benchmark shapes).
-constexpr int kPhaseStep = 2, kRowTilesPerGroup = 2;
 
 }  // namespace q4
 
@@ -898,14 +912,18 @@ extern "C" int q4_launch_gemm_group(int fwd, int n, const void* const* act, cons
     g.n = n;
     const int nr = (M + 255) / 256;
     // `count` column tiles from `first` on, in tiles of 256 x 256 (wide) or 256 x 128
+    bool all256 = true;
+    for (int i = 0; i < n; ++i) all256 = all256 && N[i] % 256 == 0;
     auto launch = [&](bool wide, int first, int count, int splits, int part_cols) {
+        const bool low = fwd && !wide && all256 && first % 2 == 0 && count % 2 == 0;     // see launch_low_tiles
         for (int i = 0; i < kGemmGroup; ++i) {
-            g.layer[i].col_tile0 = first;
+            g.layer[i].col_tile0 = low ? first / 2 : first;
+            g.layer[i].phase_step = kPhaseStep | ((low ? 2 * kRowTilesPerGroup : kRowTilesPerGroup) << 8);
             if (!fwd) g.layer[i].part_cols = part_cols;
-            g.tile_end[i] = ends[wide ? 0 : 1][i];
+            g.tile_end[i] = ends[wide || low ? 0 : 1][i];
         }
-        const dim3 grid(count, nr, splits);
-        if (wide) launch_wide_group_tiles(fwd != 0, g, grid, stream);
+        const dim3 grid(low ? count / 2 : count, low ? (M + 127) / 128 : nr, splits);
+        if (wide || low) launch_wide_group_tiles(fwd != 0, low, g, grid, stream);
         else if (fwd) launch_group_tiles<true>(g, n, grid, stream);
         else launch_group_tiles<false>(g, n, grid, stream);
         if (splits > 1) launch_reduce_cols(g.layer[0], part_cols, K, first * (wide ? 256 : BN), splits, stream);

@@ -108,8 +108,8 @@ struct GemmGroupArgs {
     int n;
 };
 
-// q4_gemm_wide.hip: grids of 256 x 256 tiles
-void launch_wide_tiles(bool fwd, const GemmArgs& a, dim3 grid, hipStream_t stream);
-void launch_wide_group_tiles(bool fwd, const GemmGroupArgs& g, dim3 grid, hipStream_t stream);
+// q4_gemm_wide.hip: grids of 256 x 256 tiles, or of 128 x 256 ones (`low`, forward only)
+void launch_wide_tiles(bool fwd, bool low, const GemmArgs& a, dim3 grid, hipStream_t stream);
+void launch_wide_group_tiles(bool fwd, bool low, const GemmGroupArgs& g, dim3 grid, hipStream_t stream);
 
 }  // namespace q4

@@ -26,6 +26,12 @@
 // us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 115 -> 108.5,
 // 4096 x (5120 -> 13824) 489 -> 468, 4096 x (13824 -> 5120) 480 -> 457; grad-input 115 -> 110, 488 -> 473, 490 -> 476; cycles per
 // step (2048 of them MFMAs) forward 2500, grad-input 2770, at 1.55 and 1.67 GHz.
+//
+// TM = 4, forward: tiles of 128 x 256 for outputs with too few of the large ones (one unsplit round of 256 x 128 tiles of
+// q4_gemm.hip before: the same area, half the activations per weight decoded, but 64 KB of fragment reads per round of 1024 MFMA
+// cycles instead of 128).  us, 256 x 128 with both operands in LDS -> 128 x 256: 2048 x (4096 -> 4096) 66.5 -> 60.4, 512 x (5120 -> 13824)
+// 72.4 -> 65.9, 1536 x (4096 -> 4096) 54.3 -> 49.6, 300 x (4096 -> 11008) 45.7 -> 41.7, the last 88 tiles of 2048 x (4096 -> 11008) 57 -> 51.
+// Grad-input it is level to 2 % slower (2048 x (4096 -> 4096) 66.9 against 66.0): the words turned around serve half the rows.
 #include "q4_gemm_args.hpp"
 
 namespace q4 {
@@ -47,6 +53,14 @@ __device__ __forceinline__ half2_t codes_of_bytes(uint32_t b) {
     return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.f, H != 0));
 }
 __device__ __forceinline__ uint32_t bfi(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
+
+// Keeps a block of accumulators in the accumulation registers: what vector operations make of it goes back there at once, instead
+// of 256 of them drifting into the registers that the loop needs.
+__device__ __forceinline__ void keep_acc(float16_t& a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+a"(a));
+#endif
+}
 
 template <int TM, bool FWD, bool MULTI>
 __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay, const TileMap tm, const StepRange share,
@@ -84,6 +98,137 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    auto keep_all = [&] {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) keep_acc(acc[i][j]);
+    };
+    if constexpr (TM == 8) keep_all();
+
+    // Adapter terms, before the main loop fills the accumulators: operands straight from memory.  Dropout on the adapter input: its
+    // share of out[m, c] exists only where the mask keeps (m, c); the kept values carry 1 / (1 - p) through lb_scale.  The masked
+    // terms of all layers are summed block by block and only written to the accumulators: adding to 256 of them behind the loop
+    // pulled them through the vector registers and spilled (13 us a round instead of 4).
+    auto adapter_here = [&](int li) {                             // the share that holds a layer's first step carries its term
+        if constexpr (!MULTI) return a0.R > 0 && zsplit == 0;
+        int base = 0;
+        for (int l = 0; l < li; ++l) base += layers[l].N / BK;
+        return layers[li].R > 0 && share.begin <= base && base < share.begin + share.cnt;
+    };
+    auto adapter_row = [&](const GemmArgs& a, int i, int ks) {    // columns past R and rows past M read as zero
+        const rsrc_t rl = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
+        return __builtin_bit_cast(half8_t, buf_load128(rl, 16 * ks + 8 * lg < a.R ? ((32 * i + lc) * a.R + 16 * ks + 8 * lg) * 2 : kFar, 0));
+    };
+    // operand of columns cw + 2 lc, + 1, rows 16 ks + 8 lg .. + 7 of the adapter matrix (zero past R)
+    auto adapter_cols = [&](const GemmArgs& a, int ks, half8_t (&b)[2]) {
+        const bool in = 16 * ks + 8 * lg < a.R;
+        const int r0 = in ? 16 * ks + 8 * lg : 0;
+        auto load = [&](auto tag) {
+            using T = decltype(tag);
+            T raw[2][8];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) raw[j][e] = reinterpret_cast<const T*>(a.lb)[(size_t)(r0 + e) * a.lb_sr + (size_t)(cw + 2 * lc + j) * a.lb_sc];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) b[j][e] = in ? (half_t)(a.lb_scale * (float)raw[j][e]) : (half_t)0.f;
+        };
+        if (a.lb_is_f32) load(float{});
+        else load(half_t{});
+    };
+    auto add_adapters = [&] {
+        bool masked = false;
+        for (int li = 0; li < nlay; ++li) masked = masked || (adapter_here(li) && layers[li].drop.thr15 != 0);
+        if (FWD || !masked) {
+#pragma unroll 1
+            for (int li = 0; li < nlay; ++li) {
+                if (!adapter_here(li)) continue;
+                const GemmArgs& a = layers[li];
+#pragma unroll 1
+                for (int ks = 0; 16 * ks < a.R; ++ks) {
+                    half8_t v[TM], b[2];
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) v[i] = adapter_row(a, i, ks);
+                    adapter_cols(a, ks, b);
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[i], b[j], acc[i][j], 0, 0, 0);
+                }
+            }
+            return;
+        }
+        if constexpr (!FWD && TM == 8) {
+            static_assert(kGemmGroup <= 4 && kTile >= 4 * 2 * 256 * 8, "a layer's operands fill one tile");
+            auto operand = [&](int li, int ks, int j) {           // the lane's own
+                half_t* const t = li == 0 ? sA0 : li == 1 ? sA1 : li == 2 ? sA2 : sA3;
+                return reinterpret_cast<half8_t*>(t + ((2 * ks + j) * 256 + threadIdx.x) * 8);
+            };
+            uint32_t here = 0;
+            for (int li = 0; li < nlay; ++li) here |= adapter_here(li) ? 1u << li : 0u;
+            for (int li = 0; li < nlay; ++li)
+                if (here >> li & 1)
+                    for (int ks = 0; 16 * ks < layers[li].R; ++ks) {
+                        half8_t b[2];
+                        adapter_cols(layers[li], ks, b);
+                        *operand(li, ks, 0) = b[0];
+                        *operand(li, ks, 1) = b[1];
+                    }
+            half8_t v[4], next[4];                                // a block's rows, and the following block's on their way
+            auto request = [&](int li, int i) {
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks)
+                    if (ks == 0 || 16 * ks < layers[li].R) next[ks] = adapter_row(layers[li], i, ks);
+            };
+            const int li0 = __builtin_ctz(here);
+            request(li0, 0);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                float16_t sum[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sum[j][r] = 0.f;
+#pragma unroll 1
+                for (uint32_t todo = here; todo; todo &= todo - 1) {
+                    const int li = __builtin_ctz(todo);
+                    const GemmArgs& a = layers[li];
+#pragma unroll
+                    for (int ks = 0; ks < 4; ++ks) v[ks] = next[ks];
+                    if (todo & (todo - 1)) request(__builtin_ctz(todo & (todo - 1)), i);
+                    else if (i + 1 < TM) request(li0, i + 1);
+                    float16_t term[2];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) term[j][r] = 0.f;
+#pragma unroll
+                    for (int ks = 0; ks < 4; ++ks)
+                        if (ks == 0 || 16 * ks < a.R) {
+#pragma unroll
+                            for (int j = 0; j < 2; ++j) term[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[ks], *operand(li, ks, j), term[j], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
+                        const uint32_t dw = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)(cw + 2 * lc) >> 1);
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) sum[j][r] += ((dw >> (16 * j)) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[j][r];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    acc[i][j] = sum[j];
+                    keep_acc(acc[i][j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();                                      // before the loads write over the operands
+        }
+    };
 
     auto run_layer = [&](const GemmArgs& a, const StepRange sr) {
         const int RED = FWD ? a.K : a.N;
@@ -229,7 +374,7 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
             }
         };
         constexpr int kAhead = FWD ? 3 : 4;                       // stage whose words, scales, zeros a step requests
-        constexpr int BAR = TM / 4;                               // slot of the last sub-step behind which the barrier sits
+        constexpr int BAR = TM / 2;                               // slot of the last sub-step behind which the barrier sits
 
         // multiplies stage s (ring position C = s % 4); on entry af[0] and bo[0] hold its sub-step 0
         auto step = [&](int s, auto ct) {
@@ -327,73 +472,14 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         if (s < sr.cnt) step(s, std::integral_constant<int, 0>{});
         if (s + 1 < sr.cnt) step(s + 1, std::integral_constant<int, 1>{});
         if (s + 2 < sr.cnt) step(s + 2, std::integral_constant<int, 2>{});
+        if constexpr (TM == 8) keep_all();
         // nothing on its way into the tiles any more, and every wavefront done with them
         __builtin_amdgcn_s_waitcnt(0x0070);
         __syncthreads();
     };
 
-    // Adapter term: its operands straight from memory, one block of 32 rows at a time, behind the main loop, where its
-    // registers are free.  Dropout on the adapter input: its share of out[m, c] exists only where the mask keeps (m, c); the kept
-    // values carry 1 / (1 - p) through lb_scale.
-    auto add_adapter = [&](const GemmArgs& a) {
-        const rsrc_t rl = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
-        const bool masked = a.drop.thr15 != 0;
-        half8_t lb[4][2];
-        uint4_t v[2][4];
-        auto load_rows = [&](uint4_t* d, int i) {
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)                    // columns past R and rows past M read as zero
-                d[ks] = buf_load128(rl, 16 * ks + 8 * lg < a.R ? ((32 * i + lc) * a.R + 16 * ks + 8 * lg) * 2 : kFar, 0);
-        };
-        load_rows(v[0], 0);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) lb[ks][j] = half8_t{};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int r0 = 16 * ks + 8 * lg;
-            if (r0 < a.R) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        lb[ks][j][e] = (half_t)(a.lb_scale * adapter_at(a, (size_t)(r0 + e) * a.lb_sr + (size_t)(cw + 2 * lc + j) * a.lb_sc));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            float16_t term[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) term[j][r] = 0.f;
-            if (i + 1 < TM) load_rows(v[(i + 1) & 1], i + 1);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-                if (16 * ks < a.R) {                          // uniform
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        term[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, v[i & 1][ks]), lb[ks][j], term[j], 0, 0, 0);
-                }
-            if (masked) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
-                    const uint32_t dw = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)(cw + 2 * lc) >> 1);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) term[j][r] = ((dw >> (16 * j)) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[j][r];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] += term[j][r];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-
     if constexpr (MULTI) {
+        add_adapters();
         int base = 0;
 #pragma unroll 1
         for (int li = 0; li < nlay; ++li) {
@@ -403,15 +489,9 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
             if (lo >= hi) continue;                               // uniform
             run_layer(layers[li], StepRange{lo, hi - lo});
         }
-        base = 0;
-#pragma unroll 1
-        for (int li = 0; li < nlay; ++li) {                       // with the share that holds a layer's first step
-            if (layers[li].R > 0 && share.begin <= base && base < share.begin + share.cnt) add_adapter(layers[li]);
-            base += (FWD ? layers[li].K : layers[li].N) / BK;
-        }
     } else {
+        add_adapters();
         run_layer(a0, share);
-        if (a0.R > 0 && zsplit == 0) add_adapter(a0);
     }
 
     // acc[i][j][r]: row 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, column cw + 2 (lane % 32) + j
@@ -474,12 +554,14 @@ __global__ __launch_bounds__(256) void gemm_wide_group_kernel(GemmGroupArgs g) {
     }
 }
 
-void launch_wide_tiles(bool fwd, const GemmArgs& a, dim3 grid, hipStream_t stream) {
-    if (fwd) hipLaunchKernelGGL((gemm_wide_kernel<8, true>), grid, dim3(256), 0, stream, a);
+void launch_wide_tiles(bool fwd, bool low, const GemmArgs& a, dim3 grid, hipStream_t stream) {
+    if (low) hipLaunchKernelGGL((gemm_wide_kernel<4, true>), grid, dim3(256), 0, stream, a);
+    else if (fwd) hipLaunchKernelGGL((gemm_wide_kernel<8, true>), grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((gemm_wide_kernel<8, false>), grid, dim3(256), 0, stream, a);
 }
-void launch_wide_group_tiles(bool fwd, const GemmGroupArgs& g, dim3 grid, hipStream_t stream) {
-    if (fwd) hipLaunchKernelGGL((gemm_wide_group_kernel<8, true>), grid, dim3(256), 0, stream, g);
+void launch_wide_group_tiles(bool fwd, bool low, const GemmGroupArgs& g, dim3 grid, hipStream_t stream) {
+    if (low) hipLaunchKernelGGL((gemm_wide_group_kernel<4, true>), grid, dim3(256), 0, stream, g);
+    else if (fwd) hipLaunchKernelGGL((gemm_wide_group_kernel<8, true>), grid, dim3(256), 0, stream, g);
     else hipLaunchKernelGGL((gemm_wide_group_kernel<8, false>), grid, dim3(256), 0, stream, g);
 }
 

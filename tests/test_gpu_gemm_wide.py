@@ -1,5 +1,5 @@
 """The tiles of the GEMMs whose operands are built in registers (csrc/q4_gemm_wide.hip) at the edges of their pipeline: reductions
-shorter than, equal to and just past the ring of activation tiles, ragged last row tiles, groups of 64, 128 and 256 rows, adapters
+shorter than, equal to and just past the ring of activation tiles, ragged last row tiles of 256 and of 128 rows, groups of 64, 128 and 256 rows, adapters
 of every number of 16-deep sub-steps in both types, with and without a dropout mask.
 Tolerance: outputs are rounded to fp16 (2^-11 of a value) and weights to fp16 twice (together at most 2^-10 of the largest
 |scale * code|, about twice the largest weight); sums of a few hundred such terms average out to below 2e-3 of the largest output."""
@@ -18,16 +18,16 @@ def _t(a):
 
 
 def _rows(M):
-    return np.unique([0, 1, 31, 32, 127, 128, 255, 256, M - 2, M - 1])
+    return np.unique(np.minimum([0, 1, 31, 32, 127, 128, 255, 256, M - 2, M - 1], M - 1))
 
 
 @pytest.mark.parametrize("red,gs,rank,f32", [(128, 128, 0, False), (128, 64, 8, True), (256, 64, 24, False), (384, 128, 0, True),
                                              (512, 256, 40, True), (640, 128, 64, False)])
-@pytest.mark.parametrize("M", [257, 300, 512])
+@pytest.mark.parametrize("M", [130, 200, 256, 257, 300, 512])
 def test_forward(oracle, M, red, gs, rank, f32):
     import torch
     from alpaca_lora_4bit_amd import quant_hip
-    N = 18432                                     # 72 column tiles, two row tiles: 144 tiles of 256 x 256
+    N = 18432                                     # 72 column tiles: 144 tiles of 256 x 256 from 257 rows on, of 128 x 256 below
     layer = oracle.make_layer(red, N, gs, seed=red + gs)
     t = to_cuda_layer(layer)
     xh = oracle.make_activations(M, red, seed=M)
