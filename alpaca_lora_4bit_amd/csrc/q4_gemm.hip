@@ -690,15 +690,15 @@ static void launch_reduce_cols(const GemmArgs& a, int part_cols, int out_cols, i
                        a.part, a.out, a.M, part_cols, out_cols, col0, splits);
 }
 
-// Forward, sequential groups, an unsplit grid of 256 x 128 tiles over an even number of column tiles: the same area as
-// 128 x 256 tiles of q4_gemm_wide.hip.
+// Forward, sequential groups, a grid of 256 x 128 tiles over an even number of column tiles: the same area, and the same shares of
+// the reduction, as 128 x 256 tiles of q4_gemm_wide.hip.
 template <bool FWD, bool GIDX>
 static bool launch_low_tiles(GemmArgs a, int first, int cols, int splits, hipStream_t stream) {
     if constexpr (!FWD || GIDX) return false;
-    if (splits > 1 || first % 2 != 0 || cols % 2 != 0) return false;
+    if (first % 2 != 0 || cols % 2 != 0) return false;
     a.col_tile0 = first / 2;
     a.phase_step = (a.phase_step & 0xff) | (2 * kRowTilesPerGroup << 8);
-    launch_wide_tiles(true, true, a, dim3(cols / 2, (a.M + 127) / 128), stream);
+    launch_wide_tiles(true, true, a, dim3(cols / 2, (a.M + 127) / 128, splits), stream);
     return true;
 }
 
@@ -707,8 +707,8 @@ template <bool FWD, bool GIDX>
 static void launch_tail(GemmArgs a, int nout, int tail_cols, int tail_splits, hipStream_t stream) {
     a.col_tile0 = nout / BN - tail_cols;
     a.part_cols = tail_cols * BN;
-    if (launch_low_tiles<FWD, GIDX>(a, a.col_tile0, tail_cols, tail_splits, stream)) return;
-    launch_tiles<256, 4, FWD, GIDX>(a, dim3(tail_cols, (a.M + 255) / 256, tail_splits), stream);
+    if (!launch_low_tiles<FWD, GIDX>(a, a.col_tile0, tail_cols, tail_splits, stream))
+        launch_tiles<256, 4, FWD, GIDX>(a, dim3(tail_cols, (a.M + 255) / 256, tail_splits), stream);
     if (tail_splits > 1) launch_reduce_cols(a, a.part_cols, nout, a.col_tile0 * BN, tail_splits, stream);
 }
 
@@ -733,6 +733,11 @@ static hipError_t launch_gemm_wide(GemmArgs a, int nout, int tail_cols, int tail
 template <int BM, int WGM, bool FWD, bool GIDX>
 static hipError_t launch_gemm(GemmArgs a, int nout, int splits, int tail_cols, int tail_splits, hipStream_t stream) {
     const int nc = nout / BN, nr = (a.M + BM - 1) / BM;
+    // whole tiles of 256 columns on both sides (launch_low_tiles), in as many shares as the plan's scratch holds of them
+    if (FWD && !GIDX && BM == 256 && nc % 2 == 0 && tail_cols % 2 == 1) {
+        tail_splits = tail_splits * tail_cols / (tail_cols + 1) > 1 ? tail_splits * tail_cols / (tail_cols + 1) : 1;
+        ++tail_cols;
+    }
     a.col_tile0 = 0;
     a.part_cols = nout;
     const bool low = BM == 256 && launch_low_tiles<FWD, GIDX>(a, 0, nc - tail_cols, splits, stream);
