@@ -87,9 +87,9 @@ struct GemvStreamGroupArgs {
 // the reads, and the atomics, of all of them are under way together.  A workgroup adds its blocks as signed integers and one
 // bias, the largest its share can be: `per` blocks of at most 2^46 (a block saturates at 2^22).  S * per of these, twice, fit in the
 // 56 bits below the arrival count up to 511; above, a share beyond +-2^23 saturates there, and S <= 255 of them fit.
-template <bool ONE, int EB>
+template <bool ONE, int EB, int TEAMS>
 __device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* slab, int n0, int nb, int per, int S) {
-    constexpr int T = 64 * kStreamWaves;
+    constexpr int T = 64 * kStreamWaves * TEAMS;
     const int M = a.M, total = M * 64, ws = M << 6;              // ws: from one wavefront's sums to the next's
     if (EB == 1 && (int)threadIdx.x >= total) return;
     unsigned long long add[EB], old[EB];
@@ -147,42 +147,43 @@ __device__ __forceinline__ void stream_finish(const GemvArgs& a, const float* sl
     }
 }
 
-template <int NG, bool ONE, int EB>
+// TEAMS = 2: eight wavefronts, the blocks of a longer share in turn to the two halves (plan_stream_teams).
+template <int NG, bool ONE, int EB, int TEAMS>
 __device__ __forceinline__ void gemv_stream_body(const GemvArgs& a, const StreamSplit& sa, int n0) {
     extern __shared__ float red[];
     const int M = a.M;
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wit = wave % kStreamWaves;
     const int kk = lane >> 4, c = lane & 15;
     const int block0 = blockIdx.y * sa.nb, nb = ONE ? 1 : min(sa.nb, sa.blocks - block0);
-    float* const slab = ONE ? red : red + kStreamLds / 4;         // ONE: over the tiles, behind a barrier
+    float* const slab = ONE ? red : red + TEAMS * kStreamLds / 4; // ONE: over the tiles, behind a barrier
     float4_t yacc[1][4];
     const GemvArgs* const layers[1] = {&a};
-    stream_blocks<1, NG, ONE>(layers, sa.group_inv, n0, block0, nb, min(a.K >> 7, (block0 + nb) * 2 * kStreamWaves),
-                              reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc, [&](int b) {
+    stream_blocks<1, NG, ONE, TEAMS>(layers, sa.group_inv, n0, block0, nb, min(a.K >> 7, (block0 + nb) * 2 * kStreamWaves),
+                                     reinterpret_cast<half_t*>(red) + wave * 2 * kStreamTile, yacc, [&](int b) {
         if constexpr (ONE) __syncthreads();
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = 4 * kk + r;
             if (m < M)
-                *reinterpret_cast<float4_t*>(slab + (((b * kStreamWaves + wave) * M + m) << 6) + 4 * c) =
+                *reinterpret_cast<float4_t*>(slab + (((b * kStreamWaves + wit) * M + m) << 6) + 4 * c) =
                     float4_t{yacc[0][0][r], yacc[0][1][r], yacc[0][2][r], yacc[0][3][r]};
         }
     });
     __syncthreads();
-    stream_finish<ONE, EB>(a, slab, n0, nb, sa.nb, gridDim.y);
+    stream_finish<ONE, EB, TEAMS>(a, slab, n0, nb, sa.nb, gridDim.y);
 }
 
-template <int NG, bool ONE, int EB>
-__global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_kernel(GemvStreamArgs sa) {
-    gemv_stream_body<NG, ONE, EB>(sa.layer, sa.split, blockIdx.x * kColsPerWave);
+template <int NG, bool ONE, int EB, int TEAMS>
+__global__ __launch_bounds__(64 * kStreamWaves * TEAMS) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_kernel(GemvStreamArgs sa) {
+    gemv_stream_body<NG, ONE, EB, TEAMS>(sa.layer, sa.split, blockIdx.x * kColsPerWave);
 }
-template <int NG, bool ONE, int EB>
-__global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_group_kernel(GemvStreamGroupArgs sa) {
+template <int NG, bool ONE, int EB, int TEAMS>
+__global__ __launch_bounds__(64 * kStreamWaves * TEAMS) __attribute__((amdgpu_waves_per_eu(2))) void gemv_stream_group_kernel(GemvStreamGroupArgs sa) {
     const GemvGroupArgs& g = sa.g;
     const int bx = blockIdx.x;
     const int li = (bx >= g.strip_end[0]) + (bx >= g.strip_end[1]) + (bx >= g.strip_end[2]);      // uniform
-    gemv_stream_body<NG, ONE, EB>(g.layer[li], sa.split, (bx - (li == 0 ? 0 : g.strip_end[li - 1])) * kColsPerWave);
+    gemv_stream_body<NG, ONE, EB, TEAMS>(g.layer[li], sa.split, (bx - (li == 0 ? 0 : g.strip_end[li - 1])) * kColsPerWave);
 }
 
 template <int NSTEP, int GSTEPS, bool TURNS = false>
@@ -1166,19 +1167,27 @@ static void launch_gidx(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds
 static bool whole_chunks(int K, int groupsize) {
     return K % 128 == 0 && (groupsize % 128 == 0 || groupsize == 64 || groupsize == 32);
 }
-template <int NG, bool ONE, int EB>
+template <int NG, bool ONE, int EB, int TEAMS>
 static void launch_stream_eb(const q4::GemvGroupArgs& g, int n, const q4::StreamSplit& split, dim3 grid, size_t lds, hipStream_t stream) {
     using namespace q4;
-    const dim3 block(64 * kStreamWaves);
-    if (n == 1) hipLaunchKernelGGL((gemv_stream_kernel<NG, ONE, EB>), grid, block, lds, stream, GemvStreamArgs{g.layer[0], split});
-    else hipLaunchKernelGGL((gemv_stream_group_kernel<NG, ONE, EB>), grid, block, lds, stream, GemvStreamGroupArgs{g, split});
+    const dim3 block(64 * kStreamWaves * TEAMS);
+    if (n == 1) hipLaunchKernelGGL((gemv_stream_kernel<NG, ONE, EB, TEAMS>), grid, block, lds, stream, GemvStreamArgs{g.layer[0], split});
+    else hipLaunchKernelGGL((gemv_stream_group_kernel<NG, ONE, EB, TEAMS>), grid, block, lds, stream, GemvStreamGroupArgs{g, split});
 }
 template <int NG, bool ONE>
 static void launch_stream_one(const q4::GemvGroupArgs& g, int n, const q4::StreamSplit& split, dim3 grid, size_t lds, hipStream_t stream) {
     const int M = g.layer[0].M;
-    if (M <= 4) launch_stream_eb<NG, ONE, 1>(g, n, split, grid, lds, stream);
-    else if (M <= 8) launch_stream_eb<NG, ONE, 2>(g, n, split, grid, lds, stream);
-    else launch_stream_eb<NG, ONE, 4>(g, n, split, grid, lds, stream);
+    if constexpr (NG == 1 && !ONE) {
+        if (q4::plan_stream_teams(M, split.nb) == 2) {
+            lds += q4::kStreamLds;
+            if (M <= 8) launch_stream_eb<NG, ONE, 1, 2>(g, n, split, grid, lds, stream);
+            else launch_stream_eb<NG, ONE, 2, 2>(g, n, split, grid, lds, stream);
+            return;
+        }
+    }
+    if (M <= 4) launch_stream_eb<NG, ONE, 1, 1>(g, n, split, grid, lds, stream);
+    else if (M <= 8) launch_stream_eb<NG, ONE, 2, 1>(g, n, split, grid, lds, stream);
+    else launch_stream_eb<NG, ONE, 4, 1>(g, n, split, grid, lds, stream);
 }
 template <int NSTEP>
 static void launch_seq_group(const q4::GemvPlan& p, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const q4::GemvGroupArgs& g) {

@@ -42,4 +42,11 @@ inline int plan_stream_blocks(int M, int blocks, int strips, int groupsize) {
     return (fill >= 80 && (share == blocks || M >= 11)) || (fill >= 66 && M >= 13) ? share : least;
 }
 
+// Teams of four wavefronts in a workgroup of gemv_stream_kernel whose share is `nb` blocks, the blocks in turn to the teams: two
+// where the sums of the blocks fit the LDS beside the second team's tiles.  Four wavefronts of one chunk ahead keep 16 KB per compute
+// unit on the way, too little for the latency of HBM; eight twice that.  us, one team / two: q|k|v of 4096 features 10.21 / 9.97 at
+// 16 rows, 11008 -> 4096 9.03 / 8.51 at 12, 9.45 / 8.99 at 16.  (Gate, up and activation in one launch move twice the words per chunk and
+// are level with two teams at 16 rows, 0.9 us slower at 4.)
+inline int plan_stream_teams(int M, int nb) { return nb >= 2 && stream_slab_bytes(M, nb) <= 96 * 1024 ? 2 : 1; }
+
 }  // namespace q4

@@ -32,11 +32,12 @@ inline uint32_t stream_group_inv(int groupsize) {
 // The reduction goes in blocks of 8 chunks, two neighbouring chunks per wavefront; `flush(b)` follows block b of the nb blocks
 // from `block0` on with the sums of this wavefront's two chunks in yacc[layer][j][r]: row 4 * (lane / 16) + r, column
 // n0 + 4 * (lane % 16) + j.  Chunks from `end` on are left out.  The layers share x, M, K, N and the group size.
+// TEAMS: teams of four wavefronts that take the blocks in turn, team t the blocks t, t + TEAMS, ... of the nb.
 // NG groups per chunk (1, 2, 4; 1: groupsize % 128 == 0).  `tile`: this wavefront's two activation tiles in LDS.  ONE: a single
 // block, in straight line and with nothing requested past it.
 // The operands are built as in gemv_core: codes as 1024 + q or 64 + q, and per group (sum x*(offset + q) - sum x*offset) -
 // (z + 1) * sum x in the same order.
-template <int NL, int NG, bool ONE, typename Flush>
+template <int NL, int NG, bool ONE, int TEAMS = 1, typename Flush>
 __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], uint32_t inv, int n0, int block0, int nb, int end,
                                               half_t* tile, float4_t (&yacc)[NL][4], Flush&& flush) {
     typedef __attribute__((address_space(3))) void lds_void;
@@ -175,7 +176,8 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
     };
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
-    int i = (block0 * kStreamWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), team = TEAMS > 1 ? wave / kStreamWaves : 0;
+    int i = ((block0 + team) * kStreamWaves + wave % kStreamWaves) * 2;
     load_x(i, 0);
     __builtin_amdgcn_sched_barrier(0);
     load_w(S0{}, i);
@@ -186,9 +188,9 @@ __device__ __forceinline__ void stream_blocks(const GemvArgs* const (&l)[NL], ui
         return;
     }
     // one copy of the two steps: with copies of their own for the last ones a launch took 0.2 to 1.2 us longer
-    for (int b = 0; b < nb; ++b) {
+    for (int b = team; b < nb; b += TEAMS) {
         step(S0{}, std::true_type{}, i + 1);
-        i += 2 * kStreamWaves;
+        i += 2 * kStreamWaves * TEAMS;
         step(S1{}, std::true_type{}, i);
         flush(b);
     }

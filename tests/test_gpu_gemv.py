@@ -365,3 +365,27 @@ def test_long_reductions_of_odd_chunks(oracle, route, K, gs, M):
     ref = oracle.matmul_recons(x, layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
     assert rel_err(y.cpu().numpy(), ref) <= 3e-3             # the gathering kernel multiplies fp16 weights
     assert quant_hip.workspaces_are_zero()
+
+
+@pytest.mark.parametrize("K", [3072, 5120, 7168])      # shares of 3 and 5 blocks in two teams, of 7 (their sums beyond the LDS) in one
+@pytest.mark.parametrize("M", [7, 8, 9, 16])
+def test_longer_shares_in_two_teams_have_the_bits_of_single_blocks(oracle, K, M):
+    """216 strips at 7 rows and more: one workgroup takes the whole reduction, its blocks in turn to two teams of wavefronts.  Up to
+    four rows every block has a workgroup of its own; the sums of a row are the same integers either way."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    N = 13824
+    layer = oracle.make_layer(K, N, 128, seed=K + M)
+    t = to_cuda_layer(layer)
+    xh = oracle.make_activations(M, K, seed=M)
+    x = torch.from_numpy(xh).cuda()
+    args = (t["qweight"], t["qzeros"], t["scales"], None, 128)
+    y = quant_hip.gemv(x, *args)
+    for lo in range(0, M, 4):
+        assert torch.equal(y[lo:lo + 4], quant_hip.gemv(x[lo:lo + 4].contiguous(), *args))
+    assert torch.equal(y, quant_hip.gemv(x, *args))
+    grouped = quant_hip.gemv_grouped(x, [(t["qweight"], t["qzeros"], t["scales"])], 128)[0]
+    assert torch.equal(y, grouped)
+    rows = [0, M - 1]
+    ref = oracle.matmul_recons(xh[rows], layer["qweight"], layer["qzeros"], layer["scales"], layer["g_idx"])
+    assert rel_err(y.cpu().numpy()[rows], ref) <= 2e-3
