@@ -61,6 +61,13 @@ __device__ __forceinline__ void unpack8_natural(uint32_t w, half2_t out[4]) {
     out[3] = codes_to_half2(__builtin_amdgcn_perm(hi, lo, 0x0c070c03u));
 }
 
+// Codes in bytes 2H, 2H + 1 of `b` as two fp16 values.  The byte 0x0q read as an 8-bit float of 4 exponent and 3 mantissa bits
+// is q * 2^-9 for every q of 0..15 (the first binade continues the subnormals), so one conversion scaled by 2^9 yields the codes.
+template <int H>
+__device__ __forceinline__ half2_t codes_of_bytes(uint32_t b) {
+    return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.f, H != 0));
+}
+
 // Buffer-resource loads: a 32-bit byte offset per lane plus a uniform byte offset; an access
 // past `bytes` returns zero instead of faulting, so tiles need no per-lane bounds branches.
 constexpr int kRsrcFlags = 0x00020000;

@@ -46,12 +46,6 @@ constexpr int kStages = 4;               // activation tiles in LDS: one being m
 constexpr int kWideCols = 256;
 constexpr int kFar = 0x70000000;         // beyond every buffer: reads as zero, without traffic
 
-// Codes in bytes 2H, 2H + 1 of `b` as two fp16 values.  The byte 0x0q read as an 8-bit float of 4 exponent and 3 mantissa bits
-// is q * 2^-9 for every q of 0..15 (the first binade continues the subnormals), so one conversion scaled by 2^9 yields the codes.
-template <int H>
-__device__ __forceinline__ half2_t codes_of_bytes(uint32_t b) {
-    return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b, 512.f, H != 0));
-}
 __device__ __forceinline__ uint32_t bfi(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
 
 // Keeps a block of accumulators in the accumulation registers: what vector operations make of it goes back there at once, instead
