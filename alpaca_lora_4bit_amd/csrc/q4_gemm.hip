@@ -2,9 +2,13 @@
 //   forward   y [M,N] = x  [M,K] @ W      (+ bias) (+ xa  [M,R] @ lora_bt [R,N])
 //   backward  dx[M,K] = dy [M,N] @ W^T             (+ dyb [M,R] @ lora_a  [R,K])
 // W is never materialised in HBM: each workgroup dequantizes the [64 x 128] slab of W its
-// current step needs straight into LDS, with the reference's three fp16 roundings
-// (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151), so the product equals
-// torch.matmul(x, recons(W)) of matmul_utils_4bit.py:122-126 up to fp32 summation order.
+// current step needs straight into LDS, so the product is torch.matmul(x, recons(W)) of
+// matmul_utils_4bit.py:122-126.  Weights are rn16(s * q - rn16(s * (z + 1))), one rounding less than
+// the reference's (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151): codes to bytes, then
+// one conversion and one fused multiply-add per pair (codes_of_bytes).  With per-row groups the
+// reference's three roundings.  Against the form that ORs the codes into 1024.0 and multiplies, subtracts
+// and rounds apart, us: grad-input 2048 x (4096 -> 4096) 67.8 -> 66.7, 512 x (5120 -> 13824) 83.0 -> 81.1,
+// 100 x (11008 -> 4096) 30.8 -> 30.0; forward 100 x (11008 -> 4096) 22.8 -> 21.3.
 //
 // Tiling.  A workgroup computes a BM x 128 output tile with 2*WGM wavefronts (WGM along M, 2
 // along N), each owning (BM/WGM) x 64 outputs as (BM/WGM/32) x 2 accumulators of
@@ -38,15 +42,6 @@ namespace q4 {
 
 constexpr int LDS_STRIDE = BK + 8;   // halves
 
-// rn16(rn16(s*q) - zero) for a pair of codes given as (0x6400 | q): one fused multiply-add
-// computes s*(1024+q) - 1024*s = s*q with a single rounding (1024*s is exact), i.e. exactly
-// rn16(s*q); the subtraction of the zero term is the third rounding.  Needs |s| < 64 so that
-// 1024*s does not overflow (checked on the host; larger scales take the unfused path).
-__device__ __forceinline__ half2_t dequant_pair_magic(uint32_t codes_or_magic, half2_t s, half2_t s1024, half2_t zero) {
-    const half2_t p = __builtin_elementwise_fma(as_half2(codes_or_magic), s, -s1024);
-    return p - zero;
-}
-
 struct SlabRsrc {
     rsrc_t w, s, z;
 };
@@ -67,7 +62,7 @@ struct FwdSlab {
     uint32_t w[NW];
     uint32_t s_raw;  // fp16 bits of the scale of (current group, own column); decoded in the slices
     uint32_t z_raw;  // packed zero word holding the own column's code
-    uint32_t o[4];
+    uint32_t o[4], bytes[2];
     int col, wr0;    // column 0..127 of the tile; first word-row within the slab, then +WSTEP per word
     int voff_w, voff_s, voff_z, wstride;
     __device__ __forceinline__ void init(int t, const GemmArgs& a, int n0) {
@@ -94,13 +89,12 @@ struct FwdSlab {
         static_for<0, kLoads>([&](auto ic) { load_part<decltype(ic)::value>(a, r, kred0); });
     }
     // what the slices of a step need of (scale, zero) of the step's group, computed once per group change
-    struct Prep { half2_t s2, zero2, s1024; };
+    struct Prep { half2_t s2, zero2; };
     __device__ __forceinline__ Prep make_prep(int n0) const {
         Prep pr;
         pr.s2 = as_half2(s_raw | (s_raw << 16));
         const uint32_t z_cur = (z_raw >> (((n0 + col) & 7) * 4)) & 0xFu;
         pr.zero2 = zero_term(pr.s2, z_cur, z_cur);
-        pr.s1024 = pr.s2 * half2_t{(half_t)1024.f, (half_t)1024.f};
         return pr;
     }
     template <int I>
@@ -131,10 +125,13 @@ struct FwdSlab {
             }
         } else {
             constexpr int i = I / 4, p = I % 4;
-            const uint32_t lo = w[i] & 0x0F0F0F0Fu;          // bytes e0 e2 e4 e6
-            const uint32_t hi = (w[i] >> 4) & 0x0F0F0F0Fu;   // bytes e1 e3 e5 e7
-            const uint32_t codes = __builtin_amdgcn_perm(hi, lo, 0x0c040c00u + 0x00010001u * p) | kMagic;
-            o[p] = as_u32(dequant_pair_magic(codes, pr.s2, pr.s1024, pr.zero2));
+            if constexpr (p == 0) {
+                const uint32_t lo = w[i] & 0x0F0F0F0Fu;          // bytes e0 e2 e4 e6
+                const uint32_t hi = (w[i] >> 4) & 0x0F0F0F0Fu;   // bytes e1 e3 e5 e7
+                bytes[0] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+                bytes[1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+            }
+            o[p] = as_u32(__builtin_elementwise_fma(codes_of_bytes<p & 1>(bytes[p >> 1]), pr.s2, -pr.zero2));
             if constexpr (p == 3)
                 *reinterpret_cast<uint4_t*>(sB + col * LDS_STRIDE + 8 * (wr0 + WSTEP * i)) = uint4_t{o[0], o[1], o[2], o[3]};
         }
@@ -166,6 +163,7 @@ struct BwdSlab {
     uint4_t w;
     uint2_t sv;
     uint32_t zw, o01;
+    uint32_t bytes[2][2];                         // [column pair][parity of the row]
     uint4_t tv;                                   // TAB: (s01, zero01, s23, zero23) of this thread's four columns
     int wr, n4, e0;
     int voff_w, voff_s, voff_z;
@@ -226,13 +224,14 @@ struct BwdSlab {
             // row e = e0 + I/2 with e0 in {0, 4}: odd/even nibble and byte-in-half are compile-time,
             // the half of the word (e0) is a per-thread shift by 0 or 16 bits
             constexpr int el = I / 2, h = I % 2, b = el >> 1;
-            constexpr uint32_t sel = 0x0c000c00u | ((4u + b) << 16) | (uint32_t)b;
             const int e = e0 + el;
             const uint32_t z4 = zw >> zsh;
-            const uint32_t wa = (h ? w.z : w.x) >> (4 * e0), wb = (h ? w.w : w.y) >> (4 * e0);   // the two columns of this piece
-            const uint32_t na = (el & 1) ? ((wa >> 4) & 0x0F0F0F0Fu) : (wa & 0x0F0F0F0Fu);
-            const uint32_t nb = (el & 1) ? ((wb >> 4) & 0x0F0F0F0Fu) : (wb & 0x0F0F0F0Fu);
-            const uint32_t codes = __builtin_amdgcn_perm(nb, na, sel) | kMagic;  // (code of column a, of column b) of row e
+            if constexpr ((b & 1) == 0) {             // codes of columns (a, b) of rows el and el + 2 as bytes
+                const uint32_t wa = (h ? w.z : w.x) >> (4 * e0), wb = (h ? w.w : w.y) >> (4 * e0);
+                const uint32_t na = (el & 1) ? ((wa >> 4) & 0x0F0F0F0Fu) : (wa & 0x0F0F0F0Fu);
+                const uint32_t nb = (el & 1) ? ((wb >> 4) & 0x0F0F0F0Fu) : (wb & 0x0F0F0F0Fu);
+                bytes[h][el & 1] = __builtin_amdgcn_perm(nb, na, b ? 0x07030602u : 0x05010400u);
+            }
             half2_t s2, zero2;
             if constexpr (TAB) {
                 s2 = as_half2(h ? tv.z : tv.x);
@@ -241,7 +240,7 @@ struct BwdSlab {
                 s2 = as_half2(h ? sv.y : sv.x);
                 zero2 = zero_term(s2, (z4 >> (8 * h)) & 0xFu, (z4 >> (8 * h + 4)) & 0xFu);
             }
-            const uint32_t r = as_u32(dequant_pair_magic(codes, s2, s2 * k1024, zero2));
+            const uint32_t r = as_u32(__builtin_elementwise_fma(codes_of_bytes<b & 1>(bytes[h][el & 1]), s2, -zero2));
             if constexpr (h == 0) o01 = r;
             else *reinterpret_cast<uint2_t*>(sB + (8 * wr + e) * LDS_STRIDE + 4 * n4) = uint2_t{o01, r};
         }
