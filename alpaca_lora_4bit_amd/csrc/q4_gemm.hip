@@ -3,12 +3,13 @@
 //   backward  dx[M,K] = dy [M,N] @ W^T             (+ dyb [M,R] @ lora_a  [R,K])
 // W is never materialised in HBM: each workgroup dequantizes the [64 x 128] slab of W its
 // current step needs straight into LDS, so the product is torch.matmul(x, recons(W)) of
-// matmul_utils_4bit.py:122-126.  Weights are rn16(s * q - rn16(s * (z + 1))), one rounding less than
-// the reference's (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151): codes to bytes, then
-// one conversion and one fused multiply-add per pair (codes_of_bytes).  With per-row groups the
-// reference's three roundings.  Against the form that ORs the codes into 1024.0 and multiplies, subtracts
-// and rounds apart, us: grad-input 2048 x (4096 -> 4096) 67.8 -> 66.7, 512 x (5120 -> 13824) 83.0 -> 81.1,
-// 100 x (11008 -> 4096) 30.8 -> 30.0; forward 100 x (11008 -> 4096) 22.8 -> 21.3.
+// matmul_utils_4bit.py:122-126.  Forward weights have the reference's three fp16 roundings
+// (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151): a small model's logits then follow those of
+// the dense fp16 model, also where its attention amplifies the last bit.  Grad-input weights are
+// rn16(s * q - rn16(s * (z + 1))), one rounding less: codes to bytes, then one conversion and one fused
+// multiply-add per pair (codes_of_bytes).  Against the form that ORs the codes into 1024.0 and multiplies,
+// subtracts and rounds apart, us: grad-input 2048 x (4096 -> 4096) 67.8 -> 66.7, 512 x (5120 -> 13824)
+// 83.0 -> 81.1, 100 x (11008 -> 4096) 30.8 -> 30.0.
 //
 // Tiling.  A workgroup computes a BM x 128 output tile with 2*WGM wavefronts (WGM along M, 2
 // along N), each owning (BM/WGM) x 64 outputs as (BM/WGM/32) x 2 accumulators of
@@ -42,6 +43,15 @@ namespace q4 {
 
 constexpr int LDS_STRIDE = BK + 8;   // halves
 
+// rn16(rn16(s*q) - zero) for a pair of codes given as (0x6400 | q): one fused multiply-add
+// computes s*(1024+q) - 1024*s = s*q with a single rounding (1024*s is exact), i.e. exactly
+// rn16(s*q); the subtraction of the zero term is the third rounding.  Needs |s| < 64 so that
+// 1024*s does not overflow (checked on the host; larger scales take the unfused path).
+__device__ __forceinline__ half2_t dequant_pair_magic(uint32_t codes_or_magic, half2_t s, half2_t s1024, half2_t zero) {
+    const half2_t p = __builtin_elementwise_fma(as_half2(codes_or_magic), s, -s1024);
+    return p - zero;
+}
+
 struct SlabRsrc {
     rsrc_t w, s, z;
 };
@@ -62,7 +72,7 @@ struct FwdSlab {
     uint32_t w[NW];
     uint32_t s_raw;  // fp16 bits of the scale of (current group, own column); decoded in the slices
     uint32_t z_raw;  // packed zero word holding the own column's code
-    uint32_t o[4], bytes[2];
+    uint32_t o[4];
     int col, wr0;    // column 0..127 of the tile; first word-row within the slab, then +WSTEP per word
     int voff_w, voff_s, voff_z, wstride;
     __device__ __forceinline__ void init(int t, const GemmArgs& a, int n0) {
@@ -89,12 +99,13 @@ struct FwdSlab {
         static_for<0, kLoads>([&](auto ic) { load_part<decltype(ic)::value>(a, r, kred0); });
     }
     // what the slices of a step need of (scale, zero) of the step's group, computed once per group change
-    struct Prep { half2_t s2, zero2; };
+    struct Prep { half2_t s2, zero2, s1024; };
     __device__ __forceinline__ Prep make_prep(int n0) const {
         Prep pr;
         pr.s2 = as_half2(s_raw | (s_raw << 16));
         const uint32_t z_cur = (z_raw >> (((n0 + col) & 7) * 4)) & 0xFu;
         pr.zero2 = zero_term(pr.s2, z_cur, z_cur);
+        pr.s1024 = pr.s2 * half2_t{(half_t)1024.f, (half_t)1024.f};
         return pr;
     }
     template <int I>
@@ -125,13 +136,10 @@ struct FwdSlab {
             }
         } else {
             constexpr int i = I / 4, p = I % 4;
-            if constexpr (p == 0) {
-                const uint32_t lo = w[i] & 0x0F0F0F0Fu;          // bytes e0 e2 e4 e6
-                const uint32_t hi = (w[i] >> 4) & 0x0F0F0F0Fu;   // bytes e1 e3 e5 e7
-                bytes[0] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-                bytes[1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-            }
-            o[p] = as_u32(__builtin_elementwise_fma(codes_of_bytes<p & 1>(bytes[p >> 1]), pr.s2, -pr.zero2));
+            const uint32_t lo = w[i] & 0x0F0F0F0Fu;          // bytes e0 e2 e4 e6
+            const uint32_t hi = (w[i] >> 4) & 0x0F0F0F0Fu;   // bytes e1 e3 e5 e7
+            const uint32_t codes = __builtin_amdgcn_perm(hi, lo, 0x0c040c00u + 0x00010001u * p) | kMagic;
+            o[p] = as_u32(dequant_pair_magic(codes, pr.s2, pr.s1024, pr.zero2));
             if constexpr (p == 3)
                 *reinterpret_cast<uint4_t*>(sB + col * LDS_STRIDE + 8 * (wr0 + WSTEP * i)) = uint4_t{o[0], o[1], o[2], o[3]};
         }
