@@ -370,13 +370,17 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         constexpr int kAhead = FWD ? 3 : 4;                       // stage whose words, scales, zeros a step requests
         constexpr int BAR = TM / 2;                               // slot of the last sub-step behind which the barrier sits
 
-        // multiplies stage s (ring position C = s % 4); on entry af[0] and bo[0] hold its sub-step 0
-        auto step = [&](int s, auto ct) {
-            constexpr int C = decltype(ct)::value;
+        // multiplies stage s (ring position C = s % 4); on entry af[0] and bo[0] hold its sub-step 0.  LEFT: most steps that can
+        // follow it.  The last three (LEFT < 3) request nothing, and their barriers await everything: a counted wait holds only
+        // while every request of the last two steps exists, and the compiler deletes those to registers that no later step reads.
+        auto step = [&](int s, auto ct, auto leftt) {
+            constexpr int C = decltype(ct)::value, LEFT = decltype(leftt)::value;
+            constexpr bool more = LEFT >= 3;
             const int red3 = red_of(s + 3, sr, phase), redx = red_of(s + kAhead, sr, phase);
             static_for<0, KS>([&](auto kt) {
                 constexpr int ks = decltype(kt)::value, kn = (ks + 1) % KS;
                 constexpr int sn = ks + 1 == KS ? C + 1 : C;      // stage of the operands built in this sub-step
+                constexpr bool next = LEFT > 0 || ks + 1 < KS;    // whether there can be such a stage
                 static_for<0, NMK>([&](auto it) {
                     constexpr int i = decltype(it)::value, g = ks * NMK + i;
                     acc[i / 2][i % 2] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks & 1][i / 2],
@@ -386,16 +390,17 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                     constexpr int SL = 3 * NMK;
                     static_for<0, kLoads>([&](auto lt) {
                         constexpr int l = decltype(lt)::value;
-                        if constexpr (l * SL / kLoads == g) {
+                        if constexpr (more && l * SL / kLoads == g) {
                             if constexpr (l < kOther) load_other(std::integral_constant<int, C + kAhead>{}, lt, redx);
                             else load_a(stage_ptr(std::integral_constant<int, C + 3>{}), l - kOther, red3);
                         }
                     });
                     // activation fragments of the next sub-step
                     constexpr int first = ks + 1 == KS ? BAR + 1 : 0, span = NMK - 1 - first;
-                    if constexpr (ks + 1 == KS && i == BAR) {
+                    if constexpr (next && ks + 1 == KS && i == BAR) {
+                        constexpr int kYounger = more ? 2 * kLoads : 0;     // requested since the next stage's activations
                         __builtin_amdgcn_sched_barrier(0);
-                        __builtin_amdgcn_s_waitcnt(0x0070 | ((2 * kLoads) & 15) | (((2 * kLoads) >> 4) << 14));
+                        __builtin_amdgcn_s_waitcnt(0x0070 | (kYounger & 15) | ((kYounger >> 4) << 14));
                         asm volatile("" ::: "memory");
                         __builtin_amdgcn_s_barrier();
                         asm volatile("" ::: "memory");
@@ -403,23 +408,23 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                     }
                     static_for<0, TM>([&](auto rt) {
                         constexpr int r = decltype(rt)::value;
-                        if constexpr (first + r * span / TM == i)
+                        if constexpr (next && first + r * span / TM == i)
                             af[kn & 1][r] = *reinterpret_cast<const half8_t*>(stage_ptr(std::integral_constant<int, sn>{}) + fo[kn] + r * 32 * BK);
                     });
                     // operands of the next sub-step
                     if constexpr (FWD) {
-                        if constexpr (ks + 1 == KS && i == 0) prep(sraw[(C + 1) & 3], zraw[(C + 1) & 3]);
+                        if constexpr (next && ks + 1 == KS && i == 0) prep(sraw[(C + 1) & 3], zraw[(C + 1) & 3]);
                     } else {
-                        if constexpr (i == 0) read_sz(std::integral_constant<int, ks + 2 >= KS ? C + 1 : C>{}, std::integral_constant<int, (ks + 2) % KS>{});
-                        if constexpr (ks == KS - 2 && i == 1) read_t(std::integral_constant<int, C + 1>{});
+                        if constexpr (i == 0 && (LEFT > 0 || ks + 2 < KS)) read_sz(std::integral_constant<int, ks + 2 >= KS ? C + 1 : C>{}, std::integral_constant<int, (ks + 2) % KS>{});
+                        if constexpr (LEFT > 0 && ks == KS - 2 && i == 1) read_t(std::integral_constant<int, C + 1>{});
                         static_for<0, kTurns>([&](auto qt) {      // words of stage s + 2
                             constexpr int q = decltype(qt)::value;
-                            if constexpr (NMK / 2 + q * 2 * NMK / kTurns == g) turn(std::integral_constant<int, C + 2>{}, std::integral_constant<int, C>{}, qt);
+                            if constexpr (LEFT > 1 && NMK / 2 + q * 2 * NMK / kTurns == g) turn(std::integral_constant<int, C + 2>{}, std::integral_constant<int, C>{}, qt);
                         });
                     }
                     static_for<0, 12>([&](auto ut) {
                         constexpr int u = decltype(ut)::value;
-                        if constexpr (u * (NMK - 1) / 12 == i) build(std::integral_constant<int, sn>{}, std::integral_constant<int, kn>{}, ut);
+                        if constexpr (next && u * (NMK - 1) / 12 == i) build(std::integral_constant<int, sn>{}, std::integral_constant<int, kn>{}, ut);
                     });
                     __builtin_amdgcn_sched_barrier(0);
                 });
@@ -458,14 +463,14 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         __builtin_amdgcn_sched_barrier(0);
         int s = 0;
         for (; s + 4 <= sr.cnt; s += 4) {
-            step(s, std::integral_constant<int, 0>{});
-            step(s + 1, std::integral_constant<int, 1>{});
-            step(s + 2, std::integral_constant<int, 2>{});
-            step(s + 3, std::integral_constant<int, 3>{});
+            step(s, std::integral_constant<int, 0>{}, std::integral_constant<int, 3>{});
+            step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 3>{});
+            step(s + 2, std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+            step(s + 3, std::integral_constant<int, 3>{}, std::integral_constant<int, 3>{});
         }
-        if (s < sr.cnt) step(s, std::integral_constant<int, 0>{});
-        if (s + 1 < sr.cnt) step(s + 1, std::integral_constant<int, 1>{});
-        if (s + 2 < sr.cnt) step(s + 2, std::integral_constant<int, 2>{});
+        if (s < sr.cnt) step(s, std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{});
+        if (s + 1 < sr.cnt) step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+        if (s + 2 < sr.cnt) step(s + 2, std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
         if constexpr (TM == 8) keep_all();
         // nothing on its way into the tiles any more, and every wavefront done with them
         __builtin_amdgcn_s_waitcnt(0x0070);
