@@ -46,6 +46,14 @@ constexpr int kStages = 4;               // activation tiles in LDS: one being m
 constexpr int kWideCols = 256;
 constexpr int kFar = 0x70000000;         // beyond every buffer: reads as zero, without traffic
 
+// Of `n` pieces of work spread over `span` places the first that goes to place i or a later one: piece l goes to place
+// l * span / n.
+constexpr int first_piece(int i, int n, int span) { return i <= 0 ? 0 : i >= span ? n : (i * n + span - 1) / span; }
+template <int I, int N, int SPAN, typename F>
+__device__ __forceinline__ void pieces_of(F&& f) {
+    static_for<first_piece(I, N, SPAN), first_piece(I + 1, N, SPAN)>(f);
+}
+
 __device__ __forceinline__ uint32_t bfi(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
 
 // Keeps a block of accumulators in the accumulation registers: what vector operations make of it goes back there at once, instead
@@ -388,12 +396,10 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                         acc[i / 2][i % 2], 0, 0, 0);
                     // requests, one at a time over the first three sub-steps
                     constexpr int SL = 3 * NMK;
-                    static_for<0, kLoads>([&](auto lt) {
+                    if constexpr (more) pieces_of<g, kLoads, SL>([&](auto lt) {
                         constexpr int l = decltype(lt)::value;
-                        if constexpr (more && l * SL / kLoads == g) {
-                            if constexpr (l < kOther) load_other(std::integral_constant<int, C + kAhead>{}, lt, redx);
-                            else load_a(stage_ptr(std::integral_constant<int, C + 3>{}), l - kOther, red3);
-                        }
+                        if constexpr (l < kOther) load_other(std::integral_constant<int, C + kAhead>{}, lt, redx);
+                        else load_a(stage_ptr(std::integral_constant<int, C + 3>{}), l - kOther, red3);
                     });
                     // activation fragments of the next sub-step
                     constexpr int first = ks + 1 == KS ? BAR + 1 : 0, span = NMK - 1 - first;
@@ -406,10 +412,9 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                         asm volatile("" ::: "memory");
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    static_for<0, TM>([&](auto rt) {
+                    if constexpr (next) pieces_of<i - first, TM, span>([&](auto rt) {
                         constexpr int r = decltype(rt)::value;
-                        if constexpr (next && first + r * span / TM == i)
-                            af[kn & 1][r] = *reinterpret_cast<const half8_t*>(stage_ptr(std::integral_constant<int, sn>{}) + fo[kn] + r * 32 * BK);
+                        af[kn & 1][r] = *reinterpret_cast<const half8_t*>(stage_ptr(std::integral_constant<int, sn>{}) + fo[kn] + r * 32 * BK);
                     });
                     // operands of the next sub-step
                     if constexpr (FWD) {
@@ -417,14 +422,12 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                     } else {
                         if constexpr (i == 0 && (LEFT > 0 || ks + 2 < KS)) read_sz(std::integral_constant<int, ks + 2 >= KS ? C + 1 : C>{}, std::integral_constant<int, (ks + 2) % KS>{});
                         if constexpr (LEFT > 0 && ks == KS - 2 && i == 1) read_t(std::integral_constant<int, C + 1>{});
-                        static_for<0, kTurns>([&](auto qt) {      // words of stage s + 2
-                            constexpr int q = decltype(qt)::value;
-                            if constexpr (LEFT > 1 && NMK / 2 + q * 2 * NMK / kTurns == g) turn(std::integral_constant<int, C + 2>{}, std::integral_constant<int, C>{}, qt);
+                        if constexpr (LEFT > 1) pieces_of<g - NMK / 2, kTurns, 2 * NMK>([&](auto qt) {      // words of stage s + 2
+                            turn(std::integral_constant<int, C + 2>{}, std::integral_constant<int, C>{}, qt);
                         });
                     }
-                    static_for<0, 12>([&](auto ut) {
-                        constexpr int u = decltype(ut)::value;
-                        if constexpr (next && u * (NMK - 1) / 12 == i) build(std::integral_constant<int, sn>{}, std::integral_constant<int, kn>{}, ut);
+                    if constexpr (next) pieces_of<i, 12, NMK - 1>([&](auto ut) {
+                        build(std::integral_constant<int, sn>{}, std::integral_constant<int, kn>{}, ut);
                     });
                     __builtin_amdgcn_sched_barrier(0);
                 });
