@@ -37,7 +37,9 @@ __device__ __forceinline__ half2_t codes_to_half2(uint32_t packed_codes) {
     return as_half2(packed_codes | kMagic) - k1024;
 }
 
-// Three-rounding dequant of a pair: rn16(rn16(s*q) - zero), zero = rn16(s*(z+1)) precomputed.
+// Three-rounding dequant of a pair: rn16(rn16(s*q) - zero), zero = rn16(s*(z+1)) precomputed.  Product and difference are
+// rounded apart in every kernel: a weight at its zero point, q = z + 1, is then exactly zero.  One fused multiply-add would
+// leave it the rounding error of the zero term, the same for all such weights of a group and column.
 __device__ __forceinline__ half2_t dequant_pair(half2_t q, half2_t s, half2_t zero) {
     half2_t p = s * q;
     return p - zero;

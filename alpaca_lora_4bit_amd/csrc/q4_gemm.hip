@@ -3,13 +3,11 @@
 //   backward  dx[M,K] = dy [M,N] @ W^T             (+ dyb [M,R] @ lora_a  [R,K])
 // W is never materialised in HBM: each workgroup dequantizes the [64 x 128] slab of W its
 // current step needs straight into LDS, so the product is torch.matmul(x, recons(W)) of
-// matmul_utils_4bit.py:122-126.  Forward weights have the reference's three fp16 roundings
-// (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151): a small model's logits then follow those of
-// the dense fp16 model, also where its attention amplifies the last bit.  Grad-input weights are
-// rn16(s * q - rn16(s * (z + 1))), one rounding less: codes to bytes, then one conversion and one fused
-// multiply-add per pair (codes_of_bytes).  Against the form that ORs the codes into 1024.0 and multiplies,
-// subtracts and rounds apart, us: grad-input 2048 x (4096 -> 4096) 67.8 -> 66.7, 512 x (5120 -> 13824)
-// 83.0 -> 81.1, 100 x (11008 -> 4096) 30.8 -> 30.0.
+// matmul_utils_4bit.py:122-126.  The weights have the reference's three fp16 roundings
+// (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151), here and in q4_gemm_wide.hip, both directions: what a
+// product multiplies does not depend on the kernel that its sizes lead to.  Forward ORs the codes into 1024.0 and takes the
+// offset off in the product; grad-input turns them into bytes and converts (codes_of_bytes), us: 2048 x (4096 -> 4096)
+// 69.5 -> 69.1, 512 x (5120 -> 13824) 83.0 -> 82.5, 100 x (11008 -> 4096) 31.1 -> 30.8.
 //
 // Tiling.  A workgroup computes a BM x 128 output tile with 2*WGM wavefronts (WGM along M, 2
 // along N), each owning (BM/WGM) x 64 outputs as (BM/WGM/32) x 2 accumulators of
@@ -248,7 +246,7 @@ struct BwdSlab {
                 s2 = as_half2(h ? sv.y : sv.x);
                 zero2 = zero_term(s2, (z4 >> (8 * h)) & 0xFu, (z4 >> (8 * h + 4)) & 0xFu);
             }
-            const uint32_t r = as_u32(__builtin_elementwise_fma(codes_of_bytes<b & 1>(bytes[h][el & 1]), s2, -zero2));
+            const uint32_t r = as_u32(dequant_pair(codes_of_bytes<b & 1>(bytes[h][el & 1]), s2, zero2));
             if constexpr (h == 0) o01 = r;
             else *reinterpret_cast<uint2_t*>(sB + (8 * wr + e) * LDS_STRIDE + 4 * n4) = uint2_t{o01, r};
         }

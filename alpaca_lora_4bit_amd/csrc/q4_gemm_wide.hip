@@ -19,19 +19,18 @@
 // that the 128-bit fragment reads meet no bank twice.  Per 256 x 256 x 64 step 32 KB are written and 128 KB read, where staging
 // both operands (8 wavefronts of 128 x 64) writes 64 KB and reads 192.
 //
-// Operand build.  13 (forward) or 11 vector operations per word: masks, permutes, one conversion per pair (codes_of_bytes) and one
-// fused multiply-add, weight = rn16(scale * code - rn16(scale * (zero + 1))) -- one rounding less than the dense kernel, and
-// less energy than the magic-number form (16: and 1.5 % of the time).  The pieces sit one by one behind the MFMAs.
+// Operand build.  17 (forward) or 15 vector operations per word: masks, permutes, one conversion per pair (codes_of_bytes), product
+// and difference rounded apart: the weights are the dense kernel's, bit for bit.  With the codes as (1024 + q, 64 + q) and the
+// offset taken off by the product's fused multiply-add (16 operations) most launches take 1 to 3 % longer.
 //
-// us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 115 -> 108.5,
-// 4096 x (5120 -> 13824) 489 -> 468, 4096 x (13824 -> 5120) 480 -> 457; grad-input 115 -> 110, 488 -> 473, 490 -> 476; cycles per
-// step (2048 of them MFMAs) forward 2500, grad-input 2770, at 1.55 and 1.67 GHz.
+// us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 120.3 -> 112.2,
+// 4096 x (5120 -> 13824) 509 -> 480, 4096 x (13824 -> 5120) 503 -> 471; grad-input 120.0 -> 114.2, 507 -> 492, 511 -> 490.
 //
 // TM = 4, forward: tiles of 128 x 256 for outputs with too few of the large ones (one unsplit round of 256 x 128 tiles of
 // q4_gemm.hip before: the same area, half the activations per weight decoded, but 64 KB of fragment reads per round of 1024 MFMA
-// cycles instead of 128).  us, 256 x 128 with both operands in LDS -> 128 x 256: 2048 x (4096 -> 4096) 66.5 -> 60.4, 512 x (5120 -> 13824)
-// 72.4 -> 65.9, 1536 x (4096 -> 4096) 54.3 -> 49.6, 300 x (4096 -> 11008) 45.7 -> 41.7, the last 88 tiles of 2048 x (4096 -> 11008) 57 -> 51.
-// Grad-input it is level to 2 % slower (2048 x (4096 -> 4096) 66.9 against 66.0): the words turned around serve half the rows.
+// cycles instead of 128).  us, 256 x 128 with both operands in LDS -> 128 x 256: 2048 x (4096 -> 4096) 68.7 -> 64.7, 512 x (5120 -> 13824)
+// 74.3 -> 73.2, 600 x (5120 -> 5120) 49.1 -> 43.1, 1024 x (11008 -> 4096) 99.3 -> 93.2, 2048 x (4096 -> 11008) 176.6 -> 169.5 (its last
+// 88 tiles).  Grad-input the form is level to 2 % slower: the words turned around serve half the rows.
 #include "q4_gemm_args.hpp"
 
 namespace q4 {
@@ -322,7 +321,7 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                 constexpr int j = u / 6, p = u % 6 - 2;
                 const half2_t q = codes_of_bytes<p & 1>(bt[j][p >> 1]);
                 const half2_t sc = FWD ? s2[j] : as_half2(so[ks & 1][p]), zt = FWD ? z2[j] : as_half2(zo[ks & 1][p]);
-                bo[ks & 1][j][p] = as_u32(__builtin_elementwise_fma(q, sc, -zt));
+                bo[ks & 1][j][p] = as_u32(dequant_pair(q, sc, zt));
             }
         };
         auto build_all = [&](auto st, auto kt) {

@@ -482,12 +482,9 @@ void skinny_seq_kernel(SkinnyArgs a) {
 // for the WHOLE reduction: wavefront w walks the chunks w, w + 8, ... of 128 reduction rows with its accumulators
 // in registers, the next chunk's words, scales and activations in flight while it multiplies the current one, and
 // the eight wavefronts are summed through LDS once, at the end, into fp16 outputs: one launch, no workspace.
-// The B operand holds the weights rn16(s*q - rn16(s*(z+1))) (one rounding less than the dense kernel,
-// quant_cuda_kernel.cu:1148-1152) in the order of the rows: codes to bytes, one conversion and one fused multiply-add per
-// pair (codes_of_bytes), so the activations go to the MFMA as they lie.  With the codes as (1024 + q, 64 + q) in the order of
-// the nibbles the activations had to be permuted and a chunk took 256 instead of 208 of the vector operations that bound it: us,
-// before -> now, 4096 -> 11008 at 17 / 32 / 48 / 64 rows 12.2 / 12.2 / 13.3 / 15.2 -> 11.0 / 11.5 / 12.5 / 15.2, 5120 -> 13824 at 48 rows
-// 16.4 -> 15.7, 4096 -> 4096 at 256 rows 16.4 -> 15.9, 11008 -> 4096 at 150 rows 28.3 -> 27.0.
+// The B operand holds the dequantized weights rn16(rn16(s*q) - rn16(s*(z+1))) (the values of the dense kernel,
+// quant_cuda_kernel.cu:1148-1152): with one scale per column of a chunk the product of code and scale is one
+// packed fused multiply-add on (1024 + q) or (64 + q) (1024*s and 64*s are exact), the zero term one subtraction.
 template <int RB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 void stream_fwd_kernel(SkinnyArgs a) {
@@ -540,6 +537,12 @@ void stream_fwd_kernel(SkinnyArgs a) {
         for (int t = 0; t < NSTEP; ++t) w1[t] = buf_load128_stream(rw, vw, off + (ch << 4) * a.N * 4 + t * wstep);
     };
     fetch(wave);
+    // mask (scalar register) and magic number (vector register) as opaque values: with two literals the compiler
+    // emits an AND and an OR, with register operands the single three-operand and-or instruction
+    uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, g_lo = 0x64006400u, g_hi = 0x54005400u;
+    asm volatile("" : "+s"(m_lo), "+s"(m_hi));
+    asm volatile("" : "+v"(g_lo), "+v"(g_hi));
+
     float4_t acc[RB][4];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
@@ -550,20 +553,28 @@ void stream_fwd_kernel(SkinnyArgs a) {
         // the loads of this chunk have landed (vmcnt 0): the tile in LDS, words, scales and zeros in registers
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // A operands in the order the nibble split below produces: (e0,e4)(e1,e5)(e2,e6)(e3,e7)
         half8_t av[RB][NSTEP];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            const half8_t* stage = reinterpret_cast<const half8_t*>(&red[rb][wave][0]);
+            const uint4_t* stage = reinterpret_cast<const uint4_t*>(&red[rb][wave][0]);
 #pragma unroll
-            for (int t = 0; t < NSTEP; ++t) av[rb][t] = stage[c * 16 + ((4 * t + kk) ^ c)];
+            for (int t = 0; t < NSTEP; ++t) {
+                const uint4_t u = stage[c * 16 + ((4 * t + kk) ^ c)];
+                av[rb][t] = make_half8(__builtin_amdgcn_perm(u.z, u.x, 0x05040100u), __builtin_amdgcn_perm(u.z, u.x, 0x07060302u),
+                                       __builtin_amdgcn_perm(u.w, u.y, 0x05040100u), __builtin_amdgcn_perm(u.w, u.y, 0x07060302u));
+            }
         }
         // scale and zero term of the four columns of this lane (one group per chunk)
         const uint32_t zw = zv >> ((c & 1) * 16);
         const uint32_t sraw[4] = {sv.x & 0xFFFFu, sv.x >> 16, sv.y & 0xFFFFu, sv.y >> 16};
-        half2_t s2[4], zero2[4];
+        half2_t s2[4], s1024[4], s64[4], zero2[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            const half2_t k1024 = {(half_t)1024.0f, (half_t)1024.0f}, k64 = {(half_t)64.0f, (half_t)64.0f};
             s2[j] = as_half2(sraw[j] | (sraw[j] << 16));
+            s1024[j] = s2[j] * k1024;
+            s64[j] = s2[j] * k64;
             const uint32_t z = (zw >> (4 * j)) & 0xFu;
             zero2[j] = zero_term(s2[j], z, z);
         }
@@ -580,12 +591,12 @@ void stream_fwd_kernel(SkinnyArgs a) {
             const uint32_t w[4] = {w0[t].x, w0[t].y, w0[t].z, w0[t].w};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const uint32_t lo = w[j] & 0x0F0F0F0Fu, hi = (w[j] >> 4) & 0x0F0F0F0Fu;
-                const uint32_t c03 = __builtin_amdgcn_perm(hi, lo, 0x05010400u), c47 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-                const half2_t b0 = __builtin_elementwise_fma(codes_of_bytes<0>(c03), s2[j], -zero2[j]);
-                const half2_t b1 = __builtin_elementwise_fma(codes_of_bytes<1>(c03), s2[j], -zero2[j]);
-                const half2_t b2 = __builtin_elementwise_fma(codes_of_bytes<0>(c47), s2[j], -zero2[j]);
-                const half2_t b3 = __builtin_elementwise_fma(codes_of_bytes<1>(c47), s2[j], -zero2[j]);
+                // a code in mantissa bits 0..3 of fp16 1024.0 reads 1024 + q, in bits 4..7 of fp16 64.0 it reads 64 + q
+                const uint32_t hi = w[j] >> 8;
+                const half2_t b0 = __builtin_elementwise_fma(as_half2((w[j] & m_lo) | g_lo), s2[j], -s1024[j]) - zero2[j];
+                const half2_t b1 = __builtin_elementwise_fma(as_half2((w[j] & m_hi) | g_hi), s2[j], -s64[j]) - zero2[j];
+                const half2_t b2 = __builtin_elementwise_fma(as_half2((hi & m_lo) | g_lo), s2[j], -s1024[j]) - zero2[j];
+                const half2_t b3 = __builtin_elementwise_fma(as_half2((hi & m_hi) | g_hi), s2[j], -s64[j]) - zero2[j];
                 const half8_t bv = make_half8(as_u32(b0), as_u32(b1), as_u32(b2), as_u32(b3));
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
