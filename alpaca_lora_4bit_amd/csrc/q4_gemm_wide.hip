@@ -20,16 +20,20 @@
 // both operands (8 wavefronts of 128 x 64) writes 64 KB and reads 192.
 //
 // Operand build.  17 (forward) or 15 vector operations per word: masks, permutes, one conversion per pair (codes_of_bytes), product
-// and difference rounded apart: the weights are the dense kernel's, bit for bit.  With the codes as (1024 + q, 64 + q) and the
-// offset taken off by the product's fused multiply-add (16 operations) most launches take 1 to 3 % longer.
+// and difference rounded apart: the weights are the dense kernel's, bit for bit.  A pair's difference comes with the next pair's
+// product: directly behind its own it waits for an issue slot (512 x (5120 -> 13824) 73 us instead of 67).  With the codes as
+// (1024 + q, 64 + q) and the offset taken off by the product (16 operations) 70.
 //
-// us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 120.3 -> 112.2,
-// 4096 x (5120 -> 13824) 509 -> 480, 4096 x (13824 -> 5120) 503 -> 471; grad-input 120.0 -> 114.2, 507 -> 492, 511 -> 490.
+// Order of the sums.  That of q4_gemm.hip: the reduction rotated per 256 rows, adapter terms behind a layer's loop, masked ones in
+// front of it, so that a product has the same bits on either file's tiles.
+//
+// us, 8 wavefronts of 128 x 64 with both operands in LDS -> now, one lease: forward 4096 x (4096 -> 4096) 113.5 -> 105.9,
+// 4096 x (5120 -> 13824) 482 -> 454, 4096 x (13824 -> 5120) 482 -> 446; grad-input 113.7 -> 109.3, 487 -> 472, 485 -> 470.
 //
 // TM = 4, forward: tiles of 128 x 256 for outputs with too few of the large ones (one unsplit round of 256 x 128 tiles of
 // q4_gemm.hip before: the same area, half the activations per weight decoded, but 64 KB of fragment reads per round of 1024 MFMA
-// cycles instead of 128).  us, 256 x 128 with both operands in LDS -> 128 x 256: 2048 x (4096 -> 4096) 68.7 -> 64.7, 512 x (5120 -> 13824)
-// 74.3 -> 73.2, 600 x (5120 -> 5120) 49.1 -> 43.1, 1024 x (11008 -> 4096) 99.3 -> 93.2, 2048 x (4096 -> 11008) 176.6 -> 169.5 (its last
+// cycles instead of 128).  us, 256 x 128 with both operands in LDS -> 128 x 256: 2048 x (4096 -> 4096) 65.2 -> 61.0, 512 x (5120 -> 13824)
+// 72.2 -> 67.4, 600 x (5120 -> 5120) 47.4 -> 41.7, 1024 x (11008 -> 4096) 95.0 -> 88.6, 2048 x (4096 -> 11008) 166.5 -> 158.6 (its last
 // 88 tiles).  Grad-input the form is level to 2 % slower: the words turned around serve half the rows.
 #include "q4_gemm_args.hpp"
 
@@ -80,8 +84,8 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
     __shared__ __attribute__((aligned(16))) uint32_t sT1[FWD ? 4 : 8 * kTw];
     __shared__ __attribute__((aligned(16))) half_t sZ[FWD ? 1 : 4][2][2][FWD ? 4 : BK];
 
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lc = lane & 31, lg = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int lane = threadIdx.x & 63, lc = lane & 31, lg = lane >> 5;
     const GemmArgs& a0 = layers[0];
     const int NOUT = FWD ? a0.N : a0.K;
     const int m0 = tm.tile_r * BM, c0 = tm.tile_c * kWideCols, cw = c0 + 64 * wave;
@@ -107,124 +111,140 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
     };
     if constexpr (TM == 8) keep_all();
 
-    // Adapter terms, before the main loop fills the accumulators: operands straight from memory.  Dropout on the adapter input: its
-    // share of out[m, c] exists only where the mask keeps (m, c); the kept values carry 1 / (1 - p) through lb_scale.  The masked
-    // terms of all layers are summed block by block and only written to the accumulators: adding to 256 of them behind the loop
-    // pulled them through the vector registers and spilled (13 us a round instead of 4).
-    auto adapter_here = [&](int li) {                             // the share that holds a layer's first step carries its term
-        if constexpr (!MULTI) return a0.R > 0 && zsplit == 0;
-        int base = 0;
-        for (int l = 0; l < li; ++l) base += layers[l].N / BK;
-        return layers[li].R > 0 && share.begin <= base && base < share.begin + share.cnt;
-    };
+    // Adapter terms: operands straight from memory, added where q4_gemm.hip adds them.
     auto adapter_row = [&](const GemmArgs& a, int i, int ks) {    // columns past R and rows past M read as zero
         const rsrc_t rl = make_rsrc(a.la + (size_t)m0 * a.R, (unsigned)rows_valid * (unsigned)a.R * 2u);
         return __builtin_bit_cast(half8_t, buf_load128(rl, 16 * ks + 8 * lg < a.R ? ((32 * i + lc) * a.R + 16 * ks + 8 * lg) * 2 : kFar, 0));
     };
-    // operand of columns cw + 2 lc, + 1, rows 16 ks + 8 lg .. + 7 of the adapter matrix (zero past R)
-    auto adapter_cols = [&](const GemmArgs& a, int ks, half8_t (&b)[2]) {
-        const bool in = 16 * ks + 8 * lg < a.R;
-        const int r0 = in ? 16 * ks + 8 * lg : 0;
+    // columns cw + 2 lc, + 1, rows 16 ks + 8 lg .. + 7 of the adapter matrix (rows past R: of row 0), as they lie in memory
+    auto adapter_load = [&](const GemmArgs& a, int ks, uint32_t (&raw)[2][8]) {
+        const int r0 = 16 * ks + 8 * lg < a.R ? 16 * ks + 8 * lg : 0;
         auto load = [&](auto tag) {
             using T = decltype(tag);
-            T raw[2][8];
+            constexpr int per = 16 / sizeof(T);
+            if (FWD && a.lb_sr == 1 && a.lb_sc % per == 0 && reinterpret_cast<uintptr_t>(a.lb) % 16 == 0) {
+                // lora_B as it is kept, [N, R]: a lane's rows of a column lie together (one by one its loads touch 64 lines each,
+                // 1024 x (4096 -> 4096) at rank 64 takes 51.9 us instead of 47.3)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int h = 0; h < 8 / per; ++h) {
+                        const uint4_t u = *reinterpret_cast<const uint4_t*>(reinterpret_cast<const T*>(a.lb) + r0 + per * h + (size_t)(cw + 2 * lc + j) * a.lb_sc);
+                        const uint32_t d[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                        for (int e = 0; e < per; ++e) raw[j][per * h + e] = sizeof(T) == 4 ? d[e & 3] : d[(e / 2) & 3] >> (16 * (e & 1));
+                    }
+                return;
+            }
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) raw[j][e] = reinterpret_cast<const T*>(a.lb)[(size_t)(r0 + e) * a.lb_sr + (size_t)(cw + 2 * lc + j) * a.lb_sc];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) b[j][e] = in ? (half_t)(a.lb_scale * (float)raw[j][e]) : (half_t)0.f;
         };
-        if (a.lb_is_f32) load(float{});
-        else load(half_t{});
+        if (a.lb_is_f32) load(uint32_t{});
+        else load((unsigned short)0);
     };
-    auto add_adapters = [&] {
-        bool masked = false;
-        for (int li = 0; li < nlay; ++li) masked = masked || (adapter_here(li) && layers[li].drop.thr15 != 0);
-        if (FWD || !masked) {
-#pragma unroll 1
-            for (int li = 0; li < nlay; ++li) {
-                if (!adapter_here(li)) continue;
-                const GemmArgs& a = layers[li];
-#pragma unroll 1
-                for (int ks = 0; 16 * ks < a.R; ++ks) {
-                    half8_t v[TM], b[2];
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) v[i] = adapter_row(a, i, ks);
-                    adapter_cols(a, ks, b);
-#pragma unroll
-                    for (int i = 0; i < TM; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[i], b[j], acc[i][j], 0, 0, 0);
-                }
+    // the operand they make (zero past R)
+    auto adapter_cols = [&](const GemmArgs& a, int ks, const uint32_t (&raw)[2][8], half8_t (&b)[2]) {
+        uint32_t in = 16 * ks + 8 * lg < a.R ? 0xFFFFFFFFu : 0u;
+        asm volatile("" : "+v"(in));                              // opaque: one mask instead of a branch around every value
+        // fp32 values scaled and rounded to fp16 at once, as q4_gemm.hip's staging of the matrix compiles (left to itself the
+        // compiler makes a product and a conversion of pairs: a rounding more)
+        auto pair = [&](uint32_t u0, uint32_t u1) -> uint32_t {
+            if (a.lb_is_f32) {                                    // uniform
+                uint32_t h = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+                asm("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0" : "=&v"(h) : "v"(u0), "v"(u1), "s"(a.lb_scale));
+#endif
+                return h;
             }
-            return;
+            return as_u32(half2_t{(half_t)(a.lb_scale * (float)__builtin_bit_cast(half_t, (unsigned short)u0)),
+                                  (half_t)(a.lb_scale * (float)__builtin_bit_cast(half_t, (unsigned short)u1))});
+        };
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t o[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) o[p] = pair(raw[j][2 * p], raw[j][2 * p + 1]) & in;
+            b[j] = __builtin_bit_cast(half8_t, uint4_t{o[0], o[1], o[2], o[3]});
         }
+    };
+    // behind the layer's loop; the next sub-step of the rank is on its way while one is multiplied
+    auto add_adapter = [&](const GemmArgs& a) {
+        uint32_t raw[2][8];
+        half8_t v[TM], b[2];
+        auto request = [&](int ks) {
+            adapter_load(a, ks, raw);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) v[i] = adapter_row(a, i, ks);
+        };
+        request(0);
+#pragma unroll 1
+        for (int ks = 0; 16 * ks < a.R; ++ks) {
+            half8_t row[TM];
+            adapter_cols(a, ks, raw, b);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) row[i] = v[i];
+            if (16 * (ks + 1) < a.R) request(ks + 1);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(row[i], b[j], acc[i][j], 0, 0, 0);
+            if constexpr (TM == 8) keep_all();
+        }
+    };
+    // Dropout on the adapter input: its share of out[m, c] exists only where the mask keeps (m, c); the kept values carry
+    // 1 / (1 - p) through lb_scale.  Summed by itself and added block by block, in front of the layer's loop, before anything
+    // of it is live.
+    auto add_masked_adapter = [&](const GemmArgs& a) {
         if constexpr (!FWD && TM == 8) {
-            static_assert(kGemmGroup <= 4 && kTile >= 4 * 2 * 256 * 8, "a layer's operands fill one tile");
-            auto operand = [&](int li, int ks, int j) {           // the lane's own
-                half_t* const t = li == 0 ? sA0 : li == 1 ? sA1 : li == 2 ? sA2 : sA3;
-                return reinterpret_cast<half8_t*>(t + ((2 * ks + j) * 256 + threadIdx.x) * 8);
+            static_assert(kTile >= 4 * 2 * 256 * 8, "a layer's operands fill one tile");
+            auto operand = [&](int ks, int j) {                   // the lane's own
+                return reinterpret_cast<half8_t*>(sA0 + ((2 * ks + j) * 256 + threadIdx.x) * 8);
             };
-            uint32_t here = 0;
-            for (int li = 0; li < nlay; ++li) here |= adapter_here(li) ? 1u << li : 0u;
-            for (int li = 0; li < nlay; ++li)
-                if (here >> li & 1)
-                    for (int ks = 0; 16 * ks < layers[li].R; ++ks) {
-                        half8_t b[2];
-                        adapter_cols(layers[li], ks, b);
-                        *operand(li, ks, 0) = b[0];
-                        *operand(li, ks, 1) = b[1];
-                    }
+            for (int ks = 0; 16 * ks < a.R; ++ks) {
+                uint32_t raw[2][8];
+                half8_t b[2];
+                adapter_load(a, ks, raw);
+                adapter_cols(a, ks, raw, b);
+                *operand(ks, 0) = b[0];
+                *operand(ks, 1) = b[1];
+            }
             half8_t v[4], next[4];                                // a block's rows, and the following block's on their way
-            auto request = [&](int li, int i) {
+            auto request = [&](int i) {
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks)
-                    if (ks == 0 || 16 * ks < layers[li].R) next[ks] = adapter_row(layers[li], i, ks);
+                    if (ks == 0 || 16 * ks < a.R) next[ks] = adapter_row(a, i, ks);
             };
-            const int li0 = __builtin_ctz(here);
-            request(li0, 0);
+            request(0);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                float16_t sum[2];
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) v[ks] = next[ks];
+                if (i + 1 < TM) request(i + 1);
+                float16_t term[2];
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) sum[j][r] = 0.f;
-#pragma unroll 1
-                for (uint32_t todo = here; todo; todo &= todo - 1) {
-                    const int li = __builtin_ctz(todo);
-                    const GemmArgs& a = layers[li];
+                    for (int r = 0; r < 16; ++r) term[j][r] = 0.f;
 #pragma unroll
-                    for (int ks = 0; ks < 4; ++ks) v[ks] = next[ks];
-                    if (todo & (todo - 1)) request(__builtin_ctz(todo & (todo - 1)), i);
-                    else if (i + 1 < TM) request(li0, i + 1);
-                    float16_t term[2];
+                for (int ks = 0; ks < 4; ++ks)
+                    if (ks == 0 || 16 * ks < a.R) {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                        for (int j = 0; j < 2; ++j) term[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[ks], *operand(ks, j), term[j], 0, 0, 0);
+                    }
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) term[j][r] = 0.f;
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
+                    const uint32_t dw = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)(cw + 2 * lc) >> 1);
 #pragma unroll
-                    for (int ks = 0; ks < 4; ++ks)
-                        if (ks == 0 || 16 * ks < a.R) {
-#pragma unroll
-                            for (int j = 0; j < 2; ++j) term[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[ks], *operand(li, ks, j), term[j], 0, 0, 0);
-                        }
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
-                        const uint32_t dw = drop_word(a.drop, drop_row_key(a.drop, (uint32_t)m), (uint32_t)(cw + 2 * lc) >> 1);
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) sum[j][r] += ((dw >> (16 * j)) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[j][r];
+                    for (int j = 0; j < 2; ++j) {
+                        const float kept = ((dw >> (16 * j)) & 0x7FFFu) < a.drop.thr15 ? 0.f : term[j][r];
+                        acc[i][j][r] = MULTI ? acc[i][j][r] + kept : 0.f + kept;
                     }
                 }
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    acc[i][j] = sum[j];
-                    keep_acc(acc[i][j]);
-                }
+                for (int j = 0; j < 2; ++j) keep_acc(acc[i][j]);
                 __builtin_amdgcn_sched_barrier(0);
             }
             __syncthreads();                                      // before the loads write over the operands
@@ -233,7 +253,7 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
 
     auto run_layer = [&](const GemmArgs& a, const StepRange sr) {
         const int RED = FWD ? a.K : a.N;
-        const int phase = (tm.tile_r * (a.phase_step & 0xff)) % sr.cnt;
+        const int phase = (tm.tile_r * TM / 8 * (a.phase_step & 0xff)) % sr.cnt;     // of the 256 rows that the tile belongs to
         const rsrc_t ra = make_rsrc(a.a + (size_t)m0 * RED, (unsigned)rows_valid * (unsigned)RED * 2u);
         const rsrc_t rw = make_rsrc(a.qweight, (unsigned)(a.K >> 3) * (unsigned)a.N * 4u);
         const rsrc_t rs = make_rsrc(a.scales, (unsigned)a.G * (unsigned)a.N * 2u);
@@ -305,6 +325,7 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         // The operands of sub-step ks of a stage in 12 pieces for as many MFMAs' shadows: the codes of column j as bytes
         // (pieces 0..3: the two halves of j = 0, of j = 1), then one pair of weights each.
         uint32_t bt[2][2];
+        half2_t bp[2];
         auto build = [&](auto st, auto kt, auto ut) {
             constexpr int ks = decltype(kt)::value, u = decltype(ut)::value, S = decltype(st)::value & (FWD ? 3 : 1);
             if constexpr (u % 6 < 2) {
@@ -318,10 +339,15 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
                     bt[j][1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
                 }
             } else {
+                // the zero term comes off with the next pair: right behind its product the difference waits for a slot
                 constexpr int j = u / 6, p = u % 6 - 2;
-                const half2_t q = codes_of_bytes<p & 1>(bt[j][p >> 1]);
-                const half2_t sc = FWD ? s2[j] : as_half2(so[ks & 1][p]), zt = FWD ? z2[j] : as_half2(zo[ks & 1][p]);
-                bo[ks & 1][j][p] = as_u32(dequant_pair(q, sc, zt));
+                bp[p & 1] = codes_of_bytes<p & 1>(bt[j][p >> 1]) * (FWD ? s2[j] : as_half2(so[ks & 1][p]));
+                auto less_zero = [&](auto pt) {
+                    constexpr int P = decltype(pt)::value;
+                    bo[ks & 1][j][P] = as_u32(bp[P & 1] - (FWD ? z2[j] : as_half2(zo[ks & 1][P])));
+                };
+                if constexpr (p > 0) less_zero(std::integral_constant<int, p - 1>{});
+                if constexpr (p == 3) less_zero(std::integral_constant<int, p>{});
             }
         };
         auto build_all = [&](auto st, auto kt) {
@@ -479,8 +505,18 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
         __syncthreads();
     };
 
+    auto layer = [&](const GemmArgs& a, const StepRange sr, const bool with_adapter) {
+        if constexpr (MULTI) {                // opaque per layer, or everything derived from it is kept in registers over the layers (and spills)
+            asm volatile("" : "+v"(lane));
+            lc = lane & 31;
+            lg = lane >> 5;
+        }
+        const bool adapter = with_adapter && a.R > 0, masked = adapter && !FWD && a.drop.thr15 != 0;     // uniform
+        if (masked) add_masked_adapter(a);
+        run_layer(a, sr);
+        if (adapter && !masked) add_adapter(a);
+    };
     if constexpr (MULTI) {
-        add_adapters();
         int base = 0;
 #pragma unroll 1
         for (int li = 0; li < nlay; ++li) {
@@ -488,11 +524,10 @@ __device__ __forceinline__ void wide_body(const GemmArgs* layers, const int nlay
             const int lo = max(share.begin, base) - base, hi = min(share.begin + share.cnt, base + steps) - base;
             base += steps;
             if (lo >= hi) continue;                               // uniform
-            run_layer(layers[li], StepRange{lo, hi - lo});
+            layer(layers[li], StepRange{lo, hi - lo}, lo == 0);   // the share that holds a layer's first step carries its adapter term
         }
     } else {
-        add_adapters();
-        run_layer(a0, share);
+        layer(a0, share, zsplit == 0);
     }
 
     // acc[i][j][r]: row 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, column cw + 2 (lane % 32) + j

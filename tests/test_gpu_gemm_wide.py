@@ -151,3 +151,107 @@ def test_weights_at_their_zero_point_are_zero(route):
         y = quant_hip.gemm_bwd_dx(x, qweight, qzeros, scales, None, gs)
         assert not y[:, none].any()
     assert float(y.double().abs().mean()) > 0.1
+
+
+def _indexed(fwd, x, layer, gs, out_cols, bias=None, la=None, lb=None, drop=None):
+    """The same product by the kernels that look every row's group up (csrc/q4_gemm.hip)."""
+    import ctypes
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    L = _lib.lib()
+    qweight, qzeros, scales = layer
+    K, N, M = 8 * qweight.shape[0], qweight.shape[1], x.shape[0]
+    g_idx = (torch.arange(K, device="cuda") // gs).to(torch.int32)
+    out = torch.empty(M, out_cols, dtype=torch.float16, device="cuda")
+    need = L.q4_gemm_workspace_bytes(int(fwd), M, K, N)
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device="cuda")
+    lora = (None, None, 0, 0, 0, 0.0, 0) if la is None else (la.data_ptr(), lb.data_ptr(), lb.stride(0), lb.stride(1),
+                                                             int(lb.dtype == torch.float32), 2.0, la.shape[1])
+    common = (x.data_ptr(), qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), g_idx.data_ptr(), gs)
+    tail = (out.data_ptr(), M, K, N, K // gs)
+    stream = torch.cuda.current_stream().cuda_stream
+    if fwd:
+        rc = L.q4_gemm_fwd_f16(*common, None if bias is None else bias.data_ptr(), *lora, *tail, ws.data_ptr(), ws.numel(), stream)
+    else:
+        d = quant_hip._drop_arg(drop)
+        rc = L.q4_gemm_bwd_dx_f16(*common, *lora, *tail, quant_hip._drop_ref(d), ws.data_ptr(), ws.numel(), stream)
+    torch.cuda.synchronize()
+    assert rc == 0
+    return out
+
+
+def _random_layer(K, N, gs, gen):
+    import torch
+    qweight = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), device="cuda", dtype=torch.int32, generator=gen)
+    qzeros = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // gs, N // 8), device="cuda", dtype=torch.int32, generator=gen)
+    return qweight, qzeros, (0.001 + 0.01 * torch.rand(K // gs, N, device="cuda", generator=gen)).half()
+
+
+# rows, reduction, outputs; which grid; reduction steps of its shares
+GRIDS = [(600, 1024, 18432, "256 x 256", {16}), (600, 1024, 10240, "128 x 256", {16}), (600, 4096, 2048, "128 x 256 in shares", {12, 13}),
+         (600, 4736, 2048, "128 x 256 in shares", {14, 15}), (1000, 4096, 8448, "128 x 256, remainder in shares", {64, 8}),
+         (300, 1152, 18432, "256 x 256", {18}), (1024, 11008, 4096, "128 x 256 in shares", {86})]
+
+
+@pytest.mark.parametrize("rank,f32", [(0, False), (8, True), (24, False), (64, True)])
+@pytest.mark.parametrize("M,red,out,what,steps", GRIDS)
+def test_bits_are_those_of_the_indexed_kernels(M, red, out, what, steps, rank, f32):
+    """Weights, the order of the reduction (rotated per 256 rows), its shares and the place of the adapter term are the same in both
+    files, so an explicit index of the same groups gives the same bits; every length of a share modulo the four steps of the loop."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    gen = torch.Generator("cuda").manual_seed(M + out + rank)
+    x = torch.randn(M, red, device="cuda", generator=gen).half()
+    for fwd, drop in ((True, None), (False, None), (False, (4321, 0.25))):
+        if drop and not rank:
+            continue
+        K, N = (red, out) if fwd else (out, red)
+        layer = _random_layer(K, N, 64, gen)
+        la = lb = None
+        if rank:
+            la = torch.randn(M, rank, device="cuda", generator=gen).half()
+            lb = (torch.randn(out, rank, device="cuda", generator=gen).t() if fwd else torch.randn(rank, out, device="cuda", generator=gen))
+            lb = lb if f32 else lb.half()
+        bias = torch.randn(out, device="cuda", generator=gen).half() if fwd else None
+        if fwd:
+            got = quant_hip.gemm_fwd(x, *layer, None, 64, bias=bias, xa=la, lora_bt=lb, lora_scale=2.0)
+            if rank:                                                  # the matrix as [N, R] rows, as [R, N] rows and off the 16-byte grid
+                other = torch.empty(rank * out + 1, dtype=lb.dtype, device="cuda")[1:].view(rank, out).copy_(lb)
+                assert torch.equal(got, quant_hip.gemm_fwd(x, *layer, None, 64, bias=bias, xa=la, lora_bt=other, lora_scale=2.0))
+                odd = torch.empty(rank * out + 1, dtype=lb.dtype, device="cuda")[1:].view(out, rank).copy_(lb.t()).t()
+                assert torch.equal(got, quant_hip.gemm_fwd(x, *layer, None, 64, bias=bias, xa=la, lora_bt=odd, lora_scale=2.0))
+        else:
+            got = quant_hip.gemm_bwd_dx(x, *layer, None, 64, dyb=la, lora_a=lb, lora_scale=2.0, dropout=drop)
+        assert torch.equal(got, _indexed(fwd, x, layer, 64, out, bias, la, lb, drop))
+
+
+@pytest.mark.parametrize("ranks", [(0, 0), (8, 64), (0, 24)])
+def test_grouped_bits(ranks):
+    """Forward: the bits of the layers one by one, whose tiles are unsplit too, in wide tiles and their remainder of 128 x 256.  Grad-input:
+    128 more outputs keep the group on the tiles of csrc/q4_gemm.hip; the outputs that both have are the same."""
+    import torch
+    from alpaca_lora_4bit_amd import _lib, quant_hip
+    gen = torch.Generator("cuda").manual_seed(sum(ranks))
+    M, K, N, gs = 300, 640, 18432, 128
+    x = torch.randn(M, K, device="cuda", generator=gen).half()
+    layers = [_random_layer(K, N, gs, gen) for _ in ranks]
+    xas = [torch.randn(M, r, device="cuda", generator=gen).half() if r else None for r in ranks]
+    Bs = [torch.randn(N, r, device="cuda", generator=gen).t() if r else None for r in ranks]
+    assert _lib.lib().q4_gemm_workspace_bytes(1, M, K, N) == 0
+    ys = quant_hip.gemm_grouped_fwd(x, [(*l, None, xa, B, 2.0) for l, xa, B in zip(layers, xas, Bs)], gs)
+    for y, l, xa, B in zip(ys, layers, xas, Bs):
+        assert torch.equal(y, _indexed(True, x, l, gs, N, None, xa, B))
+
+    Ns, K = (384, 256), 18432
+    dys = [torch.randn(M, n, device="cuda", generator=gen).half() for n in Ns]
+    more = [_random_layer(K + 128, n, gs, gen) for n in Ns]
+    less = [(q[:K // 8].contiguous(), z[:K // gs].contiguous(), s[:K // gs].contiguous()) for q, z, s in more]
+    dybs = [torch.randn(M, r, device="cuda", generator=gen).half() if r else None for r in ranks]
+    As = [torch.randn(r, K + 128, device="cuda", generator=gen) if r else None for r in ranks]
+    for drops in ((None, None), ((11, 0.1), (12, 0.5)), (None, (13, 0.25))):
+        def dx(ls, k):
+            arr = (__import__("ctypes").c_int * 2)(*Ns)
+            assert _lib.lib().q4_gemm_grouped_workspace_bytes(0, 2, M, k, arr) == 0
+            return quant_hip.gemm_grouped_bwd_dx(dys, [(*l, b, None if A is None else A[:, :k].contiguous(), 2.0, d if b is not None else None)
+                                                       for l, b, A, d in zip(ls, dybs, As, drops)], gs)
+        assert torch.equal(dx(less, K), dx(more, K + 128)[:, :K])
