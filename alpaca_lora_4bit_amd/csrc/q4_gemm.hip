@@ -738,11 +738,6 @@ static hipError_t launch_gemm_wide(GemmArgs a, int nout, int tail_cols, int tail
 template <int BM, int WGM, bool FWD, bool GIDX>
 static hipError_t launch_gemm(GemmArgs a, int nout, int splits, int tail_cols, int tail_splits, hipStream_t stream) {
     const int nc = nout / BN, nr = (a.M + BM - 1) / BM;
-    // whole tiles of 256 columns on both sides (launch_low_tiles), in as many shares as the plan's scratch holds of them
-    if (FWD && !GIDX && BM == 256 && nc % 2 == 0 && tail_cols % 2 == 1) {
-        tail_splits = tail_splits * tail_cols / (tail_cols + 1) > 1 ? tail_splits * tail_cols / (tail_cols + 1) : 1;
-        ++tail_cols;
-    }
     a.col_tile0 = 0;
     a.part_cols = nout;
     const bool low = BM == 256 && launch_low_tiles<FWD, GIDX>(a, 0, nc - tail_cols, splits, stream);
@@ -830,7 +825,7 @@ extern "C" int q4_launch_gemm(int fwd, const void* act, const int32_t* qweight, 
         workspace_bytes >= q4_skinny_dx_workspace(M, K, N))
         return q4_launch_skinny_dx(act, qweight, qzeros, scales, groupsize, out, M, K, N, G, workspace, stream);
     // tile configuration: 256-row tiles once they still give every CU a workgroup; split-K for few tiles
-    const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, workspace ? workspace_bytes : 0, gidx);
+    const GemmPlan p = plan_gemm(M, fwd ? K : N, nout, workspace ? workspace_bytes : 0, gidx, fwd && !gidx);
     a.part = reinterpret_cast<float*>(workspace);
     hipError_t e;
     if (fwd) e = gidx ? launch_gemm_cfg<true, true>(p, a, nout, stream) : launch_gemm_cfg<true, false>(p, a, nout, stream);
@@ -952,7 +947,7 @@ extern "C" size_t q4_gemm_plan_workspace(int fwd, int M, int K, int N) {
     const int nout = fwd ? N : K;
     size_t need = 0;                              // the query does not know the group order: room for either
     for (const bool indexed : {false, true}) {
-        const size_t part = plan_workspace(plan_gemm(M, fwd ? K : N, nout, ~(size_t)0, indexed), M, nout);
+        const size_t part = plan_workspace(plan_gemm(M, fwd ? K : N, nout, ~(size_t)0, indexed, fwd && !indexed), M, nout);
         need = part > need ? part : need;
     }
     if (fwd && M > 16 && M <= 64) {               // the skinny kernel's partial rows (it may or may not apply)

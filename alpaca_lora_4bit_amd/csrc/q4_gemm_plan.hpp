@@ -46,7 +46,8 @@ inline WideTail wide_tail(int M, int nsteps, int nout, bool may_split, size_t wo
 // remainder launch are slower than the narrow tiles on every shape measured (30 shapes of groups of 32): forward by 37..53 %
 // (1969 x (4352 -> 9472): 420 against 290 us), grad-input by 11..16 % (2605 x (8704 -> 4352): 318 against 279 us, where the
 // wide kernel also spills 80 bytes a lane).
-inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes, bool indexed) {
+// `paired`: the launches of 256 x 128 tiles run as 128 x 256 ones where their columns come in whole pairs (forward, sequential groups).
+inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes, bool indexed, bool paired = false) {
     GemmPlan p;
     p.tail_cols = 0; p.tail_splits = 1;
     const int nsteps = red / BK;
@@ -89,6 +90,15 @@ inline GemmPlan plan_gemm(int M, int red, int nout, size_t workspace_bytes, bool
             if (ts > 1 && (size_t)ts * (size_t)M * (size_t)tcols * BN * sizeof(float) <= workspace_bytes) {
                 p.tail_cols = tcols;
                 p.tail_splits = ts;
+                // An odd remainder of an even width takes one more column, in as many shares as the same scratch holds, so that
+                // both launches are whole pairs; not where only one share would be left.  us, odd / even: 640 x (4096 -> 11008)
+                // 76.4 / 71.9, 1536 rows 141.7 / 136.6, 3072 rows 270 / 258, 3328 x (13824 -> 5120) 460 / 434, 768 x (4096 -> 11008)
+                // 79.0 / 79.1; one share: 520 x (1024 -> 11008) 31.1 / 32.1.
+                const int fewer = ts * tcols / (tcols + 1);
+                if (paired && (nout / BN) % 2 == 0 && tcols % 2 == 1 && fewer > 1) {
+                    p.tail_cols = tcols + 1;
+                    p.tail_splits = fewer;
+                }
             }
         }
     } else if (t256 <= 128 && M > 128 && nsteps >= 8 * (int)(256 / t256) &&

@@ -10,7 +10,7 @@ from conftest import ROOT
 WRAPPER = r"""
 #include "q4_gemm_plan.hpp"
 extern "C" void plan(int M, int red, int nout, size_t workspace, int indexed, int* out) {
-    const q4::GemmPlan p = q4::plan_gemm(M, red, nout, workspace, indexed != 0);
+    const q4::GemmPlan p = q4::plan_gemm(M, red, nout, workspace, indexed == 1, indexed == 2);       // 2: forward, sequential groups
     out[0] = p.cfg; out[1] = p.splits; out[2] = p.tail_cols; out[3] = p.tail_splits;
 }
 extern "C" void group_plan(int fwd, int n, int M, int K, const int* N, int* out) {
@@ -78,8 +78,10 @@ def test_a_plan_stays_inside_its_output_and_its_workspace(plans):
     for _ in range(4000):
         M = int(2 ** rng.uniform(0, 14))
         red, nout = 128 * int(2 ** rng.uniform(0, 7.5)), 128 * int(2 ** rng.uniform(0, 10))
-        for indexed in (False, True):
+        for indexed in (False, True, 2):
             whole = _plan(plans, M, red, nout, indexed=indexed)
+            if indexed == 2 and nout % 256 == 0 and whole[0] == NARROW and whole[2] % 2:
+                assert whole[3] * whole[2] // (whole[2] + 1) < 2
             assert _partials(whole, M, nout) <= L.q4_gemm_workspace_bytes(1, M, red, nout)
             scratch = rng.choice([0, 1 << 20, _partials(whole, M, nout), max(_partials(whole, M, nout) - 1, 0)])
             for p, room in ((whole, ANY), (_plan(plans, M, red, nout, scratch, indexed), scratch)):
@@ -89,6 +91,14 @@ def test_a_plan_stays_inside_its_output_and_its_workspace(plans):
                 assert 1 <= splits <= max(red // 64, 1) and 1 <= tail_splits <= red // 64
                 assert splits == 1 or tail_cols == 0
                 assert _partials(p, M, nout) <= room
+
+
+@pytest.mark.parametrize("M,red,nout,odd,even", [(1536, 4096, 11008, (1, 8), (2, 4)), (3328, 13824, 5120, (1, 8), (2, 4)),
+                                                 (520, 1024, 11008, (1, 2), (1, 2)), (1024, 1024, 11136, (23, 2), (23, 2))])
+def test_forward_remainders_are_planned_as_they_are_launched(plans, M, red, nout, odd, even):
+    """Whole pairs of column tiles where the output has them and two shares are left; an odd width and one share keep the odd remainder."""
+    assert _plan(plans, M, red, nout) == (NARROW, 1, *odd) == _plan(plans, M, red, nout, indexed=True)
+    assert _plan(plans, M, red, nout, indexed=2) == (NARROW, 1, *even)
 
 
 @pytest.mark.parametrize("M,K,Ns,was", [

@@ -364,7 +364,10 @@ def test_gemm_remainder_tiles_run_as_a_split_second_launch(oracle, M, red, nout,
             out = out.cpu().numpy()
             assert rel_err(out, want) <= TOL
             edge = (nout // 128 - tail_cols) * 128                  # first column of the second launch
-            assert rel_err(out[:, edge - 128:edge + 128], want[:, edge - 128:edge + 128]) <= TOL
+            if fwd and not act and (nout // 128, tail_cols, tail_splits) == (86, 1, 8):
+                edge -= 128                                         # as a pair of column tiles, in four shares
+            assert rel_err(out[:, edge - 128:edge], want[:, edge - 128:edge]) <= TOL
+            assert rel_err(out[:, edge:edge + 128], want[:, edge:edge + 128]) <= TOL
             assert rel_err(out[:, -128:], want[:, -128:]) <= TOL
 
 

@@ -190,7 +190,7 @@ def _random_layer(K, N, gs, gen):
 # rows, reduction, outputs; which grid; reduction steps of its shares
 GRIDS = [(600, 1024, 18432, "256 x 256", {16}), (600, 1024, 10240, "128 x 256", {16}), (600, 4096, 2048, "128 x 256 in shares", {12, 13}),
          (600, 4736, 2048, "128 x 256 in shares", {14, 15}), (1000, 4096, 8448, "128 x 256, remainder in shares", {64, 8}),
-         (300, 1152, 18432, "256 x 256", {18}), (1024, 11008, 4096, "128 x 256 in shares", {86})]
+         (520, 1024, 11008, "256 x 128, one column left in shares", {16, 8}), (300, 1152, 18432, "256 x 256", {18}), (1024, 11008, 4096, "128 x 256 in shares", {86})]
 
 
 @pytest.mark.parametrize("rank,f32", [(0, False), (8, True), (24, False), (64, True)])
