@@ -611,19 +611,19 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_kernel(GemmArgs a) {
     gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(&a, 1, map_tile(a.phase_step, a.col_tile0), sr, blockIdx.z, gridDim.z);
 }
 
-template <int BM, int WGM, bool FWD, bool GIDX, int SZ = 0, int WGN = 2>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_group_kernel(GemmGroupArgs g) {
+template <int BM, int WGM, bool FWD, bool GIDX, int SZ = 0>
+__global__ __launch_bounds__(64 * WGM * 2) void gemm_group_kernel(GemmGroupArgs g) {
     TileMap tm = map_tile(g.layer[0].phase_step, g.layer[0].col_tile0);
     if constexpr (FWD) {
         const int li = (tm.tile_c >= g.tile_end[0]) + (tm.tile_c >= g.tile_end[1]) + (tm.tile_c >= g.tile_end[2]);   // uniform
         tm.tile_c -= li == 0 ? 0 : g.tile_end[li - 1];
         const GemmArgs a = g.layer[li];
-        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN>(&a, 1, tm, split_steps(a.K / BK, 0, 1), 0, 1);
+        gemm_body<BM, WGM, FWD, GIDX, SZ, 2>(&a, 1, tm, split_steps(a.K / BK, 0, 1), 0, 1);
     } else {
         int nsteps = 0;
         for (int i = 0; i < g.n; ++i) nsteps += g.layer[i].N / BK;
-        gemm_body<BM, WGM, FWD, GIDX, SZ, WGN, true>(g.layer, g.n, tm, split_steps(nsteps, blockIdx.z, gridDim.z),
-                                                     blockIdx.z, gridDim.z);
+        gemm_body<BM, WGM, FWD, GIDX, SZ, 2, true>(g.layer, g.n, tm, split_steps(nsteps, blockIdx.z, gridDim.z),
+                                                   blockIdx.z, gridDim.z);
     }
 }
 
@@ -755,9 +755,8 @@ template <bool FWD, bool GIDX>
 static hipError_t launch_gemm_cfg(const GemmPlan& p, const GemmArgs& a, int nout, hipStream_t stream) {
     switch (p.cfg) {
         case 0: return launch_gemm<128, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 128 x 128, 4 wavefronts of 64 x 64
-        case 1: return launch_gemm<256, 2, FWD, GIDX>(a, nout, p.splits, 0, 1, stream);    // 256 x 128, 4 wavefronts of 128 x 64
-        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, p.tail_cols, p.tail_splits, stream);   // 256 x 256, 8 wavefronts of 128 x 64
-        default: return launch_gemm<256, 4, FWD, GIDX>(a, nout, p.splits, p.tail_cols, p.tail_splits, stream);   // 256 x 128, 8 wavefronts of 64 x 64
+        case 3: return launch_gemm_wide<FWD, GIDX>(a, nout, p.tail_cols, p.tail_splits, stream);   // 256 x 256: 4 wavefronts of 256 x 64, GIDX 8 of 128 x 64
+        default: return launch_gemm<256, 4, FWD, GIDX>(a, nout, p.splits, p.tail_cols, p.tail_splits, stream);   // 256 x 128: 8 wavefronts of 64 x 64, or launch_low_tiles
     }
 }
 
