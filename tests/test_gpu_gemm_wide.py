@@ -1,12 +1,13 @@
-"""The tiles of the GEMMs whose operands are built in registers (csrc/q4_gemm_wide.hip) at the edges of their pipeline: reductions
-shorter than, equal to and just past the ring of activation tiles, ragged last row tiles of 256 and of 128 rows, groups of 64, 128 and 256 rows, adapters
-of every number of 16-deep sub-steps in both types, with and without a dropout mask.
+"""The tiles of the GEMMs whose operands are built in registers (csrc/q4_gemm_wide.hip) at the edges of their pipeline: shares of the
+reduction shorter than the ring of activation tiles and of every length modulo its four steps, ragged last row tiles of 256 and of 128 rows,
+groups of 64, 128 and 256 rows, adapters of every number of 16-deep sub-steps in both types, with and without a dropout mask.
 Tolerance: outputs are rounded to fp16 (2^-11 of a value), adapter matrices and their scaling too; sums of a few hundred such terms
 average out to below 2e-3 of the largest output.  Weights are the dense kernel's, bit for bit."""
 import numpy as np
 import pytest
 
 from conftest import rel_err, to_cuda_layer
+from test_gemm_plan import _group_plan, _plan, plans  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
@@ -187,6 +188,10 @@ def _random_layer(K, N, gs, gen):
     return qweight, qzeros, (0.001 + 0.01 * torch.rand(K // gs, N, device="cuda", generator=gen)).half()
 
 
+def _lengths(steps, shares):
+    return {steps // shares, -(-steps // shares)}
+
+
 # rows, reduction, outputs; which grid; reduction steps of its shares
 GRIDS = [(600, 1024, 18432, "256 x 256", {16}), (600, 1024, 10240, "128 x 256", {16}), (600, 4096, 2048, "128 x 256 in shares", {12, 13}),
          (600, 4736, 2048, "128 x 256 in shares", {14, 15}), (1000, 4096, 8448, "128 x 256, remainder in shares", {64, 8}),
@@ -195,11 +200,14 @@ GRIDS = [(600, 1024, 18432, "256 x 256", {16}), (600, 1024, 10240, "128 x 256", 
 
 @pytest.mark.parametrize("rank,f32", [(0, False), (8, True), (24, False), (64, True)])
 @pytest.mark.parametrize("M,red,out,what,steps", GRIDS)
-def test_bits_are_those_of_the_indexed_kernels(M, red, out, what, steps, rank, f32):
+def test_bits_are_those_of_the_indexed_kernels(plans, M, red, out, what, steps, rank, f32):
     """Weights, the order of the reduction (rotated per 256 rows), its shares and the place of the adapter term are the same in both
     files, so an explicit index of the same groups gives the same bits; every length of a share modulo the four steps of the loop."""
     import torch
     from alpaca_lora_4bit_amd import quant_hip
+    cfg, splits, tail, tail_splits = _plan(plans, M, red, out, indexed=2)
+    assert (cfg == 3) == (what == "256 x 256") and (splits > 1) == ("in shares" in what and tail == 0) and (tail > 0) == ("in shares" in what and splits == 1)
+    assert _lengths(red // 64, splits) | (_lengths(red // 64, tail_splits) if tail else set()) == steps
     gen = torch.Generator("cuda").manual_seed(M + out + rank)
     x = torch.randn(M, red, device="cuda", generator=gen).half()
     for fwd, drop in ((True, None), (False, None), (False, (4321, 0.25))):
@@ -223,6 +231,47 @@ def test_bits_are_those_of_the_indexed_kernels(M, red, out, what, steps, rank, f
         else:
             got = quant_hip.gemm_bwd_dx(x, *layer, None, 64, dyb=la, lora_a=lb, lora_scale=2.0, dropout=drop)
         assert torch.equal(got, _indexed(fwd, x, layer, 64, out, bias, la, lb, drop))
+        W = quant_hip.dequant(*layer, None, 64).double()
+        full = x.double() @ (W if fwd else W.t()) + (bias.double() if fwd else 0.0)
+        if rank:
+            term = 2.0 * la.double() @ lb.double()
+            full += term if drop is None else term * quant_hip.dropout_keep_mask(M, K, *drop, x.device).double() * quant_hip.dropout_scale(drop[1])
+        assert float((got.double() - full).abs().max() / full.abs().max()) <= TOL
+
+
+# rows, outputs, columns of the layers; steps of the shares' parts of the layers
+SHARED = [(300, 5120, (1280, 3712, 640, 2304), [20, 1, 21, 21, 15, 6, 4, 16, 20]), (300, 5120, (3200, 2048, 2688), [21, 21, 8, 13, 19, 2, 20, 20]),
+          (300, 5120, (3840, 4096), [21, 21, 18, 3, 21, 20, 20])]
+
+
+@pytest.mark.parametrize("M,K,Ns,parts", SHARED)
+@pytest.mark.parametrize("rank,p", [(0, 0.0), (16, 0.0), (40, 0.1)])
+def test_grouped_grad_input_in_shares(plans, M, K, Ns, parts, rank, p):
+    """Shares of 256 x 256 tiles that end in the middle of a layer, down to one, two and three steps of it, against float64 over all rows."""
+    import torch
+    from alpaca_lora_4bit_amd import quant_hip
+    cfg, splits, tail, _ = _group_plan(plans, 0, M, K, Ns)
+    assert cfg == 3 and splits > 1 and tail == 0
+    ends, total, begin, seen = np.cumsum([n // 64 for n in Ns]), sum(Ns) // 64, 0, []
+    for z in range(splits):
+        end = begin + total // splits + (z < total % splits)
+        seen += [int(min(end, e) - max(begin, e - n // 64)) for e, n in zip(ends, Ns) if min(end, e) > max(begin, e - n // 64)]
+        begin = end
+    assert seen == parts
+    gen = torch.Generator("cuda").manual_seed(rank + len(Ns))
+    layers = [_random_layer(K, n, 128, gen) for n in Ns]
+    dys = [torch.randn(M, n, device="cuda", generator=gen).half() for n in Ns]
+    dybs = [torch.randn(M, rank, device="cuda", generator=gen).half() if rank else None for _ in Ns]
+    As = [torch.randn(rank, K, device="cuda", generator=gen) if rank else None for _ in Ns]
+    drops = [(100 + i, p) if p and i != 1 else None for i in range(len(Ns))]
+    dx = quant_hip.gemm_grouped_bwd_dx(dys, [(*l, b, A, 2.0, d) for l, b, A, d in zip(layers, dybs, As, drops)], 128)
+    full = torch.zeros(M, K, dtype=torch.float64, device="cuda")
+    for l, dy, b, A, d in zip(layers, dys, dybs, As, drops):
+        full += dy.double() @ quant_hip.dequant(*l, None, 128).double().t()
+        if rank:
+            term = 2.0 * b.double() @ A.double()
+            full += term if d is None else term * quant_hip.dropout_keep_mask(M, K, *d, dy.device).double() * quant_hip.dropout_scale(p)
+    assert float((dx.double() - full).abs().max() / full.abs().max()) <= TOL
 
 
 @pytest.mark.parametrize("ranks", [(0, 0), (8, 64), (0, 24)])
