@@ -5,7 +5,7 @@
 // current step needs straight into LDS, so the product is torch.matmul(x, recons(W)) of
 // matmul_utils_4bit.py:122-126.  The weights have the reference's three fp16 roundings
 // (src/alpaca_lora_4bit/quant_cuda/quant_cuda_kernel.cu:1146-1151), here and in q4_gemm_wide.hip, both directions: what a
-// product multiplies does not depend on the kernel that its sizes lead to.  Forward ORs the codes into 1024.0 and takes the
+// tiled product multiplies does not depend on the tiles that its sizes lead to.  Forward ORs the codes into 1024.0 and takes the
 // offset off in the product; grad-input turns them into bytes and converts (codes_of_bytes), us: 2048 x (4096 -> 4096)
 // 69.5 -> 69.1, 512 x (5120 -> 13824) 83.0 -> 82.5, 100 x (11008 -> 4096) 31.1 -> 30.8.
 //

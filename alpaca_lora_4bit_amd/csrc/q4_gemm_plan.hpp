@@ -1,5 +1,10 @@
 // Launch plans of the tiled GEMMs: which tiles, how many shares of the reduction, which columns go to a second launch.
 // Host arithmetic on the sizes alone, without HIP, so that it also compiles by itself for the CPU tests.
+//
+// The thresholds and the estimate below were fitted to kernels with both operands in LDS, which the tiles of
+// q4_gemm_wide.hip have replaced since on sequential groups (all launches of 256 x 256, forward ones of 256 x 128 as 128 x 256); their
+// figures are of that time where they do not say otherwise.  Since then forward takes 5 to 10 % less from 250 rows on, grad-input 1 to
+// 5 %, no shape measured more; 256-row tiles are still counted where forward launches run ceil(M / 128) rows of 128 x 256 ones.
 #pragma once
 #include <stddef.h>
 
@@ -15,7 +20,8 @@ struct GemmPlan {
 
 // More 256 x 256 tiles than whole rounds of the CUs: the wide tiles of the whole rounds run as they are, and the columns
 // left over go to a second launch of 256 x 128 tiles that is one round at most, its reduction split when even that
-// leaves CUs idle.  A full round of wide tiles takes 1.75-1.85 us per reduction step, one of narrow tiles 0.9-1.05, so the
+// leaves CUs idle.  A full round of wide tiles takes 1.75-1.85 us per reduction step (1.65-1.7 in q4_gemm_wide.hip), one of
+// narrow tiles 0.9-1.05 (0.95 forward, 1.03 grad-input now), so the
 // remainder costs at most 0.6 of the round of wide tiles, or half of the two narrow ones, that it would cost otherwise:
 // 2048 x (4096 -> 11008), 344 tiles: three rounds of narrow tiles 186 us, 118 + 57 us; grad-input of 4096 x
 // (5120 -> 13824), 864 tiles: four rounds of wide tiles 561 us, 447 + 79 us.

@@ -31,7 +31,8 @@ inline bool plan_stream_takes(int M, int blocks, int strips, int groupsize) {
 // 192 strips, K = 4096 (75 %) 9.0 / 9.0 at 8 rows, 10.1 / 10.4 at 11, 10.3 / 10.4 at 12, 10.9 / 10.5 at 16.  Where several share it:
 // 64 strips, K = 11008 8.5 / 8.6 at 8 rows, 9.4 / 9.2 at 10, 9.6 / 9.2 at 11, 10.5 / 9.7 at 16; 80 strips, K = 13824 11.7 / 12.0 at 8, 12.5 / 12.7
 // at 10, 12.7 / 12.6 at 11, 14.3 / 12.8 at 16; 128 strips, K = 8192 10.6 / 10.5 at 8, 11.7 / 11.3 at 11, 12.7 / 11.8 at 16.  Shares of two blocks and
-// groups of 64 or 32 rows do not gain.
+// groups of 64 or 32 rows do not gain.  (The longer share's figures are of one team of wavefronts; with two, plan_stream_teams, it is
+// 0.2 to 0.5 us shorter.)
 inline int plan_stream_blocks(int M, int blocks, int strips, int groupsize) {
     const int least = blocks > 255 ? (blocks + 254) / 255 : 1;    // the 8-bit arrival counter
     if (strips > 256 || groupsize % 128 != 0 || M < 7) return least;

@@ -225,7 +225,7 @@ Q4_API int q4_dropout_keep_u8(uint8_t *keep, int M, int C, const q4_dropout_t *d
 
 /* Forward GEMM, any M >= 1:
  *   y fp16 [M, N] = x fp16 [M, K] @ W  (+ bias fp16 [N])  (+ lora_scale * xa fp16 [M, R] @ Bm [R, N])
- * with fp32 accumulation on MFMA; W tiles are dequantized in LDS and never written to HBM.
+ * with fp32 accumulation on MFMA; W is dequantized tile by tile, in registers or LDS, and never written to HBM.
  * Replaces vecquant4recons_v2 + torch.matmul(x, buffer) (matmul_utils_4bit.py:114-124),
  * the bias add (autograd_4bit.py:206-207) and, when xa/lora_b are given, the adapter term
  * result += lora_B(lora_A(x)) * scaling (models.py:58-66) where xa = x @ A^T.
@@ -233,7 +233,7 @@ Q4_API int q4_dropout_keep_u8(uint8_t *keep, int M, int C, const q4_dropout_t *d
  * fp32, so lora_B.weight [N, R] (ldb_r = 1, ldb_n = R) is passed in place: no cast, no transpose.
  * bias, xa, lora_b may be NULL; R is 0 or a multiple of 8, at most 64.
  * Both GEMM entry points need K % 128 == 0, N % 128 == 0, K*N < 2^33, and with g_idx == NULL also
- * groupsize % 64 == 0 and every |scale| < 64 (the sequential-group dequant forms s*q with a fused
+ * groupsize % 64 == 0 and every |scale| < 64 (some of the sequential-group kernels form s*q with a fused
  * multiply-add on 1024+q; pass g_idx to lift the restriction on the scales).
  * `workspace` (optional, may be NULL; 256-byte aligned, contents irrelevant): with few output tiles (small M),
  * and for the tiles of a last round that would fill at most half of the CUs, the reduction is split over
@@ -246,7 +246,7 @@ Q4_API int q4_dropout_keep_u8(uint8_t *keep, int M, int C, const q4_dropout_t *d
 Q4_API size_t q4_gemm_workspace_bytes(int fwd, int M, int K, int N);
 
 /* Which kernel family the two GEMM entry points run for a product WITHOUT adapter term, given a workspace of
- * q4_gemm_workspace_bytes(): Q4_ROUTE_TILED (dequantize-into-LDS MFMA tiles), Q4_ROUTE_SKINNY (17..64 rows, partial rows
+ * q4_gemm_workspace_bytes(): Q4_ROUTE_TILED (MFMA tiles), Q4_ROUTE_SKINNY (17..64 rows, partial rows
  * in the workspace), Q4_ROUTE_STREAM (some hundred rows, one launch without workspace), or a negative Q4_ERR_* code for
  * a shape neither entry point takes.  A planning query for callers and tests; it launches nothing.  No counterpart in
  * the reference, whose only route is recons + torch.matmul (matmul_utils_4bit.py:114-127). */
