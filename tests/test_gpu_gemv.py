@@ -367,7 +367,8 @@ def test_long_reductions_of_odd_chunks(oracle, route, K, gs, M):
     assert quant_hip.workspaces_are_zero()
 
 
-@pytest.mark.parametrize("K", [3072, 5120, 7168])      # shares of 3 and 5 blocks in two teams, of 7 (their sums beyond the LDS) in one
+# shares of 3, 5 and 6 blocks in two teams, of 7 and 8 (their sums beyond the LDS beside two teams' tiles) in one; 6 and 8 fill all 160 KB
+@pytest.mark.parametrize("K", [3072, 5120, 6144, 7168, 8192])
 @pytest.mark.parametrize("M", [7, 8, 9, 16])
 def test_longer_shares_in_two_teams_have_the_bits_of_single_blocks(oracle, K, M):
     """216 strips at 7 rows and more: one workgroup takes the whole reduction, its blocks in turn to two teams of wavefronts.  Up to
